@@ -482,6 +482,9 @@ int pggc_ctx_create(pggc_ctx** out, void* stream) {
         std::unique_ptr<pggc_ctx> x(new pggc_ctx());
         x->c.stream = (hipStream_t)stream;
         PGGC_HIP(hipGetDevice(&x->c.device));
+        size_t mem_free = 0, mem_total = 0;
+        PGGC_HIP(hipMemGetInfo(&mem_free, &mem_total));
+        x->c.cache_keep = mem_total / 32;
         // coherent (fine-grained) host memory: the readback kernel's stores
         // reach the host without a cache writeback the host would have to wait for
         PGGC_HIP(hipHostMalloc((void**)&x->c.pinned, 64 * sizeof(i64), hipHostMallocCoherent));

@@ -6,8 +6,9 @@
 //
 // Build: every undirected pair becomes the key (lo << B) | hi with B =
 // ceil(log2 n); a radix sort of the keys groups duplicates and orders the
-// pairs by (lo, hi), and a second sort of the transposed keys (hi << B) | lo
-// orders them by (hi, lo).  With firstF[u] / firstT[u] the positions of the
+// pairs by (lo, hi), and a stable sort of the transposed keys (hi << B) | lo by
+// their hi bits alone orders them by (hi, lo), as they come in lo order (half
+// the digit passes of a sort by all 2B bits).  With firstF[u] / firstT[u] the positions of the
 // first pair with lo >= u / hi >= u, row u of the CSR is the transposed run
 // of u (columns < u, ascending) followed by the forward run of u (columns > u,
 // ascending), so rp[u] = firstF[u] + firstT[u], and pair k lands at
@@ -113,26 +114,41 @@ __global__ void __launch_bounds__(UT) k_uniq_sums(const u64* __restrict__ keys, 
     if (threadIdx.x == 0) bsum[block_id()] = s;
 }
 
+// Bound by HBM traffic.  Consecutive lanes take consecutive keys, and a key's
+// place is the count of the (step, wave) runs before its own plus its rank in
+// the ballot of its wave, so reads and writes move whole cache lines (with 8
+// consecutive keys per thread instead, 16.3M weighted keys took 543 us).
 __global__ void __launch_bounds__(UT) k_uniq_write(const u64* __restrict__ keys, const i32* __restrict__ wk, i64 m,
                                                    u64 invalid, const i64* __restrict__ boff,
                                                    u64* __restrict__ okeys, i32* __restrict__ ow) {
-    const i64 base = block_id() * UTILE + (i64)threadIdx.x * UI;
-    int f[UI];
-    i64 s = 0;
+    constexpr int NW = UT / 64;
+    __shared__ int cnt[UI * NW];
+    const i64 base = block_id() * UTILE;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    u64 bal[UI];
 #pragma unroll
     for (int k = 0; k < UI; k++) {
-        const i64 x = base + k;
-        f[k] = (x < m && uniq_flag(keys, x, invalid)) ? 1 : 0;
-        s += f[k];
+        const i64 x = base + (i64)k * UT + threadIdx.x;
+        bal[k] = __ballot(x < m && uniq_flag(keys, x, invalid));
+        if (lane == 0) cnt[k * NW + wv] = __popcll(bal[k]);
     }
-    i64 tot;
-    i64 pre = block_excl_scan_i64(s, &tot) + boff[block_id()];
+    __syncthreads();
+    const i64 b0 = boff[block_id()];
+    int run = 0;  // kept keys of the runs before (k, wv)
 #pragma unroll
     for (int k = 0; k < UI; k++) {
-        if (f[k]) {
-            okeys[pre] = keys[base + k];
-            if (ow) ow[pre] = wk[base + k];
-            pre++;
+        int before = run;
+#pragma unroll
+        for (int w = 0; w < NW; w++) {
+            const int c = cnt[k * NW + w];
+            before += w < wv ? c : 0;
+            run += c;
+        }
+        if ((bal[k] >> lane) & 1) {
+            const i64 x = base + (i64)k * UT + threadIdx.x;
+            const i64 pos = b0 + before + __popcll(bal[k] & (((u64)1 << lane) - 1));
+            okeys[pos] = keys[x];
+            if (ow) ow[pos] = wk[x];
         }
     }
 }
@@ -214,9 +230,9 @@ static void pairs_to_csr(Ctx& c, i64 n, u64* fkeys, i32* fw, i64 M, int B, int w
     if (wmode == 1) {
         tw = Buf<i32>(c, std::max<i64>(M, 1));
         copy_dev(c, tw.p, fw, (size_t)M * sizeof(i32));
-        radix_sort_pairs(c, tkeys, tw, M, 2 * B);
+        radix_sort_pairs(c, tkeys, tw, M, 2 * B, B);
     } else {
-        radix_sort_keys(c, tkeys, M, 2 * B);
+        radix_sort_keys(c, tkeys, M, 2 * B, B);
     }
     k_first<<<grid_items(n + 1, 256), 256, 0, c.stream>>>(n, fkeys, M, B, fF);
     k_first<<<grid_items(n + 1, 256), 256, 0, c.stream>>>(n, tkeys, M, B, fT);
@@ -273,7 +289,7 @@ void rmat_csr(Ctx& c, int scale, int edge_factor, double a, double b, double cc,
     }
     pairs_to_csr(c, n, ukeys, nullptr, M, B, wmax > 0 ? 2 : 0, seed, wmin, wmax, out);
     ukeys.reset();
-    c.trim();
+    c.trim_large();
 }
 
 void edges_csr(Ctx& c, i64 n, i64 m, const i32* src, const i32* dst, const i32* w, DevCSR& out) {
@@ -304,7 +320,7 @@ void edges_csr(Ctx& c, i64 n, i64 m, const i32* src, const i32* dst, const i32* 
     pairs_to_csr(c, n, ukeys, uw.p, M, B, w ? 1 : 0, 0, 0, 0, out);
     ukeys.reset();
     uw.reset();
-    c.trim();
+    c.trim_large();
 }
 
 // ------------------------------------------------------------------ LFR
@@ -558,7 +574,7 @@ void lfr_csr(Ctx& c, const LfrParams& p, DevCSR& out, i32* gt) {
     ek.reset();
     pairs_to_csr(c, n, uk, nullptr, U, B, p.wmax > 0 ? 2 : 0, p.seed, p.wmin, p.wmax, out);
     uk.reset();
-    c.trim();
+    c.trim_large();
 }
 
 void random_labels(Ctx& c, i64 n, i64 L, u64 seed, i32* out) {

@@ -72,6 +72,10 @@ void Ctx::trim() {
     bytes_cached = 0;
 }
 
+void Ctx::trim_large() {
+    if (bytes_cached > cache_keep) trim();
+}
+
 hipEvent_t Ctx::kt_event() {
     if (!kt.pool.empty()) {
         hipEvent_t e = kt.pool.back();
@@ -350,36 +354,38 @@ i64 compact_flags(Ctx& c, const i32* flag, const i32* src, i64 n, i32* out, i64*
 }
 
 // ---------------------------------------------------------------- radix sort
-// Stable LSD sort of (key, value) pairs on the low `bits` key bits: rocPRIM's
+// Stable LSD sort of (key, value) pairs on key bits [begin, bits): rocPRIM's
 // onesweep radix sort (a plain library sort, compiled from the ROCm headers),
 // with its temporary storage and the second buffers from the context's pool.
 template <class V>
-void radix_sort_pairs_t(Ctx& c, u64* keys, V* vals, i64 n, int bits) {
-    if (n <= 1 || bits <= 0) return;
+void radix_sort_pairs_t(Ctx& c, u64* keys, V* vals, i64 n, int bits, int begin = 0) {
+    if (n <= 1 || bits <= begin) return;
     Buf<u64> k2(c, n);
     Buf<V> v2(c, n);
     rocprim::double_buffer<u64> kd(keys, k2.p);
     rocprim::double_buffer<V> vd(vals, v2.p);
     const unsigned int end_bit = (unsigned int)std::min(bits, 64);
     size_t tb = 0;
-    PGGC_HIP(rocprim::radix_sort_pairs(nullptr, tb, kd, vd, (size_t)n, 0u, end_bit, c.stream));
+    PGGC_HIP(rocprim::radix_sort_pairs(nullptr, tb, kd, vd, (size_t)n, (unsigned)begin, end_bit, c.stream));
     Buf<u64> tmp(c, std::max<size_t>((tb + 7) / 8, 1));
-    PGGC_HIP(rocprim::radix_sort_pairs((void*)tmp.p, tb, kd, vd, (size_t)n, 0u, end_bit, c.stream));
+    PGGC_HIP(rocprim::radix_sort_pairs((void*)tmp.p, tb, kd, vd, (size_t)n, (unsigned)begin, end_bit, c.stream));
     if (kd.current() != keys) copy_dev(c, keys, kd.current(), n * sizeof(u64));
     if (vd.current() != vals) copy_dev(c, vals, vd.current(), n * sizeof(V));
 }
-void radix_sort_pairs(Ctx& c, u64* keys, i32* vals, i64 n, int bits) { radix_sort_pairs_t(c, keys, vals, n, bits); }
+void radix_sort_pairs(Ctx& c, u64* keys, i32* vals, i64 n, int bits, int begin) {
+    radix_sort_pairs_t(c, keys, vals, n, bits, begin);
+}
 void radix_sort_pairs(Ctx& c, u64* keys, i64* vals, i64 n, int bits) { radix_sort_pairs_t(c, keys, vals, n, bits); }
 
-void radix_sort_keys(Ctx& c, u64* keys, i64 n, int bits) {
-    if (n <= 1 || bits <= 0) return;
+void radix_sort_keys(Ctx& c, u64* keys, i64 n, int bits, int begin) {
+    if (n <= 1 || bits <= begin) return;
     Buf<u64> k2(c, n);
     rocprim::double_buffer<u64> kd(keys, k2.p);
     const unsigned int end_bit = (unsigned int)std::min(bits, 64);
     size_t tb = 0;
-    PGGC_HIP(rocprim::radix_sort_keys(nullptr, tb, kd, (size_t)n, 0u, end_bit, c.stream));
+    PGGC_HIP(rocprim::radix_sort_keys(nullptr, tb, kd, (size_t)n, (unsigned)begin, end_bit, c.stream));
     Buf<u64> tmp(c, std::max<size_t>((tb + 7) / 8, 1));
-    PGGC_HIP(rocprim::radix_sort_keys((void*)tmp.p, tb, kd, (size_t)n, 0u, end_bit, c.stream));
+    PGGC_HIP(rocprim::radix_sort_keys((void*)tmp.p, tb, kd, (size_t)n, (unsigned)begin, end_bit, c.stream));
     if (kd.current() != keys) copy_dev(c, keys, kd.current(), n * sizeof(u64));
 }
 
