@@ -84,6 +84,7 @@ struct LevelPlan {
     // tables; he / hs: edges per build item and slots per scan item
     u64 epoch = ~(u64)0;
     i64 nlds = 0, hub0 = 0, nhub = 0;
+    i64 max_deg = 0;  // of the hub class (0 without hubs)
     i64 he = 1024, hs = 4096;
 };
 
@@ -105,7 +106,8 @@ struct MoveScratch {
     Gnn* gnn = nullptr;  // active-set predictor (null or mode off: plain sweeps)
     Buf<AbInfo> abi;
     Buf<u64> mvp;  // per vertex: cluster | moved << 31, and the cluster after this sweep's moves
-    Buf<i32> part, dest, mflag, cand, moves, flag, tmp, tmp2;
+    Buf<u64> sqpart;  // partial sums of k_finish
+    Buf<i32> part, dest, cand, moves, flag, tmp, tmp2;
     Buf<float> gain;
     Buf<i64> prio, scal;
     void ensure(Ctx& c, i64 n);

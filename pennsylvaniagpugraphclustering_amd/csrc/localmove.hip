@@ -37,12 +37,16 @@ void update_objective(Ctx& c, RefineData& rd) {
 }
 
 // ------------------------------------------------------------- scratch
+// Scalars of a sweep in MoveScratch::scal, zeroed at the start of a call:
+// SC_STALE and the MV_SLOTS words of the uncut change are zero between sweeps,
+// SC_TICKET counts k_finish's blocks (at most FIN_BLOCKS).
+constexpr int SC_STALE = 3, SC_TICKET = 4, SC_SLOTS = 16, MV_SLOTS = 64, SC_COUNT = SC_SLOTS + MV_SLOTS;
+constexpr int FIN_BLOCKS = 256;
 void MoveScratch::ensure(Ctx& c, i64 n) {
     if (cap >= n) return;
     cap = std::max<i64>(n, 1);
     part = Buf<i32>(c, cap);
     dest = Buf<i32>(c, cap);
-    mflag = Buf<i32>(c, cap);
     cand = Buf<i32>(c, cap);
     moves = Buf<i32>(c, cap);
     flag = Buf<i32>(c, cap);
@@ -52,8 +56,8 @@ void MoveScratch::ensure(Ctx& c, i64 n) {
     abi = Buf<AbInfo>(c, cap);
     mvp = Buf<u64>(c, cap);
     prio = Buf<i64>(c, cap + 1);
-    scal = Buf<i64>(c, 16);
-    fill_i32(c, mflag, cap, 0);
+    scal = Buf<i64>(c, SC_COUNT);
+    sqpart = Buf<u64>(c, 2 * FIN_BLOCKS);
 }
 
 // ------------------------------------------------------------- level plan
@@ -124,6 +128,10 @@ __global__ void k_first_above(const i64* rp, const i32* list, i64 m, i64 bound, 
         else lo = mid + 1;
     }
     *out = lo;
+}
+
+__global__ void k_list_degree(const i64* rp, const i32* entry, i64* out) {
+    if (threadIdx.x == 0) *out = rp[*entry + 1] - rp[*entry];
 }
 
 // row weight of each hub (one block per edge item)
@@ -259,6 +267,13 @@ void plan_level(Ctx& c, const DGraph& g, LevelPlan& p) {
     p.nhub = nh - p.nlds;
     const i64 m7 = p.nhub;
     p.gslots = 0;
+    p.max_deg = 0;
+    if (nh > 0) {  // (the hub class is sorted by degree)
+        Buf<i64> f(c, 1);
+        k_list_degree<<<1, 64, 0, c.stream>>>(g.rp, p.sc_list.p + p.sc_start[CL_HUB] + nh - 1, f);
+        PGGC_LAUNCH_CHECK();
+        p.max_deg = c.read1(f);
+    }
     if (m7 > 0) {
         p.goff = Buf<i64>(c, m7 + 1);
         p.items = Buf<i64>(c, m7 + 1);
@@ -927,16 +942,12 @@ __global__ void k_hub_pv(const i32* __restrict__ hubs, i64 m, const i64* __restr
                         : table_get(gkeys + goff[hi], gvals + goff[hi], gmask, hsm[hi], part[i]);
 }
 
-// Movers' edges into hubs: weight w of edge (i, u) leaves key part[i] and
-// joins key dest[i] in hub u's table (run before the moves are applied).
-// Same degree split as the uncut delta.  A failed update sets *stale.
-template <bool PACKED, class WT>
-__device__ __forceinline__ void hub_update_edge(const i32* col, WT W, const i32* hidx, const i64* goff,
-                                                const u32* hsm, i32* gkeys, i64* gvals, u64* gtab, u32* hlist,
-                                                i32* hcnt, i64 j, i32 oi, i32 ni, i64* stale) {
-    const i32 h = hidx[col[j]];
-    if (h < 0) return;
-    const i64 w = W(j);
+// A mover's edge into hub h: weight w leaves key oi and joins key ni in the
+// hub's table (run before the moves are applied).  A failed update sets
+// *stale.
+template <bool PACKED>
+__device__ __forceinline__ void hub_update_edge(i32 h, i64 w, const i64* goff, const u32* hsm, i32* gkeys, i64* gvals,
+                                                u64* gtab, u32* hlist, i32* hcnt, i32 oi, i32 ni, i64* stale) {
     const i64 g = goff[h];
     const u32 gmask = (u32)(goff[h + 1] - g - 1);
     const u32 sm = hsm[h];
@@ -949,62 +960,6 @@ __device__ __forceinline__ void hub_update_edge(const i32* col, WT W, const i32*
         ok = table_update(gkeys + g, gvals + g, gmask, sm, ni, w, hlist + g, hcnt + h) && ok;
     }
     if (!ok) *stale = 1;
-}
-template <bool PACKED, class WT>
-__global__ void __launch_bounds__(256) k_hub_update_thread(const i64* __restrict__ rp, const i32* __restrict__ col,
-                                                           WT W, const i32* __restrict__ moves, i64 k,
-                                                           const i32* __restrict__ part, const i32* __restrict__ dest,
-                                                           const i32* __restrict__ hidx, const i64* __restrict__ goff,
-                                                           const u32* __restrict__ hsm, i32* gkeys, i64* gvals,
-                                                           u64* gtab, u32* hlist, i32* hcnt, i64* stale) {
-    const i64 x = thread_item();
-    if (x >= k) return;
-    const i32 i = moves[x];
-    const i64 s = rp[i], e = rp[i + 1];
-    if (e - s >= LARGE_CUTOFF) return;
-    const i32 oi = part[i], ni = dest[i];
-    if (ni < 0) return;  // not applied (k_apply_moves)
-#pragma unroll 4
-    for (i64 j = s; j < e; j++) hub_update_edge<PACKED>(col, W, hidx, goff, hsm, gkeys, gvals, gtab, hlist, hcnt, j, oi, ni, stale);
-}
-template <bool PACKED, class WT>
-__global__ void __launch_bounds__(256) k_hub_update_wave(const i64* __restrict__ rp, const i32* __restrict__ col,
-                                                         WT W, const i32* __restrict__ moves, i64 k, i64 nw,
-                                                         const i32* __restrict__ part, const i32* __restrict__ dest,
-                                                         const i32* __restrict__ hidx, const i64* __restrict__ goff,
-                                                         const u32* __restrict__ hsm, i32* gkeys, i64* gvals,
-                                                         u64* gtab, u32* hlist, i32* hcnt, i64* stale) {
-    const int lane = threadIdx.x & 63;
-    const i64 w = block_id() * 4 + (threadIdx.x >> 6);
-    if (w >= nw) return;
-    const i32 i = moves[k - 1 - w];
-    const i64 s = rp[i], e = rp[i + 1];
-    if (e - s < LARGE_CUTOFF || e - s >= MASSIVE_CUTOFF) return;
-    const i32 oi = part[i], ni = dest[i];
-    if (ni < 0) return;  // not applied (k_apply_moves)
-    for (i64 base = s; base < e; base += 64) {  // wave-uniform loop control
-        const i64 j = base + lane;
-        if (j < e) hub_update_edge<PACKED>(col, W, hidx, goff, hsm, gkeys, gvals, gtab, hlist, hcnt, j, oi, ni, stale);
-    }
-}
-// movers of degree >= MASSIVE_CUTOFF (the last nb entries of moves at most):
-// a 1024-thread block each, so one huge row is not a single wave's serial tail
-template <bool PACKED, class WT>
-__global__ void __launch_bounds__(1024) k_hub_update_block(const i64* __restrict__ rp, const i32* __restrict__ col,
-                                                           WT W, const i32* __restrict__ moves, i64 k, i64 nb,
-                                                           const i32* __restrict__ part, const i32* __restrict__ dest,
-                                                           const i32* __restrict__ hidx, const i64* __restrict__ goff,
-                                                           const u32* __restrict__ hsm, i32* gkeys, i64* gvals,
-                                                           u64* gtab, u32* hlist, i32* hcnt, i64* stale) {
-    const i64 w = block_id();
-    if (w >= nb) return;
-    const i32 i = moves[k - 1 - w];
-    const i64 s = rp[i], e = rp[i + 1];
-    if (e - s < MASSIVE_CUTOFF) return;
-    const i32 oi = part[i], ni = dest[i];
-    if (ni < 0) return;  // not applied (k_apply_moves)
-    for (i64 j = s + threadIdx.x; j < e; j += 1024)
-        hub_update_edge<PACKED>(col, W, hidx, goff, hsm, gkeys, gvals, gtab, hlist, hcnt, j, oi, ni, stale);
 }
 
 // Scan items cover hs entries of a hub's occupied-slot list (the grid is
@@ -1431,7 +1386,7 @@ __device__ __forceinline__ void ab_term(const i32* col, WT W, const AbInfo* info
 template <class WT, class LT, class PT>
 __global__ void __launch_bounds__(256) k_ab_serial(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
                                                    const AbInfo* __restrict__ info, const i32* __restrict__ cand,
-                                                   i64 k, LT lam, PT prio, i32* keep, i32* mflag) {
+                                                   i64 k, LT lam, PT prio, i32* keep) {
     const i64 x = thread_item();
     if (x >= k) return;
     const i32 i = cand[x];
@@ -1444,15 +1399,13 @@ __global__ void __launch_bounds__(256) k_ab_serial(const i64* __restrict__ rp, c
     const i64 e = rp[i + 1];
 #pragma unroll 4  // independent neighbour gathers in flight; the adds keep their order
     for (i64 j = rp[i]; j < e; j++) ab_term(col, W, info, j, p, best, multi, igain, hi, prio, acc);
-    const int kp = (igain + acc >= 0.0f) ? 1 : 0;
-    keep[x] = kp;
-    mflag[i] = kp;  // candidates start with mflag 0: an unconditional store
+    keep[x] = (igain + acc >= 0.0f) ? 1 : 0;  // an unconditional store
 }
 
 template <class WT, class LT, class PT>
 __global__ void __launch_bounds__(256) k_ab_wave(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
                                                  const AbInfo* __restrict__ info, const i32* __restrict__ cand, i64 k0,
-                                                 i64 k1, LT lam, PT prio, i32* keep, i32* mflag) {
+                                                 i64 k1, LT lam, PT prio, i32* keep) {
     const int lane = threadIdx.x & 63;
     const i64 x = k0 + block_id() * 4 + (threadIdx.x >> 6);
     if (x >= k1) return;
@@ -1473,18 +1426,14 @@ __global__ void __launch_bounds__(256) k_ab_wave(const i64* __restrict__ rp, con
         xlane_fence(acc);
 #pragma unroll
         for (int off = 32; off >= 1; off >>= 1) acc = acc + __shfl_down(acc, off);
-        if (lane == 0) {
-            const int kp = (igain + acc >= 0.0f) ? 1 : 0;
-            keep[x] = kp;
-            if (kp) mflag[i] = 1;
-        }
+        if (lane == 0) keep[x] = (igain + acc >= 0.0f) ? 1 : 0;
     }
 }
 
 template <class WT, class LT, class PT>
 __global__ void __launch_bounds__(1024) k_ab_block(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
                                                    const AbInfo* __restrict__ info, const i32* __restrict__ cand,
-                                                   i64 k0, i64 k1, LT lam, PT prio, i32* keep, i32* mflag) {
+                                                   i64 k0, i64 k1, LT lam, PT prio, i32* keep) {
     __shared__ float sh[1024];
     const int t = threadIdx.x;
     const i64 x = k0 + block_id();
@@ -1513,11 +1462,7 @@ __global__ void __launch_bounds__(1024) k_ab_block(const i64* __restrict__ rp, c
             xlane_fence(acc);
 #pragma unroll
             for (int off = 32; off >= 1; off >>= 1) acc = acc + __shfl_down(acc, off);
-            if (t == 0) {
-                const int kp = (igain + acc >= 0.0f) ? 1 : 0;
-                keep[x] = kp;
-                if (kp) mflag[i] = 1;
-            }
+            if (t == 0) keep[x] = (igain + acc >= 0.0f) ? 1 : 0;
         }
         __syncthreads();
     }
@@ -1545,13 +1490,13 @@ static i64 afterburner(Ctx& c, MoveScratch& s, const DGraph& g, const i32* cand,
     PGGC_WDISPATCH(g, {
         if (b[0] > 0)
             k_ab_serial<<<grid_items(b[0], 256), 256, 0, c.stream>>>(g.rp, g.col, W, s.abi, cand, b[0], lam, prio,
-                                                                     s.flag, s.mflag);
+                                                                     s.flag);
         if (b[1] > b[0])
             k_ab_wave<<<grid_items(b[1] - b[0], 4), 256, 0, c.stream>>>(g.rp, g.col, W, s.abi, cand, b[0], b[1], lam,
-                                                                        prio, s.flag, s.mflag);
+                                                                        prio, s.flag);
         if (k > b[1])
             k_ab_block<<<grid_blocks(k - b[1]), 1024, 0, c.stream>>>(g.rp, g.col, W, s.abi, cand, b[1], k, lam,
-                                                                     prio, s.flag, s.mflag);
+                                                                     prio, s.flag);
     });
     c.kt_end(tk, 0.0);
     PGGC_LAUNCH_CHECK();
@@ -1641,112 +1586,190 @@ static void set_new_cluster_ids(Ctx& c, MoveScratch& s, const DGraph& g, RefineD
 }
 
 // ------------------------------------------------------------- perform moves
-// Exact uncut delta of the moves (src/local_mover.cpp:1274-1277 computes the
-// same quantity from pvals): per mover, the sum over its edges of
-// w * ([new_i == new_v] - [old_i == old_v]), counted once for mover pairs and
-// twice for edges to vertices that stay.  Move lists are in order1 order, so
-// movers of degree >= LARGE_CUTOFF form a suffix: they take one wave each
-// (counted from the end); the others one thread each.  out[x] = delta of mover x.
-// mvp[v]: low word part[v] | mflag[v] << 31 (cluster ids are >= 0), high
-// word the cluster after the moves (dest[v] for a mover, else part[v]), so
-// the delta reads one 8-byte word per edge
-__global__ void k_mv_pack(i64 n, const i32* __restrict__ part, const i32* __restrict__ dest,
-                          const i32* __restrict__ mflag, u64* __restrict__ mvp) {
+// mvp[v]: low word the cluster of v | moved << 31 (cluster ids are >= 0), high
+// word the cluster after this sweep's moves.  Between sweeps both words are
+// v's cluster (k_mvp_init at the start of a call); a sweep marks its movers
+// (k_mvp_moves) and k_apply_moves settles them, so a sweep touches the movers'
+// words only, and an edge's uncut change reads one 8-byte word.
+__global__ void __launch_bounds__(256) k_mvp_init(i64 n, const i32* __restrict__ part, u64* __restrict__ mvp,
+                                                  i64* scal) {
     const i64 i = thread_item();
+    if (i < SC_COUNT) scal[i] = 0;
     if (i >= n) return;
-    const i32 ov = part[i];
-    const u32 mv = mflag[i] ? 1u : 0u;
-    const i32 nv = mv ? dest[i] : ov;
-    mvp[i] = (u64)((u32)ov | (mv << 31)) | ((u64)(u32)nv << 32);
+    const u64 p = (u64)(u32)part[i];
+    mvp[i] = p | (p << 32);
 }
-
-template <class WT>
-__device__ __forceinline__ i64 delta_term(const i32* col, WT W, const u64* mvp, i64 j, i32 oi, i32 ni) {
-    const u64 q = mvp[col[j]];
-    const u32 lo = (u32)q;
-    const i32 ov = (i32)(lo & 0x7fffffffu);
-    const bool mv = (lo >> 31) != 0;
-    const i32 nv = (i32)(u32)(q >> 32);
-    const i64 dd = (i64)(ni == nv) - (i64)(oi == ov);
-    return dd * W(j) * (mv ? 1 : 2);
-}
-template <class WT>
-__global__ void __launch_bounds__(256) k_delta_uncut_thread(const i64* __restrict__ rp, const i32* __restrict__ col,
-                                                            WT W, const i32* __restrict__ moves, i64 k,
-                                                            const i32* __restrict__ part,
-                                                            const i32* __restrict__ dest,
-                                                            const u64* __restrict__ mvp, i64* out) {
+__global__ void __launch_bounds__(256) k_mvp_moves(const i32* __restrict__ moves, i64 k, const i32* __restrict__ part,
+                                                   const i32* __restrict__ dest, u64* __restrict__ mvp) {
     const i64 x = thread_item();
     if (x >= k) return;
     const i32 i = moves[x];
-    const i64 s = rp[i], e = rp[i + 1];
-    if (e - s >= LARGE_CUTOFF) return;
-    const i32 oi = part[i], ni = dest[i];
-    i64 acc = 0;
-#pragma unroll 4
-    for (i64 j = s; j < e; j++) acc += delta_term(col, W, mvp, j, oi, ni);
-    out[x] = acc;
+    mvp[i] = (u64)((u32)part[i] | 0x80000000u) | ((u64)(u32)dest[i] << 32);
 }
-template <class WT>
-__global__ void __launch_bounds__(256) k_delta_uncut_wave(const i64* __restrict__ rp, const i32* __restrict__ col,
-                                                          WT W, const i32* __restrict__ moves, i64 k, i64 nw,
-                                                          const i32* __restrict__ part, const i32* __restrict__ dest,
-                                                          const u64* __restrict__ mvp, i64* out) {
-    const int lane = threadIdx.x & 63;
-    const i64 w = block_id() * 4 + (threadIdx.x >> 6);
-    if (w >= nw) return;
-    const i64 x = k - 1 - w;
-    const i32 i = moves[x];
-    const i64 s = rp[i], e = rp[i + 1];
-    if (e - s < LARGE_CUTOFF || e - s >= MASSIVE_CUTOFF) return;
-    const i32 oi = part[i], ni = dest[i];
-    i64 acc = 0;
-    for (i64 base = s; base < e; base += 64) {  // wave-uniform loop control
-        const i64 j = base + lane;
-        if (j < e) acc += delta_term(col, W, mvp, j, oi, ni);
+
+// Where the uncut changes of the movers are added: AccOne spreads one sum over
+// MV_SLOTS words (summed by k_finish), AccInst adds per instance of a union
+// batch, merged per block in LDS.
+constexpr int IC_SLOTS = 512;  // LDS slots for at most 256 distinct instances per block
+struct AccOne {
+    i64* slots;
+    template <int BS>
+    __device__ __forceinline__ void add(i32, i64 acc) const {
+        acc = block_sum_i64<BS>(acc);
+        if (threadIdx.x == 0 && acc)
+            atomicAdd((unsigned long long*)&slots[block_id() & (MV_SLOTS - 1)], (unsigned long long)acc);
     }
-    acc = wave_sum_i64(acc);
-    if (lane == 0) out[x] = acc;
-}
-template <class WT>
-__global__ void __launch_bounds__(1024) k_delta_uncut_block(const i64* __restrict__ rp, const i32* __restrict__ col,
-                                                            WT W, const i32* __restrict__ moves, i64 k, i64 nb,
-                                                            const i32* __restrict__ part,
-                                                            const i32* __restrict__ dest,
-                                                            const u64* __restrict__ mvp, i64* out) {
-    const i64 w = block_id();
-    if (w >= nb) return;
-    const i64 x = k - 1 - w;
-    const i32 i = moves[x];
-    const i64 s = rp[i], e = rp[i + 1];
-    if (e - s < MASSIVE_CUTOFF) return;  // block-uniform
-    const i32 oi = part[i], ni = dest[i];
+};
+struct AccInst {
+    const i32* inst;
+    i64* sums;
+    template <int BS>
+    __device__ __forceinline__ void add(i32 i, i64 acc) const {
+        __shared__ i32 lk[IC_SLOTS];
+        __shared__ i64 lv[IC_SLOTS];
+        lds_agg_clear<BS, IC_SLOTS>(lk, lv);
+        if (i >= 0 && acc) table_add_lds(lk, lv, IC_SLOTS - 1, inst[i], acc);
+        __syncthreads();
+        for (int q = threadIdx.x; q < IC_SLOTS; q += BS)
+            if (lk[q] != EMPTY_KEY && lv[q] != 0)
+                atomicAdd((unsigned long long*)&sums[lk[q]], (unsigned long long)lv[q]);
+    }
+};
+
+// hub tables as the move kernels see them (hidx null: not kept current)
+struct HubView {
+    const i32* hidx;
+    const i64* goff;
+    const u32* hsm;
+    i32* gkeys;
+    i64* gvals;
+    u64* gtab;
+    u32* hlist;
+    i32* hcnt;
+    i64* stale;
+};
+
+// One pass over the movers' edges (src/local_mover.cpp:1274-1277, 717, 798):
+//  - the exact uncut change, per edge w * ([new_i == new_v] - [old_i ==
+//    old_v]), counted once for mover pairs and twice for neighbours that stay
+//    (the reference computes the same quantity from pvals);
+//  - RESET: the neighbour's cached destination becomes NULL_PART;
+//  - HUB: a hub neighbour's table moves the edge's weight between its keys.
+// What bounds it is latency: each edge is a chain of dependent loads (column,
+// neighbour word, hub slot, atomics).  So a mover of degree below
+// LARGE_CUTOFF takes MV_G lanes, one below MASSIVE_CUTOFF a 128-thread half
+// block, the rest chunks of MV_CHUNK edges per block, and each thread has
+// MV_U edges in flight.  As one thread per small mover and one wave per
+// mid-size one, in a kernel each for the three jobs, the hub updates alone
+// took 479 + 109 us per sweep on R-MAT scale 20 (1.04 ms at worst on scale
+// 22); this kernel does all of it in 82-98 us there (193 us on average on
+// scale 22).
+// The list is in order1 order: the movers of degree >= LARGE_CUTOFF are a
+// suffix of at most nw entries, those >= MASSIVE_CUTOFF one of at most nb.
+constexpr int MV_G = 16, MV_U = 4;
+constexpr i64 MV_CHUNK = 8192;
+template <bool HUB, bool PACKED, bool RESET, class WT, class AT>
+__global__ void __launch_bounds__(256) k_move_edges(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
+                                                    const i32* __restrict__ moves, i64 k, i64 b1, i64 b2, i64 nw,
+                                                    i64 nb, i64 cpm, const u64* __restrict__ mvp, HubView hv,
+                                                    i32* __restrict__ dest, AT at) {
+    const i64 b = block_id();
+    i64 x;         // list entry
+    int lane, gs;  // this thread among the gs threads of the entry
+    i64 lo = 0, hi = 0, c0 = 0, cl = (i64)1 << 62;
+    if (b < b1) {
+        x = b * (256 / MV_G) + threadIdx.x / MV_G;
+        lane = threadIdx.x & (MV_G - 1);
+        gs = MV_G;
+        hi = LARGE_CUTOFF;
+        if (x >= k) x = -1;
+    } else if (b < b1 + b2) {
+        const i64 w = (b - b1) * 2 + (threadIdx.x >> 7);
+        x = w < nw ? k - 1 - w : -1;
+        lane = threadIdx.x & 127;
+        gs = 128;
+        lo = LARGE_CUTOFF;
+        hi = MASSIVE_CUTOFF;
+    } else {
+        const i64 w = (b - b1 - b2) / cpm;
+        x = w < nb ? k - 1 - w : -1;
+        lane = threadIdx.x;
+        gs = 256;
+        lo = MASSIVE_CUTOFF;
+        hi = (i64)1 << 62;
+        c0 = ((b - b1 - b2) % cpm) * MV_CHUNK;
+        cl = MV_CHUNK;
+    }
     i64 acc = 0;
-    for (i64 j = s + threadIdx.x; j < e; j += 1024) acc += delta_term(col, W, mvp, j, oi, ni);
-    acc = block_sum_i64<1024>(acc);
-    if (threadIdx.x == 0) out[x] = acc;
+    i32 i = -1;
+    if (x >= 0) {
+        i = moves[x];
+        const i64 s0 = rp[i], d = rp[i + 1] - s0;
+        const u64 me = mvp[i];
+        const i32 oi = (i32)((u32)me & 0x7fffffffu), ni = (i32)(u32)(me >> 32);
+        if (d >= lo && d < hi && c0 < d) {
+            const i64 e = s0 + (d < c0 + cl ? d : c0 + cl);
+            for (i64 jb = s0 + c0 + lane; jb < e; jb += (i64)gs * MV_U) {
+                i32 v[MV_U], h[MV_U];
+                u64 q[MV_U];
+#pragma unroll
+                for (int u = 0; u < MV_U; u++) {
+                    const i64 j = jb + (i64)u * gs;
+                    v[u] = j < e ? col[j] : -1;
+                }
+#pragma unroll
+                for (int u = 0; u < MV_U; u++) {
+                    q[u] = v[u] >= 0 ? mvp[v[u]] : 0;
+                    h[u] = HUB && v[u] >= 0 ? hv.hidx[v[u]] : -1;
+                }
+#pragma unroll
+                for (int u = 0; u < MV_U; u++) {
+                    if (v[u] < 0) continue;
+                    if (RESET) dest[v[u]] = NULL_PART;
+                    const i64 w = W(jb + (i64)u * gs);
+                    const u32 ql = (u32)q[u];
+                    const i32 ov = (i32)(ql & 0x7fffffffu), nv = (i32)(u32)(q[u] >> 32);
+                    const i64 dd = (i64)(ni == nv) - (i64)(oi == ov);
+                    acc += dd * w * ((ql >> 31) ? 1 : 2);
+                    // ni < 0: an unresolved NEW_PART mover is not applied
+                    if (HUB && h[u] >= 0 && ni >= 0)
+                        hub_update_edge<PACKED>(h[u], w, hv.goff, hv.hsm, hv.gkeys, hv.gvals, hv.gtab, hv.hlist,
+                                                hv.hcnt, oi, ni, hv.stale);
+                }
+            }
+        }
+    }
+    at.template add<256>(i, acc);
 }
 
 // The volume changes of a block's 256 movers are merged per cluster in an
 // LDS table first (many movers of a sweep leave or join the same clusters),
 // then each distinct cluster gets one HBM atomic; the sums are exact
-// integers, so the order does not matter.
+// integers, so the order does not matter.  The movers' words and cached
+// destinations are settled for the next sweep.
 constexpr int AM_SLOTS = 1024;  // >= 2 keys per mover of a 256-thread block, at most half full
-__global__ void __launch_bounds__(256) k_apply_moves(const i32* moves, i64 k, const i64* vw, i32* part,
-                                                     const i32* dest, i64* vol) {
+__global__ void __launch_bounds__(256) k_apply_moves(const i32* __restrict__ moves, i64 k,
+                                                     const i64* __restrict__ vw, u64* __restrict__ mvp,
+                                                     i32* __restrict__ part, i32* __restrict__ dest, i64* vol) {
     __shared__ i32 lk[AM_SLOTS];
     __shared__ i64 lv[AM_SLOTS];
     lds_agg_clear<256, AM_SLOTS>(lk, lv);
     const i64 x = thread_item();
     if (x < k) {
         const i32 i = moves[x];
-        const i32 p = part[i], b = dest[i];
-        const i64 w = vw[i];
+        const u64 q = mvp[i];
+        const i32 p = (i32)((u32)q & 0x7fffffffu);
+        i32 b = (i32)(u32)(q >> 32);
         if (b >= 0) {  // unresolved NEW_PART cannot reach here (p_conn is 0 for singletons)
+            const i64 w = vw[i];
             table_add_lds(lk, lv, AM_SLOTS - 1, p, -w);
             table_add_lds(lk, lv, AM_SLOTS - 1, b, w);
             part[i] = b;
+        } else {
+            b = p;
         }
+        mvp[i] = (u64)(u32)b | ((u64)(u32)b << 32);
+        dest[i] = NULL_PART;
     }
     __syncthreads();
     for (int q = threadIdx.x; q < AM_SLOTS; q += 256) {
@@ -1756,169 +1779,137 @@ __global__ void __launch_bounds__(256) k_apply_moves(const i32* moves, i64 k, co
     }
 }
 
-// dest := NULL_PART for the movers and their neighbours (src/local_mover.cpp:717,798),
-// same degree split as the uncut delta
-__global__ void __launch_bounds__(256) k_reset_affected_thread(const i64* __restrict__ rp,
-                                                               const i32* __restrict__ col,
-                                                               const i32* __restrict__ moves, i64 k, i32* dest,
-                                                               i32* mflag) {
-    const i64 x = thread_item();
-    if (x >= k) return;
-    const i32 i = moves[x];
-    const i64 s = rp[i], e = rp[i + 1];
-    if (e - s >= LARGE_CUTOFF) return;
-#pragma unroll 4
-    for (i64 j = s; j < e; j++) dest[col[j]] = NULL_PART;
-    dest[i] = NULL_PART;
-    mflag[i] = 0;
-}
-__global__ void __launch_bounds__(256) k_reset_affected_wave(const i64* __restrict__ rp, const i32* __restrict__ col,
-                                                             const i32* __restrict__ moves, i64 k, i64 nw, i32* dest,
-                                                             i32* mflag) {
-    const int lane = threadIdx.x & 63;
-    const i64 w = block_id() * 4 + (threadIdx.x >> 6);
-    if (w >= nw) return;
-    const i32 i = moves[k - 1 - w];
-    const i64 s = rp[i], e = rp[i + 1];
-    if (e - s < LARGE_CUTOFF || e - s >= MASSIVE_CUTOFF) return;
-    for (i64 j = s + lane; j < e; j += 64) dest[col[j]] = NULL_PART;
-    if (lane == 0) {
-        dest[i] = NULL_PART;
-        mflag[i] = 0;
+// End of a sweep: the exact 128-bit sum of squared volumes, the uncut change
+// and the stale flag, stored to the host slots by the last block to finish
+// (host[0] = uncut change, host[1..2] = sum of squares high and low, host[3] =
+// stale).  One launch instead of seven (fills, two reductions of two
+// kernels each, read-back): on small levels the sweep is bound by launches.
+__global__ void __launch_bounds__(256) k_finish(const i64* __restrict__ vol, i64 L, u64* part, i64* scal, i64* host) {
+    u64 lo = 0, hi = 0;
+    for (i64 x = (i64)blockIdx.x * 256 + threadIdx.x; x < L; x += (i64)gridDim.x * 256) {
+        const i64 v = vol[x];
+        const u64 a = (u64)(v < 0 ? -v : v);
+        const u64 plo = a * a;
+        lo += plo;
+        hi += __umul64hi(a, a) + (lo < plo ? 1 : 0);
     }
-}
-__global__ void __launch_bounds__(1024) k_reset_affected_block(const i64* __restrict__ rp,
-                                                               const i32* __restrict__ col,
-                                                               const i32* __restrict__ moves, i64 k, i64 nb,
-                                                               i32* dest, i32* mflag) {
-    const i64 w = block_id();
-    if (w >= nb) return;
-    const i32 i = moves[k - 1 - w];
-    const i64 s = rp[i], e = rp[i + 1];
-    if (e - s < MASSIVE_CUTOFF) return;
-    for (i64 j = s + threadIdx.x; j < e; j += 1024) dest[col[j]] = NULL_PART;
+    __shared__ u64 slo[256], shi[256];
+    __shared__ int last;
+    auto tree = [&]() {
+        __syncthreads();
+        for (int o = 128; o > 0; o >>= 1) {
+            if ((int)threadIdx.x < o) {
+                const u64 a = slo[threadIdx.x], b = slo[threadIdx.x + o];
+                slo[threadIdx.x] = a + b;
+                shi[threadIdx.x] = shi[threadIdx.x] + shi[threadIdx.x + o] + (a + b < a ? 1 : 0);
+            }
+            __syncthreads();
+        }
+    };
+    slo[threadIdx.x] = lo;
+    shi[threadIdx.x] = hi;
+    tree();
     if (threadIdx.x == 0) {
-        dest[i] = NULL_PART;
-        mflag[i] = 0;
+        // agent-scope stores and loads: the blocks run on different XCDs
+        __hip_atomic_store(&part[2 * blockIdx.x], shi[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(&part[2 * blockIdx.x + 1], slo[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __threadfence();
+        last = atomicAdd((unsigned long long*)&scal[SC_TICKET], 1ull) == gridDim.x - 1;
     }
-}
-__global__ void k_clear_mflag(const i32* moves, i64 k, i32* mflag) {
-    const i64 x = thread_item();
-    if (x >= k) return;
-    mflag[moves[x]] = 0;
-}
-__global__ void k_set_mflag(const i32* moves, i64 k, i32* mflag) {
-    const i64 x = thread_item();
-    if (x >= k) return;
-    mflag[moves[x]] = 1;
+    __syncthreads();
+    if (!last) return;  // block-uniform
+    __threadfence();
+    const int t = threadIdx.x;
+    const bool in = t < (int)gridDim.x;  // gridDim.x <= FIN_BLOCKS
+    slo[t] = in ? __hip_atomic_load(&part[2 * t + 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+    shi[t] = in ? __hip_atomic_load(&part[2 * t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+    tree();
+    const u64 rlo = slo[0], rhi = shi[0];
+    __syncthreads();
+    const i64 du = block_sum_i64<256>(t < MV_SLOTS ? scal[SC_SLOTS + t] : 0);
+    if (t < MV_SLOTS) scal[SC_SLOTS + t] = 0;
+    if (t == 0) {
+        host[0] = du;
+        host[1] = (i64)rhi;
+        host[2] = (i64)rlo;
+        host[3] = scal[SC_STALE];
+        scal[SC_STALE] = 0;
+        scal[SC_TICKET] = 0;
+        __threadfence_system();
+    }
 }
 
-// perform_moves (src/local_mover.cpp:1241-1279).  moves is in order1 order,
-// so movers by degree class: below LARGE_CUTOFF (a thread each), below
-// MASSIVE_CUTOFF (a wave each), then the rest (a 1024-thread block each).
+// perform_moves (src/local_mover.cpp:1241-1279).  moves is in order1 order;
 // n_large / n_massive = vertices of the level with degree >= LARGE_CUTOFF /
-// MASSIVE_CUTOFF, which bound the movers of the last two classes.
-// The moves themselves: hub-table updates (before part changes), the exact
-// uncut delta of every mover into du[x], volume moves and part updates.  A
-// hub table that runs out of slots sets s.scal[3].
+// MASSIVE_CUTOFF, which bound the movers of the last two classes.  The uncut
+// change goes to `at`; a hub table that runs out of slots sets SC_STALE.
+// reset: the movers' neighbours are scored again in the next sweep.
+template <class AT>
 static void apply_moves_core(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, i64* vol, const i32* moves,
-                             i64 k, i64 n_large, i64 n_massive, i64* du) {
+                             i64 k, i64 n_large, i64 n_massive, bool reset, AT at) {
     const i64 nw = std::min(k, n_large);
     const i64 nb = std::min(k, n_massive);
     const int tk = c.kt_begin(KS_MOVES);
-    fill_i64(c, s.scal.p + 3, 1, 0);
     const i64 m7 = lp.nhub;
     // many movers: updating costs more than rebuilding the tables next sweep
     if (lp.hub_live && m7 > 0 && (c.hub_update_div <= 0 || k * c.hub_update_div > g.n)) lp.hub_live = false;
     const bool hub_upd = lp.hub_live && m7 > 0;
-    if (hub_upd) {  // keep the hub tables current (before part changes)
-        i64* stale = s.scal.p + 3;
-        PGGC_WDISPATCH(g, {
-            if (lp.packed) {
-                k_hub_update_thread<true><<<grid_items(k, 256), 256, 0, c.stream>>>(
-                    g.rp, g.col, W, moves, k, s.part, s.dest, lp.hidx, lp.goff, lp.hsm, nullptr, nullptr, lp.gtab, lp.hlist, lp.hcnt, stale);
-                if (nw > 0)
-                    k_hub_update_wave<true><<<grid_items(nw, 4), 256, 0, c.stream>>>(
-                        g.rp, g.col, W, moves, k, nw, s.part, s.dest, lp.hidx, lp.goff, lp.hsm, nullptr, nullptr, lp.gtab, lp.hlist, lp.hcnt,
-                        stale);
-                if (nb > 0)
-                    k_hub_update_block<true><<<grid_blocks(nb), 1024, 0, c.stream>>>(
-                        g.rp, g.col, W, moves, k, nb, s.part, s.dest, lp.hidx, lp.goff, lp.hsm, nullptr, nullptr, lp.gtab, lp.hlist, lp.hcnt,
-                        stale);
-            } else {
-                k_hub_update_thread<false><<<grid_items(k, 256), 256, 0, c.stream>>>(
-                    g.rp, g.col, W, moves, k, s.part, s.dest, lp.hidx, lp.goff, lp.hsm, lp.gkeys, lp.gvals, nullptr, lp.hlist, lp.hcnt, stale);
-                if (nw > 0)
-                    k_hub_update_wave<false><<<grid_items(nw, 4), 256, 0, c.stream>>>(
-                        g.rp, g.col, W, moves, k, nw, s.part, s.dest, lp.hidx, lp.goff, lp.hsm, lp.gkeys, lp.gvals, nullptr, lp.hlist, lp.hcnt,
-                        stale);
-                if (nb > 0)
-                    k_hub_update_block<false><<<grid_blocks(nb), 1024, 0, c.stream>>>(
-                        g.rp, g.col, W, moves, k, nb, s.part, s.dest, lp.hidx, lp.goff, lp.hsm, lp.gkeys, lp.gvals, nullptr, lp.hlist, lp.hcnt,
-                        stale);
-            }
-        });
-        PGGC_LAUNCH_CHECK();
-    }
-    {
-        k_mv_pack<<<grid_items(g.n, 256), 256, 0, c.stream>>>(g.n, s.part, s.dest, s.mflag, s.mvp);
-        PGGC_LAUNCH_CHECK();
-        PGGC_WDISPATCH(g, {
-            k_delta_uncut_thread<<<grid_items(k, 256), 256, 0, c.stream>>>(g.rp, g.col, W, moves, k, s.part, s.dest,
-                                                                          s.mvp, du);
-            if (nw > 0)
-                k_delta_uncut_wave<<<grid_items(nw, 4), 256, 0, c.stream>>>(g.rp, g.col, W, moves, k, nw, s.part,
-                                                                           s.dest, s.mvp, du);
-            if (nb > 0)
-                k_delta_uncut_block<<<grid_blocks(nb), 1024, 0, c.stream>>>(g.rp, g.col, W, moves, k, nb, s.part,
-                                                                           s.dest, s.mvp, du);
-        });
-        PGGC_LAUNCH_CHECK();
-    }
-    k_apply_moves<<<grid_items(k, 256), 256, 0, c.stream>>>(moves, k, g.vw, s.part, s.dest, vol);
+    k_mvp_moves<<<grid_items(k, 256), 256, 0, c.stream>>>(moves, k, s.part, s.dest, s.mvp);
+    PGGC_LAUNCH_CHECK();
+    const i64 cpm = nb > 0 ? ceil_div(lp.max_deg, MV_CHUNK) : 1;
+    const i64 b1 = ceil_div(k, 256 / MV_G), b2 = ceil_div(nw, 2), b3 = nb * cpm;
+    const HubView hv{hub_upd ? lp.hidx.p : nullptr, lp.goff, lp.hsm, lp.gkeys, lp.gvals, lp.gtab, lp.hlist, lp.hcnt,
+                     s.scal.p + SC_STALE};
+#define PGGC_MOVE_EDGES(HUB, PK, RS)                                                                               \
+    k_move_edges<HUB, PK, RS><<<grid_blocks(b1 + b2 + b3), 256, 0, c.stream>>>(g.rp, g.col, W, moves, k, b1, b2, nw, \
+                                                                              nb, cpm, s.mvp, hv, s.dest, at)
+    PGGC_WDISPATCH(g, {
+        if (!hub_upd && reset) PGGC_MOVE_EDGES(false, false, true);
+        else if (!hub_upd) PGGC_MOVE_EDGES(false, false, false);
+        else if (lp.packed && reset) PGGC_MOVE_EDGES(true, true, true);
+        else if (lp.packed) PGGC_MOVE_EDGES(true, true, false);
+        else if (reset) PGGC_MOVE_EDGES(true, false, true);
+        else PGGC_MOVE_EDGES(true, false, false);
+    });
+#undef PGGC_MOVE_EDGES
+    PGGC_LAUNCH_CHECK();
+    k_apply_moves<<<grid_items(k, 256), 256, 0, c.stream>>>(moves, k, g.vw, s.mvp, s.part, s.dest, vol);
     c.kt_end(tk, 0.0);
     PGGC_LAUNCH_CHECK();
     if (tk >= 0) {  // timing runs only
-        // per vertex the packed record (part, dest, flag read, 8 bytes
-        // written); per mover row bounds, part, dest, the partial delta and
-        // its sum, vertex weight, two volume updates and the part write; per
-        // mover edge column, weight and the neighbour's record, plus the
-        // column, weight and hub index again when hub tables are updated
+        // per mover its word (written, read, settled), row bounds, cluster,
+        // destination, vertex weight and two volume updates; per mover edge
+        // the column, weight, the neighbour's word and its destination reset,
+        // plus the hub index when hub tables are kept current
         const int wb = g.wk == W_UNIT ? 0 : g.wk == W_I32 ? 4 : 8;
         Buf<i64> acc(c, 1);
         fill_i64(c, acc, 1, 0);
         k_list_bytes<<<grid_items(std::max<i64>(k, 1), 256), 256, 0, c.stream>>>(
-            g.rp, moves, k, 72, 12 + wb + (hub_upd ? 8 + wb : 0), 20 * g.n, acc);
+            g.rp, moves, k, 84, 12 + wb + (reset ? 4 : 0) + (hub_upd ? 4 : 0), 0, acc);
         PGGC_LAUNCH_CHECK();
         acct_add(c, c.kt_counter(tk), acc);
     }
 }
 
+static void init_mvp(Ctx& c, MoveScratch& s, i64 n) {
+    if (n <= 0) return;
+    k_mvp_init<<<grid_items(n, 256), 256, 0, c.stream>>>(n, s.part, s.mvp, s.scal);
+    PGGC_LAUNCH_CHECK();
+}
+
 static void perform_moves(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, RefineData& curr,
                           const i32* moves, i64 k, i64 n_large, i64 n_massive, bool& tables) {
-    const i64 nw = std::min(k, n_large);
-    const i64 nb = std::min(k, n_massive);
-    {
-        Buf<i64> du(c, std::max<i64>(k, 1));
-        apply_moves_core(c, s, lp, g, curr.vol, moves, k, n_large, n_massive, du);
-        sum_i64(c, du, k, s.scal);
-    }
+    apply_moves_core(c, s, lp, g, curr.vol, moves, k, n_large, n_massive, tables, AccOne{s.scal.p + SC_SLOTS});
     if (!tables) {
         tables = true;
         fill_i32(c, s.dest, g.n, NULL_PART);
-        k_clear_mflag<<<grid_items(k, 256), 256, 0, c.stream>>>(moves, k, s.mflag);
-    } else {
-        k_reset_affected_thread<<<grid_items(k, 256), 256, 0, c.stream>>>(g.rp, g.col, moves, k, s.dest, s.mflag);
-        if (nw > 0)
-            k_reset_affected_wave<<<grid_items(nw, 4), 256, 0, c.stream>>>(g.rp, g.col, moves, k, nw, s.dest,
-                                                                           s.mflag);
-        if (nb > 0)
-            k_reset_affected_block<<<grid_blocks(nb), 1024, 0, c.stream>>>(g.rp, g.col, moves, k, nb, s.dest,
-                                                                           s.mflag);
     }
+    const i64 L = curr.label_count;
+    k_finish<<<grid_for(std::max<i64>(L, 1), 256 * 8, FIN_BLOCKS), 256, 0, c.stream>>>(curr.vol, L, s.sqpart, s.scal,
+                                                                                      c.pinned_dev);
     PGGC_LAUNCH_CHECK();
-    sum_sq_u128(c, curr.vol, curr.label_count, s.scal.p + 1);
-    const i64* h = c.read(s.scal, 4);
+    c.sync();
+    const i64* h = c.pinned;
     if (h[3]) lp.hub_live = false;  // a hub table ran out of slots: rebuild next sweep
     curr.uncut += h[0];
     curr.obj = objective_value(curr.uncut, curr.lambda, (u64)h[1], (u64)h[2]);
@@ -2047,6 +2038,7 @@ static void local_move_t(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g,
     Buf<i64> cv;
     RefineData curr = begin_curr(c, best, cv, n);
     copy_dev(c, s.part, best_part, n * sizeof(i32));
+    init_mvp(c, s, n);
     fill_i32(c, s.dest, n, NULL_PART);
     bool tables = !is_initial;
     const float ratios[2] = {0.75f, 0.25f};
@@ -2200,6 +2192,7 @@ void local_move_strict(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, i
     Buf<i64> cv;
     RefineData curr = begin_curr(c, best, cv, n);
     copy_dev(c, s.part, best_part, n * sizeof(i32));
+    init_mvp(c, s, n);
     fill_i32(c, s.dest, n, NULL_PART);
     bool tables = !is_initial;
     const i32* ccons = constrained ? cons : nullptr;
@@ -2233,8 +2226,6 @@ void local_move_strict(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, i
             trc.end(k, 0);
             break;
         }
-        k_set_mflag<<<grid_items(tr, 256), 256, 0, c.stream>>>(s.moves, tr, s.mflag);
-        PGGC_LAUNCH_CHECK();
         perform_moves(c, s, lp, g, curr, s.moves, tr, g.n - lp.ord.off_large, g.n - lp.ord.off_large2, tables);
         if (stats) stats->moves += tr;
         if (curr.obj > best.obj) {
@@ -2268,8 +2259,6 @@ i64 sweep_once(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, const i32
     i64 km = 0;
     if (k > 0) {
         km = afterburner(c, s, g, s.cand, k, b, LamOne{lam}, PrioOne{}, moves_out);
-        k_clear_mflag<<<grid_items(km, 256), 256, 0, c.stream>>>(moves_out, km, s.mflag);
-        PGGC_LAUNCH_CHECK();
     }
     copy_dev(c, dest, s.dest, n * sizeof(i32));
     copy_dev(c, gain, s.gain, n * sizeof(float));
@@ -2326,7 +2315,6 @@ static void download(Ctx& c, std::vector<T>& dst, const T* src, size_t count) {
 // of one per entry.  Per-entry atomics on a few dozen counters ran at the
 // rate of one address: 241 us per launch on average over 48 instances
 // (2.8M vertices), 6.4 ms for the largest list; merged 4-6 us.
-constexpr int IC_SLOTS = 512;  // at most 256 distinct instances per block
 __global__ void __launch_bounds__(256) k_inst_count(const i32* __restrict__ list, i64 k,
                                                     const i32* __restrict__ owner, i64* cnt) {
     __shared__ i32 lk[IC_SLOTS];
@@ -2348,19 +2336,6 @@ __global__ void k_inst_fill(i64 n, const i32* __restrict__ inst, const i32* __re
     const i64 v = thread_item();
     if (v >= n) return;
     if (mask[inst[v]]) a[v] = val;
-}
-__global__ void __launch_bounds__(256) k_inst_add(const i32* __restrict__ moves, i64 k,
-                                                  const i32* __restrict__ inst, const i64* __restrict__ du,
-                                                  i64* acc) {
-    __shared__ i32 lk[IC_SLOTS];
-    __shared__ i64 lv[IC_SLOTS];
-    lds_agg_clear<256, IC_SLOTS>(lk, lv);
-    const i64 x = thread_item();
-    if (x < k) table_add_lds(lk, lv, IC_SLOTS - 1, inst[moves[x]], du[x]);
-    __syncthreads();
-    for (int q = threadIdx.x; q < IC_SLOTS; q += 256)
-        if (lk[q] != EMPTY_KEY && lv[q] != 0)
-            atomicAdd((unsigned long long*)&acc[lk[q]], (unsigned long long)lv[q]);
 }
 // exact 128-bit sum of squared volumes over each masked instance's labels
 // [loff[k], loff[k] + L[k]); one block per instance, out[2k] = high word
@@ -2579,6 +2554,7 @@ void local_move_batch(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, co
     copy_dev(c, cvol, best.vol, NL * sizeof(i64));
     std::vector<RefineData> cur = best.rd;
     copy_dev(c, s.part, best_part, n * sizeof(i32));
+    init_mvp(c, s, n);
     fill_i32(c, s.dest, n, NULL_PART);
     Buf<i32> on(c, K), full(c, K), imp(c, K);
     Buf<float> rat(c, K);
@@ -2634,25 +2610,10 @@ void local_move_batch(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, co
         }
         if (km > 0) {
             set_new_cluster_ids_batch(c, s, g, bl, best, cur, cvol, s.moves, km);
-            {
-                Buf<i64> du(c, km);
-                apply_moves_core(c, s, lp, g, cvol, s.moves, km, n_large, n_massive, du);
-                fill_i64(c, acc, K, 0);
-                k_inst_add<<<grid_items(km, 256), 256, 0, c.stream>>>(s.moves, km, bl.inst, du, acc);
-                PGGC_LAUNCH_CHECK();
-            }
-            // dest := NULL_PART for movers and their neighbours, and for
-            // every vertex of an instance whose first moves these are
-            const i64 nw = std::min(km, n_large), nb = std::min(km, n_massive);
-            k_reset_affected_thread<<<grid_items(km, 256), 256, 0, c.stream>>>(g.rp, g.col, s.moves, km, s.dest,
-                                                                              s.mflag);
-            if (nw > 0)
-                k_reset_affected_wave<<<grid_items(nw, 4), 256, 0, c.stream>>>(g.rp, g.col, s.moves, km, nw, s.dest,
-                                                                               s.mflag);
-            if (nb > 0)
-                k_reset_affected_block<<<grid_blocks(nb), 1024, 0, c.stream>>>(g.rp, g.col, s.moves, km, nb, s.dest,
-                                                                               s.mflag);
-            PGGC_LAUNCH_CHECK();
+            fill_i64(c, acc, K, 0);
+            // resets the movers and their neighbours; every vertex of an
+            // instance whose first moves these are follows below
+            apply_moves_core(c, s, lp, g, cvol, s.moves, km, n_large, n_massive, true, AccInst{bl.inst, acc});
             bool anyfull = false;
             for (i64 q = 0; q < K; q++) {
                 const bool moved = hc[K + q] > 0;
@@ -2670,7 +2631,8 @@ void local_move_batch(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, co
             upload(c, imp.p, himp);
             k_inst_sumsq<<<grid_blocks(K), 256, 0, c.stream>>>(cvol, best.dloff, Ld, imp, K, sq);
             PGGC_LAUNCH_CHECK();
-            const i64 stale = c.read1(s.scal.p + 3);
+            const i64 stale = c.read1(s.scal.p + SC_STALE);
+            if (stale) fill_i64(c, s.scal.p + SC_STALE, 1, 0);
             if (stale) lp.hub_live = false;  // a hub table ran out of slots: rebuild next sweep
             download(c, hacc, acc.p, K);
             download(c, hsq, sq.p, 2 * K);
