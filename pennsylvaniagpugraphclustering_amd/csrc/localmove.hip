@@ -360,20 +360,36 @@ __device__ __forceinline__ u64 pack_cand(float jc, i32 key) {
     return ((u64)ord_f32(jc) << 32) | (u64)(0xFFFFFFFFu - (u32)(key + 4));
 }
 
-__device__ __forceinline__ void decide(i32 i, float p_conn, u64 bk, i32* dest, float* gain) {
+// What scoring writes per scored vertex: the cached destination, the gain
+// (when some caller reads the array) and the afterburner's record.  A vertex
+// that is not scored keeps its record: it is NO_MOVE, and its cluster cannot
+// have changed since that was decided.
+struct ScoreOut {
+    i32* dest;
+    float* gain;   // nullable
+    AbInfo* info;  // nullable: k_ab_pack builds the records from the arrays
+};
+
+__device__ __forceinline__ void decide(i32 i, float p_conn, u64 bk, i32 p, i64 wv, const ScoreOut& o) {
     bool have = bk != 0;
     float bj = have ? unord_f32((u32)(bk >> 32)) : 0.0f;
     i32 bc = have ? (i32)(0xFFFFFFFFu - (u32)(bk & 0xffffffffull)) - 4 : 0;
+    AbInfo a;
+    a.part = p;
+    a.vwf = (float)wv;
     if (p_conn < 0.0f && (!have || !(bj > 0.0f))) {
-        gain[i] = 0.0f - p_conn;
-        dest[i] = NEW_PART;
+        a.gain = 0.0f - p_conn;
+        a.dest = NEW_PART;
     } else if (have) {
-        gain[i] = bj - p_conn;
-        dest[i] = bc;
+        a.gain = bj - p_conn;
+        a.dest = bc;
     } else {
-        gain[i] = -FLT_MAX;
-        dest[i] = NO_MOVE;
+        a.gain = -FLT_MAX;
+        a.dest = NO_MOVE;
     }
+    o.dest[i] = a.dest;
+    if (o.gain) o.gain[i] = a.gain;
+    if (o.info) o.info[i] = a;
 }
 
 // lambda of a vertex's objective and the sweep's filter ratio: one value
@@ -423,14 +439,14 @@ __global__ void __launch_bounds__(256) k_score_group(const i64* __restrict__ rp,
                                                      const i64* __restrict__ vw, const i32* __restrict__ list, i64 m,
                                                      const i32* __restrict__ part, const i64* __restrict__ vol,
                                                      const i32* __restrict__ cons, int raw, LT lam, float ratio,
-                                                     i32* __restrict__ dest, float* __restrict__ gain) {
+                                                     ScoreOut out) {
     constexpr int GPB = 256 / G;
     const int gl = threadIdx.x & (G - 1);
     const i64 gi = block_id() * GPB + threadIdx.x / G;
     if (gi >= m) return;
     {
         const i32 i = list[gi];
-        if (dest[i] == NO_MOVE) return;
+        if (out.dest[i] == NO_MOVE) return;
         const i64 s = rp[i];
         const int d = (int)(rp[i + 1] - s);
         const i32 p = part[i];
@@ -467,7 +483,7 @@ __global__ void __launch_bounds__(256) k_score_group(const i64* __restrict__ rp,
             if (jc >= b) bk = pack_cand(jc, key);
         }
         bk = group_max_u64<G>(bk);
-        if (gl == 0) decide(i, p_conn, bk, dest, gain);
+        if (gl == 0) decide(i, p_conn, bk, p, wv, out);
     }
 }
 
@@ -479,8 +495,8 @@ __global__ void __launch_bounds__(BS) k_score_table(const i64* __restrict__ rp, 
                                                     const i64* __restrict__ vw, const i32* __restrict__ list, i64 m,
                                                     const i32* __restrict__ part, const i64* __restrict__ vol,
                                                     const i32* __restrict__ cons, int raw, LT lam, float ratio,
-                                                    i32* __restrict__ dest, float* __restrict__ gain, i32* gkeys,
-                                                    i64* gvals, const i64* __restrict__ goff) {
+                                                    ScoreOut out, i32* gkeys, i64* gvals,
+                                                    const i64* __restrict__ goff) {
     __shared__ i32 skeys[GLOBAL ? 1 : SLOTS];
     __shared__ i64 svals[GLOBAL ? 1 : SLOTS];
     const int t = threadIdx.x;
@@ -488,7 +504,7 @@ __global__ void __launch_bounds__(BS) k_score_table(const i64* __restrict__ rp, 
     if (li >= m) return;
     {
         const i32 i = list[li];
-        if (dest[i] == NO_MOVE) return;
+        if (out.dest[i] == NO_MOVE) return;
         const i64 s = rp[i];
         const i64 d = rp[i + 1] - s;
         const i64 S = tslots(d, SPE);
@@ -543,7 +559,8 @@ __global__ void __launch_bounds__(BS) k_score_table(const i64* __restrict__ rp, 
         if (GLOBAL) __threadfence();
         pv = block_sum_i64<BS>(pv);
         float multi, p_conn, b;
-        own_terms(pv, vol[p], vw[i], lam(i), lam.rt(i, ratio), multi, p_conn, b);
+        const i64 wi = vw[i];
+        own_terms(pv, vol[p], wi, lam(i), lam.rt(i, ratio), multi, p_conn, b);
         u64 bk = 0;
         for (i64 qb = 0; qb < S; qb += BS) {  // block-uniform loop control
             const i64 q = qb + t;
@@ -568,7 +585,7 @@ __global__ void __launch_bounds__(BS) k_score_table(const i64* __restrict__ rp, 
             }
         }
         bk = block_max_u64<BS>(bk);
-        if (t == 0) decide(i, p_conn, bk, dest, gain);
+        if (t == 0) decide(i, p_conn, bk, p, wi, out);
         __syncthreads();
     }
 }
@@ -597,16 +614,17 @@ __global__ void __launch_bounds__(BS) k_score_raw(const i64* __restrict__ rp, co
                                                   const i64* __restrict__ vw, const i32* __restrict__ list, i64 m,
                                                   const i32* __restrict__ part, const i64* __restrict__ vol,
                                                   const i32* __restrict__ cons, const i32* __restrict__ lab, LT lam,
-                                                  float ratio, i32* __restrict__ dest, float* __restrict__ gain) {
+                                                  float ratio, ScoreOut out) {
     const i64 li = block_id();
     if (li >= m) return;
     const i32 i = list[li];
-    if (dest[i] == NO_MOVE) return;
+    if (out.dest[i] == NO_MOVE) return;
     const i64 s = rp[i], e = rp[i + 1];
     const i32 p = part[i];
     const i32 cp = cons ? cons[p] : 0;
     float multi, p_conn, b;
-    own_terms(0, vol[p], vw[i], lam(i), lam.rt(i, ratio), multi, p_conn, b);
+    const i64 wi = vw[i];
+    own_terms(0, vol[p], wi, lam(i), lam.rt(i, ratio), multi, p_conn, b);
     u64 bk = 0;
     for (i64 jb = s; jb < e; jb += BS) {  // block-uniform loop control
         const i64 j = jb + threadIdx.x;
@@ -616,7 +634,7 @@ __global__ void __launch_bounds__(BS) k_score_raw(const i64* __restrict__ rp, co
         }
     }
     bk = block_max_u64<BS>(bk);
-    if (threadIdx.x == 0) decide(i, p_conn, bk, dest, gain);
+    if (threadIdx.x == 0) decide(i, p_conn, bk, p, wi, out);
 }
 
 // hubs: one block per edge item, folded into hub_best with atomicMax
@@ -1018,14 +1036,16 @@ __global__ void __launch_bounds__(256) k_hub_scan(const i32* __restrict__ hubs, 
 
 template <class LT>
 __global__ void k_hub_decide(const i32* hubs, i64 m, const i32* part, const i64* vw, const i64* vol, LT lam,
-                             float ratio, const i64* hub_pv, const u64* hub_best, i32* dest, float* gain) {
+                             float ratio, const i64* hub_pv, const u64* hub_best, ScoreOut out) {
     const i64 hi = thread_item();
     if (hi >= m) return;
     const i32 i = hubs[hi];
-    if (dest[i] == NO_MOVE) return;
+    if (out.dest[i] == NO_MOVE) return;
+    const i32 p = part[i];
+    const i64 wi = vw[i];
     float multi, p_conn, bth;
-    own_terms(hub_pv[hi], vol[part[i]], vw[i], lam(i), lam.rt(i, ratio), multi, p_conn, bth);
-    decide(i, p_conn, hub_best[hi], dest, gain);
+    own_terms(hub_pv[hi], vol[p], wi, lam(i), lam.rt(i, ratio), multi, p_conn, bth);
+    decide(i, p_conn, hub_best[hi], p, wi, out);
 }
 
 
@@ -1094,25 +1114,25 @@ __global__ void __launch_bounds__(256) k_list_bytes(const i64* __restrict__ rp, 
 // BS threads, SLOTS LDS slots, SPE slots per edge of the degree bound.
 template <int BS, int SLOTS, int SPE, class WT, class LT>
 static void launch_table(Ctx& c, const DGraph& g, WT W, const i32* L, i64 x0, i64 x1, const i32* part,
-                         const i64* vol, const i32* cons, LT lam, float ratio, i32* dest, float* gain) {
+                         const i64* vol, const i32* cons, LT lam, float ratio, const ScoreOut& out) {
     const i64 m = x1 - x0;
     if (m <= 0) return;
     k_score_table<BS, SLOTS, SPE, false><<<grid_blocks(m), BS, 0, c.stream>>>(
-        g.rp, g.col, W, g.vw, L + x0, m, part, vol, cons, 0, lam, ratio, dest, gain, nullptr, nullptr, nullptr);
+        g.rp, g.col, W, g.vw, L + x0, m, part, vol, cons, 0, lam, ratio, out, nullptr, nullptr, nullptr);
 }
 // class with degree bound D (128, 256, 512): threads per vertex and slots per
 // edge from the knobs
 template <int D, class WT, class LT>
 static void launch_table_class(Ctx& c, const DGraph& g, WT W, const i32* L, i64 x0, i64 x1, const i32* part,
-                               const i64* vol, const i32* cons, LT lam, float ratio, i32* dest, float* gain) {
+                               const i64* vol, const i32* cons, LT lam, float ratio, const ScoreOut& out) {
     const int bs = c.table_threads, spe = c.table_spe;
-    if (bs == 64 && spe == 2) launch_table<64, 2 * D, 2>(c, g, W, L, x0, x1, part, vol, cons, lam, ratio, dest, gain);
-    else if (bs == 64) launch_table<64, 4 * D, 4>(c, g, W, L, x0, x1, part, vol, cons, lam, ratio, dest, gain);
+    if (bs == 64 && spe == 2) launch_table<64, 2 * D, 2>(c, g, W, L, x0, x1, part, vol, cons, lam, ratio, out);
+    else if (bs == 64) launch_table<64, 4 * D, 4>(c, g, W, L, x0, x1, part, vol, cons, lam, ratio, out);
     else if (bs == 128 && spe == 2)
-        launch_table<128, 2 * D, 2>(c, g, W, L, x0, x1, part, vol, cons, lam, ratio, dest, gain);
-    else if (bs == 128) launch_table<128, 4 * D, 4>(c, g, W, L, x0, x1, part, vol, cons, lam, ratio, dest, gain);
-    else if (spe == 2) launch_table<256, 2 * D, 2>(c, g, W, L, x0, x1, part, vol, cons, lam, ratio, dest, gain);
-    else launch_table<256, 4 * D, 4>(c, g, W, L, x0, x1, part, vol, cons, lam, ratio, dest, gain);
+        launch_table<128, 2 * D, 2>(c, g, W, L, x0, x1, part, vol, cons, lam, ratio, out);
+    else if (bs == 128) launch_table<128, 4 * D, 4>(c, g, W, L, x0, x1, part, vol, cons, lam, ratio, out);
+    else if (spe == 2) launch_table<256, 2 * D, 2>(c, g, W, L, x0, x1, part, vol, cons, lam, ratio, out);
+    else launch_table<256, 4 * D, 4>(c, g, W, L, x0, x1, part, vol, cons, lam, ratio, out);
 }
 
 // Hub tables of the current clustering: slices built in LDS, then the
@@ -1221,7 +1241,8 @@ static void hub_build_all(Ctx& c, const DGraph& g, WT W, LevelPlan& lp, const i3
 
 template <class LT>
 static void score_all(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, const i32* part, const i64* vol,
-                      const i32* cons, int raw, LT lam, float ratio, i32* dest, float* gain) {
+                      const i32* cons, int raw, LT lam, float ratio, const ScoreOut& out) {
+    i32* dest = out.dest;
     // raw 1: singletons labelled by vertex id; raw 2: singletons whose labels
     // are read from part (a renumbered graph); 0: any clustering
     const i32* lab = raw == 2 ? part : nullptr;
@@ -1245,45 +1266,45 @@ static void score_all(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, co
         int tk = c.kt_begin(KS_SCORE_GROUP);
         if ((m = st[1] - st[0]) > 0)
             k_score_group<4><<<grid_items(m, 64), 256, 0, c.stream>>>(
-                g.rp, g.col, W, g.vw, L + st[0], m, part, vol, cons, raw, lam, ratio, dest, gain);
+                g.rp, g.col, W, g.vw, L + st[0], m, part, vol, cons, raw, lam, ratio, out);
         if ((m = st[2] - st[1]) > 0)
             k_score_group<8><<<grid_items(m, 32), 256, 0, c.stream>>>(
-                g.rp, g.col, W, g.vw, L + st[1], m, part, vol, cons, raw, lam, ratio, dest, gain);
+                g.rp, g.col, W, g.vw, L + st[1], m, part, vol, cons, raw, lam, ratio, out);
         if ((m = st[3] - st[2]) > 0)
             k_score_group<16><<<grid_items(m, 16), 256, 0, c.stream>>>(
-                g.rp, g.col, W, g.vw, L + st[2], m, part, vol, cons, raw, lam, ratio, dest, gain);
+                g.rp, g.col, W, g.vw, L + st[2], m, part, vol, cons, raw, lam, ratio, out);
         if ((m = st[4] - st[3]) > 0)
             k_score_group<32><<<grid_items(m, 8), 256, 0, c.stream>>>(
-                g.rp, g.col, W, g.vw, L + st[3], m, part, vol, cons, raw, lam, ratio, dest, gain);
+                g.rp, g.col, W, g.vw, L + st[3], m, part, vol, cons, raw, lam, ratio, out);
         if ((m = st[5] - st[4]) > 0)
             k_score_group<64><<<grid_items(m, 4), 256, 0, c.stream>>>(
-                g.rp, g.col, W, g.vw, L + st[4], m, part, vol, cons, raw, lam, ratio, dest, gain);
+                g.rp, g.col, W, g.vw, L + st[4], m, part, vol, cons, raw, lam, ratio, out);
         c.kt_end(tk, 0.0);
         if (tk >= 0) acct_add(c, c.kt_counter(tk), acct.p);
         tk = c.kt_begin(KS_SCORE_TABLE);
         if (raw) {
             if ((m = st[CL_BIG] - st[CL_TABLE]) > 0)
                 k_score_raw<64><<<grid_blocks(m), 64, 0, c.stream>>>(g.rp, g.col, W, g.vw, L + st[CL_TABLE], m,
-                                                                     part, vol, cons, lab, lam, ratio, dest, gain);
+                                                                     part, vol, cons, lab, lam, ratio, out);
             if ((m = lp.hub0 - st[CL_BIG]) > 0)  // big rows and the LDS-scored hubs
                 k_score_raw<256><<<grid_blocks(m), 256, 0, c.stream>>>(g.rp, g.col, W, g.vw, L + st[CL_BIG], m,
-                                                                       part, vol, cons, lab, lam, ratio, dest, gain);
+                                                                       part, vol, cons, lab, lam, ratio, out);
         } else {
             // LDS tables sized for the class, so the many low-degree rows keep
             // more waves resident per CU; threads per vertex and slots per
             // edge are knobs
-            launch_table_class<128>(c, g, W, L, st[5], st[6], part, vol, cons, lam, ratio, dest, gain);
-            launch_table_class<256>(c, g, W, L, st[6], st[7], part, vol, cons, lam, ratio, dest, gain);
-            launch_table_class<512>(c, g, W, L, st[7], st[8], part, vol, cons, lam, ratio, dest, gain);
+            launch_table_class<128>(c, g, W, L, st[5], st[6], part, vol, cons, lam, ratio, out);
+            launch_table_class<256>(c, g, W, L, st[6], st[7], part, vol, cons, lam, ratio, out);
+            launch_table_class<512>(c, g, W, L, st[7], st[8], part, vol, cons, lam, ratio, out);
             if (c.table_spe == 2) {
-                launch_table<256, 2048, 2>(c, g, W, L, st[8], st[9], part, vol, cons, lam, ratio, dest, gain);
-                launch_table<512, 4096, 2>(c, g, W, L, st[9], st[10], part, vol, cons, lam, ratio, dest, gain);
+                launch_table<256, 2048, 2>(c, g, W, L, st[8], st[9], part, vol, cons, lam, ratio, out);
+                launch_table<512, 4096, 2>(c, g, W, L, st[9], st[10], part, vol, cons, lam, ratio, out);
             } else {
-                launch_table<256, 4096, 4>(c, g, W, L, st[8], st[9], part, vol, cons, lam, ratio, dest, gain);
-                launch_table<512, 8192, 4>(c, g, W, L, st[9], st[10], part, vol, cons, lam, ratio, dest, gain);
+                launch_table<256, 4096, 4>(c, g, W, L, st[8], st[9], part, vol, cons, lam, ratio, out);
+                launch_table<512, 8192, 4>(c, g, W, L, st[9], st[10], part, vol, cons, lam, ratio, out);
             }
             // hubs of degree <= hub_lds_max: 8192 LDS slots (96 KB of LDS)
-            launch_table<512, 8192, 2>(c, g, W, L, st[CL_HUB], lp.hub0, part, vol, cons, lam, ratio, dest, gain);
+            launch_table<512, 8192, 2>(c, g, W, L, st[CL_HUB], lp.hub0, part, vol, cons, lam, ratio, out);
         }
         c.kt_end(tk, 0.0);
         if (tk >= 0) acct_add(c, c.kt_counter(tk), acct.p + 1);
@@ -1316,7 +1337,7 @@ static void score_all(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, co
                 }
             }
             k_hub_decide<<<grid_items(m, 256), 256, 0, c.stream>>>(hubs, m, part, g.vw, vol, lam, ratio, lp.hub_pv,
-                                                                       lp.hub_best, dest, gain);
+                                                                       lp.hub_best, out);
             c.kt_end(tk, 0.0);
             if (tk >= 0) acct_add(c, c.kt_counter(tk), acct.p + 2);
         }
@@ -1365,106 +1386,158 @@ static i64 gather_candidates(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph
 // ------------------------------------------------------------- afterburner
 // afterburner_filter (src/local_mover.cpp:374-433): the change in the
 // candidate's gain if every neighbour with a larger gain (ties broken by the
-// xorshift hash) also makes its move
-template <class WT, class PT>
-__device__ __forceinline__ void ab_term(const i32* col, WT W, const AbInfo* info, i64 j, i32 p, i32 best,
-                                        float multi, float igain, i32 hi, PT prio, float& acc) {
-    const i32 v = col[j];
-    const AbInfo q4 = info[v];
+// xorshift hash) also makes its move.  An edge gives two FP32 terms, added in
+// this order: what the neighbour's destination means for the candidate's own
+// and best cluster, then what its leaving its cluster means.  (At most one
+// comparison of each pair holds, as the best cluster is never the own one;
+// an edge without effect adds zeros.)
+struct AbSelf {
+    i32 p, best, hi;
+    float multi, igain;
+};
+template <class LT, class PT>
+__device__ __forceinline__ AbSelf ab_self(const AbInfo* info, i32 i, LT lam, PT prio) {
+    const AbInfo me = info[i];
+    return AbSelf{me.part, me.dest, prio(i), me.vwf * lam(i), me.gain};
+}
+template <class PT>
+__device__ __forceinline__ float2 ab_terms(const AbInfo& q4, i32 v, i64 w, const AbSelf& m, PT prio) {
+    float2 t = make_float2(0.0f, 0.0f);
     const float vg = q4.gain;
-    if ((vg - igain) >= AFTERBURNER_EPS || (fabsf(vg - igain) < AFTERBURNER_EPS && prio(v) < hi)) {
-        i32 vpart = q4.dest;
-        const float q = fmaf(-multi, q4.vwf, (float)W(j));
-        acc = acc - ((vpart == p) ? q : 0.0f);
-        acc = acc + ((vpart == best && best != NEW_PART) ? q : 0.0f);
-        vpart = q4.part;
-        acc = acc + ((vpart == p) ? q : 0.0f);
-        acc = acc - ((vpart == best) ? q : 0.0f);
+    if ((vg - m.igain) >= AFTERBURNER_EPS || (fabsf(vg - m.igain) < AFTERBURNER_EPS && prio(v) < m.hi)) {
+        const float q = fmaf(-m.multi, q4.vwf, (float)w);
+        t.x = q4.dest == m.p ? -q : ((q4.dest == m.best && m.best != NEW_PART) ? q : 0.0f);
+        t.y = q4.part == m.p ? q : (q4.part == m.best ? -q : 0.0f);
+    }
+    return t;
+}
+
+// Degree below LARGE_CUTOFF: the terms are added in adjacency order.  The
+// gathers of the neighbours' records bound it, so AB_G lanes gather a
+// candidate's edges (AB_U in flight per lane) and leave the terms in LDS, and
+// one lane adds them in order.  With one thread per candidate, which also
+// gathered in order, a sweep of R-MAT scale 20 took 137 us here on the top
+// level (unit weights), now 53 us; on scale 24 1804 -> 1007 us.  16 lanes: most
+// candidates have at most a few dozen edges.
+constexpr int AB_G = 16, AB_U = 4, AB_PB = 256 / AB_G;
+template <class WT, class LT, class PT>
+__global__ void __launch_bounds__(256) k_ab_small(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
+                                                  const AbInfo* __restrict__ info, const i32* __restrict__ cand,
+                                                  i64 k, LT lam, PT prio, i32* __restrict__ keep) {
+    __shared__ float2 term[AB_PB][LARGE_CUTOFF + 1];
+    const int lane = threadIdx.x & (AB_G - 1), grp = threadIdx.x / AB_G;
+    const i64 x = block_id() * AB_PB + grp;
+    int d = 0;
+    float igain = 0.0f;
+    if (x < k) {
+        const i32 i = cand[x];
+        const AbSelf m = ab_self(info, i, lam, prio);
+        igain = m.igain;
+        const i64 s = rp[i];
+        d = (int)(rp[i + 1] - s);
+        for (int jb = lane; jb < d; jb += AB_G * AB_U) {
+            i32 v[AB_U];
+            AbInfo q[AB_U];
+#pragma unroll
+            for (int u = 0; u < AB_U; u++) v[u] = jb + u * AB_G < d ? col[s + jb + u * AB_G] : -1;
+#pragma unroll
+            for (int u = 0; u < AB_U; u++)
+                if (v[u] >= 0) q[u] = info[v[u]];
+#pragma unroll
+            for (int u = 0; u < AB_U; u++)
+                if (v[u] >= 0) term[grp][jb + u * AB_G] = ab_terms(q[u], v[u], W(s + jb + u * AB_G), m, prio);
+        }
+    }
+    __syncthreads();
+    if (lane == 0 && x < k) {
+        float acc = 0.0f;
+#pragma unroll 8
+        for (int e = 0; e < d; e++) {
+            const float2 t = term[grp][e];
+            acc = acc + t.x;
+            acc = acc + t.y;
+        }
+        keep[x] = (igain + acc >= 0.0f) ? 1 : 0;
     }
 }
 
-template <class WT, class LT, class PT>
-__global__ void __launch_bounds__(256) k_ab_serial(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
-                                                   const AbInfo* __restrict__ info, const i32* __restrict__ cand,
-                                                   i64 k, LT lam, PT prio, i32* keep) {
-    const i64 x = thread_item();
-    if (x >= k) return;
-    const i32 i = cand[x];
-    const AbInfo me = info[i];
-    const i32 best = me.dest, p = me.part;
-    const float multi = me.vwf * lam(i);
-    const float igain = me.gain;
-    const i32 hi = prio(i);
-    float acc = 0.0f;
-    const i64 e = rp[i + 1];
-#pragma unroll 4  // independent neighbour gathers in flight; the adds keep their order
-    for (i64 j = rp[i]; j < e; j++) ab_term(col, W, info, j, p, best, multi, igain, hi, prio, acc);
-    keep[x] = (igain + acc >= 0.0f) ? 1 : 0;  // an unconditional store
-}
-
+// One wave per candidate: 64 strided partials and a halving tree.
 template <class WT, class LT, class PT>
 __global__ void __launch_bounds__(256) k_ab_wave(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
                                                  const AbInfo* __restrict__ info, const i32* __restrict__ cand, i64 k0,
-                                                 i64 k1, LT lam, PT prio, i32* keep) {
+                                                 i64 k1, LT lam, PT prio, i32* __restrict__ keep) {
     const int lane = threadIdx.x & 63;
     const i64 x = k0 + block_id() * 4 + (threadIdx.x >> 6);
     if (x >= k1) return;
-    {
-        const i32 i = cand[x];
-        const AbInfo me = info[i];
-        const i32 best = me.dest, p = me.part;
-        const float multi = me.vwf * lam(i);
-        const float igain = me.gain;
-        const i32 hi = prio(i);
-        float acc = 0.0f;
-        const i64 e = rp[i + 1];
-#pragma unroll 4
-        for (i64 base = rp[i]; base < e; base += 64) {  // wave-uniform loop control
-            const i64 j = base + lane;
-            if (j < e) ab_term(col, W, info, j, p, best, multi, igain, hi, prio, acc);
-        }
-        xlane_fence(acc);
+    const i32 i = cand[x];
+    const AbSelf m = ab_self(info, i, lam, prio);
+    float acc = 0.0f;
+    const i64 e = rp[i + 1];
+    constexpr int U = 4;
+    for (i64 base = rp[i]; base < e; base += 64 * U) {  // wave-uniform loop control
+        i32 v[U];
+        AbInfo q[U];
 #pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) acc = acc + __shfl_down(acc, off);
-        if (lane == 0) keep[x] = (igain + acc >= 0.0f) ? 1 : 0;
+        for (int u = 0; u < U; u++) v[u] = base + u * 64 + lane < e ? col[base + u * 64 + lane] : -1;
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (v[u] >= 0) q[u] = info[v[u]];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (v[u] < 0) continue;
+            const float2 t = ab_terms(q[u], v[u], W(base + u * 64 + lane), m, prio);
+            acc = acc + t.x;
+            acc = acc + t.y;
+        }
     }
+    xlane_fence(acc);
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) acc = acc + __shfl_down(acc, off);
+    if (lane == 0) keep[x] = (m.igain + acc >= 0.0f) ? 1 : 0;
 }
 
+// A 1024-thread block per candidate: 1024 strided partials and a halving tree.
 template <class WT, class LT, class PT>
 __global__ void __launch_bounds__(1024) k_ab_block(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
                                                    const AbInfo* __restrict__ info, const i32* __restrict__ cand,
-                                                   i64 k0, i64 k1, LT lam, PT prio, i32* keep) {
+                                                   i64 k0, i64 k1, LT lam, PT prio, i32* __restrict__ keep) {
     __shared__ float sh[1024];
     const int t = threadIdx.x;
     const i64 x = k0 + block_id();
     if (x >= k1) return;
-    {
-        const i32 i = cand[x];
-        const AbInfo me = info[i];
-        const i32 best = me.dest, p = me.part;
-        const float multi = me.vwf * lam(i);
-        const float igain = me.gain;
-        const i32 hi = prio(i);
-        float acc = 0.0f;
-        const i64 e = rp[i + 1];
-        for (i64 base = rp[i]; base < e; base += 1024) {  // block-uniform loop control
-            const i64 j = base + t;
-            if (j < e) ab_term(col, W, info, j, p, best, multi, igain, hi, prio, acc);
-        }
-        sh[t] = acc;
-        __syncthreads();
-        for (int off = 512; off >= 64; off >>= 1) {
-            if (t < off) sh[t] = sh[t] + sh[t + off];
-            __syncthreads();
-        }
-        if (t < 64) {
-            acc = sh[t];
-            xlane_fence(acc);
+    const i32 i = cand[x];
+    const AbSelf m = ab_self(info, i, lam, prio);
+    float acc = 0.0f;
+    const i64 e = rp[i + 1];
+    constexpr int U = 4;
+    for (i64 base = rp[i]; base < e; base += 1024 * U) {  // block-uniform loop control
+        i32 v[U];
+        AbInfo q[U];
 #pragma unroll
-            for (int off = 32; off >= 1; off >>= 1) acc = acc + __shfl_down(acc, off);
-            if (t == 0) keep[x] = (igain + acc >= 0.0f) ? 1 : 0;
+        for (int u = 0; u < U; u++) v[u] = base + u * 1024 + t < e ? col[base + u * 1024 + t] : -1;
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (v[u] >= 0) q[u] = info[v[u]];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (v[u] < 0) continue;
+            const float2 tt = ab_terms(q[u], v[u], W(base + u * 1024 + t), m, prio);
+            acc = acc + tt.x;
+            acc = acc + tt.y;
         }
+    }
+    sh[t] = acc;
+    __syncthreads();
+    for (int off = 512; off >= 64; off >>= 1) {
+        if (t < off) sh[t] = sh[t] + sh[t + off];
         __syncthreads();
+    }
+    if (t < 64) {
+        acc = sh[t];
+        xlane_fence(acc);
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) acc = acc + __shfl_down(acc, off);
+        if (t == 0) keep[x] = (m.igain + acc >= 0.0f) ? 1 : 0;
     }
 }
 
@@ -1483,14 +1556,16 @@ __global__ void __launch_bounds__(256) k_ab_pack(i64 n, const float* __restrict_
 
 template <class LT, class PT>
 static i64 afterburner(Ctx& c, MoveScratch& s, const DGraph& g, const i32* cand, i64 k, const i64* b, LT lam, PT prio,
-                       i32* moves) {
+                       i32* moves, bool pack) {
     const int tk = c.kt_begin(KS_AFTERBURNER);
-    k_ab_pack<<<grid_items(g.n, 256), 256, 0, c.stream>>>(g.n, s.gain, s.dest, s.part, g.vw, s.abi);
-    PGGC_LAUNCH_CHECK();
+    if (pack) {
+        k_ab_pack<<<grid_items(g.n, 256), 256, 0, c.stream>>>(g.n, s.gain, s.dest, s.part, g.vw, s.abi);
+        PGGC_LAUNCH_CHECK();
+    }
     PGGC_WDISPATCH(g, {
         if (b[0] > 0)
-            k_ab_serial<<<grid_items(b[0], 256), 256, 0, c.stream>>>(g.rp, g.col, W, s.abi, cand, b[0], lam, prio,
-                                                                     s.flag);
+            k_ab_small<<<grid_items(b[0], AB_PB), 256, 0, c.stream>>>(g.rp, g.col, W, s.abi, cand, b[0], lam, prio,
+                                                                      s.flag);
         if (b[1] > b[0])
             k_ab_wave<<<grid_items(b[1] - b[0], 4), 256, 0, c.stream>>>(g.rp, g.col, W, s.abi, cand, b[0], b[1], lam,
                                                                         prio, s.flag);
@@ -1501,14 +1576,13 @@ static i64 afterburner(Ctx& c, MoveScratch& s, const DGraph& g, const i32* cand,
     c.kt_end(tk, 0.0);
     PGGC_LAUNCH_CHECK();
     if (tk >= 0) {  // timing runs only: count the bytes outside the timed region
-        // the pack reads gain, dest, part and vertex weight and writes a
-        // 16-byte record per vertex; the filter reads per candidate edge the
-        // column, weight and the neighbour's record, per candidate its id, row
-        // bounds and keep flag
+        // per candidate edge the column, weight and the neighbour's record,
+        // per candidate its id, record, row bounds and keep flag; a pack reads
+        // gain, dest, part and vertex weight and writes a record per vertex
         Buf<i64> acc(c, 1);
         fill_i64(c, acc, 1, 0);
         k_list_bytes<<<grid_items(std::max<i64>(k, 1), 256), 256, 0, c.stream>>>(
-            g.rp, cand, k, 24, 20 + (g.wk == W_UNIT ? 0 : g.wk == W_I32 ? 4 : 8), 36 * g.n, acc);
+            g.rp, cand, k, 40, 20 + (g.wk == W_UNIT ? 0 : g.wk == W_I32 ? 4 : 8), pack ? 36 * g.n : 0, acc);
         PGGC_LAUNCH_CHECK();
         acct_add(c, c.kt_counter(tk), acc);
     }
@@ -2056,6 +2130,9 @@ static void local_move_t(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g,
     // active set is mostly the movers' neighbourhood and little is to gain)
     Gnn* G = (s.gnn && s.gnn->cfg.mode != GNN_OFF && g.nnz >= s.gnn->cfg.min_nnz) ? s.gnn : nullptr;
     const bool train = G && G->cfg.mode == GNN_TRAIN;
+    // pruned vertices are not scored, so with the predictor on the records
+    // are packed from the arrays
+    const ScoreOut so = G ? ScoreOut{s.dest, s.gain, nullptr} : ScoreOut{s.dest, nullptr, s.abi};
     if (G) gnn_begin(c, *G, n, train);
     i64 kprev = n;
     i64 npred = 0;  // predicted sweeps in this call
@@ -2074,16 +2151,16 @@ static void local_move_t(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g,
                 npred++;
             }
             tr.begin(s.dest, iter == 1 && !use);
-            score_all(c, s, lp, g, s.part, curr.vol, ccons, tables ? 0 : raw_mode, lam, fr, s.dest, s.gain);
+            score_all(c, s, lp, g, s.part, curr.vol, ccons, tables ? 0 : raw_mode, lam, fr, so);
             i64 b[2];
             i64 k = gather_candidates(c, s, lp, g, s.dest, s.cand, b);
-            i64 km = k > 0 ? afterburner(c, s, g, s.cand, k, b, lam, prio, s.moves) : 0;
+            i64 km = k > 0 ? afterburner(c, s, g, s.cand, k, b, lam, prio, s.moves, so.info == nullptr) : 0;
             if (km == 0 && G && gnn_restore(c, *G, n, s.dest)) {
                 // nothing to move among the vertices let through: score the
                 // pruned ones too, so the call ends as the plain method does
-                score_all(c, s, lp, g, s.part, curr.vol, ccons, tables ? 0 : raw_mode, lam, fr, s.dest, s.gain);
+                score_all(c, s, lp, g, s.part, curr.vol, ccons, tables ? 0 : raw_mode, lam, fr, so);
                 k = gather_candidates(c, s, lp, g, s.dest, s.cand, b);
-                km = k > 0 ? afterburner(c, s, g, s.cand, k, b, lam, prio, s.moves) : 0;
+                km = k > 0 ? afterburner(c, s, g, s.cand, k, b, lam, prio, s.moves, so.info == nullptr) : 0;
             }
             if (stats) {
                 stats->sweeps++;
@@ -2201,7 +2278,8 @@ void local_move_strict(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, i
     for (int it = 0; it < 6; it++) {
         const float lam = (float)curr.lambda;
         trc.begin(s.dest, true);
-        score_all(c, s, lp, g, s.part, curr.vol, ccons, !tables && c.raw_sweeps, LamOne{lam}, 0.0f, s.dest, s.gain);
+        score_all(c, s, lp, g, s.part, curr.vol, ccons, !tables && c.raw_sweeps, LamOne{lam}, 0.0f,
+                  ScoreOut{s.dest, s.gain, nullptr});
         i64 b[2];
         i64 k = gather_candidates(c, s, lp, g, s.dest, s.moves, b);
         if (stats) {
@@ -2252,13 +2330,14 @@ i64 sweep_once(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, const i32
     copy_dev(c, s.dest, dest, n * sizeof(i32));
     copy_dev(c, s.gain, gain, n * sizeof(float));
     const float lam = (float)lambda;
-    score_all(c, s, lp, g, s.part, vol, cons, raw, LamOne{lam}, ratio, s.dest, s.gain);
+    score_all(c, s, lp, g, s.part, vol, cons, raw, LamOne{lam}, ratio,
+              ScoreOut{s.dest, s.gain, nullptr});
     i64 b[2];
     i64 k = gather_candidates(c, s, lp, g, s.dest, s.cand, b);
     *ncand = k;
     i64 km = 0;
     if (k > 0) {
-        km = afterburner(c, s, g, s.cand, k, b, LamOne{lam}, PrioOne{}, moves_out);
+        km = afterburner(c, s, g, s.cand, k, b, LamOne{lam}, PrioOne{}, moves_out, true);
     }
     copy_dev(c, dest, s.dest, n * sizeof(i32));
     copy_dev(c, gain, s.gain, n * sizeof(float));
@@ -2590,12 +2669,12 @@ void local_move_batch(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, co
         }
         // table scoring throughout: on a singleton clustering it gives what
         // the raw first sweep gives (every neighbour its own cluster)
-        score_all(c, s, lp, g, s.part, cvol, nullptr, false, lam, 0.0f, s.dest, s.gain);
+        score_all(c, s, lp, g, s.part, cvol, nullptr, false, lam, 0.0f, ScoreOut{s.dest, nullptr, s.abi});
         i64 b[2];
         const i64 kc = gather_candidates(c, s, lp, g, s.dest, s.cand, b);
         i64 km = 0;
         if (kc > 0) {
-            km = afterburner(c, s, g, s.cand, kc, b, lam, prio, s.moves);
+            km = afterburner(c, s, g, s.cand, kc, b, lam, prio, s.moves, false);
         }
         fill_i64(c, cnt2, 2 * K, 0);
         if (kc > 0) k_inst_count<<<grid_items(kc, 256), 256, 0, c.stream>>>(s.cand, kc, bl.inst, cnt2);
