@@ -72,6 +72,7 @@ struct DGraph {
     const void* w = nullptr;   // weights [nnz] (null when W_UNIT)
     int wk = W_UNIT;
     const i64* vw = nullptr;   // vertex weights [n]
+    bool wsmall = false;       // all weights together are known to sum to less than 2^32
 };
 
 #define PGGC_WDISPATCH(G, ...)                               \

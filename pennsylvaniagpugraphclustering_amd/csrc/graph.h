@@ -13,6 +13,7 @@ struct OwnedGraph {
     Buf<i32> w32;  // the same weights in 32 bits when every one fits (narrow_weights)
     Buf<i64> vw;
     i64 n = 0, nnz = 0;
+    bool wsmall = false;  // DGraph::wsmall
     DGraph view() const {
         DGraph g;
         g.n = n;
@@ -27,6 +28,7 @@ struct OwnedGraph {
             g.wk = W_I64;
         }
         g.vw = vw.p;
+        g.wsmall = wsmall;
         return g;
     }
 };
@@ -59,6 +61,9 @@ void contract(Ctx& c, const DGraph& g, const i32* vcmap, i64 nc, OwnedGraph& out
 // sweeps read 4 instead of 8 weight bytes per edge and the level holds 8
 // instead of 12 bytes per nonzero.
 void narrow_weights(Ctx& c, const DGraph& fine, OwnedGraph& g);
+
+// largest weight of g as an unsigned value (a negative weight is huge); g.nnz > 0
+u64 max_weight(Ctx& c, const DGraph& g);
 
 // next.vw[map[i]] += g.vw[i]  (src/clustering_methods.cpp:33-38)
 void coarsen_vertex_weights(Ctx& c, const DGraph& g, const i32* map, i64 nc, i64* out);

@@ -687,12 +687,13 @@ static int bits_for(i64 v) {
     return b;
 }
 
-__global__ void __launch_bounds__(256) k_max_i64(const i64* __restrict__ in, i64 n, u64* out) {
+template <class T>
+__global__ void __launch_bounds__(256) k_max(const T* __restrict__ in, i64 n, u64* out) {
     u64 m = 0;
     // block-uniform loop control (the reduction below is cross-lane)
     for (i64 base = (i64)blockIdx.x * blockDim.x; base < n; base += (i64)gridDim.x * blockDim.x) {
         const i64 x = base + threadIdx.x;
-        if (x < n) m = (u64)in[x] > m ? (u64)in[x] : m;  // weights are positive
+        if (x < n) m = (u64)in[x] > m ? (u64)in[x] : m;
     }
     m = block_max_u64<256>(m);
     if (threadIdx.x == 0 && m) atomicMax((unsigned long long*)out, (unsigned long long)m);
@@ -702,15 +703,22 @@ __global__ void k_narrow(const i64* __restrict__ in, i64 n, i32* __restrict__ ou
         out[x] = (i32)in[x];
 }
 
+u64 max_weight(Ctx& c, const DGraph& g) {
+    if (g.wk == W_UNIT) return 1;
+    Buf<u64> mx(c, 1);
+    fill_i64(c, (i64*)mx.p, 1, 0);
+    const int grid = grid_for(g.nnz, 256 * 8, 8192);
+    if (g.wk == W_I32) k_max<i32><<<grid, 256, 0, c.stream>>>((const i32*)g.w, g.nnz, mx);
+    else k_max<i64><<<grid, 256, 0, c.stream>>>((const i64*)g.w, g.nnz, mx);
+    PGGC_LAUNCH_CHECK();
+    return (u64)c.read1((const i64*)mx.p);
+}
+
 void narrow_weights(Ctx& c, const DGraph& fine, OwnedGraph& g) {
     if (g.nnz == 0 || !g.w.p) return;
     bool fits = fine.wk == W_UNIT && fine.nnz < ((i64)1 << 31);
     if (!fits) {
-        Buf<u64> mx(c, 1);
-        fill_i64(c, (i64*)mx.p, 1, 0);
-        k_max_i64<<<grid_for(g.nnz, 256 * 8, 8192), 256, 0, c.stream>>>(g.w, g.nnz, mx);
-        PGGC_LAUNCH_CHECK();
-        fits = (u64)c.read1((const i64*)mx.p) <= 0x7fffffffull;
+        fits = max_weight(c, g.view()) <= 0x7fffffffull;
     }
     if (!fits) return;
     g.w32 = Buf<i32>(c, g.nnz);
@@ -823,6 +831,8 @@ void contract(Ctx& c, const DGraph& g, const i32* vcmap, i64 nc, OwnedGraph& out
         contract_bytes(c, tk, big, n2, mstart, bound, ccnt, wb);
     }
     out.n = nc;
+    // (a coarse graph's weights sum to at most the finer level's)
+    out.wsmall = g.wsmall || (g.wk == W_UNIT && g.nnz < ((i64)1 << 32));
     out.rp = Buf<i64>(c, nc + 1);
     scan_i64(c, ccnt, out.rp, nc);
     out.nnz = c.read1(out.rp.p + nc);

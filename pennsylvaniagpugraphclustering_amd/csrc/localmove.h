@@ -84,6 +84,7 @@ struct LevelPlan {
     // tables; he / hs: edges per build item and slots per scan item
     u64 epoch = ~(u64)0;
     i64 nlds = 0, hub0 = 0, nhub = 0;
+    bool agg32 = false;  // sums of rows of degree <= 4096 fit 32 bits
     i64 max_deg = 0;  // of the hub class (0 without hubs)
     i64 he = 1024, hs = 4096;
 };
@@ -106,6 +107,8 @@ struct MoveScratch {
     Gnn* gnn = nullptr;  // active-set predictor (null or mode off: plain sweeps)
     Buf<AbInfo> abi;
     Buf<u64> mvp;  // per vertex: cluster | moved << 31, and the cluster after this sweep's moves
+    Buf<u64> rec;     // per vertex: cluster and its volume as fp32 (scoring)
+    Buf<uint4> rec16; // the same with the cluster's constraint value, when there is one
     Buf<u64> sqpart;  // partial sums of k_finish
     Buf<i32> part, dest, cand, moves, flag, tmp, tmp2;
     Buf<float> gain;

@@ -13,6 +13,7 @@
 #include <cfloat>
 #include <cstdio>
 #include <chrono>
+#include <type_traits>
 
 #include "device.h"
 #include "gnn.h"
@@ -55,6 +56,8 @@ void MoveScratch::ensure(Ctx& c, i64 n) {
     gain = Buf<float>(c, cap);
     abi = Buf<AbInfo>(c, cap);
     mvp = Buf<u64>(c, cap);
+    rec = Buf<u64>(c, cap);
+    rec16.reset();
     prio = Buf<i64>(c, cap + 1);
     scal = Buf<i64>(c, SC_COUNT);
     sqpart = Buf<u64>(c, 2 * FIN_BLOCKS);
@@ -65,6 +68,10 @@ __host__ __device__ __forceinline__ int score_class(i64 d) {
     return d <= 4 ? 0 : d <= 8 ? 1 : d <= 16 ? 2 : d <= 32 ? 3 : d <= 64 ? 4 : d <= 128 ? 5 : d <= 256 ? 6
          : d <= 512 ? 7 : d <= 1024 ? 8 : d <= 2048 ? 9 : 10;
 }
+// Level of at most this many rows in the LDS-table classes: one launch for all
+// (the chip holds 5 of its 256-thread blocks per CU, 1,280 at once, so two
+// rounds of blocks cost less than the four launches saved).
+constexpr i64 TABLE_ONE_LAUNCH = 2048;
 // LDS table of a vertex of degree d: the power of two >= spe * d slots
 __host__ __device__ __forceinline__ i64 tslots(i64 d, int spe) {
     i64 s = 2;
@@ -263,6 +270,14 @@ void plan_level(Ctx& c, const DGraph& g, LevelPlan& p) {
         PGGC_LAUNCH_CHECK();
         p.nlds = c.read1(f);
     }
+    // 32-bit sums for the rows scored in registers and LDS (degree at most
+    // HUB_LDS_BOUND): unit weights, a level whose weights sum to less than
+    // 2^32 (contracted from a unit-weight graph), or small weights
+    p.agg32 = g.wk == W_UNIT || g.wsmall;
+    if (!p.agg32 && g.nnz > 0) {
+        const u64 mx = max_weight(c, g);
+        p.agg32 = mx <= 0xffffffffull / HUB_LDS_BOUND;
+    }
     p.hub0 = p.sc_start[CL_HUB] + p.nlds;
     p.nhub = nh - p.nlds;
     const i64 m7 = p.nhub;
@@ -432,162 +447,343 @@ __device__ __forceinline__ void own_terms(i64 pv, i64 volp, i64 wv, float lam, f
     if (p_conn < 0.0f) b = 0.0f;
 }
 
-// G lanes per vertex, one edge per lane (degree <= G): duplicate clusters
-// are merged with in-group shuffles.
-template <int G, class WT, class LT>
-__global__ void __launch_bounds__(256) k_score_group(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
-                                                     const i64* __restrict__ vw, const i32* __restrict__ list, i64 m,
-                                                     const i32* __restrict__ part, const i64* __restrict__ vol,
-                                                     const i32* __restrict__ cons, int raw, LT lam, float ratio,
-                                                     ScoreOut out) {
-    constexpr int GPB = 256 / G;
-    const int gl = threadIdx.x & (G - 1);
-    const i64 gi = block_id() * GPB + threadIdx.x / G;
-    if (gi >= m) return;
-    {
-        const i32 i = list[gi];
-        if (out.dest[i] == NO_MOVE) return;
-        const i64 s = rp[i];
-        const int d = (int)(rp[i + 1] - s);
-        const i32 p = part[i];
-        const i64 wv = vw[i];
-        i32 key = -5;
-        i64 wt = 0;
-        const bool has = gl < d;
-        if (has) {
-            i32 v = col[s + gl];
-            key = raw == 1 ? v : part[v];
-            wt = W(s + gl);
-        }
-        i64 agg = wt;
-        bool own = false;
-        i64 pv = 0;
-        if (!raw) {  // raw rows have distinct columns and no own-cluster edge
-            agg = 0;
-            xlane_fence(key);
-            xlane_fence(wt);
-#pragma unroll
-            for (int k = 0; k < G; k++) {
-                i32 kk = __shfl(key, k, G);
-                i64 ww = __shfl(wt, k, G);
-                agg += (kk == key) ? ww : 0;
-            }
-            own = has && key == p;
-            pv = group_max_i64<G>(own ? agg : (i64)0);
-        }
-        float multi, p_conn, b;
-        own_terms(pv, vol[p], wv, lam(i), lam.rt(i, ratio), multi, p_conn, b);
-        u64 bk = 0;
-        if (has && !own && agg > 0 && (float)agg >= b && (cons == nullptr || cons[key] == cons[p])) {
-            float jc = fmaf(-(float)vol[key], multi, (float)agg);
-            if (jc >= b) bk = pack_cand(jc, key);
-        }
-        bk = group_max_u64<G>(bk);
-        if (gl == 0) decide(i, p_conn, bk, p, wv, out);
+// What scoring reads of a neighbour, packed per vertex once per sweep
+// (k_rec_pack): its cluster and that cluster's volume as the fp32 value the
+// gain arithmetic uses, in 8 bytes; with a constraint also the cluster's
+// constraint value, in 16.  The gathers at random neighbour ids bound the
+// scoring kernels, so an edge costs one of them instead of one for the cluster
+// and another, at a random label, for each distinct cluster's volume (and a
+// third for its constraint).
+struct RecView {
+    const u64* r8;
+    const uint4* r16;  // set (instead of r8) when there is a constraint
+};
+struct NbRec {
+    i32 part;
+    float volf;
+    i32 cons;
+};
+__device__ __forceinline__ NbRec load_rec(const RecView& rv, i32 v) {
+    NbRec r;
+    if (rv.r16) {  // kernel-uniform
+        const uint4 q = rv.r16[v];
+        r.part = (i32)q.x;
+        r.volf = __uint_as_float(q.y);
+        r.cons = (i32)q.z;
+    } else {
+        const u64 q = rv.r8[v];
+        r.part = (i32)(u32)q;
+        r.volf = __uint_as_float((u32)(q >> 32));
+        r.cons = 0;
+    }
+    return r;
+}
+__global__ void __launch_bounds__(256) k_rec_pack(i64 n, const i32* __restrict__ part, const i64* __restrict__ vol,
+                                                  const i32* __restrict__ cons, u64* __restrict__ r8,
+                                                  uint4* __restrict__ r16) {
+    const i64 i = thread_item();
+    if (i >= n) return;
+    const i32 p = part[i];
+    const u32 vf = __float_as_uint((float)vol[p]);
+    if (r16) {
+        r16[i] = make_uint4((u32)p, vf, (u32)cons[p], 0u);
+    } else {
+        r8[i] = (u64)(u32)p | ((u64)vf << 32);
     }
 }
 
-// One block per vertex with a hash table in LDS (or HBM for the largest
-// degrees): SLOTS slots of LDS hold the table of any degree up to
-// SLOTS / SPE, each table the power of two >= SPE * degree.
-template <int BS, int SLOTS, int SPE, bool GLOBAL, class WT, class LT>
+// Lane exchange inside groups of G consecutive lanes.  DPP moves cover 16
+// lanes (quad permutes, half-row and row mirrors, row rotations); shuffles
+// reach the other 16-lane rows.
+template <int CTRL>
+__device__ __forceinline__ i32 dpp(i32 v) {
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
+}
+template <int CTRL>
+__device__ __forceinline__ u32 dpp(u32 v) {
+    return (u32)dpp<CTRL>((i32)v);
+}
+template <int CTRL>
+__device__ __forceinline__ i64 dpp(i64 v) {
+    const u32 lo = dpp<CTRL>((u32)(u64)v), hi = dpp<CTRL>((u32)((u64)v >> 32));
+    return (i64)(((u64)hi << 32) | lo);
+}
+template <int CTRL>
+__device__ __forceinline__ u64 dpp(u64 v) {
+    return (u64)dpp<CTRL>((i64)v);
+}
+constexpr int DPP_X1 = 0xB1, DPP_X2 = 0x4E, DPP_X3 = 0x1B, DPP_HMIRROR = 0x141, DPP_MIRROR = 0x140;
+
+// reduction over the group with `op` (commutative); every lane gets the result
+template <int G, class T, class Op>
+__device__ __forceinline__ T group_reduce(T v, Op op) {
+    xlane_fence(v);
+    v = op(v, dpp<DPP_X1>(v));
+    v = op(v, dpp<DPP_X2>(v));
+    if (G >= 8) v = op(v, dpp<DPP_HMIRROR>(v));
+    if (G >= 16) v = op(v, dpp<DPP_MIRROR>(v));
+    if (G >= 32) v = op(v, (T)__shfl_xor(v, 16));
+    if (G >= 64) v = op(v, (T)__shfl_xor(v, 32));
+    return v;
+}
+template <int G, class T>
+__device__ __forceinline__ T group_max(T v) {
+    return group_reduce<G>(v, [](T a, T b) { return a > b ? a : b; });
+}
+template <int G, class T>
+__device__ __forceinline__ T group_add(T v) {
+    return group_reduce<G>(v, [](T a, T b) { return a + b; });
+}
+// over the block; every thread gets the result
+template <int BS, class T, class Op>
+__device__ __forceinline__ T block_reduce(T v, Op op) {
+    v = group_reduce<64>(v, op);
+    if (BS > 64) {
+        __shared__ T sh[BS / 64];
+        if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+        __syncthreads();
+        v = sh[0];
+#pragma unroll
+        for (int w = 1; w < BS / 64; w++) v = op(v, sh[w]);
+        __syncthreads();
+    }
+    return v;
+}
+
+// agg += w of the lanes of the 16-lane row (or 4 / 8 lane group) whose key
+// equals `key`, given this lane's partner values (kk, ww) of one offset
+template <bool UNIT, class AT>
+__device__ __forceinline__ void merge_one(i32 kk, AT ww, i32 key, AT& agg) {
+    agg += kk == key ? (UNIT ? (AT)1 : ww) : (AT)0;
+}
+template <bool UNIT, class AT, int C>
+__device__ __forceinline__ void merge_dpp(i32 k, AT w, i32 key, AT& agg) {
+    merge_one<UNIT>(dpp<C>(k), UNIT ? (AT)0 : dpp<C>(w), key, agg);
+}
+// rotations 1..15 of a 16-lane row
+template <bool UNIT, class AT>
+__device__ __forceinline__ void merge_row(i32 k, AT w, i32 key, AT& agg) {
+    merge_dpp<UNIT, AT, 0x121>(k, w, key, agg);
+    merge_dpp<UNIT, AT, 0x122>(k, w, key, agg);
+    merge_dpp<UNIT, AT, 0x123>(k, w, key, agg);
+    merge_dpp<UNIT, AT, 0x124>(k, w, key, agg);
+    merge_dpp<UNIT, AT, 0x125>(k, w, key, agg);
+    merge_dpp<UNIT, AT, 0x126>(k, w, key, agg);
+    merge_dpp<UNIT, AT, 0x127>(k, w, key, agg);
+    merge_dpp<UNIT, AT, 0x128>(k, w, key, agg);
+    merge_dpp<UNIT, AT, 0x129>(k, w, key, agg);
+    merge_dpp<UNIT, AT, 0x12A>(k, w, key, agg);
+    merge_dpp<UNIT, AT, 0x12B>(k, w, key, agg);
+    merge_dpp<UNIT, AT, 0x12C>(k, w, key, agg);
+    merge_dpp<UNIT, AT, 0x12D>(k, w, key, agg);
+    merge_dpp<UNIT, AT, 0x12E>(k, w, key, agg);
+    merge_dpp<UNIT, AT, 0x12F>(k, w, key, agg);
+}
+// sum of the weights of the group's lanes that hold this lane's key
+template <int G, bool UNIT, class AT>
+__device__ __forceinline__ AT merge_group(i32 key, AT w) {
+    xlane_fence(key);
+    xlane_fence(w);
+    AT agg = w;
+    if (G == 4 || G == 8) {
+        merge_dpp<UNIT, AT, DPP_X1>(key, w, key, agg);
+        merge_dpp<UNIT, AT, DPP_X2>(key, w, key, agg);
+        merge_dpp<UNIT, AT, DPP_X3>(key, w, key, agg);
+        if (G == 8) {  // the mirrored half row is offset 7, its quad permutes 6, 5, 4
+            const i32 k7 = dpp<DPP_HMIRROR>(key);
+            const AT w7 = UNIT ? (AT)0 : dpp<DPP_HMIRROR>(w);
+            merge_one<UNIT>(k7, w7, key, agg);
+            merge_dpp<UNIT, AT, DPP_X1>(k7, w7, key, agg);
+            merge_dpp<UNIT, AT, DPP_X2>(k7, w7, key, agg);
+            merge_dpp<UNIT, AT, DPP_X3>(k7, w7, key, agg);
+        }
+        return agg;
+    }
+    merge_row<UNIT>(key, w, key, agg);
+#pragma unroll
+    for (int r = 16; r < G; r += 16) {  // the other rows of the group
+        const i32 kr = __shfl_xor(key, r);
+        const AT wr = UNIT ? (AT)0 : (AT)__shfl_xor(w, r);
+        merge_one<UNIT>(kr, wr, key, agg);
+        merge_row<UNIT>(kr, wr, key, agg);
+    }
+    return agg;
+}
+
+template <class WT>
+struct IsUnit {
+    static constexpr bool v = false;
+};
+template <>
+struct IsUnit<WUnit> {
+    static constexpr bool v = true;
+};
+
+// G lanes per vertex, one edge per lane (degree <= G): duplicate clusters are
+// merged in registers.  AT: u32 when every row sum of the level's small
+// degrees fits 32 bits (LevelPlan::agg32), else i64; the sums are the same
+// integers.  raw rows have distinct columns and no own-cluster edge.  Merging
+// by DPP moves in 32 bits instead of three shuffles per partner lane took the
+// five classes from 50.4 to 31.5 ms (R-MAT scale 24, two passes), 84 to 33 ms
+// on scale 20, where the 64-lane class was instruction bound.
+template <int G, class AT, class WT, class LT>
+__device__ __forceinline__ void score_group(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
+                                            const i64* __restrict__ vw, const i32* __restrict__ list, i64 x0, i64 x1,
+                                            i64 blk, const i32* __restrict__ part, const i64* __restrict__ vol,
+                                            const RecView& rv, const i32* __restrict__ cons, int raw, LT lam,
+                                            float ratio, const ScoreOut& out) {
+    const int gl = threadIdx.x & (G - 1);
+    const i64 gi = x0 + blk * (256 / G) + threadIdx.x / G;
+    if (gi >= x1) return;
+    const i32 i = list[gi];
+    if (out.dest[i] == NO_MOVE) return;
+    const i64 s = rp[i];
+    const int d = (int)(rp[i + 1] - s);
+    const i32 p = part[i];
+    const i64 wv = vw[i];
+    const i32 cp = cons ? cons[p] : 0;
+    NbRec r;
+    r.part = -5;
+    r.volf = 0.0f;
+    r.cons = 0;
+    AT wt = 0;
+    const bool has = gl < d;
+    if (has) {
+        r = load_rec(rv, col[s + gl]);
+        wt = (AT)W(s + gl);
+    }
+    const i32 key = r.part;
+    AT agg = wt;
+    bool own = false;
+    AT pv = 0;
+    if (!raw) {
+        agg = merge_group<G, IsUnit<WT>::v>(key, wt);
+        own = has && key == p;
+        pv = group_max<G>(own ? agg : (AT)0);
+    }
+    float multi, p_conn, b;
+    own_terms((i64)pv, vol[p], wv, lam(i), lam.rt(i, ratio), multi, p_conn, b);
+    u64 bk = 0;
+    if (has && !own && agg > 0 && (float)agg >= b && r.cons == cp) {
+        const float jc = fmaf(-r.volf, multi, (float)agg);
+        if (jc >= b) bk = pack_cand(jc, key);
+    }
+    bk = group_max<G>(bk);
+    if (gl == 0) decide(i, p_conn, bk, p, wv, out);
+}
+
+// the five group classes in one launch: blocks [blk[q], blk[q + 1]) score the
+// list entries [s[q], s[q + 1]) with 4 << q lanes each
+struct GroupRanges {
+    i64 s[CL_TABLE + 1], blk[CL_TABLE + 1];
+};
+template <class AT, class WT, class LT>
+__global__ void __launch_bounds__(256) k_score_groups(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
+                                                      const i64* __restrict__ vw, const i32* __restrict__ list,
+                                                      GroupRanges gr, const i32* __restrict__ part,
+                                                      const i64* __restrict__ vol, RecView rv,
+                                                      const i32* __restrict__ cons, int raw, LT lam, float ratio,
+                                                      ScoreOut out) {
+    const i64 b = block_id();
+#define PGGC_GROUP(q, G)                                                                                              \
+    score_group<G, AT>(rp, col, W, vw, list, gr.s[q], gr.s[q + 1], b - gr.blk[q], part, vol, rv, cons, raw, lam, ratio, \
+                       out)
+    if (b < gr.blk[1]) PGGC_GROUP(0, 4);
+    else if (b < gr.blk[2]) PGGC_GROUP(1, 8);
+    else if (b < gr.blk[3]) PGGC_GROUP(2, 16);
+    else if (b < gr.blk[4]) PGGC_GROUP(3, 32);
+    else if (b < gr.blk[5]) PGGC_GROUP(4, 64);
+#undef PGGC_GROUP
+}
+
+// One block per vertex with a hash table in LDS: SLOTS slots hold the table
+// of any degree up to SLOTS / SPE, each table the power of two >= SPE * degree.
+// A thread gathers the records of all its (at most R) edges first, so the
+// gathers are in flight together, inserts them, and after the barrier looks
+// each edge's slot up again: its record still holds the cluster's volume, so
+// the arg-max needs neither a scan of the table nor another gather (a cluster
+// met by several edges is evaluated by each; the packed maximum is the same).
+// AT as in score_group: with u32 sums a slot takes 8 bytes of LDS.  The
+// 65..2048 classes went from 148 to 93 ms on R-MAT scale 24 (two passes) and
+// from 147 to 78 ms on scale 20.
+template <class AT>
+__device__ __forceinline__ u32 table_add_slot(i32* keys, AT* vals, u32 mask, i32 key, AT w) {
+    u32 h = slot_hash(key, mask);
+    while (true) {  // at most mask / SPE keys: an empty slot is always found
+        const i32 old = atomicCAS(&keys[h], EMPTY_KEY, key);
+        if (old == EMPTY_KEY || old == key) break;
+        h = (h + 1) & mask;
+    }
+    if (sizeof(AT) == 4) atomicAdd((u32*)&vals[h], (u32)w);
+    else atomicAdd((unsigned long long*)&vals[h], (unsigned long long)w);
+    return h;
+}
+template <int BS, int SLOTS, int SPE, class AT, class WT, class LT>
 __global__ void __launch_bounds__(BS) k_score_table(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
                                                     const i64* __restrict__ vw, const i32* __restrict__ list, i64 m,
                                                     const i32* __restrict__ part, const i64* __restrict__ vol,
-                                                    const i32* __restrict__ cons, int raw, LT lam, float ratio,
-                                                    ScoreOut out, i32* gkeys, i64* gvals,
-                                                    const i64* __restrict__ goff) {
-    __shared__ i32 skeys[GLOBAL ? 1 : SLOTS];
-    __shared__ i64 svals[GLOBAL ? 1 : SLOTS];
+                                                    RecView rv, const i32* __restrict__ cons, LT lam, float ratio,
+                                                    ScoreOut out) {
+    __shared__ i32 keys[SLOTS];
+    __shared__ AT vals[SLOTS];
+    constexpr int R = (SLOTS / SPE + BS - 1) / BS;
     const int t = threadIdx.x;
     const i64 li = block_id();
     if (li >= m) return;
-    {
-        const i32 i = list[li];
-        if (out.dest[i] == NO_MOVE) return;
-        const i64 s = rp[i];
-        const i64 d = rp[i + 1] - s;
-        const i64 S = tslots(d, SPE);
-        const u32 mask = (u32)(S - 1);
-        i32* keys = GLOBAL ? gkeys + goff[li] : skeys;
-        i64* vals = GLOBAL ? gvals + goff[li] : svals;
-        for (i64 q = t; q < S; q += BS) {
-            keys[q] = EMPTY_KEY;
-            vals[q] = 0;
-        }
-        if (GLOBAL) __threadfence();
-        __syncthreads();
-        const i32 p = part[i];
-        i64 pv = 0;
-        // LDS classes hold d <= SLOTS / SPE: a thread first gathers the
-        // clusters of all its (at most R) edges, so the gathers are in flight
-        // together, then inserts them
-        constexpr int R = GLOBAL ? 0 : (SLOTS / SPE + BS - 1) / BS;
-        i64 e_done = 0;
-        if (!GLOBAL) {
-            i32 kk[R > 0 ? R : 1];
-            i64 wv[R > 0 ? R : 1];
+    const i32 i = list[li];
+    if (out.dest[i] == NO_MOVE) return;
+    const i64 s = rp[i];
+    const int d = (int)(rp[i + 1] - s);
+    const int S = (int)tslots(d, SPE);
+    const u32 mask = (u32)(S - 1);
+    const i32 p = part[i];
+    const i64 wi = vw[i];
+    NbRec r[R];
+    AT w[R];
 #pragma unroll
-            for (int r = 0; r < R; r++) {
-                const i64 e = (i64)r * BS + t;
-                kk[r] = EMPTY_KEY;
-                wv[r] = 0;
-                if (e < d) {
-                    const i32 v = col[s + e];
-                    kk[r] = raw == 1 ? v : part[v];
-                    wv[r] = W(s + e);
-                }
-            }
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                if (kk[r] == EMPTY_KEY) continue;
-                if (!raw && kk[r] == p) pv += wv[r];
-                else table_add_lds(keys, vals, mask, kk[r], wv[r]);
-            }
-            e_done = (i64)R * BS;
+    for (int q = 0; q < R; q++) {
+        const int e = q * BS + t;
+        r[q].part = EMPTY_KEY;
+        w[q] = 0;
+        if (e < d) {
+            r[q] = load_rec(rv, col[s + e]);
+            w[q] = (AT)W(s + e);
         }
-        for (i64 eb = e_done; eb < d; eb += BS) {  // block-uniform loop control
-            const i64 e = eb + t;
-            if (e >= d) continue;
-            i32 v = col[s + e];
-            i32 key = raw == 1 ? v : part[v];
-            i64 ww = W(s + e);
-            if (!raw && key == p) pv += ww;
-            else if (GLOBAL) table_add_global(keys, vals, mask, key, ww);
-            else table_add_lds(keys, vals, mask, key, ww);
-        }
-        if (GLOBAL) __threadfence();
-        pv = block_sum_i64<BS>(pv);
-        float multi, p_conn, b;
-        const i64 wi = vw[i];
-        own_terms(pv, vol[p], wi, lam(i), lam.rt(i, ratio), multi, p_conn, b);
-        u64 bk = 0;
-        for (i64 qb = 0; qb < S; qb += BS) {  // block-uniform loop control
-            const i64 q = qb + t;
-            if (q >= S) continue;
-            i32 key;
-            i64 agg;
-            if (GLOBAL) {
-                key = __hip_atomic_load(&keys[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (key == EMPTY_KEY) continue;
-                agg = __hip_atomic_load(&vals[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            } else {
-                key = keys[q];
-                if (key == EMPTY_KEY) continue;
-                agg = vals[q];
-            }
-            if (agg > 0 && (float)agg >= b && (cons == nullptr || cons[key] == cons[p])) {
-                float jc = fmaf(-(float)vol[key], multi, (float)agg);
-                if (jc >= b) {
-                    u64 k2 = pack_cand(jc, key);
-                    bk = k2 > bk ? k2 : bk;
-                }
-            }
-        }
-        bk = block_max_u64<BS>(bk);
-        if (t == 0) decide(i, p_conn, bk, p, wi, out);
-        __syncthreads();
     }
+    for (int q = t; q < S; q += BS) {
+        keys[q] = EMPTY_KEY;
+        vals[q] = 0;
+    }
+    __syncthreads();
+    AT pv = 0;
+    u32 h[R];
+#pragma unroll
+    for (int q = 0; q < R; q++) {
+        h[q] = 0;
+        if (r[q].part == EMPTY_KEY) continue;
+        if (r[q].part == p) pv += w[q];
+        else h[q] = table_add_slot(keys, vals, mask, r[q].part, w[q]);
+    }
+    pv = block_reduce<BS>(pv, [](AT a, AT b) { return a + b; });
+    __syncthreads();
+    float multi, p_conn, b;
+    own_terms((i64)pv, vol[p], wi, lam(i), lam.rt(i, ratio), multi, p_conn, b);
+    const i32 cp = cons ? cons[p] : 0;
+    u64 bk = 0;
+#pragma unroll
+    for (int q = 0; q < R; q++) {
+        if (r[q].part == EMPTY_KEY || r[q].part == p) continue;
+        const AT agg = vals[h[q]];
+        if (agg > 0 && (float)agg >= b && r[q].cons == cp) {
+            const float jc = fmaf(-r[q].volf, multi, (float)agg);
+            if (jc >= b) {
+                const u64 k2 = pack_cand(jc, r[q].part);
+                bk = k2 > bk ? k2 : bk;
+            }
+        }
+    }
+    bk = block_reduce<BS>(bk, [](u64 a, u64 b2) { return a > b2 ? a : b2; });
+    if (t == 0) decide(i, p_conn, bk, p, wi, out);
 }
 
 // Raw sweep (first sweep of an initial local_move, src/local_mover.cpp:1391-1395):
@@ -596,16 +792,32 @@ __global__ void __launch_bounds__(BS) k_score_table(const i64* __restrict__ rp, 
 // candidate is a streaming arg-max over the adjacency, with the same packed
 // (gain, smallest label) order as the table path.
 template <class WT>
-__device__ __forceinline__ u64 raw_cand(const i32* __restrict__ col, WT W, const i64* __restrict__ vol,
-                                        const i32* __restrict__ cons, const i32* __restrict__ lab, i32 cp, i64 j,
+__device__ __forceinline__ u64 raw_cand(const i32* __restrict__ col, WT W, const RecView& rv, i32 cp, i64 j,
                                         float multi, float b) {
-    const i32 v = lab ? lab[col[j]] : col[j];  // the neighbour's (singleton) cluster
+    const NbRec r = load_rec(rv, col[j]);
     const i64 agg = W(j);
-    if (agg > 0 && (float)agg >= b && (cons == nullptr || cons[v] == cp)) {
-        const float jc = fmaf(-(float)vol[v], multi, (float)agg);
-        if (jc >= b) return pack_cand(jc, v);
+    if (agg > 0 && (float)agg >= b && r.cons == cp) {
+        const float jc = fmaf(-r.volf, multi, (float)agg);
+        if (jc >= b) return pack_cand(jc, r.part);
     }
     return 0;
+}
+// arg-max over the edges [jlo, jhi) by a block
+template <int BS, class WT>
+__device__ __forceinline__ u64 raw_best(const i32* __restrict__ col, WT W, const RecView& rv, i32 cp, i64 jlo, i64 jhi,
+                                        float multi, float b) {
+    u64 bk = 0;
+    for (i64 jb = jlo; jb < jhi; jb += 4 * BS) {  // block-uniform loop control
+#pragma unroll
+        for (int u = 0; u < 4; u++) {  // independent gathers in flight
+            const i64 j = jb + u * BS + threadIdx.x;
+            if (j < jhi) {
+                const u64 k2 = raw_cand(col, W, rv, cp, j, multi, b);
+                bk = k2 > bk ? k2 : bk;
+            }
+        }
+    }
+    return block_max_u64<BS>(bk);
 }
 
 // one block per vertex (64 < degree <= 2048)
@@ -613,27 +825,18 @@ template <int BS, class WT, class LT>
 __global__ void __launch_bounds__(BS) k_score_raw(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
                                                   const i64* __restrict__ vw, const i32* __restrict__ list, i64 m,
                                                   const i32* __restrict__ part, const i64* __restrict__ vol,
-                                                  const i32* __restrict__ cons, const i32* __restrict__ lab, LT lam,
-                                                  float ratio, ScoreOut out) {
+                                                  RecView rv, const i32* __restrict__ cons, LT lam, float ratio,
+                                                  ScoreOut out) {
     const i64 li = block_id();
     if (li >= m) return;
     const i32 i = list[li];
     if (out.dest[i] == NO_MOVE) return;
-    const i64 s = rp[i], e = rp[i + 1];
     const i32 p = part[i];
     const i32 cp = cons ? cons[p] : 0;
     float multi, p_conn, b;
     const i64 wi = vw[i];
     own_terms(0, vol[p], wi, lam(i), lam.rt(i, ratio), multi, p_conn, b);
-    u64 bk = 0;
-    for (i64 jb = s; jb < e; jb += BS) {  // block-uniform loop control
-        const i64 j = jb + threadIdx.x;
-        if (j < e) {
-            const u64 k2 = raw_cand(col, W, vol, cons, lab, cp, j, multi, b);
-            bk = k2 > bk ? k2 : bk;
-        }
-    }
-    bk = block_max_u64<BS>(bk);
+    const u64 bk = raw_best<BS>(col, W, rv, cp, rp[i], rp[i + 1], multi, b);
     if (threadIdx.x == 0) decide(i, p_conn, bk, p, wi, out);
 }
 
@@ -642,8 +845,8 @@ template <class WT, class LT>
 __global__ void __launch_bounds__(256) k_hub_raw(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
                                                  const i64* __restrict__ vw, const i32* __restrict__ hubs, i64 m,
                                                  const i64* __restrict__ items, const i32* __restrict__ part,
-                                                 const i64* __restrict__ vol, const i32* __restrict__ cons,
-                                                 const i32* __restrict__ lab, LT lam, float ratio,
+                                                 const i64* __restrict__ vol, RecView rv,
+                                                 const i32* __restrict__ cons, LT lam, float ratio,
                                                  const i32* __restrict__ dest, i64 he, u64* hub_best) {
     const i64 b = block_id();
     if (b >= items[m]) return;
@@ -657,15 +860,7 @@ __global__ void __launch_bounds__(256) k_hub_raw(const i64* __restrict__ rp, con
     const i32 cp = cons ? cons[p] : 0;
     float multi, p_conn, bth;
     own_terms(0, vol[p], vw[i], lam(i), lam.rt(i, ratio), multi, p_conn, bth);
-    u64 bk = 0;
-    for (i64 jb = j_lo; jb < j_hi; jb += 256) {  // block-uniform loop control
-        const i64 j = jb + threadIdx.x;
-        if (j < j_hi) {
-            const u64 k2 = raw_cand(col, W, vol, cons, lab, cp, j, multi, bth);
-            bk = k2 > bk ? k2 : bk;
-        }
-    }
-    bk = block_max_u64<256>(bk);
+    const u64 bk = raw_best<256>(col, W, rv, cp, j_lo, j_hi, multi, bth);
     if (threadIdx.x == 0 && bk) atomicMax((unsigned long long*)&hub_best[hi], (unsigned long long)bk);
 }
 
@@ -1052,9 +1247,9 @@ __global__ void k_hub_decide(const i32* hubs, i64 m, const i32* part, const i64*
 // Algorithmic bytes of one scoring sweep, counted (on timing runs only)
 // before it runs, since dest decides which vertices it scores.  A scored
 // vertex reads its row bounds, destination, cluster, vertex weight and its
-// cluster's volume, every edge's column (and weight) and, after the first
-// sweep, the neighbour's cluster, and writes its destination and gain:
-// 48 + d (4 + weight bytes + 4) bytes.  A hub whose table is kept current reads
+// cluster's volume, every edge's column (and weight) and the neighbour's
+// record, and writes its destination, gain and record: 48 + d (4 + weight
+// bytes + 8) bytes.  A hub whose table is kept current reads
 // the table instead of its edges: 48 + 8 per slot, plus the edge bytes on the
 // sweep that builds the table.  Every listed vertex also costs its list entry
 // and destination read.  acc3[0..2] = group, table and hub classes.
@@ -1073,7 +1268,7 @@ __global__ void __launch_bounds__(256) k_score_bytes(const i64* __restrict__ rp,
         const int grp = x < sb.s[CL_TABLE] ? 0 : (x < sb.hub0 ? 1 : 2);
         i64 by = 8;
         if (dest[i] != NO_MOVE) {
-            const i64 eb = (rp[i + 1] - rp[i]) * (4 + WB + (raw == 1 ? 0 : 4));
+            const i64 eb = (rp[i + 1] - rp[i]) * (4 + WB + 8);
             if (grp < 2 || raw) {
                 by += 48 + eb;
             } else {
@@ -1110,29 +1305,75 @@ __global__ void __launch_bounds__(256) k_list_bytes(const i64* __restrict__ rp, 
     if (threadIdx.x == 0 && b) atomicAdd((unsigned long long*)acc, (unsigned long long)b);
 }
 
+// What the scoring launches share.
+template <class LT>
+struct ScoreArgs {
+    const i32* L;
+    const i32* part;
+    const i64* vol;
+    RecView rv;
+    const i32* cons;
+    LT lam;
+    float ratio;
+    ScoreOut out;
+};
 // LDS-table scoring of the list entries [x0, x1) (one block per vertex):
 // BS threads, SLOTS LDS slots, SPE slots per edge of the degree bound.
-template <int BS, int SLOTS, int SPE, class WT, class LT>
-static void launch_table(Ctx& c, const DGraph& g, WT W, const i32* L, i64 x0, i64 x1, const i32* part,
-                         const i64* vol, const i32* cons, LT lam, float ratio, const ScoreOut& out) {
+template <class AT, int BS, int SLOTS, int SPE, class WT, class LT>
+static void launch_table(Ctx& c, const DGraph& g, WT W, const ScoreArgs<LT>& a, i64 x0, i64 x1) {
     const i64 m = x1 - x0;
     if (m <= 0) return;
-    k_score_table<BS, SLOTS, SPE, false><<<grid_blocks(m), BS, 0, c.stream>>>(
-        g.rp, g.col, W, g.vw, L + x0, m, part, vol, cons, 0, lam, ratio, out, nullptr, nullptr, nullptr);
+    k_score_table<BS, SLOTS, SPE, AT><<<grid_blocks(m), BS, 0, c.stream>>>(
+        g.rp, g.col, W, g.vw, a.L + x0, m, a.part, a.vol, a.rv, a.cons, a.lam, a.ratio, a.out);
 }
 // class with degree bound D (128, 256, 512): threads per vertex and slots per
 // edge from the knobs
-template <int D, class WT, class LT>
-static void launch_table_class(Ctx& c, const DGraph& g, WT W, const i32* L, i64 x0, i64 x1, const i32* part,
-                               const i64* vol, const i32* cons, LT lam, float ratio, const ScoreOut& out) {
+template <class AT, int D, class WT, class LT>
+static void launch_table_class(Ctx& c, const DGraph& g, WT W, const ScoreArgs<LT>& a, i64 x0, i64 x1) {
     const int bs = c.table_threads, spe = c.table_spe;
-    if (bs == 64 && spe == 2) launch_table<64, 2 * D, 2>(c, g, W, L, x0, x1, part, vol, cons, lam, ratio, out);
-    else if (bs == 64) launch_table<64, 4 * D, 4>(c, g, W, L, x0, x1, part, vol, cons, lam, ratio, out);
-    else if (bs == 128 && spe == 2)
-        launch_table<128, 2 * D, 2>(c, g, W, L, x0, x1, part, vol, cons, lam, ratio, out);
-    else if (bs == 128) launch_table<128, 4 * D, 4>(c, g, W, L, x0, x1, part, vol, cons, lam, ratio, out);
-    else if (spe == 2) launch_table<256, 2 * D, 2>(c, g, W, L, x0, x1, part, vol, cons, lam, ratio, out);
-    else launch_table<256, 4 * D, 4>(c, g, W, L, x0, x1, part, vol, cons, lam, ratio, out);
+    if (bs == 64 && spe == 2) launch_table<AT, 64, 2 * D, 2>(c, g, W, a, x0, x1);
+    else if (bs == 64) launch_table<AT, 64, 4 * D, 4>(c, g, W, a, x0, x1);
+    else if (bs == 128 && spe == 2) launch_table<AT, 128, 2 * D, 2>(c, g, W, a, x0, x1);
+    else if (bs == 128) launch_table<AT, 128, 4 * D, 4>(c, g, W, a, x0, x1);
+    else if (spe == 2) launch_table<AT, 256, 2 * D, 2>(c, g, W, a, x0, x1);
+    else launch_table<AT, 256, 4 * D, 4>(c, g, W, a, x0, x1);
+}
+template <class AT, class WT, class LT>
+static void launch_groups(Ctx& c, const DGraph& g, WT W, const ScoreArgs<LT>& a, const i64* st, int raw) {
+    GroupRanges gr;
+    i64 nb = 0;
+    for (int q = 0; q <= CL_TABLE; q++) {
+        gr.s[q] = st[q];
+        gr.blk[q] = nb;
+        if (q < CL_TABLE) nb += ceil_div(st[q + 1] - st[q], 256 / (4 << q));
+    }
+    if (nb == 0) return;
+    k_score_groups<AT><<<grid_blocks(nb), 256, 0, c.stream>>>(g.rp, g.col, W, g.vw, a.L, gr, a.part, a.vol, a.rv,
+                                                              a.cons, raw, a.lam, a.ratio, a.out);
+}
+template <class AT, class WT, class LT>
+static void launch_tables(Ctx& c, const LevelPlan& lp, const DGraph& g, WT W, const ScoreArgs<LT>& a) {
+    const i64* st = lp.sc_start;
+    // few rows: one launch for all classes (the widest block), as launches
+    // then cost more than the lower occupancy
+    if (lp.hub0 - st[CL_TABLE] <= TABLE_ONE_LAUNCH && lp.hub0 == st[CL_HUB]) {
+        launch_table<AT, 256, 4096, 2>(c, g, W, a, st[CL_TABLE], st[CL_HUB]);
+        return;
+    }
+    // LDS tables sized for the class, so the many low-degree rows keep more
+    // waves resident per CU; threads per vertex and slots per edge are knobs
+    launch_table_class<AT, 128>(c, g, W, a, st[5], st[6]);
+    launch_table_class<AT, 256>(c, g, W, a, st[6], st[7]);
+    launch_table_class<AT, 512>(c, g, W, a, st[7], st[8]);
+    if (c.table_spe == 2) {
+        launch_table<AT, 256, 2048, 2>(c, g, W, a, st[8], st[9]);
+        launch_table<AT, 512, 4096, 2>(c, g, W, a, st[9], st[10]);
+    } else {
+        launch_table<AT, 256, 4096, 4>(c, g, W, a, st[8], st[9]);
+        launch_table<AT, 512, 8192, 4>(c, g, W, a, st[9], st[10]);
+    }
+    // hubs of degree <= hub_lds_max: 8192 LDS slots
+    launch_table<AT, 512, 8192, 2>(c, g, W, a, st[CL_HUB], lp.hub0);
 }
 
 // Hub tables of the current clustering: slices built in LDS, then the
@@ -1243,9 +1484,7 @@ template <class LT>
 static void score_all(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, const i32* part, const i64* vol,
                       const i32* cons, int raw, LT lam, float ratio, const ScoreOut& out) {
     i32* dest = out.dest;
-    // raw 1: singletons labelled by vertex id; raw 2: singletons whose labels
-    // are read from part (a renumbered graph); 0: any clustering
-    const i32* lab = raw == 2 ? part : nullptr;
+    // raw: every vertex a cluster of its own; 0: any clustering
     const i64* st = lp.sc_start;
     const i32* L = lp.sc_list.p;
     Buf<i64> acct;
@@ -1261,50 +1500,33 @@ static void score_all(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, co
                               g.rp, L, sb, dest, raw, build, goff, acct)));
         PGGC_LAUNCH_CHECK();
     }
+    if (g.n > 0) {
+        if (cons && s.rec16.n < (size_t)g.n) s.rec16 = Buf<uint4>(c, s.cap);
+        k_rec_pack<<<grid_items(g.n, 256), 256, 0, c.stream>>>(g.n, part, vol, cons, s.rec, cons ? s.rec16.p : nullptr);
+        PGGC_LAUNCH_CHECK();
+    }
+    const ScoreArgs<LT> a{L, part, vol, RecView{s.rec.p, cons ? s.rec16.p : nullptr}, cons, lam, ratio, out};
     PGGC_WDISPATCH(g, {
+        using WT = decltype(W);
+        using A64 = typename std::conditional<IsUnit<WT>::v, u32, i64>::type;  // sums of unit rows fit 32 bits
         i64 m;
         int tk = c.kt_begin(KS_SCORE_GROUP);
-        if ((m = st[1] - st[0]) > 0)
-            k_score_group<4><<<grid_items(m, 64), 256, 0, c.stream>>>(
-                g.rp, g.col, W, g.vw, L + st[0], m, part, vol, cons, raw, lam, ratio, out);
-        if ((m = st[2] - st[1]) > 0)
-            k_score_group<8><<<grid_items(m, 32), 256, 0, c.stream>>>(
-                g.rp, g.col, W, g.vw, L + st[1], m, part, vol, cons, raw, lam, ratio, out);
-        if ((m = st[3] - st[2]) > 0)
-            k_score_group<16><<<grid_items(m, 16), 256, 0, c.stream>>>(
-                g.rp, g.col, W, g.vw, L + st[2], m, part, vol, cons, raw, lam, ratio, out);
-        if ((m = st[4] - st[3]) > 0)
-            k_score_group<32><<<grid_items(m, 8), 256, 0, c.stream>>>(
-                g.rp, g.col, W, g.vw, L + st[3], m, part, vol, cons, raw, lam, ratio, out);
-        if ((m = st[5] - st[4]) > 0)
-            k_score_group<64><<<grid_items(m, 4), 256, 0, c.stream>>>(
-                g.rp, g.col, W, g.vw, L + st[4], m, part, vol, cons, raw, lam, ratio, out);
+        if (lp.agg32) launch_groups<u32>(c, g, W, a, st, raw);
+        else launch_groups<A64>(c, g, W, a, st, raw);
         c.kt_end(tk, 0.0);
         if (tk >= 0) acct_add(c, c.kt_counter(tk), acct.p);
         tk = c.kt_begin(KS_SCORE_TABLE);
         if (raw) {
             if ((m = st[CL_BIG] - st[CL_TABLE]) > 0)
                 k_score_raw<64><<<grid_blocks(m), 64, 0, c.stream>>>(g.rp, g.col, W, g.vw, L + st[CL_TABLE], m,
-                                                                     part, vol, cons, lab, lam, ratio, out);
+                                                                     part, vol, a.rv, cons, lam, ratio, out);
             if ((m = lp.hub0 - st[CL_BIG]) > 0)  // big rows and the LDS-scored hubs
                 k_score_raw<256><<<grid_blocks(m), 256, 0, c.stream>>>(g.rp, g.col, W, g.vw, L + st[CL_BIG], m,
-                                                                       part, vol, cons, lab, lam, ratio, out);
+                                                                       part, vol, a.rv, cons, lam, ratio, out);
+        } else if (lp.agg32) {
+            launch_tables<u32>(c, lp, g, W, a);
         } else {
-            // LDS tables sized for the class, so the many low-degree rows keep
-            // more waves resident per CU; threads per vertex and slots per
-            // edge are knobs
-            launch_table_class<128>(c, g, W, L, st[5], st[6], part, vol, cons, lam, ratio, out);
-            launch_table_class<256>(c, g, W, L, st[6], st[7], part, vol, cons, lam, ratio, out);
-            launch_table_class<512>(c, g, W, L, st[7], st[8], part, vol, cons, lam, ratio, out);
-            if (c.table_spe == 2) {
-                launch_table<256, 2048, 2>(c, g, W, L, st[8], st[9], part, vol, cons, lam, ratio, out);
-                launch_table<512, 4096, 2>(c, g, W, L, st[9], st[10], part, vol, cons, lam, ratio, out);
-            } else {
-                launch_table<256, 4096, 4>(c, g, W, L, st[8], st[9], part, vol, cons, lam, ratio, out);
-                launch_table<512, 8192, 4>(c, g, W, L, st[9], st[10], part, vol, cons, lam, ratio, out);
-            }
-            // hubs of degree <= hub_lds_max: 8192 LDS slots (96 KB of LDS)
-            launch_table<512, 8192, 2>(c, g, W, L, st[CL_HUB], lp.hub0, part, vol, cons, lam, ratio, out);
+            launch_tables<A64>(c, lp, g, W, a);
         }
         c.kt_end(tk, 0.0);
         if (tk >= 0) acct_add(c, c.kt_counter(tk), acct.p + 1);
@@ -1315,7 +1537,7 @@ static void score_all(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, co
             fill_i64(c, (i64*)lp.hub_best.p, m, 0);
             if (raw) {
                 k_hub_raw<<<grid_blocks(lp.nitems), 256, 0, c.stream>>>(g.rp, g.col, W, g.vw, hubs, m, lp.items, part,
-                                                                       vol, cons, lab, lam, ratio, dest, lp.he,
+                                                                       vol, a.rv, cons, lam, ratio, dest, lp.he,
                                                                        lp.hub_best);
             } else {
                 if (!lp.hub_live) {  // first table sweep of the call (or stale tables): build
@@ -2119,9 +2341,7 @@ static void local_move_t(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g,
     const int limits[2] = {4, 2};
     int iter = 0;
     const i32* ccons = constrained ? cons : nullptr;
-    // the raw first sweep (every neighbour its own cluster) reads a
-    // neighbour's cluster from part when the graph is renumbered
-    const int raw_mode = c.raw_sweeps ? (ids ? 2 : 1) : 0;
+    const int raw_mode = c.raw_sweeps ? 1 : 0;
     SweepTrace tr(c, g, is_initial ? 0 : 1);
     // active-set predictor: on levels of at least min_nnz nonzeros, from the
     // second sweep of a call that starts at singletons (whose first sweep
