@@ -167,14 +167,14 @@ int pggc_ctx_set_sweep_trace(pggc_ctx* ctx, pggc_sweep_fn fn, void* user);
  *     edge work items); 1 every table by edge work items adding into the HBM
  *     table with atomics; 2 the tables of odd hub index by edge items, the
  *     rest by slices (the same tables' contents in every mode).
- *   PGGC_KNOB_RENUMBER: where the local mover of the top level runs: on an
- *     internal copy of the graph with vertices in descending degree order
- *     (rows keep their entry order; labels, priorities and new cluster ids
- *     follow the caller's ids, so results are identical) or on the caller's
- *     graph.  1: always the copy; 2 (default): the copy when the call makes
- *     more than one top-level pass (pggc_cluster with ex_iters != 0), which
- *     pays for building it; 0: never.  Not used with the active-set
- *     predictor on.
+ *   PGGC_KNOB_RENUMBER: where the local mover of a level runs: on an internal
+ *     copy of the level with vertices in descending degree order (rows keep
+ *     their entry order; labels, priorities and new cluster ids follow the
+ *     original ids, so results are identical) or on the level itself.  1:
+ *     always the copy; 2 (default): the copy on large levels whose edges
+ *     gather on few vertices, and on the top level when the call makes more
+ *     than one top-level pass (pggc_cluster with ex_iters != 0); 0: never.
+ *     Not used with the active-set predictor on.
  *   PGGC_KNOB_CONTRACT_BATCH: the contraction merges its largest coarse rows
  *     in HBM hash tables and sorts them in batches of rows holding at most
  *     this many table slots (default 2^30) and a quarter as many sort

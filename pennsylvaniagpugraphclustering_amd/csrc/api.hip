@@ -134,6 +134,7 @@ struct Level {
     DGraph g;
     std::unique_ptr<OwnedGraph> own;
     std::unique_ptr<LevelPlan> plan;
+    std::unique_ptr<Renum> rn;  // renumbered copy of a coarse level (coarse_renum)
 };
 
 static Level top_level(const DGraph& g) {
@@ -149,6 +150,7 @@ static Level top_level(const DGraph& g) {
 static void release_level(Level& l, Buf<i32>& part) {
     l.own.reset();
     l.plan.reset();
+    l.rn.reset();
     part.reset();
 }
 
@@ -164,14 +166,30 @@ static Level owned_level(std::unique_ptr<OwnedGraph> og) {
 constexpr int LEIDEN_MAX_STALLS = 8;
 
 // The top level renumbered by degree for the local mover (results are the
-// caller's order's, bit for bit): always with the renumber knob at 1, with
-// it at 2 (the default) when the copy serves several top-level passes
-// (reuse), never at 0 or with the active-set predictor on, whose features
-// follow the vertex order.
+// caller's order's, bit for bit): always with the renumber knob at 1, where it
+// pays (renum_build) or the call makes several top-level passes (reuse) with
+// it at 2 (the default), never at 0 or with the active-set predictor on, whose
+// features follow the vertex order.
 static Renum* top_renum(Ctx& c, MoveScratch& ms, const DGraph& g, Renum& r, bool reuse) {
-    if (c.renumber == 0 || (c.renumber == 2 && !reuse) || (ms.gnn && ms.gnn->cfg.mode != GNN_OFF)) return nullptr;
-    renum_build(c, g, r);
-    return &r;
+    if (c.renumber == 0 || (ms.gnn && ms.gnn->cfg.mode != GNN_OFF)) return nullptr;
+    return renum_build(c, g, r, c.renumber == 1 || reuse) ? &r : nullptr;
+}
+// The same for a coarse level, built once and kept for the way back up.  The
+// copies of a run hold at most RN_MEM of the device's memory together: on
+// graphs of billions of edges the finer levels go without.
+constexpr double RN_MEM = 1.0 / 8;
+static Renum* coarse_renum(Ctx& c, MoveScratch& ms, std::vector<Level>& levels, size_t li) {
+    Level& l = levels[li];
+    if (c.renumber == 0 || (ms.gnn && ms.gnn->cfg.mode != GNN_OFF)) return nullptr;
+    if (!l.rn) {
+        auto bytes = [](const DGraph& g) { return 32.0 * g.n + (g.wk == W_I64 ? 12.0 : 8.0) * g.nnz; };
+        double held = bytes(l.g);
+        for (size_t k = 0; k < li; k++)
+            if (levels[k].rn && levels[k].rn->copied) held += bytes(levels[k].g);
+        l.rn.reset(new Renum());
+        if (held <= RN_MEM * (double)c.mem_total) renum_build(c, l.g, *l.rn, c.renumber == 1);
+    }
+    return l.rn->copied ? l.rn.get() : nullptr;
 }
 
 // local_move at one level; rn (when set) is the top level renumbered
@@ -219,7 +237,8 @@ static void louvain_part(Ctx& c, MoveScratch& ms, const DGraph& top, RefineData&
         Buf<i32> part(c, std::max<i64>(g.n, 1));
         iota_i32(c, part, g.n);
         c.mem_note("louvain: level start");
-        move_level(c, ms, lp, g, part, rfd, true, constrained, cons, true, rs, levels.size() == 1 ? rn : nullptr);
+        Renum* lr = levels.size() == 1 ? rn : coarse_renum(c, ms, levels, levels.size() - 1);
+        move_level(c, ms, lp, g, part, rfd, true, constrained, cons, true, rs, lr);
         c.mem_note("louvain: after local move");
         if (constrained && rfd.label_count == g.n) local_move_strict(c, ms, lp, g, part, rfd, true, constrained, cons, &rs.mv);
         const i32* pp = part.p;
@@ -228,7 +247,7 @@ static void louvain_part(Ctx& c, MoveScratch& ms, const DGraph& top, RefineData&
             const i64 nc = rfd.label_count;
             std::unique_ptr<OwnedGraph> og(new OwnedGraph());
             auto t0 = std::chrono::steady_clock::now();
-            contract_level(c, g, pp, nc, *og, levels.size() == 1 ? rn : nullptr);
+            contract_level(c, g, pp, nc, *og, lr);
             c.sync();
             rs.contract_s += since(t0);
             og->vw = Buf<i64>(c, std::max<i64>(nc, 1));
@@ -260,7 +279,8 @@ static void louvain_part(Ctx& c, MoveScratch& ms, const DGraph& top, RefineData&
         LevelPlan& lp = (i == 0 && top_plan) ? *top_plan : *levels[i].plan;
         project(c, g.n, parts[i + 1], parts[i]);
         release_level(levels[i + 1], parts[i + 1]);  // done with the coarser level
-        move_level(c, ms, lp, g, parts[i], rfd, false, false, nullptr, true, rs, i == 0 ? rn : nullptr);
+        move_level(c, ms, lp, g, parts[i], rfd, false, false, nullptr, true, rs,
+                   i == 0 ? rn : coarse_renum(c, ms, levels, (size_t)i));
     }
     copy_dev(c, part_out, parts[0].p, top.n * sizeof(i32));
     c.sync();
@@ -282,7 +302,7 @@ static void leiden_part(Ctx& c, MoveScratch& ms, const DGraph& top, RefineData& 
         LevelPlan& lp = (li == 0 && top_plan) ? *top_plan : *levels[li].plan;
         const double old_obj = rfd.obj;
         const bool init = !improve && levels.size() == 1;
-        Renum* r0 = li == 0 ? rn : nullptr;
+        Renum* r0 = li == 0 ? rn : coarse_renum(c, ms, levels, li);
         c.mem_note("leiden: level start");
         move_level(c, ms, lp, g, part, rfd, init, false, nullptr, true, rs, r0);
         c.mem_note("leiden: after local move");
@@ -350,7 +370,9 @@ static void leiden_part(Ctx& c, MoveScratch& ms, const DGraph& top, RefineData& 
         LevelPlan& lp = (i == 0 && top_plan) ? *top_plan : *levels[i].plan;
         project(c, g.n, parts[i + 1], parts[i]);
         release_level(levels[i + 1], parts[i + 1]);  // done with the coarser level
-        if (plus) move_level(c, ms, lp, g, parts[i], rfd, false, false, nullptr, true, rs, i == 0 ? rn : nullptr);
+        if (plus)
+            move_level(c, ms, lp, g, parts[i], rfd, false, false, nullptr, true, rs,
+                       i == 0 ? rn : coarse_renum(c, ms, levels, (size_t)i));
     }
     copy_dev(c, part_out, parts[0].p, top.n * sizeof(i32));
     c.sync();
@@ -485,6 +507,7 @@ int pggc_ctx_create(pggc_ctx** out, void* stream) {
         size_t mem_free = 0, mem_total = 0;
         PGGC_HIP(hipMemGetInfo(&mem_free, &mem_total));
         x->c.cache_keep = mem_total / 32;
+        x->c.mem_total = mem_total;
         // coherent (fine-grained) host memory: the readback kernel's stores
         // reach the host without a cache writeback the host would have to wait for
         PGGC_HIP(hipHostMalloc((void**)&x->c.pinned, 64 * sizeof(i64), hipHostMallocCoherent));

@@ -118,6 +118,7 @@ struct Ctx {
     // millions of edges.  Below that the blocks serve the next call: freeing
     // and allocating them again took 18 of the 25 ms of a 16M-edge build.
     size_t cache_keep = 0;
+    size_t mem_total = 0;  // of the device
     void trim_large();
     void sync() { PGGC_HIP(hipStreamSynchronize(stream)); }
     // copy `count` int64 device values to the pinned slots and wait

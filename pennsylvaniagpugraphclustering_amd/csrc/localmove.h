@@ -123,8 +123,11 @@ void plan_level(Ctx& c, const DGraph& g, LevelPlan& p);
 // ids (optional, device, n): g is a renumbering of the caller's graph and
 // ids[i] is vertex i's caller id, which then stands in for i wherever the
 // result depends on vertex ids (afterburner priorities, new cluster ids).
+// nfull (optional, >= g.n): best_part has nfull entries, the ones from g.n on
+// those of inert vertices without neighbours, which keep their clusters.
 void local_move(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, i32* best_part, RefineData& best,
-                bool is_initial, bool constrained, i32* cons, bool SA, MoveStats* st, const i32* ids = nullptr);
+                bool is_initial, bool constrained, i32* cons, bool SA, MoveStats* st, const i32* ids = nullptr,
+                i64 nfull = -1);
 void local_move_strict(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, i32* best_part, RefineData& best,
                        bool is_initial, bool constrained, i32* cons, MoveStats* st);
 

@@ -1852,7 +1852,7 @@ __global__ void k_newid_keys(const i32* newv, i64 K, const i64* rp, const i32* i
 // graph is renumbered and ids[i] is vertex i's id in the caller's order; the
 // movers are then taken in the caller's move order.
 static void set_new_cluster_ids(Ctx& c, MoveScratch& s, const DGraph& g, RefineData& rd, const i32* moves, i64 k,
-                                i32* cons, const i32* ids) {
+                                i32* cons, const i32* ids, i64 nfull) {
     k_new_flags<<<grid_items(k, 256), 256, 0, c.stream>>>(moves, k, s.dest, s.flag);
     PGGC_LAUNCH_CHECK();
     i64 K = compact_flags(c, s.flag, moves, k, s.tmp, s.scal);
@@ -1865,7 +1865,7 @@ static void set_new_cluster_ids(Ctx& c, MoveScratch& s, const DGraph& g, RefineD
     }
     const i32 curr = rd.label_count;
     fill_i32(c, s.flag, curr, 0);
-    k_mark_used<<<grid_items(g.n, 256), 256, 0, c.stream>>>(s.part, g.n, s.flag);
+    k_mark_used<<<grid_items(nfull, 256), 256, 0, c.stream>>>(s.part, nfull, s.flag);
     PGGC_LAUNCH_CHECK();
     Buf<i32> uf(c, std::max<i64>(curr, 1));
     k_unused_flags<<<grid_items(curr, 256), 256, 0, c.stream>>>(s.flag, curr, uf);
@@ -2142,13 +2142,13 @@ __global__ void __launch_bounds__(256) k_finish(const i64* __restrict__ vol, i64
 // reset: the movers' neighbours are scored again in the next sweep.
 template <class AT>
 static void apply_moves_core(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, i64* vol, const i32* moves,
-                             i64 k, i64 n_large, i64 n_massive, bool reset, AT at) {
+                             i64 k, i64 n_large, i64 n_massive, bool reset, AT at, i64 nfull) {
     const i64 nw = std::min(k, n_large);
     const i64 nb = std::min(k, n_massive);
     const int tk = c.kt_begin(KS_MOVES);
     const i64 m7 = lp.nhub;
     // many movers: updating costs more than rebuilding the tables next sweep
-    if (lp.hub_live && m7 > 0 && (c.hub_update_div <= 0 || k * c.hub_update_div > g.n)) lp.hub_live = false;
+    if (lp.hub_live && m7 > 0 && (c.hub_update_div <= 0 || k * c.hub_update_div > nfull)) lp.hub_live = false;
     const bool hub_upd = lp.hub_live && m7 > 0;
     k_mvp_moves<<<grid_items(k, 256), 256, 0, c.stream>>>(moves, k, s.part, s.dest, s.mvp);
     PGGC_LAUNCH_CHECK();
@@ -2194,8 +2194,8 @@ static void init_mvp(Ctx& c, MoveScratch& s, i64 n) {
 }
 
 static void perform_moves(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, RefineData& curr,
-                          const i32* moves, i64 k, i64 n_large, i64 n_massive, bool& tables) {
-    apply_moves_core(c, s, lp, g, curr.vol, moves, k, n_large, n_massive, tables, AccOne{s.scal.p + SC_SLOTS});
+                          const i32* moves, i64 k, i64 n_large, i64 n_massive, bool& tables, i64 nfull) {
+    apply_moves_core(c, s, lp, g, curr.vol, moves, k, n_large, n_massive, tables, AccOne{s.scal.p + SC_SLOTS}, nfull);
     if (!tables) {
         tables = true;
         fill_i32(c, s.dest, g.n, NULL_PART);
@@ -2270,12 +2270,14 @@ struct SweepTrace {
     Ctx& c;
     const DGraph& g;
     i64 phase, sweep = 0, active = 0;
+    i64 n;      // vertices of the level
+    i64 inert;  // of them left out of g, and counted while every vertex is active
     std::chrono::steady_clock::time_point t0;
-    SweepTrace(Ctx& cc, const DGraph& gg, i64 ph) : c(cc), g(gg), phase(ph) {}
-    void begin(const i32* dest, bool all) {
+    SweepTrace(Ctx& cc, const DGraph& gg, i64 ph, i64 nfull) : c(cc), g(gg), phase(ph), n(nfull), inert(nfull - gg.n) {}
+    void begin(const i32* dest, bool all, bool fresh = false) {
         if (!c.sweep_trace) return;
         if (all) {
-            active = g.n;
+            active = n;
         } else {
             Buf<i64> cnt(c, 1);
             fill_i64(c, cnt, 1, 0);
@@ -2283,7 +2285,7 @@ struct SweepTrace {
                 k_count_active<<<grid_items(g.n, 256), 256, 0, c.stream>>>(dest, g.n, cnt);
                 PGGC_LAUNCH_CHECK();
             }
-            active = c.read1(cnt);
+            active = c.read1(cnt) + (fresh ? inert : 0);
         }
         c.sync();
         t0 = std::chrono::steady_clock::now();
@@ -2292,7 +2294,7 @@ struct SweepTrace {
         if (!c.sweep_trace) return;
         c.sync();
         const double us = std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - t0).count();
-        const int64_t rec[8] = {g.n, g.nnz, phase, sweep++, active, cands, moves, (int64_t)us};
+        const int64_t rec[8] = {n, g.nnz, phase, sweep++, active, cands, moves, (int64_t)us};
         c.sweep_trace(c.sweep_user, rec, 8);
     }
 };
@@ -2310,30 +2312,33 @@ static RefineData begin_curr(Ctx& c, const RefineData& best, Buf<i64>& cv, i64 n
 template <class PT>
 static void local_move_t(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, i32* best_part, RefineData& best,
                          bool is_initial, bool constrained, i32* cons, bool SA, MoveStats* stats, PT prio,
-                         const i32* ids);
+                         const i32* ids, i64 nfull);
 
 void local_move(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, i32* best_part, RefineData& best,
-                bool is_initial, bool constrained, i32* cons, bool SA, MoveStats* stats, const i32* ids) {
+                bool is_initial, bool constrained, i32* cons, bool SA, MoveStats* stats, const i32* ids, i64 nfull) {
+    if (nfull < 0) nfull = g.n;
     if (ids) {
-        local_move_t(c, s, lp, g, best_part, best, is_initial, constrained, cons, SA, stats, PrioInst{ids}, ids);
+        local_move_t(c, s, lp, g, best_part, best, is_initial, constrained, cons, SA, stats, PrioInst{ids}, ids,
+                     nfull);
     } else {
-        local_move_t(c, s, lp, g, best_part, best, is_initial, constrained, cons, SA, stats, PrioOne{}, nullptr);
+        local_move_t(c, s, lp, g, best_part, best, is_initial, constrained, cons, SA, stats, PrioOne{}, nullptr,
+                     nfull);
     }
 }
 
 template <class PT>
 static void local_move_t(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, i32* best_part, RefineData& best,
                          bool is_initial, bool constrained, i32* cons, bool SA, MoveStats* stats, PT prio,
-                         const i32* ids) {
+                         const i32* ids, i64 nfull) {
     const i64 n = g.n;
-    s.ensure(c, n);
+    s.ensure(c, nfull);
     plan_level(c, g, lp);
     hub_tables_acquire(c, lp);
     lp.hub_live = false;  // the clustering changed since the last call
     c.mem_note("local move: plan ready");
     Buf<i64> cv;
-    RefineData curr = begin_curr(c, best, cv, n);
-    copy_dev(c, s.part, best_part, n * sizeof(i32));
+    RefineData curr = begin_curr(c, best, cv, nfull);
+    copy_dev(c, s.part, best_part, nfull * sizeof(i32));
     init_mvp(c, s, n);
     fill_i32(c, s.dest, n, NULL_PART);
     bool tables = !is_initial;
@@ -2342,7 +2347,7 @@ static void local_move_t(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g,
     int iter = 0;
     const i32* ccons = constrained ? cons : nullptr;
     const int raw_mode = c.raw_sweeps ? 1 : 0;
-    SweepTrace tr(c, g, is_initial ? 0 : 1);
+    SweepTrace tr(c, g, is_initial ? 0 : 1, nfull);
     // active-set predictor: on levels of at least min_nnz nonzeros, from the
     // second sweep of a call that starts at singletons (whose first sweep
     // moves most vertices), from the first sweep otherwise, and only while
@@ -2356,6 +2361,7 @@ static void local_move_t(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g,
     if (G) gnn_begin(c, *G, n, train);
     i64 kprev = n;
     i64 npred = 0;  // predicted sweeps in this call
+    bool fresh = false;  // every vertex was made active by the last sweep
     for (int x = 0; x < 2; x++) {
         const float fr = SA ? ratios[x] : 0.0f;
         for (int cnt = 0; cnt < limits[x]; cnt++) {
@@ -2370,7 +2376,8 @@ static void local_move_t(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g,
                             G->cfg.mode == GNN_PRUNE, train);
                 npred++;
             }
-            tr.begin(s.dest, iter == 1 && !use);
+            tr.begin(s.dest, iter == 1 && !use, fresh);
+            fresh = false;
             score_all(c, s, lp, g, s.part, curr.vol, ccons, tables ? 0 : raw_mode, lam, fr, so);
             i64 b[2];
             i64 k = gather_candidates(c, s, lp, g, s.dest, s.cand, b);
@@ -2398,8 +2405,9 @@ static void local_move_t(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g,
                 break;
             }
             if (iter > 1 || !is_initial)
-                set_new_cluster_ids(c, s, g, curr, s.moves, km, constrained ? cons : nullptr, ids);
-            perform_moves(c, s, lp, g, curr, s.moves, km, g.n - lp.ord.off_large, g.n - lp.ord.off_large2, tables);
+                set_new_cluster_ids(c, s, g, curr, s.moves, km, constrained ? cons : nullptr, ids, nfull);
+            fresh = !tables;
+            perform_moves(c, s, lp, g, curr, s.moves, km, g.n - lp.ord.off_large, g.n - lp.ord.off_large2, tables, nfull);
             if (stats) stats->moves += km;
             if (c.verbose >= 3)
                 fprintf(stderr, "sweep n=%lld it=%d cands=%lld moves=%lld labels=%d uncut=%lld obj=%.17g\n",
@@ -2412,7 +2420,7 @@ static void local_move_t(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g,
             tr.end(k, km);
         }
     }
-    relabel(c, s, n, best_part, best);
+    relabel(c, s, nfull, best_part, best);
     hub_tables_settle(c, lp);
 }
 
@@ -2494,7 +2502,7 @@ void local_move_strict(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, i
     bool tables = !is_initial;
     const i32* ccons = constrained ? cons : nullptr;
     Buf<float> sg(c, std::max<i64>(n, 1));
-    SweepTrace trc(c, g, 2);
+    SweepTrace trc(c, g, 2, n);
     for (int it = 0; it < 6; it++) {
         const float lam = (float)curr.lambda;
         trc.begin(s.dest, true);
@@ -2510,7 +2518,7 @@ void local_move_strict(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, i
             trc.end(0, 0);
             break;
         }
-        if (it > 0 || !is_initial) set_new_cluster_ids(c, s, g, curr, s.moves, k, constrained ? cons : nullptr, nullptr);
+        if (it > 0 || !is_initial) set_new_cluster_ids(c, s, g, curr, s.moves, k, constrained ? cons : nullptr, nullptr, n);
         fill_i64(c, s.prio, n, n + 1);
         k_prio<<<grid_items(k, 256), 256, 0, c.stream>>>(s.moves, k, s.prio);
         PGGC_LAUNCH_CHECK();
@@ -2524,7 +2532,7 @@ void local_move_strict(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, i
             trc.end(k, 0);
             break;
         }
-        perform_moves(c, s, lp, g, curr, s.moves, tr, g.n - lp.ord.off_large, g.n - lp.ord.off_large2, tables);
+        perform_moves(c, s, lp, g, curr, s.moves, tr, g.n - lp.ord.off_large, g.n - lp.ord.off_large2, tables, n);
         if (stats) stats->moves += tr;
         if (curr.obj > best.obj) {
             copy_state(c, best, curr);
@@ -2912,7 +2920,7 @@ void local_move_batch(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, co
             fill_i64(c, acc, K, 0);
             // resets the movers and their neighbours; every vertex of an
             // instance whose first moves these are follows below
-            apply_moves_core(c, s, lp, g, cvol, s.moves, km, n_large, n_massive, true, AccInst{bl.inst, acc});
+            apply_moves_core(c, s, lp, g, cvol, s.moves, km, n_large, n_massive, true, AccInst{bl.inst, acc}, n);
             bool anyfull = false;
             for (i64 q = 0; q < K; q++) {
                 const bool moved = hc[K + q] > 0;
