@@ -48,6 +48,7 @@ def test_improve_with_isolated_vertices(gpu_ctx, objective, labels, plus):
             st.uncut, st.label_count = uncut, L
             st.obj = float(uncut) - st.lambda_ * float(sq)
             print(f"improve {objective} {labels} plus={plus} renumber={knob}", flush=True)
+            C.check(gpu_ctx.lib.pggc_ctx_set_seed(gpu_ctx.h, 5, 0))  # the refinement's draws
             out = C.leiden_part(dg, st, plus=plus, improve=True, input=part)
             res.append((out.cpu().numpy(), st.obj, st.uncut, st.label_count))
         finally:
