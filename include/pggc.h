@@ -100,10 +100,10 @@ int pggc_ctx_set_verbose(pggc_ctx* ctx, int level);
  * resets the totals; kernel_stats waits for the stream and returns the
  * launches, summed milliseconds and summed algorithmic bytes of one slot. */
 #define PGGC_KS_SCORE_GROUP 0    /* neighbour-cluster scoring, d <= 64 */
-#define PGGC_KS_SCORE_TABLE 1    /* scoring with LDS tables, 64 < d <= 2048 */
-#define PGGC_KS_SCORE_HUB 2      /* hub scoring (HBM table build or scan), d > 2048 */
+#define PGGC_KS_SCORE_TABLE 1    /* scoring with one LDS table per vertex, 64 < d <= 8192 */
+#define PGGC_KS_SCORE_HUB 2      /* hub scoring (several LDS tables per vertex), d > 8192 */
 #define PGGC_KS_AFTERBURNER 3    /* conflict filter */
-#define PGGC_KS_MOVES 4          /* hub-table updates, exact uncut delta, volume moves */
+#define PGGC_KS_MOVES 4          /* exact uncut delta, destination resets, volume moves */
 #define PGGC_KS_CONTRACT_AGG 5   /* coarse-row merge in LDS */
 #define PGGC_KS_CONTRACT_BIG 6   /* coarse-row merge in HBM tables */
 #define PGGC_KS_CONTRACT_COPY 7  /* coarse-row copy-out */
@@ -137,10 +137,6 @@ int pggc_ctx_set_sweep_trace(pggc_ctx* ctx, pggc_sweep_fn fn, void* user);
 /* Tuning knobs of the HIP path (no counterpart in the reference, whose
  * equivalents are compile-time constants: src/header/ordering.h:17-19,
  * src/local_mover.cpp:985,1312).
- *   PGGC_KNOB_HUB_UPDATE_DIV: the hash tables of the highest-degree vertices
- *     are kept current from the movers while a sweep moves at most
- *     n / value vertices and rebuilt otherwise; 0 rebuilds every sweep.
- *     Default 32.
  *   PGGC_KNOB_GNN_MAX_SWEEPS: the active-set predictor runs on at most this
  *     many sweeps of a local-move call; 0 (default) runs it on every
  *     eligible sweep.  (It changes which vertices are pruned, so with
@@ -152,21 +148,14 @@ int pggc_ctx_set_sweep_trace(pggc_ctx* ctx, pggc_sweep_fn fn, void* user);
  *     scoring of vertices with 64 < degree <= 512: 64 (default), 128, 256.
  *   PGGC_KNOB_TABLE_SLOTS_PER_EDGE: LDS hash-table slots per edge of a degree
  *     class's bound, 64 < degree <= 2048: 2 (default) or 4.
- *   PGGC_KNOB_HUB_LDS_MAX_DEGREE: vertices of degree 2049..value are scored
- *     from an 8192-slot LDS table instead of an HBM hub table: 2048
- *     (default, none) or 4096.
- *   PGGC_KNOB_HUB_EDGES_PER_ITEM: edges per hub-table build work item:
- *     512, 1024 (default), 2048.
- *   PGGC_KNOB_HUB_SLOTS_PER_ITEM: hub-table slots per scan work item:
- *     2048, 4096 (default), 8192.
+ *   PGGC_KNOB_HUB_UPDATE_DIV, PGGC_KNOB_HUB_LDS_MAX_DEGREE (2048 or 4096),
+ *     PGGC_KNOB_HUB_EDGES_PER_ITEM (512, 1024, 2048),
+ *     PGGC_KNOB_HUB_SLOTS_PER_ITEM (2048, 4096, 8192) and PGGC_KNOB_HUB_BUILD:
+ *     accepted and kept, without effect: they shaped hash tables in device
+ *     memory for the highest degrees, which are now scored from LDS alone.
  *   PGGC_KNOB_RAW_SWEEPS: 1 (default) scores the first sweep of a local move
  *     from singletons on the raw adjacency (src/local_mover.cpp:1391-1395),
  *     0 with the neighbour-cluster tables (the same result, more work).
- *   PGGC_KNOB_HUB_BUILD: how HBM hub tables are built: 0 (default) one LDS
- *     slice of a table per block, written out whole (the largest tables by
- *     edge work items); 1 every table by edge work items adding into the HBM
- *     table with atomics; 2 the tables of odd hub index by edge items, the
- *     rest by slices (the same tables' contents in every mode).
  *   PGGC_KNOB_RENUMBER: where the local mover of a level runs: on an internal
  *     copy of the level with vertices in descending degree order (rows keep
  *     their entry order; labels, priorities and new cluster ids follow the

@@ -146,7 +146,7 @@ static Level top_level(const DGraph& g) {
 // On the way back up the hierarchy a level is done once its clustering is
 // projected onto the finer one: its graph, plan and clustering are freed,
 // so the finer levels' local moves have that memory (the whole hierarchy of
-// a billion-edge graph does not fit next to the top level's hub tables).
+// a billion-edge graph does not fit next to the top level's scratch).
 static void release_level(Level& l, Buf<i32>& part) {
     l.own.reset();
     l.plan.reset();

@@ -15,11 +15,11 @@ namespace pggc {
 // launches of the kernels named here, with the algorithmic bytes each launch
 // moves (measurement hooks; off unless enabled).
 enum KSlot {
-    KS_SCORE_GROUP = 0,  // k_score_group<G>
+    KS_SCORE_GROUP = 0,  // k_score_groups
     KS_SCORE_TABLE,      // k_score_table / k_score_raw (LDS tables, block arg-max)
-    KS_SCORE_HUB,        // hub scoring: table build (k_hub_insert), k_hub_pv, k_hub_scan, k_hub_decide
-    KS_AFTERBURNER,      // k_ab_pack + k_ab_serial / k_ab_wave / k_ab_block
-    KS_MOVES,            // hub-table updates + k_delta_uncut + k_apply_moves
+    KS_SCORE_HUB,        // hub scoring: k_hub_gather, k_hub_score (k_hub_raw), k_hub_decide
+    KS_AFTERBURNER,      // k_ab_small / k_ab_wave / k_ab_block
+    KS_MOVES,            // k_mvp_moves + k_move_edges + k_apply_moves
     KS_CONTRACT_AGG,     // k_cagg (LDS merge of coarse rows)
     KS_CONTRACT_BIG,     // k_cbig_insert + k_cbig_extract
     KS_CONTRACT_COPY,    // k_crow_copy
@@ -70,21 +70,14 @@ struct Ctx {
     void (*sweep_trace)(void*, const int64_t*, int) = nullptr;
     void* sweep_user = nullptr;
     double last_contract_s = 0.0, last_refine_s = 0.0;  // of the last clustering call
-    // tuning knobs (pggc_ctx_set_knob): hub tables are updated from the
-    // movers while a sweep moves at most n / hub_update_div vertices and
-    // rebuilt otherwise (0: always rebuilt)
-    i64 hub_update_div = 32;
-    // Execution-shape knobs of the scoring kernels (results do not depend on
-    // them; pggc_autotune picks them by timing):
+    // tuning knobs (pggc_ctx_set_knob); the execution shape of the scoring
+    // kernels does not change results, pggc_autotune picks it by timing:
     //   table_threads: threads per vertex of the LDS-table classes with
     //     64 < degree <= 512 (64, 128 or 256);
     //   table_spe: LDS hash-table slots per edge of a class's degree bound
     //     (2 or 4), classes 64 < degree <= 2048;
-    //   hub_lds_max: vertices of degree 2049..hub_lds_max are scored from an
-    //     8192-slot LDS table instead of an HBM hub table (2048 or 4096);
-    //   hub_edges_item / hub_slots_item: edges per hub-table build item
-    //     (512, 1024 or 2048) and table slots per hub scan item (2048, 4096
-    //     or 8192).
+    //   the hub knobs are kept for callers that set them and have no effect
+    i64 hub_update_div = 32;
     int table_threads = 64;
     int table_spe = 2;
     i64 hub_lds_max = 2048;
@@ -93,11 +86,9 @@ struct Ctx {
     // the first sweep of a call from singletons scores the raw adjacency
     // (every neighbour its own cluster); 0 scores it with the tables
     int raw_sweeps = 1;
-    // hub tables: 0 builds each table slice in LDS and writes it out whole,
-    // 1 adds edge work items into the HBM tables with atomics
     int hub_build = 0;
-    // the top level's local mover runs on a copy renumbered by degree:
-    // 0 never, 1 always, 2 when a call makes several top-level passes
+    // levels' local movers run on a copy renumbered by degree: 0 never, 1
+    // always, 2 where it pays
     int renumber = 2;
     // big-row contraction batches: table slots per batch (sort entries per
     // batch: a quarter of it)

@@ -44,49 +44,20 @@ struct LevelPlan {
     Orders ord;
     Buf<i32> sc_list;           // vertices grouped by scoring class
     i64 sc_start[NCLS + 1] = {0};
-    // hubs (largest degree class): HBM hash tables of neighbour-cluster
-    // weights (own cluster included), edge and slot work items per hub.
-    // A table is built at the first table sweep of a local-move call and
-    // then kept current by the movers of each sweep (weight moved from the
-    // old to the new cluster key), so later sweeps only scan it; a table that
-    // runs out of slots marks the set stale and the next sweep rebuilds it.
-    // packed: one u64 per slot (key << 32 | weight), used when every hub's
-    // row weight fits 32 bits; otherwise separate key / int64 weight arrays.
-    // A table is split into slices of at most hub_slice(packed) slots: a key
-    // probes within the slice its hash falls in, so a build holds one slice
-    // in LDS per block (soff: slice prefix per hub) and writes it out whole.
-    // A slice that cannot hold its keys (or the hub_build knob) sends its
-    // hub to the fallback build, edge items adding into the table with
-    // atomics and probing over the whole table: hflag[h] = 1, and hsm[h]
-    // (the slice mask every table user probes with) becomes the table mask.
-    // imap / smap / bmap: block -> build item, scan item or slice, so that
-    // all work of one hub runs on one XCD (blocks are dispatched round-robin
-    // over the 8 XCDs) and its table stays in that XCD's L2; -1 = idle block.
-    // hidx: vertex -> hub index, -1 for other vertices.
-    Buf<i64> goff, items, sitems, soff, hub_pv;
+    // hubs (the class above 2048, sorted by degree): the first nlds of them
+    // (degree <= 8192; the first nhalf <= 4096) are scored from LDS tables like
+    // the smaller classes, the others (from list entry hub0 on) by one block
+    // per slice of their clusters' hash range: hub_groups is the slice prefix
+    // over groups of 8 hubs, hub_blocks the grid, hub_eoff the prefix of their
+    // degrees (hub_edges in all).  hub_pv and hub_best are zero between sweeps.
+    Buf<i64> hub_groups, hub_pv, hub_eoff;
     Buf<u64> hub_best;
-    Buf<i32> gkeys;
-    Buf<i64> gvals;
-    Buf<u64> gtab;
-    Buf<i32> imap, smap, bmap, hidx, hflag, hovf;
-    Buf<u32> hsm;
-    // occupied-slot list per table (slot indices from goff[h] on, hcnt[h]
-    // of them, in no particular order): scans read occupied slots only
-    Buf<u32> hlist;
-    Buf<i32> hcnt;
-    bool packed = false;
-    bool hub_live = false;  // tables match the current clustering
-    i64 gslots = 0, nitems = 0, nsitems = 0, nslices = 0, igrid = 0, sgrid = 0, bgrid = 0;
-    i64 hs1 = 0, hs2 = 0;  // slice-class bounds (xcd_maps)
-    i64 hg = 0, ghg = 0, ihg = 0, shg = 0;  // first fallback-built hub, its first slot, build item and slice
-    // the hub class is sorted by degree; its first nlds vertices (degree <=
-    // Ctx::hub_lds_max) are scored in LDS, the rest (from hub0 on) in HBM
-    // tables; he / hs: edges per build item and slots per scan item
+    i64 hub_blocks = 0, hub_edges = 0, nhalf = 0;
+    bool hub32 = false;   // their row sums fit 32 bits
     u64 epoch = ~(u64)0;
     i64 nlds = 0, hub0 = 0, nhub = 0;
-    bool agg32 = false;  // sums of rows of degree <= 4096 fit 32 bits
+    bool agg32 = false;  // sums of rows of degree <= 8192 fit 32 bits
     i64 max_deg = 0;  // of the hub class (0 without hubs)
-    i64 he = 1024, hs = 4096;
 };
 
 // Device scratch sized for the top level, shared by every level.
@@ -109,6 +80,7 @@ struct MoveScratch {
     Buf<u64> mvp;  // per vertex: cluster | moved << 31, and the cluster after this sweep's moves
     Buf<u64> rec;     // per vertex: cluster and its volume as fp32 (scoring)
     Buf<uint4> rec16; // the same with the cluster's constraint value, when there is one
+    Buf<u64> hub_kv;  // the large hubs' gathered records, while a local move runs
     Buf<u64> sqpart;  // partial sums of k_finish
     Buf<i32> part, dest, cand, moves, flag, tmp, tmp2;
     Buf<float> gain;

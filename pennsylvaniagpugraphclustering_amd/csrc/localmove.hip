@@ -39,9 +39,8 @@ void update_objective(Ctx& c, RefineData& rd) {
 
 // ------------------------------------------------------------- scratch
 // Scalars of a sweep in MoveScratch::scal, zeroed at the start of a call:
-// SC_STALE and the MV_SLOTS words of the uncut change are zero between sweeps,
-// SC_TICKET counts k_finish's blocks (at most FIN_BLOCKS).
-constexpr int SC_STALE = 3, SC_TICKET = 4, SC_SLOTS = 16, MV_SLOTS = 64, SC_COUNT = SC_SLOTS + MV_SLOTS;
+// the MV_SLOTS words of the uncut change are zero between sweeps, SC_TICKET counts k_finish's blocks (at most FIN_BLOCKS).
+constexpr int SC_TICKET = 4, SC_SLOTS = 16, MV_SLOTS = 64, SC_COUNT = SC_SLOTS + MV_SLOTS;
 constexpr int FIN_BLOCKS = 256;
 void MoveScratch::ensure(Ctx& c, i64 n) {
     if (cap >= n) return;
@@ -72,51 +71,59 @@ __host__ __device__ __forceinline__ int score_class(i64 d) {
 // (the chip holds 5 of its 256-thread blocks per CU, 1,280 at once, so two
 // rounds of blocks cost less than the four launches saved).
 constexpr i64 TABLE_ONE_LAUNCH = 2048;
-// LDS table of a vertex of degree d: the power of two >= spe * d slots
-__host__ __device__ __forceinline__ i64 tslots(i64 d, int spe) {
-    i64 s = 2;
+// LDS table of a vertex of degree d: the power of two >= spe * d slots, at most
+// `most`
+__host__ __device__ __forceinline__ int tslots(i64 d, int spe, int most) {
+    int s = 2;
     while (s < spe * d) s <<= 1;
-    return s;
+    return s < most ? s : most;
 }
-// vertices of the hub class scored from an LDS table (degree <= HUB_LDS_BOUND)
-constexpr i64 HUB_LDS_BOUND = 4096;
-// HBM hub tables: power of two >= 1.5 d, so at most 2/3 full (a hub has at
-// most d distinct neighbour clusters); every probe loop ends at an empty slot
-__host__ __device__ __forceinline__ i64 hub_slots(i64 d) {
-    i64 s = 2;
-    while (2 * s < 3 * d) s <<= 1;
-    return s;
-}
+// Vertices of the hub class scored from one LDS table each: degree at most
+// HUB_HALF from 8,192 slots (two blocks per CU with 32-bit sums), at most
+// HUB_LDS_BOUND from 10,112 slots, which is the most that still lets two
+// 1,024-thread blocks share a CU's LDS (at most 81% full)
+constexpr i64 HUB_HALF = 4096, HUB_LDS_BOUND = 8192;
+constexpr int HUB_LDS_SLOTS = 10112;
+// Larger hubs (k_hub_score): slots of the LDS table of one slice, 12 bytes each
+// with 32-bit sums, 16 with 64-bit ones (144 and 128 KB of LDS), and the
+// slices of a hub: 1.5 slots per edge, so a slice is at most 2/3 full on average
+constexpr int HUB_SLOTS32 = 12288, HUB_SLOTS64 = 8192;
+__host__ __device__ __forceinline__ i64 hub_slices(i64 d, int slots) { return (3 * d + 2 * slots - 1) / (2 * slots); }
 
 __global__ void k_score_classes(const i64* rp, i64 n, i32* cls) {
     const i64 i = thread_item();
     if (i >= n) return;
     cls[i] = score_class(rp[i + 1] - rp[i]);
 }
-__global__ void k_global_sizes(const i64* rp, const i32* list, i64 m, i64 he, i64* sz, i64* items) {
+// Work of the large hubs: groups of NXCD consecutive hubs (sorted by degree, so
+// of similar size), each hub with as many blocks as the group's largest hub
+// has slices.  Block ids go round-robin over the XCDs, so with the blocks of a
+// group interleaved all slices of one hub run on one XCD and read the hub's
+// edges and records through its L2.
+constexpr int NXCD = 8;
+__global__ void k_hub_groups(const i64* rp, const i32* hubs, i64 m, int slots, i64* gs) {
+    const i64 g = thread_item();
+    if (g >= (m + NXCD - 1) / NXCD) return;
+    const i64 last = (g + 1) * NXCD < m ? (g + 1) * NXCD - 1 : m - 1;
+    const i32 i = hubs[last];
+    gs[g] = hub_slices(rp[i + 1] - rp[i], slots);
+}
+// block -> hub and slice; false for padding.  The largest hubs come first.
+__global__ void k_hub_degrees(const i64* rp, const i32* hubs, i64 m, i64* deg) {
     const i64 x = thread_item();
     if (x >= m) return;
-    i32 i = list[x];
-    i64 d = rp[i + 1] - rp[i];
-    sz[x] = hub_slots(d);
-    items[x] = (d + he - 1) / he;
+    deg[x] = rp[hubs[x] + 1] - rp[hubs[x]];
 }
-__global__ void k_slot_items(const i64* goff, i64 m, i64 hs, i64* sitems) {
-    const i64 x = thread_item();
-    if (x >= m) return;
-    sitems[x] = (goff[x + 1] - goff[x] + hs - 1) / hs;
+__device__ __forceinline__ bool hub_block(const i64* gpre, i64 ng, i64 m, i64 bid, i64 nblk, i64& h, i64& sl) {
+    if (bid >= nblk) return false;
+    const i64 b = nblk - 1 - bid;
+    const i64 q = b / NXCD;
+    const i64 g = upper_row(gpre, 0, ng, q);
+    h = g * NXCD + b % NXCD;
+    sl = q - gpre[g];
+    return h < m;
 }
-// Slots per hub-table slice: one slice is built in LDS by one block, 128 KB
-// of LDS for packed u64 slots, 96 KB for separate i32 keys and i64 weights.
-constexpr i64 HUB_SLICE_PACKED = 16384, HUB_SLICE_WIDE = 8192;
-constexpr i64 HUB_MAX_SLICES = 16;  // larger tables are built by the fallback
-__host__ __device__ __forceinline__ i64 hub_slice(bool packed) { return packed ? HUB_SLICE_PACKED : HUB_SLICE_WIDE; }
-__global__ void k_slice_counts(const i64* goff, i64 m, i64 sl, i64* soff) {
-    const i64 x = thread_item();
-    if (x >= m) return;
-    const i64 S = goff[x + 1] - goff[x];
-    soff[x] = S > sl ? S / sl : 1;
-}
+
 __global__ void k_hub_deg_keys(const i64* rp, const i32* list, i64 m, u64* keys, i32* vals) {
     const i64 x = thread_item();
     if (x >= m) return;
@@ -124,9 +131,11 @@ __global__ void k_hub_deg_keys(const i64* rp, const i32* list, i64 m, u64* keys,
     keys[x] = (u64)(rp[i + 1] - rp[i]);
     vals[x] = i;
 }
-// first x with degree(list[x]) > bound (list sorted by degree)
-__global__ void k_first_above(const i64* rp, const i32* list, i64 m, i64 bound, i64* out) {
-    if (threadIdx.x != 0) return;
+// of a list sorted by degree: out[0] and out[1] = first x with degree(list[x]) >
+// HUB_HALF and HUB_LDS_BOUND, out[2] = the largest degree
+__global__ void k_hub_shape(const i64* rp, const i32* list, i64 m, i64* out) {
+    if (threadIdx.x >= 2) return;
+    const i64 bound = threadIdx.x == 0 ? HUB_HALF : HUB_LDS_BOUND;
     i64 lo = 0, hi = m;
     while (lo < hi) {
         const i64 mid = (lo + hi) >> 1;
@@ -134,108 +143,8 @@ __global__ void k_first_above(const i64* rp, const i32* list, i64 m, i64 bound, 
         if (rp[i + 1] - rp[i] > bound) hi = mid;
         else lo = mid + 1;
     }
-    *out = lo;
-}
-
-__global__ void k_list_degree(const i64* rp, const i32* entry, i64* out) {
-    if (threadIdx.x == 0) *out = rp[*entry + 1] - rp[*entry];
-}
-
-// row weight of each hub (one block per edge item)
-template <class WT>
-__global__ void __launch_bounds__(256) k_hub_wsum(const i64* __restrict__ rp, WT W, const i32* __restrict__ hubs,
-                                                  i64 m, const i64* __restrict__ items, i64 he, i64* hsum) {
-    const i64 b = block_id();
-    if (b >= items[m]) return;
-    const i64 hi = upper_row(items, 0, m, b);
-    const i32 i = hubs[hi];
-    const i64 e = rp[i + 1];
-    const i64 j_lo = rp[i] + (b - items[hi]) * he;
-    const i64 j_hi = j_lo + he < e ? j_lo + he : e;
-    i64 acc = 0;
-    for (i64 jb = j_lo; jb < j_hi; jb += 256) {
-        const i64 j = jb + threadIdx.x;
-        if (j < j_hi) acc += W(j);
-    }
-    acc = block_sum_i64<256>(acc);
-    if (threadIdx.x == 0) atomicAdd((unsigned long long*)&hsum[hi], (unsigned long long)acc);
-}
-
-// Block -> work-item maps that keep each hub on one XCD: hubs are assigned
-// longest-first to the least loaded of the 8 XCDs (load = insert items + scan
-// items); block 8k + x runs the k-th item of XCD x.
-constexpr int NXCD = 8;
-static void build_map(const std::vector<i64>& pre, const std::vector<int>& xcd_of, i64 m, std::vector<i32>& map,
-                      i64& grid, i64 lo = 0, bool largest_first = false) {
-    std::vector<std::vector<i32>> per(NXCD);
-    for (i64 k = 0; k < m; k++) {
-        const i64 h = largest_first ? m - 1 - k : k;  // hubs are sorted by degree
-        for (i64 it = std::max(pre[h], lo); it < pre[h + 1]; it++) per[xcd_of[h]].push_back((i32)it);
-    }
-    size_t mx = 0;
-    for (auto& v : per) mx = std::max(mx, v.size());
-    grid = (i64)mx * NXCD;
-    map.assign(std::max<i64>(grid, 1), -1);
-    for (int x = 0; x < NXCD; x++)
-        for (size_t k = 0; k < per[x].size(); k++) map[k * NXCD + x] = per[x][k];
-}
-
-static void xcd_maps(Ctx& c, LevelPlan& p, i64 m) {
-    std::vector<i64> it(m + 1), st(m + 1), so(m + 1), go(m + 1);
-    PGGC_HIP(hipMemcpyAsync(go.data(), p.goff, (m + 1) * sizeof(i64), hipMemcpyDeviceToHost, c.stream));
-    PGGC_HIP(hipMemcpyAsync(it.data(), p.items, (m + 1) * sizeof(i64), hipMemcpyDeviceToHost, c.stream));
-    PGGC_HIP(hipMemcpyAsync(st.data(), p.sitems, (m + 1) * sizeof(i64), hipMemcpyDeviceToHost, c.stream));
-    PGGC_HIP(hipMemcpyAsync(so.data(), p.soff, (m + 1) * sizeof(i64), hipMemcpyDeviceToHost, c.stream));
-    c.sync();
-    std::vector<i64> order(m);
-    for (i64 h = 0; h < m; h++) order[h] = h;
-    auto load = [&](i64 h) { return (it[h + 1] - it[h]) + (st[h + 1] - st[h]); };
-    std::stable_sort(order.begin(), order.end(), [&](i64 a, i64 b) { return load(a) > load(b); });
-    std::vector<i64> tot(NXCD, 0);
-    std::vector<int> xcd_of(m, 0);
-    for (i64 h : order) {
-        int best = 0;
-        for (int x = 1; x < NXCD; x++)
-            if (tot[x] < tot[best]) best = x;
-        xcd_of[h] = best;
-        tot[best] += load(h);
-    }
-    std::vector<i32> imap, smap;
-    build_map(it, xcd_of, m, imap, p.igrid);
-    p.imap = Buf<i32>(c, imap.size());
-    copy_h2d(c, p.imap, imap.data(), imap.size() * sizeof(i32));
-    build_map(st, xcd_of, m, smap, p.sgrid);
-    p.smap = Buf<i32>(c, smap.size());
-    copy_h2d(c, p.smap, smap.data(), smap.size() * sizeof(i32));
-    // slice classes (hubs are sorted by degree, so table sizes ascend):
-    // [0, hs1) tables of at most 4096 slots, [hs1, hs2) packed tables of
-    // 8192, then the tables of more slots than one block's slice class
-    // (several slices each), which go through the XCD map
-    auto first_above = [&](i64 slots) {
-        i64 h = 0;
-        while (h < m && go[h + 1] - go[h] <= slots) h++;
-        return so[h];
-    };
-    p.hs1 = first_above(4096);
-    p.hs2 = p.packed ? first_above(8192) : p.hs1;
-    // the largest hubs (more than HUB_MAX_SLICES slices) are built by the
-    // fallback: first such hub, its first table slot and first build item
-    p.hg = 0;
-    while (p.hg < m && go[p.hg + 1] - go[p.hg] <= HUB_MAX_SLICES * hub_slice(p.packed)) p.hg++;
-    p.ghg = go[p.hg];
-    p.ihg = it[p.hg];
-    p.shg = so[p.hg];
-    std::vector<i32> bmap;
-    build_map(so, xcd_of, m, bmap, p.bgrid, p.hs2, true);
-    if (p.hs2 == so[m]) p.bgrid = 0;
-    p.bmap = Buf<i32>(c, bmap.size());
-    copy_h2d(c, p.bmap, bmap.data(), bmap.size() * sizeof(i32));
-}
-
-__global__ void k_hub_index(const i32* hubs, i64 m, i32* hidx) {
-    const i64 x = thread_item();
-    if (x >= m) return;
-    hidx[hubs[x]] = (i32)x;
+    out[threadIdx.x] = lo;
+    out[2] = rp[list[m - 1] + 1] - rp[list[m - 1]];
 }
 
 void plan_level(Ctx& c, const DGraph& g, LevelPlan& p) {
@@ -243,8 +152,6 @@ void plan_level(Ctx& c, const DGraph& g, LevelPlan& p) {
     p.key = g.rp;
     p.n = g.n;
     p.epoch = c.knob_epoch;
-    p.he = c.hub_edges_item;
-    p.hs = c.hub_slots_item;
     make_orders(c, g, p.ord);
     Buf<i32> cls(c, std::max<i64>(g.n, 1));
     p.sc_list = Buf<i32>(c, std::max<i64>(g.n, 1));
@@ -255,119 +162,53 @@ void plan_level(Ctx& c, const DGraph& g, LevelPlan& p) {
     // LDS form a prefix; every hub is scored on its own, so the order within
     // the class does not change results
     const i64 nh = p.sc_start[CL_HUB + 1] - p.sc_start[CL_HUB];
-    p.nlds = 0;
-    if (nh > 1) {
+    p.nlds = p.nhalf = 0;
+    p.max_deg = 0;
+    if (nh > 0) {
         i32* hl = p.sc_list.p + p.sc_start[CL_HUB];
         Buf<u64> hk(c, nh);
+        Buf<i64> f(c, 3);
         k_hub_deg_keys<<<grid_items(nh, 256), 256, 0, c.stream>>>(g.rp, hl, nh, hk, hl);
         PGGC_LAUNCH_CHECK();
         radix_sort_pairs(c, hk, hl, nh, 40);
-    }
-    if (nh > 0 && c.hub_lds_max > 2048) {
-        Buf<i64> f(c, 1);
-        k_first_above<<<1, 64, 0, c.stream>>>(g.rp, p.sc_list.p + p.sc_start[CL_HUB], nh,
-                                               std::min<i64>(c.hub_lds_max, HUB_LDS_BOUND), f);
+        k_hub_shape<<<1, 64, 0, c.stream>>>(g.rp, hl, nh, f);
         PGGC_LAUNCH_CHECK();
-        p.nlds = c.read1(f);
+        const i64* h = c.read(f, 3);
+        p.nhalf = h[0];
+        p.nlds = h[1];
+        p.max_deg = h[2];
     }
     // 32-bit sums for the rows scored in registers and LDS (degree at most
-    // HUB_LDS_BOUND): unit weights, a level whose weights sum to less than
-    // 2^32 (contracted from a unit-weight graph), or small weights
-    p.agg32 = g.wk == W_UNIT || g.wsmall;
+    // HUB_LDS_BOUND) and for the larger hubs: unit weights, a level whose
+    // weights sum to less than 2^32 (contracted from a unit-weight graph), or
+    // weights small enough for the degrees
+    p.agg32 = p.hub32 = g.wk == W_UNIT || g.wsmall;
     if (!p.agg32 && g.nnz > 0) {
         const u64 mx = max_weight(c, g);
         p.agg32 = mx <= 0xffffffffull / HUB_LDS_BOUND;
+        p.hub32 = mx <= 0xffffffffull / (u64)std::max(p.max_deg, HUB_LDS_BOUND);
     }
     p.hub0 = p.sc_start[CL_HUB] + p.nlds;
     p.nhub = nh - p.nlds;
-    const i64 m7 = p.nhub;
-    p.gslots = 0;
-    p.max_deg = 0;
-    if (nh > 0) {  // (the hub class is sorted by degree)
-        Buf<i64> f(c, 1);
-        k_list_degree<<<1, 64, 0, c.stream>>>(g.rp, p.sc_list.p + p.sc_start[CL_HUB] + nh - 1, f);
+    p.hub_blocks = 0;
+    if (p.nhub > 0) {
+        const i64 ng = ceil_div(p.nhub, NXCD);
+        p.hub_groups = Buf<i64>(c, ng + 1);
+        p.hub_pv = Buf<i64>(c, p.nhub);
+        p.hub_best = Buf<u64>(c, p.nhub);
+        k_hub_groups<<<grid_items(ng, 256), 256, 0, c.stream>>>(g.rp, p.sc_list.p + p.hub0, p.nhub,
+                                                                p.hub32 ? HUB_SLOTS32 : HUB_SLOTS64, p.hub_groups);
         PGGC_LAUNCH_CHECK();
-        p.max_deg = c.read1(f);
+        scan_i64(c, p.hub_groups, p.hub_groups, ng);
+        p.hub_eoff = Buf<i64>(c, p.nhub + 1);
+        k_hub_degrees<<<grid_items(p.nhub, 256), 256, 0, c.stream>>>(g.rp, p.sc_list.p + p.hub0, p.nhub, p.hub_eoff);
+        PGGC_LAUNCH_CHECK();
+        scan_i64(c, p.hub_eoff, p.hub_eoff, p.nhub);
+        fill_i64(c, (i64*)p.hub_best.p, p.nhub, 0);  // zero between sweeps (k_hub_decide)
+        fill_i64(c, p.hub_pv, p.nhub, 0);
+        p.hub_blocks = c.read1(p.hub_groups.p + ng) * NXCD;
+        p.hub_edges = c.read1(p.hub_eoff.p + p.nhub);
     }
-    if (m7 > 0) {
-        p.goff = Buf<i64>(c, m7 + 1);
-        p.items = Buf<i64>(c, m7 + 1);
-        p.sitems = Buf<i64>(c, m7 + 1);
-        p.hub_pv = Buf<i64>(c, m7);
-        p.hub_best = Buf<u64>(c, m7);
-        k_global_sizes<<<grid_items(m7, 256), 256, 0, c.stream>>>(g.rp, p.sc_list.p + p.hub0, m7, p.he, p.goff,
-                                                                        p.items);
-        PGGC_LAUNCH_CHECK();
-        scan_i64(c, p.goff, p.goff, m7);
-        scan_i64(c, p.items, p.items, m7);
-        k_slot_items<<<grid_items(m7, 256), 256, 0, c.stream>>>(p.goff, m7, p.hs, p.sitems);
-        PGGC_LAUNCH_CHECK();
-        scan_i64(c, p.sitems, p.sitems, m7);
-        p.gslots = c.read1(p.goff.p + m7);
-        p.nitems = c.read1(p.items.p + m7);
-        p.nsitems = c.read1(p.sitems.p + m7);
-        const i32* hubs = p.sc_list.p + p.hub0;
-        // packed slots need every hub row weight below 2^32
-        p.packed = true;
-        if (g.wk != W_UNIT) {
-            Buf<i64> hsum(c, m7);
-            fill_i64(c, hsum, m7, 0);
-            PGGC_WDISPATCH(g, (k_hub_wsum<<<grid_blocks(p.nitems), 256, 0, c.stream>>>(g.rp, W, hubs, m7, p.items,
-                                                                                    p.he, hsum)));
-            PGGC_LAUNCH_CHECK();
-            std::vector<i64> hs(m7);
-            PGGC_HIP(hipMemcpyAsync(hs.data(), hsum, m7 * sizeof(i64), hipMemcpyDeviceToHost, c.stream));
-            c.sync();
-            for (i64 x = 0; x < m7; x++)
-                if (hs[x] >= ((i64)1 << 32) - 1) p.packed = false;
-        }
-        // the tables themselves (and their slot lists) are allocated by
-        // hub_tables_acquire when a local move starts
-        p.gtab.reset();
-        p.gkeys.reset();
-        p.gvals.reset();
-        p.hlist.reset();
-        p.soff = Buf<i64>(c, m7 + 1);
-        k_slice_counts<<<grid_items(m7, 256), 256, 0, c.stream>>>(p.goff, m7, hub_slice(p.packed), p.soff);
-        PGGC_LAUNCH_CHECK();
-        scan_i64(c, p.soff, p.soff, m7);
-        p.nslices = c.read1(p.soff.p + m7);
-        p.hflag = Buf<i32>(c, m7);
-        p.hovf = Buf<i32>(c, 1);
-        p.hcnt = Buf<i32>(c, m7);
-        p.hsm = Buf<u32>(c, m7);
-        xcd_maps(c, p, m7);
-        p.hidx = Buf<i32>(c, std::max<i64>(g.n, 1));
-        fill_i32(c, p.hidx, g.n, -1);
-        k_hub_index<<<grid_items(m7, 256), 256, 0, c.stream>>>(hubs, m7, p.hidx);
-        PGGC_LAUNCH_CHECK();
-    }
-    p.hub_live = false;
-}
-
-// Hub tables and slot lists, the bulk of a plan (about 1.5-3 slots per hub
-// edge), exist only while a local move of the level runs; they are rebuilt
-// at the first table sweep of every call anyway.  Released at the end of
-// the call (to the context's cache, which usually hands the same block back
-// at the level's next call), they leave the room to the contraction and the
-// other levels of the hierarchy on graphs of billions of edges.
-static void hub_tables_acquire(Ctx& c, LevelPlan& p) {
-    if (p.nhub == 0 || p.gslots == 0) return;
-    if (p.packed) {
-        if (!p.gtab.p) p.gtab = Buf<u64>(c, p.gslots);
-    } else if (!p.gkeys.p) {
-        p.gkeys = Buf<i32>(c, p.gslots);
-        p.gvals = Buf<i64>(c, p.gslots);
-    }
-    if (!p.hlist.p) p.hlist = Buf<u32>(c, p.gslots);
-}
-static void hub_tables_settle(Ctx& c, LevelPlan& p) {
-    (void)c;
-    p.gtab.reset();
-    p.gkeys.reset();
-    p.gvals.reset();
-    p.hlist.reset();
-    p.hub_live = false;
 }
 
 // ------------------------------------------------------------- scoring
@@ -696,8 +537,8 @@ __global__ void __launch_bounds__(256) k_score_groups(const i64* __restrict__ rp
 #undef PGGC_GROUP
 }
 
-// One block per vertex with a hash table in LDS: SLOTS slots hold the table
-// of any degree up to SLOTS / SPE, each table the power of two >= SPE * degree.
+// One block per vertex with a hash table in LDS, for degrees up to D: the power
+// of two >= SPE * degree slots, at most SLOTS (> D).
 // A thread gathers the records of all its (at most R) edges first, so the
 // gathers are in flight together, inserts them, and after the barrier looks
 // each edge's slot up again: its record still holds the cluster's volume, so
@@ -707,18 +548,18 @@ __global__ void __launch_bounds__(256) k_score_groups(const i64* __restrict__ rp
 // 65..2048 classes went from 148 to 93 ms on R-MAT scale 24 (two passes) and
 // from 147 to 78 ms on scale 20.
 template <class AT>
-__device__ __forceinline__ u32 table_add_slot(i32* keys, AT* vals, u32 mask, i32 key, AT w) {
-    u32 h = slot_hash(key, mask);
-    while (true) {  // at most mask / SPE keys: an empty slot is always found
+__device__ __forceinline__ u32 table_add_slot(i32* keys, AT* vals, u32 S, i32 key, AT w) {
+    u32 h = __umulhi((u32)key * 0x9E3779B1u, S);
+    while (true) {  // fewer keys than slots: an empty slot is always found
         const i32 old = atomicCAS(&keys[h], EMPTY_KEY, key);
         if (old == EMPTY_KEY || old == key) break;
-        h = (h + 1) & mask;
+        h = h + 1 < S ? h + 1 : 0;
     }
     if (sizeof(AT) == 4) atomicAdd((u32*)&vals[h], (u32)w);
     else atomicAdd((unsigned long long*)&vals[h], (unsigned long long)w);
     return h;
 }
-template <int BS, int SLOTS, int SPE, class AT, class WT, class LT>
+template <int BS, int D, int SLOTS, int SPE, class AT, class WT, class LT>
 __global__ void __launch_bounds__(BS) k_score_table(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
                                                     const i64* __restrict__ vw, const i32* __restrict__ list, i64 m,
                                                     const i32* __restrict__ part, const i64* __restrict__ vol,
@@ -726,7 +567,7 @@ __global__ void __launch_bounds__(BS) k_score_table(const i64* __restrict__ rp, 
                                                     ScoreOut out) {
     __shared__ i32 keys[SLOTS];
     __shared__ AT vals[SLOTS];
-    constexpr int R = (SLOTS / SPE + BS - 1) / BS;
+    constexpr int R = (D + BS - 1) / BS;
     const int t = threadIdx.x;
     const i64 li = block_id();
     if (li >= m) return;
@@ -734,8 +575,7 @@ __global__ void __launch_bounds__(BS) k_score_table(const i64* __restrict__ rp, 
     if (out.dest[i] == NO_MOVE) return;
     const i64 s = rp[i];
     const int d = (int)(rp[i + 1] - s);
-    const int S = (int)tslots(d, SPE);
-    const u32 mask = (u32)(S - 1);
+    const int S = tslots(d, SPE, SLOTS);
     const i32 p = part[i];
     const i64 wi = vw[i];
     NbRec r[R];
@@ -762,7 +602,7 @@ __global__ void __launch_bounds__(BS) k_score_table(const i64* __restrict__ rp, 
         h[q] = 0;
         if (r[q].part == EMPTY_KEY) continue;
         if (r[q].part == p) pv += w[q];
-        else h[q] = table_add_slot(keys, vals, mask, r[q].part, w[q]);
+        else h[q] = table_add_slot(keys, vals, (u32)S, r[q].part, w[q]);
     }
     pv = block_reduce<BS>(pv, [](AT a, AT b) { return a + b; });
     __syncthreads();
@@ -840,407 +680,220 @@ __global__ void __launch_bounds__(BS) k_score_raw(const i64* __restrict__ rp, co
     if (threadIdx.x == 0) decide(i, p_conn, bk, p, wi, out);
 }
 
-// hubs: one block per edge item, folded into hub_best with atomicMax
-template <class WT, class LT>
-__global__ void __launch_bounds__(256) k_hub_raw(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
-                                                 const i64* __restrict__ vw, const i32* __restrict__ hubs, i64 m,
-                                                 const i64* __restrict__ items, const i32* __restrict__ part,
-                                                 const i64* __restrict__ vol, RecView rv,
-                                                 const i32* __restrict__ cons, LT lam, float ratio,
-                                                 const i32* __restrict__ dest, i64 he, u64* hub_best) {
-    const i64 b = block_id();
-    if (b >= items[m]) return;
-    const i64 hi = upper_row(items, 0, m, b);
-    const i32 i = hubs[hi];
+// Hubs of degree above HUB_LDS_BOUND: a block per slice of a hub's hash range
+// (hub_block), folded into hub_best with atomicMax.
+//
+// First the hubs' edges are gathered: k_hub_gather leaves the (cluster, volume)
+// record of every edge at hub_eoff[h] + edge, so that each edge costs one
+// random access, and sums the own-cluster weights, which the candidates'
+// threshold needs (own edges and edges that the constraint rules out are left
+// empty).  A slice block then streams all of its hub's records (the slices of
+// one hub share an XCD's L2), keeps the clusters whose hash falls in its slice
+// in an LDS table with their weight and volume, and takes the best candidate
+// from the table.  Nothing but the best candidate leaves the chip.  LDS limits
+// it to one 1024-thread block per CU.  With tables in HBM, built slice by slice
+// and kept current from the movers, the same scoring wrote and listed 1.5-3
+// slots per edge, gathered a volume per cluster, and the updates were a chain of
+// dependent atomics per mover edge: scoring all degrees above
+// 2048 and the updates took about 200 ms on R-MAT scale 24 (two passes), now 135
+// (78 here: 64M edges gathered in 0.6 ms and streamed 5.7 times each in 1.2 ms a
+// sweep, 57 in the LDS tables of the degrees up to 8192).  Without the gather
+// pass, each slice reading records at random, a sweep took 3.0 ms.
+//
+// The hash is a bijection of the 32-bit id, split by range: a slice whose keys
+// do not fit (never seen with 1.5 slots per edge) is done again in 2, 4, ...
+// parts, which ends at the latest when a part covers fewer ids than slots.
+__device__ __forceinline__ u32 mix32(u32 x) {  // the finalizer of MurmurHash3
+    x ^= x >> 16;
+    x *= 0x85ebca6bu;
+    x ^= x >> 13;
+    x *= 0xc2b2ae35u;
+    x ^= x >> 16;
+    return x;
+}
+// the share [j_lo, j_hi) of a hub's edges that block sl of ns handles
+__device__ __forceinline__ void hub_share(i64 s, i64 e, i64 ns, i64 sl, i64& j_lo, i64& j_hi) {
+    const i64 share = (e - s + ns - 1) / ns;
+    j_lo = s + sl * share;
+    j_hi = j_lo + share < e ? j_lo + share : e;
+}
+template <int SL, class WT>
+__global__ void __launch_bounds__(256) k_hub_gather(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
+                                                    const i32* __restrict__ hubs, i64 m, const i64* __restrict__ gpre,
+                                                    i64 ng, i64 nblk, const i64* __restrict__ eoff,
+                                                    const i32* __restrict__ part, RecView rv,
+                                                    const i32* __restrict__ cons, const i32* __restrict__ dest,
+                                                    u64* __restrict__ kv, i64* hub_pv) {
+    i64 h, sl;
+    if (!hub_block(gpre, ng, m, block_id(), nblk, h, sl)) return;
+    const i32 i = hubs[h];
     if (dest[i] == NO_MOVE) return;
     const i64 s = rp[i], e = rp[i + 1];
-    const i64 j_lo = s + (b - items[hi]) * he;
-    const i64 j_hi = j_lo + he < e ? j_lo + he : e;
+    const i64 ns = hub_slices(e - s, SL);
+    if (sl >= ns) return;
+    i64 j_lo, j_hi;
+    hub_share(s, e, ns, sl, j_lo, j_hi);
+    const i32 p = part[i];
+    const i32 cp = cons ? cons[p] : 0;
+    u64* out = kv + eoff[h];
+    const int t = threadIdx.x;
+    i64 own = 0;
+    constexpr int U = 8;  // edges in flight per thread
+    for (i64 jb = j_lo; jb < j_hi; jb += 256 * U) {  // block-uniform loop control
+        i32 v[U];
+        NbRec r[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) v[u] = jb + u * 256 + t < j_hi ? col[jb + u * 256 + t] : -1;
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (v[u] >= 0) r[u] = load_rec(rv, v[u]);
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (v[u] < 0) continue;
+            const i64 j = jb + u * 256 + t;
+            if (r[u].part == p) own += W(j);
+            const i32 key = (r[u].part == p || r[u].cons != cp) ? EMPTY_KEY : r[u].part;
+            out[j - s] = (u64)(u32)key | ((u64)__float_as_uint(r[u].volf) << 32);
+        }
+    }
+    own = block_sum_i64<256>(own);
+    if (t == 0 && own) atomicAdd((unsigned long long*)&hub_pv[h], (unsigned long long)own);
+}
+
+template <int SL, int BS, class AT, class WT, class LT>
+__global__ void __launch_bounds__(BS) k_hub_score(const i64* __restrict__ rp, WT W, const i64* __restrict__ vw,
+                                                  const i32* __restrict__ hubs, i64 m, const i64* __restrict__ gpre,
+                                                  i64 ng, i64 nblk, const i64* __restrict__ eoff,
+                                                  const i32* __restrict__ part, const i64* __restrict__ vol, LT lam,
+                                                  float ratio, const i32* __restrict__ dest,
+                                                  const u64* __restrict__ kv, const i64* __restrict__ hub_pv,
+                                                  u64* hub_best) {
+    __shared__ i32 lk[SL];
+    __shared__ AT lv[SL];
+    __shared__ float lf[SL];
+    __shared__ int full;
+    i64 h, sl;
+    if (!hub_block(gpre, ng, m, block_id(), nblk, h, sl)) return;
+    const i32 i = hubs[h];
+    if (dest[i] == NO_MOVE) return;
+    const i64 s = rp[i], d = rp[i + 1] - s;
+    const i64 ns = hub_slices(d, SL);
+    if (sl >= ns) return;
+    const int t = threadIdx.x;
+    const u64* in = kv + eoff[h];
+    float multi, p_conn, b;
+    own_terms(hub_pv[h], vol[part[i]], vw[i], lam(i), lam.rt(i, ratio), multi, p_conn, b);
+    u64 bk = 0;
+    for (u64 parts = 1;; parts *= 2) {  // block-uniform
+        bool over = false;
+        bk = 0;
+        for (u64 part_no = 0; part_no < parts; part_no++) {
+            const u64 total = (u64)ns * parts, want = (u64)sl * parts + part_no;
+            for (int q = t; q < SL; q += BS) {
+                lk[q] = EMPTY_KEY;
+                lv[q] = 0;
+            }
+            if (t == 0) full = 0;
+            __syncthreads();
+            bool ok = true;
+            constexpr int U = 8;  // records in flight per thread
+            for (i64 xb = 0; xb < d; xb += (i64)BS * U) {  // block-uniform loop control
+                u64 r[U];
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const i64 x = xb + (i64)u * BS + t;
+                    r[u] = x < d ? in[x] : (u64)(u32)EMPTY_KEY;
+                }
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const i32 key = (i32)(u32)r[u];
+                    if (key == EMPTY_KEY) continue;
+                    const u64 y = (u64)mix32((u32)key) * total;
+                    if ((y >> 32) != want) continue;
+                    const i64 w = W(s + xb + (i64)u * BS + t);
+                    u32 q = __umulhi((u32)y, (u32)SL);
+                    int probe = 0;
+                    for (; probe < SL; probe++) {
+                        const i32 old = atomicCAS(&lk[q], EMPTY_KEY, key);
+                        if (old == EMPTY_KEY) lf[q] = __uint_as_float((u32)(r[u] >> 32));
+                        if (old == EMPTY_KEY || old == key) {
+                            if (sizeof(AT) == 4) atomicAdd((u32*)&lv[q], (u32)w);
+                            else atomicAdd((unsigned long long*)&lv[q], (unsigned long long)w);
+                            break;
+                        }
+                        q = q + 1 < (u32)SL ? q + 1 : 0;
+                    }
+                    ok = ok && probe < SL;
+                }
+            }
+            if (!ok) full = 1;
+            __syncthreads();
+            if (full) {  // block-uniform
+                over = true;
+                break;
+            }
+            for (int q = t; q < SL; q += BS) {
+                const i32 key = lk[q];
+                if (key == EMPTY_KEY) continue;
+                const AT agg = lv[q];
+                if (agg > 0 && (float)agg >= b) {
+                    const float jc = fmaf(-lf[q], multi, (float)agg);
+                    if (jc >= b) {
+                        const u64 k2 = pack_cand(jc, key);
+                        bk = k2 > bk ? k2 : bk;
+                    }
+                }
+            }
+            __syncthreads();  // the next part clears the table
+        }
+        if (!over) break;
+        __syncthreads();
+    }
+    bk = block_reduce<BS>(bk, [](u64 x, u64 y) { return x > y ? x : y; });
+    if (t == 0 && bk) atomicMax((unsigned long long*)&hub_best[h], (unsigned long long)bk);
+}
+
+// raw sweep: the same blocks, each with an equal share of the hub's edges
+template <int SL, class WT, class LT>
+__global__ void __launch_bounds__(256) k_hub_raw(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
+                                                 const i64* __restrict__ vw, const i32* __restrict__ hubs, i64 m,
+                                                 const i64* __restrict__ gpre, i64 ng, i64 nblk,
+                                                 const i32* __restrict__ part, const i64* __restrict__ vol,
+                                                 RecView rv, const i32* __restrict__ cons, LT lam, float ratio,
+                                                 const i32* __restrict__ dest, u64* hub_best) {
+    i64 h, sl;
+    if (!hub_block(gpre, ng, m, block_id(), nblk, h, sl)) return;
+    const i32 i = hubs[h];
+    if (dest[i] == NO_MOVE) return;
+    const i64 s = rp[i], e = rp[i + 1];
+    const i64 ns = hub_slices(e - s, SL);
+    if (sl >= ns) return;
+    i64 j_lo, j_hi;
+    hub_share(s, e, ns, sl, j_lo, j_hi);
     const i32 p = part[i];
     const i32 cp = cons ? cons[p] : 0;
     float multi, p_conn, bth;
     own_terms(0, vol[p], vw[i], lam(i), lam.rt(i, ratio), multi, p_conn, bth);
     const u64 bk = raw_best<256>(col, W, rv, cp, j_lo, j_hi, multi, bth);
-    if (threadIdx.x == 0 && bk) atomicMax((unsigned long long*)&hub_best[hi], (unsigned long long)bk);
-}
-
-// Hubs: an HBM table per hub of its neighbour-cluster weights (own cluster
-// included), built at the first table sweep of a call and kept current from
-// the movers by later sweeps (k_hub_update_*).  Per sweep, k_hub_pv reads
-// the own-cluster weight, slot work items scan the table and fold the packed
-// best candidate with atomicMax, and a last pass decides.
-//
-// Build: one block per table slice (k_hub_build) reads all of its hub's
-// edges, keeps the (cluster, weight) pairs whose hash falls in its slice in
-// an LDS table with the slice's probe sequence, and writes the slice out
-// whole (empty slots included), so the build needs no fill, no HBM atomics
-// and only coalesced stores.  The slices of one hub run on one XCD, where
-// the hub's edges and neighbour clusters are read from L2 after the first
-// slice.  A slice whose keys do not fit flags its hub (hflag), which is then
-// cleared (k_hub_clear) and built by edge items with HBM atomics and
-// whole-table probing (k_hub_insert).
-
-// Slice masks and fallback flags before a build.  hflag 1: built by the
-// fallback from the start (hub_build mode 1: every hub, mode 2: the hubs of
-// odd index, a mixed set; mode 0: the hubs from hg on, whose tables have
-// more than HUB_MAX_SLICES slices: every slice block reads all of a hub's
-// edges, and for the largest hubs the fallback's edge items spread better
-// over the CUs).  hflag 2: a slice of the hub was full (k_hub_build), and
-// *hovf is set.
-__global__ void k_hub_sm_init(const i64* __restrict__ goff, i64 m, i64 sl, int mode, i64 hg, u32* hsm, i32* hflag,
-                              i32* hovf, i32* hcnt) {
-    const i64 h = thread_item();
-    if (h == 0) *hovf = 0;
-    if (h >= m) return;
-    hcnt[h] = 0;
-    const i64 S = goff[h + 1] - goff[h];
-    const bool fb = mode == 1 || (mode == 2 && (h & 1)) || (mode == 0 && h >= hg);
-    hflag[h] = fb ? 1 : 0;
-    hsm[h] = (u32)((fb || S < sl ? S : sl) - 1);
-}
-
-// LDS insert with the slice's probe sequence; false when the slice is full
-__device__ __forceinline__ bool slice_add_packed(u64* lt, u32 smask, u32 q, i32 key, u64 w) {
-    for (u32 probe = 0; probe <= smask; probe++) {
-        const u64 cur = __hip_atomic_load(&lt[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        if ((u32)(cur >> 32) == (u32)key) {
-            atomicAdd((unsigned long long*)&lt[q], (unsigned long long)w);
-            return true;
-        }
-        if (cur == PEMPTY) {
-            const u64 old = atomicCAS((unsigned long long*)&lt[q], (unsigned long long)PEMPTY,
-                                      (unsigned long long)(((u64)(u32)key << 32) | w));
-            if (old == PEMPTY) return true;
-            if ((u32)(old >> 32) == (u32)key) {
-                atomicAdd((unsigned long long*)&lt[q], (unsigned long long)w);
-                return true;
-            }
-        }
-        q = (q + 1) & smask;
-    }
-    return false;
-}
-__device__ __forceinline__ bool slice_add_wide(i32* lk, i64* lv, u32 smask, u32 q, i32 key, i64 w) {
-    for (u32 probe = 0; probe <= smask; probe++) {
-        const i32 cur = __hip_atomic_load(&lk[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        bool hit = cur == key;
-        if (!hit && cur == EMPTY_KEY) {
-            const i32 old = atomicCAS(&lk[q], EMPTY_KEY, key);
-            hit = old == EMPTY_KEY || old == key;
-        }
-        if (hit) {
-            atomicAdd((unsigned long long*)&lv[q], (unsigned long long)w);
-            return true;
-        }
-        q = (q + 1) & smask;
-    }
-    return false;
-}
-
-// SL: LDS slots of the block (>= the slice size of every slice it builds),
-// BS threads.  Slice b0 + block id, or bmap[block id] when bmap is given.
-template <bool PACKED, int SL, int BS, class WT>
-__global__ void __launch_bounds__(BS) k_hub_build(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
-                                                  const i32* __restrict__ hubs, i64 m,
-                                                  const i64* __restrict__ soff, i64 b0, const i32* __restrict__ bmap,
-                                                  i64 nblk, const i64* __restrict__ goff,
-                                                  const i32* __restrict__ part, u32* hsm, i32* hflag,
-                                                  i32* hovf, i32* gkeys, i64* gvals, u64* gtab, u32* hlist,
-                                                  i32* hcnt) {
-    constexpr i64 SLMAX = PACKED ? HUB_SLICE_PACKED : HUB_SLICE_WIDE;
-    __shared__ u64 lt[PACKED ? SL : 1];
-    __shared__ i32 lk[PACKED ? 1 : SL];
-    __shared__ i64 lv[PACKED ? 1 : SL];
-    __shared__ int full, nocc, lbase;
-    const i64 bb = block_id();
-    if (bb >= nblk) return;
-    const i64 b = bmap ? (i64)bmap[bb] : b0 + bb;
-    if (b < 0) return;
-    const i64 hi = upper_row(soff, 0, m, b);
-    if (hflag[hi]) return;  // built by the fallback
-    const int t = threadIdx.x;
-    const i32 i = hubs[hi];
-    const i64 S = goff[hi + 1] - goff[hi];
-    const u32 mask = (u32)(S - 1);
-    const u32 smask = (u32)((S < SLMAX ? S : SLMAX) - 1);
-    if (smask >= (u32)SL) return;  // not this instance's slices (never launched so)
-    const u32 base = (u32)(b - soff[hi]) * (smask + 1);  // first slot of the slice
-    for (u32 q = t; q <= smask; q += BS) {
-        if (PACKED) {
-            lt[q] = PEMPTY;
-        } else {
-            lk[q] = EMPTY_KEY;
-            lv[q] = 0;
-        }
-    }
-    if (t == 0) {
-        full = 0;
-        nocc = 0;
-    }
-    __syncthreads();
-    const i64 s = rp[i], e = rp[i + 1];
-    bool ok = true;
-    constexpr int U = 4;  // edges per thread in flight
-    for (i64 jb = s; jb < e; jb += (i64)BS * U) {  // block-uniform loop control
-        i32 kk[U];
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            const i64 j = jb + (i64)u * BS + t;
-            kk[u] = j < e ? col[j] : -1;
-        }
-#pragma unroll
-        for (int u = 0; u < U; u++) kk[u] = kk[u] >= 0 ? part[kk[u]] : EMPTY_KEY;
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            if (kk[u] == EMPTY_KEY) continue;
-            const u32 h = slot_hash(kk[u], mask);
-            if ((h & ~smask) != base) continue;
-            const i64 w = W(jb + (i64)u * BS + t);
-            ok = (PACKED ? slice_add_packed(lt, smask, h & smask, kk[u], (u64)w)
-                         : slice_add_wide(lk, lv, smask, h & smask, kk[u], w)) && ok;
-        }
-    }
-    if (!ok) full = 1;
-    __syncthreads();
-    if (full) {  // the hub goes to the fallback build
-        if (t == 0) {
-            hflag[hi] = 2;
-            hsm[hi] = mask;
-            *hovf = 1;
-        }
-        return;
-    }
-    const i64 g0 = goff[hi] + base;
-    int mine = 0;
-    for (u32 q = t; q <= smask; q += BS) {
-        if (PACKED) {
-            gtab[g0 + q] = lt[q];
-            mine += lt[q] != PEMPTY;
-        } else {
-            gkeys[g0 + q] = lk[q];
-            gvals[g0 + q] = lv[q];
-            mine += lk[q] != EMPTY_KEY;
-        }
-    }
-    // the slice's occupied slots join the hub's list (in any order)
-    if (mine) atomicAdd(&nocc, mine);
-    __syncthreads();
-    if (t == 0) {
-        lbase = nocc ? atomicAdd(&hcnt[hi], nocc) : 0;
-        nocc = 0;
-    }
-    __syncthreads();
-    u32* lst = hlist + goff[hi] + lbase;
-    for (u32 q = t; q <= smask; q += BS)
-        if (PACKED ? lt[q] != PEMPTY : lk[q] != EMPTY_KEY) lst[atomicAdd(&nocc, 1)] = base + q;
-}
-
-// empty every slice of a hub flagged for the fallback build
-// after a full slice (grid-stride over the slices; nothing to do unless
-// *hovf)
-template <bool PACKED>
-__global__ void __launch_bounds__(256) k_hub_clear(i64 m, const i64* __restrict__ soff, i64 nslices,
-                                                   const i64* __restrict__ goff, const i32* __restrict__ hflag,
-                                                   const i32* __restrict__ hovf, i32* gkeys, i64* gvals, u64* gtab,
-                                                   i32* hcnt) {
-    if (*hovf == 0) return;
-    const i64 nblk = (i64)gridDim.x * gridDim.y;
-    for (i64 b = block_id(); b < nslices; b += nblk) {
-        const i64 hi = upper_row(soff, 0, m, b);
-        if (hflag[hi] != 2) continue;
-        if (b == soff[hi] && threadIdx.x == 0) hcnt[hi] = 0;  // relisted after the fallback build
-        const i64 S = goff[hi + 1] - goff[hi];
-        const i64 ns = soff[hi + 1] - soff[hi];
-        const i64 len = S / ns;
-        const i64 g0 = goff[hi] + (b - soff[hi]) * len;
-        for (i64 q = threadIdx.x; q < len; q += 256) {
-            if (PACKED) {
-                gtab[g0 + q] = PEMPTY;
-            } else {
-                gkeys[g0 + q] = EMPTY_KEY;
-                gvals[g0 + q] = 0;
-            }
-        }
-    }
-}
-
-// Occupied-slot lists of the tables the fallback built: the slices
-// b0 + k (grid-stride, n of them) of hubs with hflag == want; nothing to do
-// when gate is given and *gate is 0.
-template <bool PACKED>
-__global__ void __launch_bounds__(256) k_hub_relist(i64 m, const i64* __restrict__ soff, i64 b0, i64 n,
-                                                    const i64* __restrict__ goff, const i32* __restrict__ hflag,
-                                                    i32 want, const i32* __restrict__ gate,
-                                                    const i32* __restrict__ gkeys, const u64* __restrict__ gtab,
-                                                    u32* hlist, i32* hcnt) {
-    if (gate && *gate == 0) return;
-    __shared__ int nocc, lbase;
-    const i64 nblk = (i64)gridDim.x * gridDim.y;
-    for (i64 k = block_id(); k < n; k += nblk) {  // block-uniform loop control
-        const i64 b = b0 + k;
-        const i64 hi = upper_row(soff, 0, m, b);
-        if (hflag[hi] != want) continue;
-        const i64 S = goff[hi + 1] - goff[hi];
-        const i64 len = S / (soff[hi + 1] - soff[hi]);
-        const i64 s0 = (b - soff[hi]) * len;
-        const i64 g0 = goff[hi] + s0;
-        if (threadIdx.x == 0) nocc = 0;
-        __syncthreads();
-        int mine = 0;
-        for (i64 q = threadIdx.x; q < len; q += 256) mine += PACKED ? gtab[g0 + q] != PEMPTY : gkeys[g0 + q] != EMPTY_KEY;
-        if (mine) atomicAdd(&nocc, mine);
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            lbase = nocc ? atomicAdd(&hcnt[hi], nocc) : 0;
-            nocc = 0;
-        }
-        __syncthreads();
-        u32* lst = hlist + goff[hi] + lbase;
-        for (i64 q = threadIdx.x; q < len; q += 256)
-            if (PACKED ? gtab[g0 + q] != PEMPTY : gkeys[g0 + q] != EMPTY_KEY) lst[atomicAdd(&nocc, 1)] = (u32)(s0 + q);
-        __syncthreads();
-    }
-}
-
-// Fallback build of the hubs with hflag == want (into emptied tables): edge
-// work items (he = HL / 2 edges each) pre-aggregate in LDS, then add into
-// the HBM table with atomics, probing over the whole table.  Grid-stride
-// over the items b0 + k, or imap[k] when imap is given; nothing to do when
-// gate is given and *gate is 0.
-template <bool PACKED, int HL, class WT>
-__global__ void __launch_bounds__(256) k_hub_insert(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
-                                                    const i32* __restrict__ hubs, i64 m, const i64* __restrict__ items,
-                                                    const i32* __restrict__ imap, i64 b0, i64 nmap,
-                                                    const i64* __restrict__ goff, const i32* __restrict__ part,
-                                                    const i32* __restrict__ hflag, i32 want,
-                                                    const i32* __restrict__ gate, i32* gkeys, i64* gvals, u64* gtab) {
-    if (gate && *gate == 0) return;
-    constexpr i64 he = HL / 2;
-    __shared__ i32 lk[HL];
-    __shared__ i64 lv[HL];
-    const i64 nblk = (i64)gridDim.x * gridDim.y;
-    for (i64 bb = block_id(); bb < nmap; bb += nblk) {  // block-uniform loop control
-        const i64 b = imap ? (i64)imap[bb] : b0 + bb;
-        if (b < 0) continue;
-        const i64 hi = upper_row(items, 0, m, b);
-        if (hflag[hi] != want) continue;
-        const i32 i = hubs[hi];
-        const i64 s = rp[i], e = rp[i + 1];
-        const i64 j_lo = s + (b - items[hi]) * he;
-        const i64 j_hi = j_lo + he < e ? j_lo + he : e;
-        lds_agg_clear<256, HL>(lk, lv);
-        for (i64 jb = j_lo; jb < j_hi; jb += 256) {  // block-uniform loop control
-            const i64 j = jb + threadIdx.x;
-            if (j >= j_hi) continue;
-            table_add_lds(lk, lv, HL - 1, part[col[j]], W(j));
-        }
-        const u32 gmask = (u32)(goff[hi + 1] - goff[hi] - 1);
-        if (PACKED) lds_agg_flush_packed<256, HL>(lk, lv, gtab + goff[hi], gmask);
-        else lds_agg_flush<256, HL>(lk, lv, gkeys + goff[hi], gvals + goff[hi], gmask);
-        __syncthreads();  // the flush reads LDS the next item clears
-    }
-}
-
-// own-cluster weight of every active hub, read from its table
-template <bool PACKED>
-__global__ void k_hub_pv(const i32* __restrict__ hubs, i64 m, const i64* __restrict__ goff,
-                         const u32* __restrict__ hsm, const i32* __restrict__ part, const i32* __restrict__ dest,
-                         const i32* gkeys, const i64* gvals, const u64* gtab, i64* hub_pv) {
-    const i64 hi = thread_item();
-    if (hi >= m) return;
-    const i32 i = hubs[hi];
-    if (dest[i] == NO_MOVE) return;
-    const u32 gmask = (u32)(goff[hi + 1] - goff[hi] - 1);
-    hub_pv[hi] = PACKED ? ptable_get(gtab + goff[hi], gmask, hsm[hi], part[i])
-                        : table_get(gkeys + goff[hi], gvals + goff[hi], gmask, hsm[hi], part[i]);
-}
-
-// A mover's edge into hub h: weight w leaves key oi and joins key ni in the
-// hub's table (run before the moves are applied).  A failed update sets
-// *stale.
-template <bool PACKED>
-__device__ __forceinline__ void hub_update_edge(i32 h, i64 w, const i64* goff, const u32* hsm, i32* gkeys, i64* gvals,
-                                                u64* gtab, u32* hlist, i32* hcnt, i32 oi, i32 ni, i64* stale) {
-    const i64 g = goff[h];
-    const u32 gmask = (u32)(goff[h + 1] - g - 1);
-    const u32 sm = hsm[h];
-    bool ok;
-    if (PACKED) {
-        ok = ptable_update(gtab + g, gmask, sm, oi, -w, hlist + g, hcnt + h);
-        ok = ptable_update(gtab + g, gmask, sm, ni, w, hlist + g, hcnt + h) && ok;
-    } else {
-        ok = table_update(gkeys + g, gvals + g, gmask, sm, oi, -w, hlist + g, hcnt + h);
-        ok = table_update(gkeys + g, gvals + g, gmask, sm, ni, w, hlist + g, hcnt + h) && ok;
-    }
-    if (!ok) *stale = 1;
-}
-
-// Scan items cover hs entries of a hub's occupied-slot list (the grid is
-// sized for full tables; items past the list's end exit at once).
-template <bool PACKED, class LT>
-__global__ void __launch_bounds__(256) k_hub_scan(const i32* __restrict__ hubs, i64 m, const i64* __restrict__ sitems,
-                                                  const i32* __restrict__ smap, i64 nmap,
-                                                  const i64* __restrict__ goff, const i32* __restrict__ part,
-                                                  const i32* __restrict__ dest, const i64* __restrict__ vw,
-                                                  const i64* __restrict__ vol, const i32* __restrict__ cons, LT lam,
-                                                  float ratio, const i32* gkeys, const i64* gvals, const u64* gtab,
-                                                  const u32* __restrict__ hlist, const i32* __restrict__ hcnt,
-                                                  const i64* __restrict__ hub_pv, i64 hs, u64* hub_best) {
-    const i64 bb = block_id();
-    if (bb >= nmap) return;
-    const i64 b = smap[bb];
-    if (b < 0) return;
-    const i64 hi = upper_row(sitems, 0, m, b);
-    const i64 k_lo = (b - sitems[hi]) * hs;
-    const i64 cnt = hcnt[hi];
-    if (k_lo >= cnt) return;
-    const i32 i = hubs[hi];
-    if (dest[i] == NO_MOVE) return;
-    const i64 k_hi = k_lo + hs < cnt ? k_lo + hs : cnt;
-    const i64 g0 = goff[hi];
-    const u32* lst = hlist + g0;
-    const i32 p = part[i];
-    float multi, p_conn, bth;
-    own_terms(hub_pv[hi], vol[p], vw[i], lam(i), lam.rt(i, ratio), multi, p_conn, bth);
-    u64 bk = 0;
-    for (i64 kb = k_lo; kb < k_hi; kb += 256) {  // block-uniform loop control
-        const i64 k = kb + threadIdx.x;
-        if (k >= k_hi) continue;
-        const i64 q = g0 + lst[k];
-        i32 key;
-        i64 agg;
-        if (PACKED) {
-            const u64 e = gtab[q];
-            key = (i32)(e >> 32);
-            agg = (i64)(e & 0xffffffffull);
-        } else {
-            key = gkeys[q];
-            agg = gvals[q];
-        }
-        if (key != p && agg > 0 && (float)agg >= bth && (cons == nullptr || cons[key] == cons[p])) {
-            const float jc = fmaf(-(float)vol[key], multi, (float)agg);
-            if (jc >= bth) {
-                const u64 k2 = pack_cand(jc, key);
-                bk = k2 > bk ? k2 : bk;
-            }
-        }
-    }
-    bk = block_max_u64<256>(bk);
-    if (threadIdx.x == 0 && bk) atomicMax((unsigned long long*)&hub_best[hi], (unsigned long long)bk);
+    if (threadIdx.x == 0 && bk) atomicMax((unsigned long long*)&hub_best[h], (unsigned long long)bk);
 }
 
 template <class LT>
 __global__ void k_hub_decide(const i32* hubs, i64 m, const i32* part, const i64* vw, const i64* vol, LT lam,
-                             float ratio, const i64* hub_pv, const u64* hub_best, ScoreOut out) {
+                             float ratio, i64* hub_pv, u64* hub_best, ScoreOut out) {
     const i64 hi = thread_item();
     if (hi >= m) return;
     const i32 i = hubs[hi];
     if (out.dest[i] == NO_MOVE) return;
+    const u64 bk = hub_best[hi];
+    const i64 pv = hub_pv[hi];
+    hub_best[hi] = 0;  // for the next sweep
+    hub_pv[hi] = 0;
     const i32 p = part[i];
     const i64 wi = vw[i];
     float multi, p_conn, bth;
-    own_terms(hub_pv[hi], vol[p], wi, lam(i), lam.rt(i, ratio), multi, p_conn, bth);
-    decide(i, p_conn, hub_best[hi], p, wi, out);
+    own_terms(pv, vol[p], wi, lam(i), lam.rt(i, ratio), multi, p_conn, bth);
+    decide(i, p_conn, bk, p, wi, out);
 }
 
 
@@ -1249,33 +902,22 @@ __global__ void k_hub_decide(const i32* hubs, i64 m, const i32* part, const i64*
 // vertex reads its row bounds, destination, cluster, vertex weight and its
 // cluster's volume, every edge's column (and weight) and the neighbour's
 // record, and writes its destination, gain and record: 48 + d (4 + weight
-// bytes + 8) bytes.  A hub whose table is kept current reads
-// the table instead of its edges: 48 + 8 per slot, plus the edge bytes on the
-// sweep that builds the table.  Every listed vertex also costs its list entry
+// bytes + 8) bytes.  Every listed vertex also costs its list entry
 // and destination read.  acc3[0..2] = group, table and hub classes.
 struct ScoreBounds {
     i64 s[NCLS + 1];
-    i64 hub0;  // first HBM-table hub (the hubs before it are scored in LDS)
+    i64 hub0;  // first hub of k_hub_score
 };
 template <int WB>
 __global__ void __launch_bounds__(256) k_score_bytes(const i64* __restrict__ rp, const i32* __restrict__ list,
-                                                     ScoreBounds sb, const i32* __restrict__ dest, int raw, int build,
-                                                     const i64* __restrict__ goff, i64* acc3) {
+                                                     ScoreBounds sb, const i32* __restrict__ dest, i64* acc3) {
     const i64 x = thread_item();
     i64 b0 = 0, b1 = 0, b2 = 0;
     if (x < sb.s[NCLS]) {
         const i32 i = list[x];
         const int grp = x < sb.s[CL_TABLE] ? 0 : (x < sb.hub0 ? 1 : 2);
         i64 by = 8;
-        if (dest[i] != NO_MOVE) {
-            const i64 eb = (rp[i + 1] - rp[i]) * (4 + WB + 8);
-            if (grp < 2 || raw) {
-                by += 48 + eb;
-            } else {
-                const i64 h = x - sb.hub0;
-                by += 48 + 8 * (goff[h + 1] - goff[h]) + (build ? eb : 0);
-            }
-        }
+        if (dest[i] != NO_MOVE) by += 48 + (rp[i + 1] - rp[i]) * (4 + WB + 8);
         if (grp == 0) b0 = by;
         else if (grp == 1) b1 = by;
         else b2 = by;
@@ -1318,12 +960,12 @@ struct ScoreArgs {
     ScoreOut out;
 };
 // LDS-table scoring of the list entries [x0, x1) (one block per vertex):
-// BS threads, SLOTS LDS slots, SPE slots per edge of the degree bound.
-template <class AT, int BS, int SLOTS, int SPE, class WT, class LT>
+// degrees up to D, BS threads, SPE slots per edge, at most SLOTS.
+template <class AT, int BS, int D, int SLOTS, int SPE, class WT, class LT>
 static void launch_table(Ctx& c, const DGraph& g, WT W, const ScoreArgs<LT>& a, i64 x0, i64 x1) {
     const i64 m = x1 - x0;
     if (m <= 0) return;
-    k_score_table<BS, SLOTS, SPE, AT><<<grid_blocks(m), BS, 0, c.stream>>>(
+    k_score_table<BS, D, SLOTS, SPE, AT><<<grid_blocks(m), BS, 0, c.stream>>>(
         g.rp, g.col, W, g.vw, a.L + x0, m, a.part, a.vol, a.rv, a.cons, a.lam, a.ratio, a.out);
 }
 // class with degree bound D (128, 256, 512): threads per vertex and slots per
@@ -1331,12 +973,12 @@ static void launch_table(Ctx& c, const DGraph& g, WT W, const ScoreArgs<LT>& a, 
 template <class AT, int D, class WT, class LT>
 static void launch_table_class(Ctx& c, const DGraph& g, WT W, const ScoreArgs<LT>& a, i64 x0, i64 x1) {
     const int bs = c.table_threads, spe = c.table_spe;
-    if (bs == 64 && spe == 2) launch_table<AT, 64, 2 * D, 2>(c, g, W, a, x0, x1);
-    else if (bs == 64) launch_table<AT, 64, 4 * D, 4>(c, g, W, a, x0, x1);
-    else if (bs == 128 && spe == 2) launch_table<AT, 128, 2 * D, 2>(c, g, W, a, x0, x1);
-    else if (bs == 128) launch_table<AT, 128, 4 * D, 4>(c, g, W, a, x0, x1);
-    else if (spe == 2) launch_table<AT, 256, 2 * D, 2>(c, g, W, a, x0, x1);
-    else launch_table<AT, 256, 4 * D, 4>(c, g, W, a, x0, x1);
+    if (bs == 64 && spe == 2) launch_table<AT, 64, D, 2 * D, 2>(c, g, W, a, x0, x1);
+    else if (bs == 64) launch_table<AT, 64, D, 4 * D, 4>(c, g, W, a, x0, x1);
+    else if (bs == 128 && spe == 2) launch_table<AT, 128, D, 2 * D, 2>(c, g, W, a, x0, x1);
+    else if (bs == 128) launch_table<AT, 128, D, 4 * D, 4>(c, g, W, a, x0, x1);
+    else if (spe == 2) launch_table<AT, 256, D, 2 * D, 2>(c, g, W, a, x0, x1);
+    else launch_table<AT, 256, D, 4 * D, 4>(c, g, W, a, x0, x1);
 }
 template <class AT, class WT, class LT>
 static void launch_groups(Ctx& c, const DGraph& g, WT W, const ScoreArgs<LT>& a, const i64* st, int raw) {
@@ -1357,7 +999,7 @@ static void launch_tables(Ctx& c, const LevelPlan& lp, const DGraph& g, WT W, co
     // few rows: one launch for all classes (the widest block), as launches
     // then cost more than the lower occupancy
     if (lp.hub0 - st[CL_TABLE] <= TABLE_ONE_LAUNCH && lp.hub0 == st[CL_HUB]) {
-        launch_table<AT, 256, 4096, 2>(c, g, W, a, st[CL_TABLE], st[CL_HUB]);
+        launch_table<AT, 256, 2048, 4096, 2>(c, g, W, a, st[CL_TABLE], st[CL_HUB]);
         return;
     }
     // LDS tables sized for the class, so the many low-degree rows keep more
@@ -1366,118 +1008,14 @@ static void launch_tables(Ctx& c, const LevelPlan& lp, const DGraph& g, WT W, co
     launch_table_class<AT, 256>(c, g, W, a, st[6], st[7]);
     launch_table_class<AT, 512>(c, g, W, a, st[7], st[8]);
     if (c.table_spe == 2) {
-        launch_table<AT, 256, 2048, 2>(c, g, W, a, st[8], st[9]);
-        launch_table<AT, 512, 4096, 2>(c, g, W, a, st[9], st[10]);
+        launch_table<AT, 256, 1024, 2048, 2>(c, g, W, a, st[8], st[9]);
+        launch_table<AT, 512, 2048, 4096, 2>(c, g, W, a, st[9], st[10]);
     } else {
-        launch_table<AT, 256, 4096, 4>(c, g, W, a, st[8], st[9]);
-        launch_table<AT, 512, 8192, 4>(c, g, W, a, st[9], st[10]);
+        launch_table<AT, 256, 1024, 4096, 4>(c, g, W, a, st[8], st[9]);
+        launch_table<AT, 512, 2048, 8192, 4>(c, g, W, a, st[9], st[10]);
     }
-    // hubs of degree <= hub_lds_max: 8192 LDS slots
-    launch_table<AT, 512, 8192, 2>(c, g, W, a, st[CL_HUB], lp.hub0);
-}
-
-// Hub tables of the current clustering: slices built in LDS, then the
-// fallback build of the hubs flagged (by a full slice or the hub_build knob).
-// occupied-slot lists of the fallback-built tables (slices b0 .. b0+n-1)
-static void hub_relist(Ctx& c, LevelPlan& lp, i64 m, i64 b0, i64 n, i64 cap, i32 want, const i32* gate) {
-    if (n <= 0) return;
-    const dim3 grid = grid_blocks(cap > 0 ? std::min(n, cap) : n);
-    if (lp.packed)
-        k_hub_relist<true><<<grid, 256, 0, c.stream>>>(m, lp.soff, b0, n, lp.goff, lp.hflag, want, gate, nullptr,
-                                                       lp.gtab, lp.hlist, lp.hcnt);
-    else
-        k_hub_relist<false><<<grid, 256, 0, c.stream>>>(m, lp.soff, b0, n, lp.goff, lp.hflag, want, gate, lp.gkeys,
-                                                        nullptr, lp.hlist, lp.hcnt);
-    PGGC_LAUNCH_CHECK();
-}
-
-// fallback insert launch over n item slots (b0 + k, or imap[k]); grid
-// capped at cap blocks (grid-stride) when cap > 0
-template <class WT>
-static void hub_insert_items(Ctx& c, const DGraph& g, WT W, LevelPlan& lp, const i32* hubs, i64 m, const i32* part,
-                             const i32* imap, i64 b0, i64 n, i64 cap, i32 want, const i32* gate) {
-    if (n <= 0) return;
-    i32* gk = lp.packed ? nullptr : lp.gkeys.p;
-    i64* gv = lp.packed ? nullptr : lp.gvals.p;
-    u64* gt = lp.packed ? lp.gtab.p : nullptr;
-    const dim3 grid = grid_blocks(cap > 0 ? std::min(n, cap) : n);
-#define PGGC_HUB_INSERT(PK, HL)                                                                                   \
-    k_hub_insert<PK, HL><<<grid, 256, 0, c.stream>>>(g.rp, g.col, W, hubs, m, lp.items, imap, b0, n, lp.goff, part, \
-                                                     lp.hflag, want, gate, gk, gv, gt)
-    if (lp.packed) {
-        if (lp.he == 512) PGGC_HUB_INSERT(true, 1024);
-        else if (lp.he == 2048) PGGC_HUB_INSERT(true, 4096);
-        else PGGC_HUB_INSERT(true, 2048);
-    } else {
-        if (lp.he == 512) PGGC_HUB_INSERT(false, 1024);
-        else if (lp.he == 2048) PGGC_HUB_INSERT(false, 4096);
-        else PGGC_HUB_INSERT(false, 2048);
-    }
-#undef PGGC_HUB_INSERT
-    PGGC_LAUNCH_CHECK();
-}
-
-template <class WT>
-static void hub_build_all(Ctx& c, const DGraph& g, WT W, LevelPlan& lp, const i32* hubs, i64 m, const i32* part) {
-    i32* gk = lp.packed ? nullptr : lp.gkeys.p;
-    i64* gv = lp.packed ? nullptr : lp.gvals.p;
-    u64* gt = lp.packed ? lp.gtab.p : nullptr;
-    const int mode = c.hub_build;
-    k_hub_sm_init<<<grid_items(m, 256), 256, 0, c.stream>>>(lp.goff, m, hub_slice(lp.packed), mode, lp.hg, lp.hsm,
-                                                            lp.hflag, lp.hovf, lp.hcnt);
-    // empty the tables the fallback builds from the start (before the slice
-    // builds, which write the other tables whole)
-    const i64 f0 = mode == 0 ? lp.ghg : 0;
-    if (lp.gslots > f0) {
-        if (lp.packed) {
-            fill_i64(c, (i64*)lp.gtab.p + f0, lp.gslots - f0, (i64)PEMPTY);
-        } else {
-            fill_i32(c, lp.gkeys.p + f0, lp.gslots - f0, EMPTY_KEY);
-            fill_i64(c, lp.gvals.p + f0, lp.gslots - f0, 0);
-        }
-    }
-    if (mode != 1) {
-        // single-slice tables of 4096 and (packed) 8192 slots in smaller
-        // blocks, so several run per CU; the multi-slice tables through the
-        // XCD map
-        const i64 n1 = lp.hs1, n2 = lp.hs2 - lp.hs1;
-#define PGGC_HUB_BUILD(PK, SL, BS, B0, MAP, N)                                                                    \
-    k_hub_build<PK, SL, BS><<<grid_blocks(N), BS, 0, c.stream>>>(g.rp, g.col, W, hubs, m, lp.soff, B0, MAP, N, lp.goff, \
-                                                                 part, lp.hsm, lp.hflag, lp.hovf, gk, gv, gt, lp.hlist, \
-                                                                 lp.hcnt)
-        if (lp.packed) {
-            if (n1 > 0) PGGC_HUB_BUILD(true, 4096, 256, 0, nullptr, n1);
-            if (n2 > 0) PGGC_HUB_BUILD(true, 8192, 512, lp.hs1, nullptr, n2);
-            if (lp.bgrid > 0) PGGC_HUB_BUILD(true, 16384, 1024, 0, lp.bmap.p, lp.bgrid);
-        } else {
-            if (n1 > 0) PGGC_HUB_BUILD(false, 4096, 256, 0, nullptr, n1);
-            if (lp.bgrid > 0) PGGC_HUB_BUILD(false, 8192, 512, 0, lp.bmap.p, lp.bgrid);
-        }
-#undef PGGC_HUB_BUILD
-        // hubs with a full slice (normally none: the gated kernels exit)
-        constexpr i64 FB_GRID = 4096;
-        const dim3 cgrid = grid_blocks(std::min(lp.nslices, FB_GRID));
-        if (lp.packed)
-            k_hub_clear<true><<<cgrid, 256, 0, c.stream>>>(m, lp.soff, lp.nslices, lp.goff, lp.hflag, lp.hovf, gk, gv,
-                                                           gt, lp.hcnt);
-        else
-            k_hub_clear<false><<<cgrid, 256, 0, c.stream>>>(m, lp.soff, lp.nslices, lp.goff, lp.hflag, lp.hovf, gk,
-                                                            gv, gt, lp.hcnt);
-        hub_insert_items(c, g, W, lp, hubs, m, part, lp.imap.p, 0, lp.igrid, FB_GRID, 2, lp.hovf.p);
-        hub_relist(c, lp, m, 0, lp.nslices, FB_GRID, 2, lp.hovf.p);
-    }
-    // the hubs built by the fallback from the start: in mode 0 the items
-    // from the first of the largest hubs on, else all items through the map
-    if (mode == 0) {
-        if (lp.nitems > lp.ihg) {
-            hub_insert_items(c, g, W, lp, hubs, m, part, nullptr, lp.ihg, lp.nitems - lp.ihg, 0, 1, nullptr);
-            hub_relist(c, lp, m, lp.shg, lp.nslices - lp.shg, 0, 1, nullptr);
-        }
-    } else {
-        hub_insert_items(c, g, W, lp, hubs, m, part, lp.imap.p, 0, lp.igrid, 0, 1, nullptr);
-        hub_relist(c, lp, m, 0, lp.nslices, 0, 1, nullptr);
-    }
-    PGGC_LAUNCH_CHECK();
+    launch_table<AT, 1024, HUB_HALF, 8192, 2>(c, g, W, a, st[CL_HUB], st[CL_HUB] + lp.nhalf);
+    launch_table<AT, 1024, HUB_LDS_BOUND, HUB_LDS_SLOTS, 2>(c, g, W, a, st[CL_HUB] + lp.nhalf, lp.hub0);
 }
 
 template <class LT>
@@ -1494,10 +1032,8 @@ static void score_all(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, co
         ScoreBounds sb;
         for (int k = 0; k <= NCLS; k++) sb.s[k] = st[k];
         sb.hub0 = lp.hub0;
-        const int build = (!raw && !lp.hub_live) ? 1 : 0;
-        const i64* goff = lp.nhub > 0 ? lp.goff.p : nullptr;
         PGGC_WDISPATCH(g, (k_score_bytes<decltype(W)::bytes><<<grid_items(g.n, 256), 256, 0, c.stream>>>(
-                              g.rp, L, sb, dest, raw, build, goff, acct)));
+                              g.rp, L, sb, dest, acct)));
         PGGC_LAUNCH_CHECK();
     }
     if (g.n > 0) {
@@ -1505,6 +1041,19 @@ static void score_all(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, co
         k_rec_pack<<<grid_items(g.n, 256), 256, 0, c.stream>>>(g.n, part, vol, cons, s.rec, cons ? s.rec16.p : nullptr);
         PGGC_LAUNCH_CHECK();
     }
+#define PGGC_HUB_RAW(SL)                                                                                              \
+    k_hub_raw<SL><<<grid_blocks(lp.hub_blocks), 256, 0, c.stream>>>(g.rp, g.col, W, g.vw, hubs, m, lp.hub_groups, ng, \
+                                                                    lp.hub_blocks, part, vol, a.rv, cons, lam, ratio, \
+                                                                    dest, lp.hub_best)
+#define PGGC_HUB(SL, AT)                                                                                              \
+    do {                                                                                                              \
+        k_hub_gather<SL><<<grid_blocks(lp.hub_blocks), 256, 0, c.stream>>>(                                           \
+            g.rp, g.col, W, hubs, m, lp.hub_groups, ng, lp.hub_blocks, lp.hub_eoff, part, a.rv, cons, dest, s.hub_kv, \
+            lp.hub_pv);                                                                                               \
+        k_hub_score<SL, 1024, AT><<<grid_blocks(lp.hub_blocks), 1024, 0, c.stream>>>(                                 \
+            g.rp, W, g.vw, hubs, m, lp.hub_groups, ng, lp.hub_blocks, lp.hub_eoff, part, vol, lam, ratio, dest,       \
+            s.hub_kv, lp.hub_pv, lp.hub_best);                                                                        \
+    } while (0)
     const ScoreArgs<LT> a{L, part, vol, RecView{s.rec.p, cons ? s.rec16.p : nullptr}, cons, lam, ratio, out};
     PGGC_WDISPATCH(g, {
         using WT = decltype(W);
@@ -1533,37 +1082,23 @@ static void score_all(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, co
         if ((m = lp.nhub) > 0) {
             const i32* hubs = L + lp.hub0;
             tk = c.kt_begin(KS_SCORE_HUB);
-            fill_i64(c, lp.hub_pv, m, 0);
-            fill_i64(c, (i64*)lp.hub_best.p, m, 0);
-            if (raw) {
-                k_hub_raw<<<grid_blocks(lp.nitems), 256, 0, c.stream>>>(g.rp, g.col, W, g.vw, hubs, m, lp.items, part,
-                                                                       vol, a.rv, cons, lam, ratio, dest, lp.he,
-                                                                       lp.hub_best);
-            } else {
-                if (!lp.hub_live) {  // first table sweep of the call (or stale tables): build
-                    hub_build_all(c, g, W, lp, hubs, m, part);
-                    lp.hub_live = true;
-                }
-                if (lp.packed) {
-                    k_hub_pv<true><<<grid_items(m, 256), 256, 0, c.stream>>>(hubs, m, lp.goff, lp.hsm, part, dest, nullptr,
-                                                                            nullptr, lp.gtab, lp.hub_pv);
-                    k_hub_scan<true><<<grid_blocks(lp.sgrid), 256, 0, c.stream>>>(
-                        hubs, m, lp.sitems, lp.smap, lp.sgrid, lp.goff, part, dest, g.vw, vol, cons, lam, ratio,
-                        nullptr, nullptr, lp.gtab, lp.hlist, lp.hcnt, lp.hub_pv, lp.hs, lp.hub_best);
-                } else {
-                    k_hub_pv<false><<<grid_items(m, 256), 256, 0, c.stream>>>(hubs, m, lp.goff, lp.hsm, part, dest, lp.gkeys,
-                                                                             lp.gvals, nullptr, lp.hub_pv);
-                    k_hub_scan<false><<<grid_blocks(lp.sgrid), 256, 0, c.stream>>>(
-                        hubs, m, lp.sitems, lp.smap, lp.sgrid, lp.goff, part, dest, g.vw, vol, cons, lam, ratio,
-                        lp.gkeys, lp.gvals, nullptr, lp.hlist, lp.hcnt, lp.hub_pv, lp.hs, lp.hub_best);
-                }
+            const i64 ng = ceil_div(m, NXCD);
+            if (!raw && s.hub_kv.n < (size_t)lp.hub_edges) {
+                s.hub_kv.reset();
+                s.hub_kv = Buf<u64>(c, lp.hub_edges);
             }
+            if (raw && lp.hub32) PGGC_HUB_RAW(HUB_SLOTS32);
+            else if (raw) PGGC_HUB_RAW(HUB_SLOTS64);
+            else if (lp.hub32) PGGC_HUB(HUB_SLOTS32, u32);
+            else PGGC_HUB(HUB_SLOTS64, A64);
             k_hub_decide<<<grid_items(m, 256), 256, 0, c.stream>>>(hubs, m, part, g.vw, vol, lam, ratio, lp.hub_pv,
                                                                        lp.hub_best, out);
             c.kt_end(tk, 0.0);
             if (tk >= 0) acct_add(c, c.kt_counter(tk), acct.p + 2);
         }
     });
+#undef PGGC_HUB
+#undef PGGC_HUB_RAW
     PGGC_LAUNCH_CHECK();
 }
 
@@ -1932,42 +1467,25 @@ struct AccInst {
     }
 };
 
-// hub tables as the move kernels see them (hidx null: not kept current)
-struct HubView {
-    const i32* hidx;
-    const i64* goff;
-    const u32* hsm;
-    i32* gkeys;
-    i64* gvals;
-    u64* gtab;
-    u32* hlist;
-    i32* hcnt;
-    i64* stale;
-};
-
 // One pass over the movers' edges (src/local_mover.cpp:1274-1277, 717, 798):
 //  - the exact uncut change, per edge w * ([new_i == new_v] - [old_i ==
 //    old_v]), counted once for mover pairs and twice for neighbours that stay
 //    (the reference computes the same quantity from pvals);
-//  - RESET: the neighbour's cached destination becomes NULL_PART;
-//  - HUB: a hub neighbour's table moves the edge's weight between its keys.
+//  - RESET: the neighbour's cached destination becomes NULL_PART.
 // What bounds it is latency: each edge is a chain of dependent loads (column,
-// neighbour word, hub slot, atomics).  So a mover of degree below
-// LARGE_CUTOFF takes MV_G lanes, one below MASSIVE_CUTOFF a 128-thread half
-// block, the rest chunks of MV_CHUNK edges per block, and each thread has
-// MV_U edges in flight.  As one thread per small mover and one wave per
-// mid-size one, in a kernel each for the three jobs, the hub updates alone
-// took 479 + 109 us per sweep on R-MAT scale 20 (1.04 ms at worst on scale
-// 22); this kernel does all of it in 82-98 us there (193 us on average on
-// scale 22).
+// neighbour word).  So a mover of degree below LARGE_CUTOFF takes MV_G lanes, one
+// below MASSIVE_CUTOFF a 128-thread half block, the rest chunks of MV_CHUNK edges
+// per block, and each thread has MV_U edges in flight.  As one thread per small
+// mover and one wave per mid-size one, in a kernel each for the two jobs, they
+// took 86 ms on R-MAT scale 20 (to stable), now 39 ms.
 // The list is in order1 order: the movers of degree >= LARGE_CUTOFF are a
 // suffix of at most nw entries, those >= MASSIVE_CUTOFF one of at most nb.
 constexpr int MV_G = 16, MV_U = 4;
 constexpr i64 MV_CHUNK = 8192;
-template <bool HUB, bool PACKED, bool RESET, class WT, class AT>
+template <bool RESET, class WT, class AT>
 __global__ void __launch_bounds__(256) k_move_edges(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
                                                     const i32* __restrict__ moves, i64 k, i64 b1, i64 b2, i64 nw,
-                                                    i64 nb, i64 cpm, const u64* __restrict__ mvp, HubView hv,
+                                                    i64 nb, i64 cpm, const u64* __restrict__ mvp,
                                                     i32* __restrict__ dest, AT at) {
     const i64 b = block_id();
     i64 x;         // list entry
@@ -2006,7 +1524,7 @@ __global__ void __launch_bounds__(256) k_move_edges(const i64* __restrict__ rp, 
         if (d >= lo && d < hi && c0 < d) {
             const i64 e = s0 + (d < c0 + cl ? d : c0 + cl);
             for (i64 jb = s0 + c0 + lane; jb < e; jb += (i64)gs * MV_U) {
-                i32 v[MV_U], h[MV_U];
+                i32 v[MV_U];
                 u64 q[MV_U];
 #pragma unroll
                 for (int u = 0; u < MV_U; u++) {
@@ -2014,10 +1532,7 @@ __global__ void __launch_bounds__(256) k_move_edges(const i64* __restrict__ rp, 
                     v[u] = j < e ? col[j] : -1;
                 }
 #pragma unroll
-                for (int u = 0; u < MV_U; u++) {
-                    q[u] = v[u] >= 0 ? mvp[v[u]] : 0;
-                    h[u] = HUB && v[u] >= 0 ? hv.hidx[v[u]] : -1;
-                }
+                for (int u = 0; u < MV_U; u++) q[u] = v[u] >= 0 ? mvp[v[u]] : 0;
 #pragma unroll
                 for (int u = 0; u < MV_U; u++) {
                     if (v[u] < 0) continue;
@@ -2027,10 +1542,6 @@ __global__ void __launch_bounds__(256) k_move_edges(const i64* __restrict__ rp, 
                     const i32 ov = (i32)(ql & 0x7fffffffu), nv = (i32)(u32)(q[u] >> 32);
                     const i64 dd = (i64)(ni == nv) - (i64)(oi == ov);
                     acc += dd * w * ((ql >> 31) ? 1 : 2);
-                    // ni < 0: an unresolved NEW_PART mover is not applied
-                    if (HUB && h[u] >= 0 && ni >= 0)
-                        hub_update_edge<PACKED>(h[u], w, hv.goff, hv.hsm, hv.gkeys, hv.gvals, hv.gtab, hv.hlist,
-                                                hv.hcnt, oi, ni, hv.stale);
                 }
             }
         }
@@ -2075,10 +1586,9 @@ __global__ void __launch_bounds__(256) k_apply_moves(const i32* __restrict__ mov
     }
 }
 
-// End of a sweep: the exact 128-bit sum of squared volumes, the uncut change
-// and the stale flag, stored to the host slots by the last block to finish
-// (host[0] = uncut change, host[1..2] = sum of squares high and low, host[3] =
-// stale).  One launch instead of seven (fills, two reductions of two
+// End of a sweep: the exact 128-bit sum of squared volumes and the uncut
+// change, stored to the host slots by the last block to finish (host[0] =
+// uncut change, host[1..2] = sum of squares high and low).  One launch instead of seven (fills, two reductions of two
 // kernels each, read-back): on small levels the sweep is bound by launches.
 __global__ void __launch_bounds__(256) k_finish(const i64* __restrict__ vol, i64 L, u64* part, i64* scal, i64* host) {
     u64 lo = 0, hi = 0;
@@ -2128,8 +1638,6 @@ __global__ void __launch_bounds__(256) k_finish(const i64* __restrict__ vol, i64
         host[0] = du;
         host[1] = (i64)rhi;
         host[2] = (i64)rlo;
-        host[3] = scal[SC_STALE];
-        scal[SC_STALE] = 0;
         scal[SC_TICKET] = 0;
         __threadfence_system();
     }
@@ -2138,34 +1646,24 @@ __global__ void __launch_bounds__(256) k_finish(const i64* __restrict__ vol, i64
 // perform_moves (src/local_mover.cpp:1241-1279).  moves is in order1 order;
 // n_large / n_massive = vertices of the level with degree >= LARGE_CUTOFF /
 // MASSIVE_CUTOFF, which bound the movers of the last two classes.  The uncut
-// change goes to `at`; a hub table that runs out of slots sets SC_STALE.
+// change goes to `at`.
 // reset: the movers' neighbours are scored again in the next sweep.
 template <class AT>
-static void apply_moves_core(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, i64* vol, const i32* moves,
-                             i64 k, i64 n_large, i64 n_massive, bool reset, AT at, i64 nfull) {
+static void apply_moves_core(Ctx& c, MoveScratch& s, const LevelPlan& lp, const DGraph& g, i64* vol, const i32* moves,
+                             i64 k, i64 n_large, i64 n_massive, bool reset, AT at) {
     const i64 nw = std::min(k, n_large);
     const i64 nb = std::min(k, n_massive);
     const int tk = c.kt_begin(KS_MOVES);
-    const i64 m7 = lp.nhub;
-    // many movers: updating costs more than rebuilding the tables next sweep
-    if (lp.hub_live && m7 > 0 && (c.hub_update_div <= 0 || k * c.hub_update_div > nfull)) lp.hub_live = false;
-    const bool hub_upd = lp.hub_live && m7 > 0;
     k_mvp_moves<<<grid_items(k, 256), 256, 0, c.stream>>>(moves, k, s.part, s.dest, s.mvp);
     PGGC_LAUNCH_CHECK();
     const i64 cpm = nb > 0 ? ceil_div(lp.max_deg, MV_CHUNK) : 1;
     const i64 b1 = ceil_div(k, 256 / MV_G), b2 = ceil_div(nw, 2), b3 = nb * cpm;
-    const HubView hv{hub_upd ? lp.hidx.p : nullptr, lp.goff, lp.hsm, lp.gkeys, lp.gvals, lp.gtab, lp.hlist, lp.hcnt,
-                     s.scal.p + SC_STALE};
-#define PGGC_MOVE_EDGES(HUB, PK, RS)                                                                               \
-    k_move_edges<HUB, PK, RS><<<grid_blocks(b1 + b2 + b3), 256, 0, c.stream>>>(g.rp, g.col, W, moves, k, b1, b2, nw, \
-                                                                              nb, cpm, s.mvp, hv, s.dest, at)
+#define PGGC_MOVE_EDGES(RS)                                                                                          \
+    k_move_edges<RS><<<grid_blocks(b1 + b2 + b3), 256, 0, c.stream>>>(g.rp, g.col, W, moves, k, b1, b2, nw, nb, cpm,  \
+                                                                      s.mvp, s.dest, at)
     PGGC_WDISPATCH(g, {
-        if (!hub_upd && reset) PGGC_MOVE_EDGES(false, false, true);
-        else if (!hub_upd) PGGC_MOVE_EDGES(false, false, false);
-        else if (lp.packed && reset) PGGC_MOVE_EDGES(true, true, true);
-        else if (lp.packed) PGGC_MOVE_EDGES(true, true, false);
-        else if (reset) PGGC_MOVE_EDGES(true, false, true);
-        else PGGC_MOVE_EDGES(true, false, false);
+        if (reset) PGGC_MOVE_EDGES(true);
+        else PGGC_MOVE_EDGES(false);
     });
 #undef PGGC_MOVE_EDGES
     PGGC_LAUNCH_CHECK();
@@ -2175,13 +1673,12 @@ static void apply_moves_core(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph
     if (tk >= 0) {  // timing runs only
         // per mover its word (written, read, settled), row bounds, cluster,
         // destination, vertex weight and two volume updates; per mover edge
-        // the column, weight, the neighbour's word and its destination reset,
-        // plus the hub index when hub tables are kept current
+        // the column, weight, the neighbour's word and its destination reset
         const int wb = g.wk == W_UNIT ? 0 : g.wk == W_I32 ? 4 : 8;
         Buf<i64> acc(c, 1);
         fill_i64(c, acc, 1, 0);
         k_list_bytes<<<grid_items(std::max<i64>(k, 1), 256), 256, 0, c.stream>>>(
-            g.rp, moves, k, 84, 12 + wb + (reset ? 4 : 0) + (hub_upd ? 4 : 0), 0, acc);
+            g.rp, moves, k, 84, 12 + wb + (reset ? 4 : 0), 0, acc);
         PGGC_LAUNCH_CHECK();
         acct_add(c, c.kt_counter(tk), acc);
     }
@@ -2194,8 +1691,8 @@ static void init_mvp(Ctx& c, MoveScratch& s, i64 n) {
 }
 
 static void perform_moves(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, RefineData& curr,
-                          const i32* moves, i64 k, i64 n_large, i64 n_massive, bool& tables, i64 nfull) {
-    apply_moves_core(c, s, lp, g, curr.vol, moves, k, n_large, n_massive, tables, AccOne{s.scal.p + SC_SLOTS}, nfull);
+                          const i32* moves, i64 k, i64 n_large, i64 n_massive, bool& tables) {
+    apply_moves_core(c, s, lp, g, curr.vol, moves, k, n_large, n_massive, tables, AccOne{s.scal.p + SC_SLOTS});
     if (!tables) {
         tables = true;
         fill_i32(c, s.dest, g.n, NULL_PART);
@@ -2206,7 +1703,6 @@ static void perform_moves(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g
     PGGC_LAUNCH_CHECK();
     c.sync();
     const i64* h = c.pinned;
-    if (h[3]) lp.hub_live = false;  // a hub table ran out of slots: rebuild next sweep
     curr.uncut += h[0];
     curr.obj = objective_value(curr.uncut, curr.lambda, (u64)h[1], (u64)h[2]);
 }
@@ -2333,8 +1829,6 @@ static void local_move_t(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g,
     const i64 n = g.n;
     s.ensure(c, nfull);
     plan_level(c, g, lp);
-    hub_tables_acquire(c, lp);
-    lp.hub_live = false;  // the clustering changed since the last call
     c.mem_note("local move: plan ready");
     Buf<i64> cv;
     RefineData curr = begin_curr(c, best, cv, nfull);
@@ -2407,7 +1901,7 @@ static void local_move_t(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g,
             if (iter > 1 || !is_initial)
                 set_new_cluster_ids(c, s, g, curr, s.moves, km, constrained ? cons : nullptr, ids, nfull);
             fresh = !tables;
-            perform_moves(c, s, lp, g, curr, s.moves, km, g.n - lp.ord.off_large, g.n - lp.ord.off_large2, tables, nfull);
+            perform_moves(c, s, lp, g, curr, s.moves, km, g.n - lp.ord.off_large, g.n - lp.ord.off_large2, tables);
             if (stats) stats->moves += km;
             if (c.verbose >= 3)
                 fprintf(stderr, "sweep n=%lld it=%d cands=%lld moves=%lld labels=%d uncut=%lld obj=%.17g\n",
@@ -2421,7 +1915,7 @@ static void local_move_t(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g,
         }
     }
     relabel(c, s, nfull, best_part, best);
-    hub_tables_settle(c, lp);
+    s.hub_kv.reset();
 }
 
 // afterburner_filter_strict (src/local_mover.cpp:131-213): exact sequential
@@ -2492,8 +1986,6 @@ void local_move_strict(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, i
     const i64 n = g.n;
     s.ensure(c, n);
     plan_level(c, g, lp);
-    hub_tables_acquire(c, lp);
-    lp.hub_live = false;  // the clustering changed since the last call
     Buf<i64> cv;
     RefineData curr = begin_curr(c, best, cv, n);
     copy_dev(c, s.part, best_part, n * sizeof(i32));
@@ -2532,7 +2024,7 @@ void local_move_strict(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, i
             trc.end(k, 0);
             break;
         }
-        perform_moves(c, s, lp, g, curr, s.moves, tr, g.n - lp.ord.off_large, g.n - lp.ord.off_large2, tables, n);
+        perform_moves(c, s, lp, g, curr, s.moves, tr, g.n - lp.ord.off_large, g.n - lp.ord.off_large2, tables);
         if (stats) stats->moves += tr;
         if (curr.obj > best.obj) {
             copy_state(c, best, curr);
@@ -2542,7 +2034,7 @@ void local_move_strict(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, i
         trc.end(k, tr);
     }
     relabel(c, s, n, best_part, best);
-    hub_tables_settle(c, lp);
+    s.hub_kv.reset();
 }
 
 i64 sweep_once(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, const i32* part, const i64* vol, i64 L,
@@ -2552,8 +2044,6 @@ i64 sweep_once(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, const i32
     (void)L;
     s.ensure(c, n);
     plan_level(c, g, lp);
-    hub_tables_acquire(c, lp);
-    lp.hub_live = false;
     copy_dev(c, s.part, part, n * sizeof(i32));
     copy_dev(c, s.dest, dest, n * sizeof(i32));
     copy_dev(c, s.gain, gain, n * sizeof(float));
@@ -2570,7 +2060,7 @@ i64 sweep_once(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, const i32
     copy_dev(c, dest, s.dest, n * sizeof(i32));
     copy_dev(c, gain, s.gain, n * sizeof(float));
     c.sync();
-    hub_tables_settle(c, lp);
+    s.hub_kv.reset();
     return km;
 }
 
@@ -2855,8 +2345,6 @@ void local_move_batch(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, co
     const i64 n = g.n, K = bl.K, NL = best.loff[K];
     s.ensure(c, std::max(n, NL));
     plan_level(c, g, lp);
-    hub_tables_acquire(c, lp);
-    lp.hub_live = false;
     Buf<i64> cvol(c, std::max<i64>(NL, 1));
     copy_dev(c, cvol, best.vol, NL * sizeof(i64));
     std::vector<RefineData> cur = best.rd;
@@ -2920,7 +2408,7 @@ void local_move_batch(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, co
             fill_i64(c, acc, K, 0);
             // resets the movers and their neighbours; every vertex of an
             // instance whose first moves these are follows below
-            apply_moves_core(c, s, lp, g, cvol, s.moves, km, n_large, n_massive, true, AccInst{bl.inst, acc}, n);
+            apply_moves_core(c, s, lp, g, cvol, s.moves, km, n_large, n_massive, true, AccInst{bl.inst, acc});
             bool anyfull = false;
             for (i64 q = 0; q < K; q++) {
                 const bool moved = hc[K + q] > 0;
@@ -2938,9 +2426,6 @@ void local_move_batch(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, co
             upload(c, imp.p, himp);
             k_inst_sumsq<<<grid_blocks(K), 256, 0, c.stream>>>(cvol, best.dloff, Ld, imp, K, sq);
             PGGC_LAUNCH_CHECK();
-            const i64 stale = c.read1(s.scal.p + SC_STALE);
-            if (stale) fill_i64(c, s.scal.p + SC_STALE, 1, 0);
-            if (stale) lp.hub_live = false;  // a hub table ran out of slots: rebuild next sweep
             download(c, hacc, acc.p, K);
             download(c, hsq, sq.p, 2 * K);
             bool anyimp = false;
@@ -2983,7 +2468,7 @@ void local_move_batch(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, co
         }
     }
     relabel_batch(c, s, bl, best_part, best, active);
-    hub_tables_settle(c, lp);
+    s.hub_kv.reset();
 }
 
 }  // namespace pggc
