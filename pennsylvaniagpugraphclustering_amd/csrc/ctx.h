@@ -175,9 +175,6 @@ void copy_h2d(Ctx& c, void* dst, const void* src, size_t bytes);
 // out[0..n] = exclusive scan of in[0..n); out[n] = total.  in may alias out.
 void scan_i64(Ctx& c, const i64* in, i64* out, i64 n);
 void scan_i32_to_i64(Ctx& c, const i32* in, i64* out, i64 n);
-// Ordered compaction of the indices x in [0,n) with flag[x] != 0, writing
-// src ? src[x] : x; returns the count (read back to the host).
-i64 compact_flags(Ctx& c, const i32* flag, const i32* src, i64 n, i32* out, i64* count_dev);
 // Stable LSD radix sort of (key, val) pairs on key bits [begin, bits).
 void radix_sort_pairs(Ctx& c, u64* keys, i32* vals, i64 n, int bits, int begin = 0);
 void radix_sort_pairs(Ctx& c, u64* keys, i64* vals, i64 n, int bits);

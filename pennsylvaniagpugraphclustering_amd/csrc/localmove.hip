@@ -19,6 +19,7 @@
 #include "gnn.h"
 #include "hash.h"
 #include "localmove.h"
+#include "select.h"
 
 namespace pggc {
 
@@ -40,7 +41,7 @@ void update_objective(Ctx& c, RefineData& rd) {
 // ------------------------------------------------------------- scratch
 // Scalars of a sweep in MoveScratch::scal, zeroed at the start of a call:
 // the MV_SLOTS words of the uncut change are zero between sweeps, SC_TICKET counts k_finish's blocks (at most FIN_BLOCKS).
-constexpr int SC_TICKET = 4, SC_SLOTS = 16, MV_SLOTS = 64, SC_COUNT = SC_SLOTS + MV_SLOTS;
+constexpr int SC_EXTRA = 0, SC_TICKET = 4, SC_SLOTS = 16, MV_SLOTS = 64, SC_COUNT = SC_SLOTS + MV_SLOTS;
 constexpr int FIN_BLOCKS = 256;
 void MoveScratch::ensure(Ctx& c, i64 n) {
     if (cap >= n) return;
@@ -67,6 +68,8 @@ __host__ __device__ __forceinline__ int score_class(i64 d) {
     return d <= 4 ? 0 : d <= 8 ? 1 : d <= 16 ? 2 : d <= 32 ? 3 : d <= 64 ? 4 : d <= 128 ? 5 : d <= 256 ? 6
          : d <= 512 ? 7 : d <= 1024 ? 8 : d <= 2048 ? 9 : 10;
 }
+// small levels, bound by launches (find_movers)
+constexpr i64 DIRECT_MAX = (i64)1 << 18;
 // Level of at most this many rows in the LDS-table classes: one launch for all
 // (the chip holds 5 of its 256-thread blocks per CU, 1,280 at once, so two
 // rounds of blocks cost less than the four launches saved).
@@ -209,6 +212,11 @@ void plan_level(Ctx& c, const DGraph& g, LevelPlan& p) {
         p.hub_blocks = c.read1(p.hub_groups.p + ng) * NXCD;
         p.hub_edges = c.read1(p.hub_eoff.p + p.nhub);
     }
+}
+
+// a mover's word in MoveScratch::mvp
+__device__ __forceinline__ u64 mvp_moved(i32 from, i32 to) {
+    return (u64)((u32)from | 0x80000000u) | ((u64)(u32)to << 32);
 }
 
 // ------------------------------------------------------------- scoring
@@ -933,14 +941,16 @@ __global__ void __launch_bounds__(256) k_score_bytes(const i64* __restrict__ rp,
 }
 
 // alpha + beta * degree bytes per listed vertex (per candidate of the
-// afterburner, per mover of perform_moves), plus `extra` once
-__global__ void __launch_bounds__(256) k_list_bytes(const i64* __restrict__ rp, const i32* __restrict__ list, i64 k,
-                                                    i64 alpha, i64 beta, i64 extra, i64* acc) {
+// afterburner, per mover of perform_moves) that is not NO_MOVE in dest (when
+// given), plus `extra` once
+__global__ void __launch_bounds__(256) k_list_bytes(const i64* __restrict__ rp, const i32* __restrict__ list,
+                                                    const i32* __restrict__ dest, i64 k, i64 alpha, i64 beta,
+                                                    i64 extra, i64* acc) {
     const i64 x = thread_item();
     i64 b = 0;
     if (x < k) {
         const i32 i = list[x];
-        b = alpha + beta * (rp[i + 1] - rp[i]);
+        if (!dest || dest[i] != NO_MOVE) b = alpha + beta * (rp[i + 1] - rp[i]);
     }
     if (x == 0) b += extra;
     b = block_sum_i64<256>(b);
@@ -1103,41 +1113,20 @@ static void score_all(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, co
 }
 
 // ------------------------------------------------------------- candidates
-__global__ void k_cand_flags(const i32* o1, i64 n, const i32* dest, i32* flag) {
-    const i64 x = thread_item();
-    if (x >= n) return;
-    flag[x] = dest[o1[x]] != NO_MOVE ? 1 : 0;
-}
-// first list positions whose degree reaches LARGE_CUTOFF / MASSIVE_CUTOFF
-__global__ void k_list_bounds(const i32* list, i64 k, const i64* rp, i64* out) {
-    if (threadIdx.x >= 2) return;
-    i64 cut = threadIdx.x == 0 ? LARGE_CUTOFF : MASSIVE_CUTOFF;
-    i64 lo = 0, hi = k;
-    while (lo < hi) {
-        i64 m = (lo + hi) >> 1;
-        i32 i = list[m];
-        if (rp[i + 1] - rp[i] >= cut) hi = m;
-        else lo = m + 1;
-    }
-    out[threadIdx.x] = lo;
-}
-
-// candidates in order1 order; returns count, b[0]/b[1] = class boundaries
-static i64 gather_candidates(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, const i32* dest, i32* out,
-                             i64* b) {
-    k_cand_flags<<<grid_items(g.n, 256), 256, 0, c.stream>>>(lp.ord.o1, g.n, dest, s.flag);
-    PGGC_LAUNCH_CHECK();
-    i64 k = compact_flags(c, s.flag, lp.ord.o1, g.n, out, s.scal);
-    if (k > 0) {
-        k_list_bounds<<<1, 64, 0, c.stream>>>(out, k, g.rp, s.scal.p + 1);
-        PGGC_LAUNCH_CHECK();
-        const i64* h = c.read(s.scal.p + 1, 2);
-        b[0] = h[0];
-        b[1] = h[1];
-    } else {
-        b[0] = b[1] = 0;
-    }
-    return k;
+struct SelCands {
+    static constexpr bool extra = false;
+    const i32* o1;
+    const i32* dest;
+    i32* out;
+    __device__ __forceinline__ bool test(i64 x) const { return dest[o1[x]] != NO_MOVE; }
+    __device__ __forceinline__ void emit(i64 pos, i64 x) const { out[pos] = o1[x]; }
+};
+// candidates in order1 order; returns the count, b[0]/b[1] = class boundaries
+static i64 gather_candidates(Ctx& c, const LevelPlan& lp, const DGraph& g, const i32* dest, i32* out, i64* b) {
+    const i64* h = select_items(c, SelCands{lp.ord.o1, dest, out}, g.n, SelBounds{lp.ord.off_large, lp.ord.off_large2});
+    b[0] = h[1];
+    b[1] = h[2];
+    return h[0];
 }
 
 // ------------------------------------------------------------- afterburner
@@ -1147,7 +1136,8 @@ static i64 gather_candidates(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph
 // this order: what the neighbour's destination means for the candidate's own
 // and best cluster, then what its leaving its cluster means.  (At most one
 // comparison of each pair holds, as the best cluster is never the own one;
-// an edge without effect adds zeros.)
+// an edge without effect adds zeros.)  The kernels take a list of candidates,
+// or all vertices in order1 order and skip those whose record says NO_MOVE.
 struct AbSelf {
     i32 p, best, hi;
     float multi, igain;
@@ -1178,12 +1168,12 @@ __device__ __forceinline__ float2 ab_terms(const AbInfo& q4, i32 v, i64 w, const
 // candidates have at most a few dozen edges.
 constexpr int AB_G = 16, AB_U = 4, AB_PB = 256 / AB_G;
 template <class WT, class LT, class PT>
-__global__ void __launch_bounds__(256) k_ab_small(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
-                                                  const AbInfo* __restrict__ info, const i32* __restrict__ cand,
-                                                  i64 k, LT lam, PT prio, i32* __restrict__ keep) {
+__device__ __forceinline__ void ab_small(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
+                                         const AbInfo* __restrict__ info, const i32* __restrict__ cand, i64 blk, i64 k,
+                                         LT lam, PT prio, i32* __restrict__ keep) {
     __shared__ float2 term[AB_PB][LARGE_CUTOFF + 1];
     const int lane = threadIdx.x & (AB_G - 1), grp = threadIdx.x / AB_G;
-    const i64 x = block_id() * AB_PB + grp;
+    const i64 x = blk * AB_PB + grp;
     int d = 0;
     float igain = 0.0f;
     if (x < k) {
@@ -1191,7 +1181,7 @@ __global__ void __launch_bounds__(256) k_ab_small(const i64* __restrict__ rp, co
         const AbSelf m = ab_self(info, i, lam, prio);
         igain = m.igain;
         const i64 s = rp[i];
-        d = (int)(rp[i + 1] - s);
+        d = m.best == NO_MOVE ? -1 : (int)(rp[i + 1] - s);
         for (int jb = lane; jb < d; jb += AB_G * AB_U) {
             i32 v[AB_U];
             AbInfo q[AB_U];
@@ -1214,20 +1204,23 @@ __global__ void __launch_bounds__(256) k_ab_small(const i64* __restrict__ rp, co
             acc = acc + t.x;
             acc = acc + t.y;
         }
-        keep[x] = (igain + acc >= 0.0f) ? 1 : 0;
+        keep[x] = (d >= 0 && igain + acc >= 0.0f) ? 1 : 0;
     }
 }
 
 // One wave per candidate: 64 strided partials and a halving tree.
 template <class WT, class LT, class PT>
-__global__ void __launch_bounds__(256) k_ab_wave(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
-                                                 const AbInfo* __restrict__ info, const i32* __restrict__ cand, i64 k0,
-                                                 i64 k1, LT lam, PT prio, i32* __restrict__ keep) {
+__device__ __forceinline__ void ab_wave(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
+                                        const AbInfo* __restrict__ info, const i32* __restrict__ cand, i64 x, i64 k1,
+                                        LT lam, PT prio, i32* __restrict__ keep) {
     const int lane = threadIdx.x & 63;
-    const i64 x = k0 + block_id() * 4 + (threadIdx.x >> 6);
     if (x >= k1) return;
     const i32 i = cand[x];
     const AbSelf m = ab_self(info, i, lam, prio);
+    if (m.best == NO_MOVE) {  // wave-uniform
+        if (lane == 0) keep[x] = 0;
+        return;
+    }
     float acc = 0.0f;
     const i64 e = rp[i + 1];
     constexpr int U = 4;
@@ -1253,6 +1246,17 @@ __global__ void __launch_bounds__(256) k_ab_wave(const i64* __restrict__ rp, con
     if (lane == 0) keep[x] = (m.igain + acc >= 0.0f) ? 1 : 0;
 }
 
+// both classes in one launch: list entries [0, k0) in the first b0 blocks
+// (AB_PB each), [k0, k1) in the others (a wave each)
+template <class WT, class LT, class PT>
+__global__ void __launch_bounds__(256) k_ab_lanes(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
+                                                  const AbInfo* __restrict__ info, const i32* __restrict__ cand,
+                                                  i64 k0, i64 k1, i64 b0, LT lam, PT prio, i32* __restrict__ keep) {
+    const i64 b = block_id();
+    if (b < b0) ab_small(rp, col, W, info, cand, b, k0, lam, prio, keep);
+    else ab_wave(rp, col, W, info, cand, k0 + (b - b0) * 4 + (threadIdx.x >> 6), k1, lam, prio, keep);
+}
+
 // A 1024-thread block per candidate: 1024 strided partials and a halving tree.
 template <class WT, class LT, class PT>
 __global__ void __launch_bounds__(1024) k_ab_block(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
@@ -1264,6 +1268,10 @@ __global__ void __launch_bounds__(1024) k_ab_block(const i64* __restrict__ rp, c
     if (x >= k1) return;
     const i32 i = cand[x];
     const AbSelf m = ab_self(info, i, lam, prio);
+    if (m.best == NO_MOVE) {  // block-uniform
+        if (t == 0) keep[x] = 0;
+        return;
+    }
     float acc = 0.0f;
     const i64 e = rp[i + 1];
     constexpr int U = 4;
@@ -1311,21 +1319,46 @@ __global__ void __launch_bounds__(256) k_ab_pack(i64 n, const float* __restrict_
     info[i] = a;
 }
 
+// The kept candidates become the sweep's movers, in order1 order, and are
+// marked in mvp.  first counts the movers that take a new cluster, second the
+// candidates.
+struct SelMoves {
+    static constexpr bool extra = true;
+    const i32* cand;
+    const i32* keep;
+    const i32* dest;
+    const i32* part;
+    i32* moves;
+    u64* mvp;
+    __device__ __forceinline__ bool test(i64 x) const { return keep[x] != 0; }
+    __device__ __forceinline__ bool first(i64 x, bool sel) const { return sel && dest[cand[x]] == NEW_PART; }
+    __device__ __forceinline__ bool second(i64 x, bool) const { return dest[cand[x]] != NO_MOVE; }
+    __device__ __forceinline__ void emit(i64 pos, i64 x) const {
+        const i32 i = cand[x];
+        moves[pos] = i;
+        mvp[i] = mvp_moved(part[i], dest[i]);
+    }
+};
+struct Movers {
+    i64 k;      // movers
+    i64 knew;   // of them with destination NEW_PART
+    i64 cands;  // candidates
+};
+
+// cand: k candidates, or every vertex, in order1 order; b: class boundaries
 template <class LT, class PT>
-static i64 afterburner(Ctx& c, MoveScratch& s, const DGraph& g, const i32* cand, i64 k, const i64* b, LT lam, PT prio,
-                       i32* moves, bool pack) {
+static Movers afterburner(Ctx& c, MoveScratch& s, const DGraph& g, const i32* cand, i64 k, const i64* b, LT lam,
+                          PT prio, i32* moves, bool pack) {
     const int tk = c.kt_begin(KS_AFTERBURNER);
     if (pack) {
         k_ab_pack<<<grid_items(g.n, 256), 256, 0, c.stream>>>(g.n, s.gain, s.dest, s.part, g.vw, s.abi);
         PGGC_LAUNCH_CHECK();
     }
+    const i64 nb0 = ceil_div(b[0], AB_PB), nb1 = ceil_div(b[1] - b[0], 4);
     PGGC_WDISPATCH(g, {
-        if (b[0] > 0)
-            k_ab_small<<<grid_items(b[0], AB_PB), 256, 0, c.stream>>>(g.rp, g.col, W, s.abi, cand, b[0], lam, prio,
-                                                                      s.flag);
-        if (b[1] > b[0])
-            k_ab_wave<<<grid_items(b[1] - b[0], 4), 256, 0, c.stream>>>(g.rp, g.col, W, s.abi, cand, b[0], b[1], lam,
-                                                                        prio, s.flag);
+        if (nb0 + nb1 > 0)
+            k_ab_lanes<<<grid_blocks(nb0 + nb1), 256, 0, c.stream>>>(g.rp, g.col, W, s.abi, cand, b[0], b[1], nb0, lam,
+                                                                     prio, s.flag);
         if (k > b[1])
             k_ab_block<<<grid_blocks(k - b[1]), 1024, 0, c.stream>>>(g.rp, g.col, W, s.abi, cand, b[1], k, lam,
                                                                      prio, s.flag);
@@ -1339,11 +1372,13 @@ static i64 afterburner(Ctx& c, MoveScratch& s, const DGraph& g, const i32* cand,
         Buf<i64> acc(c, 1);
         fill_i64(c, acc, 1, 0);
         k_list_bytes<<<grid_items(std::max<i64>(k, 1), 256), 256, 0, c.stream>>>(
-            g.rp, cand, k, 40, 20 + (g.wk == W_UNIT ? 0 : g.wk == W_I32 ? 4 : 8), pack ? 36 * g.n : 0, acc);
+            g.rp, cand, s.dest, k, 40, 20 + (g.wk == W_UNIT ? 0 : g.wk == W_I32 ? 4 : 8), pack ? 36 * g.n : 0, acc);
         PGGC_LAUNCH_CHECK();
         acct_add(c, c.kt_counter(tk), acc);
     }
-    return compact_flags(c, s.flag, cand, k, moves, s.scal);
+    const i64* h = select_items(c, SelMoves{cand, s.flag, s.dest, s.part, moves, s.mvp}, k, SelBounds{0, 0},
+                                s.scal.p + SC_EXTRA);
+    return Movers{h[0], h[3], h[4]};
 }
 
 // ------------------------------------------------------------- new labels
@@ -1390,7 +1425,7 @@ static void set_new_cluster_ids(Ctx& c, MoveScratch& s, const DGraph& g, RefineD
                                 i32* cons, const i32* ids, i64 nfull) {
     k_new_flags<<<grid_items(k, 256), 256, 0, c.stream>>>(moves, k, s.dest, s.flag);
     PGGC_LAUNCH_CHECK();
-    i64 K = compact_flags(c, s.flag, moves, k, s.tmp, s.scal);
+    i64 K = compact_flags(c, s.flag, moves, k, s.tmp);
     if (K == 0) return;
     if (ids && K > 1) {
         Buf<u64> key(c, K);
@@ -1405,7 +1440,7 @@ static void set_new_cluster_ids(Ctx& c, MoveScratch& s, const DGraph& g, RefineD
     Buf<i32> uf(c, std::max<i64>(curr, 1));
     k_unused_flags<<<grid_items(curr, 256), 256, 0, c.stream>>>(s.flag, curr, uf);
     PGGC_LAUNCH_CHECK();
-    i64 A = compact_flags(c, uf, nullptr, curr, s.tmp2, s.scal);
+    i64 A = compact_flags(c, uf, nullptr, curr, s.tmp2);
     if (K > A) {
         i64 need = K - A;
         if (curr + need > rd.cap) throw Error(-4, "label capacity exceeded while assigning new clusters");
@@ -1420,7 +1455,7 @@ static void set_new_cluster_ids(Ctx& c, MoveScratch& s, const DGraph& g, RefineD
 // mvp[v]: low word the cluster of v | moved << 31 (cluster ids are >= 0), high
 // word the cluster after this sweep's moves.  Between sweeps both words are
 // v's cluster (k_mvp_init at the start of a call); a sweep marks its movers
-// (k_mvp_moves) and k_apply_moves settles them, so a sweep touches the movers'
+// (SelMoves, or k_mvp_moves once new cluster ids are known) and k_apply_moves settles them, so a sweep touches the movers'
 // words only, and an edge's uncut change reads one 8-byte word.
 __global__ void __launch_bounds__(256) k_mvp_init(i64 n, const i32* __restrict__ part, u64* __restrict__ mvp,
                                                   i64* scal) {
@@ -1435,7 +1470,7 @@ __global__ void __launch_bounds__(256) k_mvp_moves(const i32* __restrict__ moves
     const i64 x = thread_item();
     if (x >= k) return;
     const i32 i = moves[x];
-    mvp[i] = (u64)((u32)part[i] | 0x80000000u) | ((u64)(u32)dest[i] << 32);
+    mvp[i] = mvp_moved(part[i], dest[i]);
 }
 
 // Where the uncut changes of the movers are added: AccOne spreads one sum over
@@ -1647,15 +1682,18 @@ __global__ void __launch_bounds__(256) k_finish(const i64* __restrict__ vol, i64
 // n_large / n_massive = vertices of the level with degree >= LARGE_CUTOFF /
 // MASSIVE_CUTOFF, which bound the movers of the last two classes.  The uncut
 // change goes to `at`.
-// reset: the movers' neighbours are scored again in the next sweep.
+// reset: the movers' neighbours are scored again in the next sweep.  marked:
+// the movers' words are in mvp already.
 template <class AT>
 static void apply_moves_core(Ctx& c, MoveScratch& s, const LevelPlan& lp, const DGraph& g, i64* vol, const i32* moves,
-                             i64 k, i64 n_large, i64 n_massive, bool reset, AT at) {
+                             i64 k, bool marked, i64 n_large, i64 n_massive, bool reset, AT at) {
     const i64 nw = std::min(k, n_large);
     const i64 nb = std::min(k, n_massive);
     const int tk = c.kt_begin(KS_MOVES);
-    k_mvp_moves<<<grid_items(k, 256), 256, 0, c.stream>>>(moves, k, s.part, s.dest, s.mvp);
-    PGGC_LAUNCH_CHECK();
+    if (!marked) {
+        k_mvp_moves<<<grid_items(k, 256), 256, 0, c.stream>>>(moves, k, s.part, s.dest, s.mvp);
+        PGGC_LAUNCH_CHECK();
+    }
     const i64 cpm = nb > 0 ? ceil_div(lp.max_deg, MV_CHUNK) : 1;
     const i64 b1 = ceil_div(k, 256 / MV_G), b2 = ceil_div(nw, 2), b3 = nb * cpm;
 #define PGGC_MOVE_EDGES(RS)                                                                                          \
@@ -1678,7 +1716,7 @@ static void apply_moves_core(Ctx& c, MoveScratch& s, const LevelPlan& lp, const 
         Buf<i64> acc(c, 1);
         fill_i64(c, acc, 1, 0);
         k_list_bytes<<<grid_items(std::max<i64>(k, 1), 256), 256, 0, c.stream>>>(
-            g.rp, moves, k, 84, 12 + wb + (reset ? 4 : 0), 0, acc);
+            g.rp, moves, nullptr, k, 84, 12 + wb + (reset ? 4 : 0), 0, acc);
         PGGC_LAUNCH_CHECK();
         acct_add(c, c.kt_counter(tk), acc);
     }
@@ -1691,8 +1729,8 @@ static void init_mvp(Ctx& c, MoveScratch& s, i64 n) {
 }
 
 static void perform_moves(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, RefineData& curr,
-                          const i32* moves, i64 k, i64 n_large, i64 n_massive, bool& tables) {
-    apply_moves_core(c, s, lp, g, curr.vol, moves, k, n_large, n_massive, tables, AccOne{s.scal.p + SC_SLOTS});
+                          const i32* moves, i64 k, bool marked, i64 n_large, i64 n_massive, bool& tables) {
+    apply_moves_core(c, s, lp, g, curr.vol, moves, k, marked, n_large, n_massive, tables, AccOne{s.scal.p + SC_SLOTS});
     if (!tables) {
         tables = true;
         fill_i32(c, s.dest, g.n, NULL_PART);
@@ -1708,15 +1746,23 @@ static void perform_moves(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g
 }
 
 // ------------------------------------------------------------- relabel
-__global__ void k_relabel_vol(const i32* used, const i64* pos, i64 L, const i64* vol, i64* nvol) {
-    const i64 l = thread_item();
-    if (l >= L) return;
-    if (used[l]) nvol[pos[l]] = vol[l];
-}
-__global__ void k_relabel_part(const i64* pos, i64 n, i32* part) {
+// the pos-th used label becomes label pos
+struct SelLabels {
+    static constexpr bool extra = false;
+    const i32* used;
+    const i64* vol;
+    i64* nvol;
+    i32* map;
+    __device__ __forceinline__ bool test(i64 l) const { return used[l] != 0; }
+    __device__ __forceinline__ void emit(i64 pos, i64 l) const {
+        nvol[pos] = vol[l];
+        map[l] = (i32)pos;
+    }
+};
+__global__ void k_relabel_part(const i32* map, i64 n, i32* part) {
     const i64 i = thread_item();
     if (i >= n) return;
-    part[i] = (i32)pos[part[i]];
+    part[i] = map[part[i]];
 }
 
 // relabel_contiguously (src/local_mover.cpp:100-129)
@@ -1725,13 +1771,11 @@ static void relabel(Ctx& c, MoveScratch& s, i64 n, i32* labels, RefineData& rd) 
     fill_i32(c, s.flag, L, 0);
     k_mark_used<<<grid_items(n, 256), 256, 0, c.stream>>>(labels, n, s.flag);
     PGGC_LAUNCH_CHECK();
-    Buf<i64> pos(c, L + 1), nvol(c, std::max<i64>(L, 1));
-    scan_i32_to_i64(c, s.flag, pos, L);
-    k_relabel_vol<<<grid_items(L, 256), 256, 0, c.stream>>>(s.flag, pos, L, rd.vol, nvol);
-    PGGC_LAUNCH_CHECK();
-    i64 t = c.read1(pos.p + L);
+    Buf<i32> map(c, std::max<i64>(L, 1));
+    Buf<i64> nvol(c, std::max<i64>(L, 1));
+    const i64 t = select_items(c, SelLabels{s.flag, rd.vol, nvol, map}, L)[0];
     copy_dev(c, rd.vol, nvol, t * sizeof(i64));
-    k_relabel_part<<<grid_items(n, 256), 256, 0, c.stream>>>(pos, n, labels);
+    k_relabel_part<<<grid_items(n, 256), 256, 0, c.stream>>>(map, n, labels);
     PGGC_LAUNCH_CHECK();
     rd.label_count = (i32)t;
 }
@@ -1746,10 +1790,34 @@ static void copy_state(Ctx& c, RefineData& dst, const RefineData& src) {
     dst.lambda = src.lambda;
 }
 
+// the best state so far: volumes and clusters, on small levels in one launch
+__global__ void __launch_bounds__(256) k_copy_best(const i64* __restrict__ vol, i64 L, i64* __restrict__ bvol,
+                                                   const i32* __restrict__ part, i64 n, i32* __restrict__ bpart) {
+    const i64 x = thread_item();
+    if (x < L) bvol[x] = vol[x];
+    if (x < n) bpart[x] = part[x];
+}
+static void copy_best(Ctx& c, RefineData& best, const RefineData& curr, i32* best_part, const i32* part, i64 n) {
+    const i64 L = curr.label_count;
+    if (std::max(n, L) > DIRECT_MAX) {  // 16-byte words
+        copy_state(c, best, curr);
+        copy_dev(c, best_part, part, n * sizeof(i32));
+        return;
+    }
+    if (L > best.cap) throw Error(-4, "label capacity exceeded");
+    k_copy_best<<<grid_items(std::max(n, L), 256), 256, 0, c.stream>>>(curr.vol, L, best.vol, part, n, best_part);
+    PGGC_LAUNCH_CHECK();
+    i64* vol = best.vol;
+    const i64 cap = best.cap;
+    const double scale = best.scale, offset = best.offset;
+    best = curr;
+    best.vol = vol;
+    best.cap = cap;
+    best.scale = scale;
+    best.offset = offset;
+}
+
 // ------------------------------------------------------------- drivers
-struct CurrVol {
-    Buf<i64> v;
-};
 
 // ------------------------------------------------------------ sweep trace
 __global__ void __launch_bounds__(256) k_count_active(const i32* dest, i64 n, i64* out) {
@@ -1803,6 +1871,23 @@ static RefineData begin_curr(Ctx& c, const RefineData& best, Buf<i64>& cv, i64 n
     curr.cap = cap;
     copy_state(c, curr, best);
     return curr;
+}
+
+// The sweep's movers from its scored vertices.  Levels of at most
+// DIRECT_MAX vertices run the afterburner over all vertices and skip the
+// others, which saves a selection, its launches and a read-back; larger ones
+// list the candidates first, so that lanes are not spent on the others.
+// DIRECT
+template <class LT, class PT>
+static Movers find_movers(Ctx& c, MoveScratch& s, const LevelPlan& lp, const DGraph& g, LT lam, PT prio, bool pack) {
+    i64 b[2];
+    if (g.n <= DIRECT_MAX && !pack) {
+        b[0] = lp.ord.off_large;
+        b[1] = lp.ord.off_large2;
+        return afterburner(c, s, g, lp.ord.o1, g.n, b, lam, prio, s.moves, false);
+    }
+    const i64 k = gather_candidates(c, lp, g, s.dest, s.cand, b);
+    return k > 0 ? afterburner(c, s, g, s.cand, k, b, lam, prio, s.moves, pack) : Movers{0, 0, 0};
 }
 
 template <class PT>
@@ -1873,16 +1958,14 @@ static void local_move_t(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g,
             tr.begin(s.dest, iter == 1 && !use, fresh);
             fresh = false;
             score_all(c, s, lp, g, s.part, curr.vol, ccons, tables ? 0 : raw_mode, lam, fr, so);
-            i64 b[2];
-            i64 k = gather_candidates(c, s, lp, g, s.dest, s.cand, b);
-            i64 km = k > 0 ? afterburner(c, s, g, s.cand, k, b, lam, prio, s.moves, so.info == nullptr) : 0;
-            if (km == 0 && G && gnn_restore(c, *G, n, s.dest)) {
+            Movers mv = find_movers(c, s, lp, g, lam, prio, so.info == nullptr);
+            if (mv.k == 0 && G && gnn_restore(c, *G, n, s.dest)) {
                 // nothing to move among the vertices let through: score the
                 // pruned ones too, so the call ends as the plain method does
                 score_all(c, s, lp, g, s.part, curr.vol, ccons, tables ? 0 : raw_mode, lam, fr, so);
-                k = gather_candidates(c, s, lp, g, s.dest, s.cand, b);
-                km = k > 0 ? afterburner(c, s, g, s.cand, k, b, lam, prio, s.moves, so.info == nullptr) : 0;
+                mv = find_movers(c, s, lp, g, lam, prio, so.info == nullptr);
             }
+            const i64 k = mv.cands, km = mv.k;
             if (stats) {
                 stats->sweeps++;
                 stats->cands += k;
@@ -1898,19 +1981,18 @@ static void local_move_t(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g,
                 tr.end(k, 0);
                 break;
             }
-            if (iter > 1 || !is_initial)
+            // (the first sweep of an initial call has no NEW_PART movers)
+            const bool fresh_ids = mv.knew > 0 && (iter > 1 || !is_initial);
+            if (fresh_ids)
                 set_new_cluster_ids(c, s, g, curr, s.moves, km, constrained ? cons : nullptr, ids, nfull);
             fresh = !tables;
-            perform_moves(c, s, lp, g, curr, s.moves, km, g.n - lp.ord.off_large, g.n - lp.ord.off_large2, tables);
+            perform_moves(c, s, lp, g, curr, s.moves, km, !fresh_ids, g.n - lp.ord.off_large, g.n - lp.ord.off_large2, tables);
             if (stats) stats->moves += km;
             if (c.verbose >= 3)
                 fprintf(stderr, "sweep n=%lld it=%d cands=%lld moves=%lld labels=%d uncut=%lld obj=%.17g\n",
                         (long long)n, iter, (long long)k, (long long)km, curr.label_count, (long long)curr.uncut,
                         curr.obj);
-            if (curr.obj > best.obj) {
-                copy_state(c, best, curr);
-                copy_dev(c, best_part, s.part, n * sizeof(i32));
-            }
+            if (curr.obj > best.obj) copy_best(c, best, curr, best_part, s.part, n);
             tr.end(k, km);
         }
     }
@@ -2001,7 +2083,7 @@ void local_move_strict(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, i
         score_all(c, s, lp, g, s.part, curr.vol, ccons, !tables && c.raw_sweeps, LamOne{lam}, 0.0f,
                   ScoreOut{s.dest, s.gain, nullptr});
         i64 b[2];
-        i64 k = gather_candidates(c, s, lp, g, s.dest, s.moves, b);
+        i64 k = gather_candidates(c, lp, g, s.dest, s.moves, b);
         if (stats) {
             stats->sweeps++;
             stats->cands += k;
@@ -2024,12 +2106,9 @@ void local_move_strict(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, i
             trc.end(k, 0);
             break;
         }
-        perform_moves(c, s, lp, g, curr, s.moves, tr, g.n - lp.ord.off_large, g.n - lp.ord.off_large2, tables);
+        perform_moves(c, s, lp, g, curr, s.moves, tr, false, g.n - lp.ord.off_large, g.n - lp.ord.off_large2, tables);
         if (stats) stats->moves += tr;
-        if (curr.obj > best.obj) {
-            copy_state(c, best, curr);
-            copy_dev(c, best_part, s.part, n * sizeof(i32));
-        }
+        if (curr.obj > best.obj) copy_best(c, best, curr, best_part, s.part, n);
         fill_i32(c, s.dest, n, NULL_PART);
         trc.end(k, tr);
     }
@@ -2047,15 +2126,16 @@ i64 sweep_once(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, const i32
     copy_dev(c, s.part, part, n * sizeof(i32));
     copy_dev(c, s.dest, dest, n * sizeof(i32));
     copy_dev(c, s.gain, gain, n * sizeof(float));
+    init_mvp(c, s, n);
     const float lam = (float)lambda;
     score_all(c, s, lp, g, s.part, vol, cons, raw, LamOne{lam}, ratio,
               ScoreOut{s.dest, s.gain, nullptr});
     i64 b[2];
-    i64 k = gather_candidates(c, s, lp, g, s.dest, s.cand, b);
+    i64 k = gather_candidates(c, lp, g, s.dest, s.cand, b);
     *ncand = k;
     i64 km = 0;
     if (k > 0) {
-        km = afterburner(c, s, g, s.cand, k, b, LamOne{lam}, PrioOne{}, moves_out, true);
+        km = afterburner(c, s, g, s.cand, k, b, LamOne{lam}, PrioOne{}, moves_out, true).k;
     }
     copy_dev(c, dest, s.dest, n * sizeof(i32));
     copy_dev(c, gain, s.gain, n * sizeof(float));
@@ -2252,7 +2332,7 @@ static void set_new_cluster_ids_batch(Ctx& c, MoveScratch& s, const DGraph& g, c
     const i64 K = bl.K, NL = st.loff[K];
     k_new_flags<<<grid_items(k, 256), 256, 0, c.stream>>>(moves, k, s.dest, s.flag);
     PGGC_LAUNCH_CHECK();
-    const i64 KN = compact_flags(c, s.flag, moves, k, s.tmp, s.scal);
+    const i64 KN = compact_flags(c, s.flag, moves, k, s.tmp);
     if (KN == 0) return;
     Buf<i64> Ld(c, K);
     upload(c, Ld.p, label_counts(cur));
@@ -2261,7 +2341,7 @@ static void set_new_cluster_ids_batch(Ctx& c, MoveScratch& s, const DGraph& g, c
     Buf<i32> uf(c, std::max<i64>(NL, 1));
     k_unused_inst<<<grid_items(NL, 256), 256, 0, c.stream>>>(NL, s.flag, st.linst, st.dloff, Ld, uf);
     PGGC_LAUNCH_CHECK();
-    const i64 A = compact_flags(c, uf, nullptr, NL, s.tmp2, s.scal);
+    const i64 A = compact_flags(c, uf, nullptr, NL, s.tmp2);
     Buf<i64> acnt(c, K), kcnt(c, K);
     fill_i64(c, acnt, K, 0);
     fill_i64(c, kcnt, K, 0);
@@ -2387,11 +2467,10 @@ void local_move_batch(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, co
         // the raw first sweep gives (every neighbour its own cluster)
         score_all(c, s, lp, g, s.part, cvol, nullptr, false, lam, 0.0f, ScoreOut{s.dest, nullptr, s.abi});
         i64 b[2];
-        const i64 kc = gather_candidates(c, s, lp, g, s.dest, s.cand, b);
-        i64 km = 0;
-        if (kc > 0) {
-            km = afterburner(c, s, g, s.cand, kc, b, lam, prio, s.moves, false);
-        }
+        const i64 kc = gather_candidates(c, lp, g, s.dest, s.cand, b);
+        Movers mv{0, 0, 0};
+        if (kc > 0) mv = afterburner(c, s, g, s.cand, kc, b, lam, prio, s.moves, false);
+        const i64 km = mv.k;
         fill_i64(c, cnt2, 2 * K, 0);
         if (kc > 0) k_inst_count<<<grid_items(kc, 256), 256, 0, c.stream>>>(s.cand, kc, bl.inst, cnt2);
         if (km > 0) k_inst_count<<<grid_items(km, 256), 256, 0, c.stream>>>(s.moves, km, bl.inst, cnt2.p + K);
@@ -2404,11 +2483,11 @@ void local_move_batch(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, co
             stats[q].cands += hc[q];
         }
         if (km > 0) {
-            set_new_cluster_ids_batch(c, s, g, bl, best, cur, cvol, s.moves, km);
+            if (mv.knew > 0) set_new_cluster_ids_batch(c, s, g, bl, best, cur, cvol, s.moves, km);
             fill_i64(c, acc, K, 0);
             // resets the movers and their neighbours; every vertex of an
             // instance whose first moves these are follows below
-            apply_moves_core(c, s, lp, g, cvol, s.moves, km, n_large, n_massive, true, AccInst{bl.inst, acc});
+            apply_moves_core(c, s, lp, g, cvol, s.moves, km, mv.knew == 0, n_large, n_massive, true, AccInst{bl.inst, acc});
             bool anyfull = false;
             for (i64 q = 0; q < K; q++) {
                 const bool moved = hc[K + q] > 0;

@@ -1,5 +1,5 @@
-// Context allocator and data-parallel primitives: fill, scan, ordered
-// compaction, stable LSD radix sort, exact integer reductions.
+// Context allocator and data-parallel primitives: fill, scan, stable LSD
+// radix sort, exact integer reductions.
 #include <algorithm>
 #include <cstdio>
 #include <cstring>
@@ -282,11 +282,6 @@ struct LoadI32 {
     const i32* p;
     __device__ __forceinline__ i64 operator()(i64 x) const { return p[x]; }
 };
-struct LoadFlag {
-    const i32* p;
-    __device__ __forceinline__ i64 operator()(i64 x) const { return p[x] != 0 ? 1 : 0; }
-};
-
 template <class Load>
 static void scan_generic(Ctx& c, Load ld, i64* out, i64 n) {
     if (n <= 0) {
@@ -315,43 +310,6 @@ void scan_i64(Ctx& c, const i64* in, i64* out, i64 n) {
     scan_generic(c, LoadI64{in}, out, n);
 }
 void scan_i32_to_i64(Ctx& c, const i32* in, i64* out, i64 n) { scan_generic(c, LoadI32{in}, out, n); }
-
-// ---------------------------------------------------------- ordered compaction
-__global__ void __launch_bounds__(ST) k_compact_write(const i32* flag, const i32* src, i64 n, const i64* boff,
-                                                       i32* out, i64* count) {
-    i64 base = (i64)blockIdx.x * STILE + (i64)threadIdx.x * SI;
-    int f[SI];
-    i64 s = 0;
-#pragma unroll
-    for (int k = 0; k < SI; k++) {
-        i64 x = base + k;
-        f[k] = (x < n && flag[x] != 0) ? 1 : 0;
-        s += f[k];
-    }
-    i64 tot;
-    i64 pre = block_excl_scan_i64(s, &tot) + boff[blockIdx.x];
-#pragma unroll
-    for (int k = 0; k < SI; k++) {
-        i64 x = base + k;
-        if (f[k]) out[pre++] = src ? src[x] : (i32)x;
-    }
-    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *count = boff[blockIdx.x] + tot;
-}
-
-i64 compact_flags(Ctx& c, const i32* flag, const i32* src, i64 n, i32* out, i64* count_dev) {
-    if (n <= 0) {
-        fill_i64(c, count_dev, 1, 0);
-        return 0;
-    }
-    i64 nb = ceil_div(n, STILE);
-    Buf<i64> bs(c, nb + 1);
-    k_tile_sums<LoadFlag><<<(int)nb, ST, 0, c.stream>>>(LoadFlag{flag}, n, bs);
-    PGGC_LAUNCH_CHECK();
-    scan_i64(c, bs, bs, nb);
-    k_compact_write<<<(int)nb, ST, 0, c.stream>>>(flag, src, n, bs, out, count_dev);
-    PGGC_LAUNCH_CHECK();
-    return c.read1(count_dev);
-}
 
 // ---------------------------------------------------------------- radix sort
 // Stable LSD sort of (key, value) pairs on key bits [begin, bits): rocPRIM's
