@@ -40,10 +40,6 @@ struct Orders {
 };
 void make_orders(Ctx& c, const DGraph& g, Orders& o);
 
-// Stable K-way partition of [0,n) by a per-vertex class (class array given);
-// out receives the vertex ids, starts[0..K] the class boundaries (host).
-void partition_classes(Ctx& c, const i32* cls, i64 n, int K, i32* out, i64* starts);
-
 // Evaluator (app/verify_objective.cpp:64-89): vol[l] += vw[i], uncut.
 // vol must hold L entries; result scalars are left in dev_out[0] (uncut).
 void evaluate(Ctx& c, const DGraph& g, const i32* labels, i64 L, i64* vol, i64* dev_uncut);

@@ -83,17 +83,6 @@ static void partition_k(Ctx& c, const i32* cls, i64 n, i32* out, i64* starts) {
     for (int k = 0; k <= K; k++) starts[k] = h[k];
 }
 
-void partition_classes(Ctx& c, const i32* cls, i64 n, int K, i32* out, i64* starts) {
-    switch (K) {
-        case 2: partition_k<2>(c, cls, n, out, starts); break;
-        case 3: partition_k<3>(c, cls, n, out, starts); break;
-        case 4: partition_k<4>(c, cls, n, out, starts); break;
-        case 8: partition_k<8>(c, cls, n, out, starts); break;
-        case 11: partition_k<11>(c, cls, n, out, starts); break;
-        default: throw Error(-1, "partition_classes: unsupported class count");
-    }
-}
-
 // ------------------------------------------------------------------ orderings
 __global__ void k_order_classes(const i64* rp, i64 n, i32* c1, i32* c2) {
     const i64 i = thread_item();

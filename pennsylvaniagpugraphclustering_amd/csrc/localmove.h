@@ -41,7 +41,7 @@ constexpr int CL_TABLE = 5, CL_BIG = 8, CL_HUB = 10;
 struct LevelPlan {
     const void* key = nullptr;  // graph identity (row offsets pointer)
     i64 n = -1;
-    Orders ord;
+    Orders ord;                 // order1 only
     Buf<i32> sc_list;           // vertices grouped by scoring class
     i64 sc_start[NCLS + 1] = {0};
     // hubs (the class above 2048, sorted by degree): the first nlds of them

@@ -39,9 +39,13 @@ void update_objective(Ctx& c, RefineData& rd) {
 }
 
 // ------------------------------------------------------------- scratch
-// Scalars of a sweep in MoveScratch::scal, zeroed at the start of a call:
-// the MV_SLOTS words of the uncut change are zero between sweeps, SC_TICKET counts k_finish's blocks (at most FIN_BLOCKS).
-constexpr int SC_EXTRA = 0, SC_TICKET = 4, SC_SLOTS = 16, MV_SLOTS = 64, SC_COUNT = SC_SLOTS + MV_SLOTS;
+// Scalars of a sweep in MoveScratch::scal, zero at the start of a call and
+// between sweeps: SC_EXTRA the two words of select_items, SC_NEW the movers that
+// need a new cluster (direct sweeps), SC_TICKET k_finish's blocks (at most
+// FIN_BLOCKS), then MV_SLOTS words each over which the uncut change, and in
+// direct sweeps the movers and the candidates, are summed.
+constexpr int SC_EXTRA = 0, SC_NEW = 2, SC_TICKET = 4, MV_SLOTS = 64, SC_SLOTS = 16, SC_KM = SC_SLOTS + MV_SLOTS,
+              SC_CAND = SC_KM + MV_SLOTS, SC_COUNT = SC_CAND + MV_SLOTS;
 constexpr int FIN_BLOCKS = 256;
 void MoveScratch::ensure(Ctx& c, i64 n) {
     if (cap >= n) return;
@@ -68,8 +72,8 @@ __host__ __device__ __forceinline__ int score_class(i64 d) {
     return d <= 4 ? 0 : d <= 8 ? 1 : d <= 16 ? 2 : d <= 32 ? 3 : d <= 64 ? 4 : d <= 128 ? 5 : d <= 256 ? 6
          : d <= 512 ? 7 : d <= 1024 ? 8 : d <= 2048 ? 9 : 10;
 }
-// small levels, bound by launches (find_movers)
-constexpr i64 DIRECT_MAX = (i64)1 << 18;
+// small levels, bound by launches (direct_sweep)
+constexpr i64 DIRECT_MAX = (i64)1 << 18, DIRECT_NNZ = (i64)1 << 22;
 // Level of at most this many rows in the LDS-table classes: one launch for all
 // (the chip holds 5 of its 256-thread blocks per CU, 1,280 at once, so two
 // rounds of blocks cost less than the four launches saved).
@@ -93,11 +97,91 @@ constexpr int HUB_LDS_SLOTS = 10112;
 constexpr int HUB_SLOTS32 = 12288, HUB_SLOTS64 = 8192;
 __host__ __device__ __forceinline__ i64 hub_slices(i64 d, int slots) { return (3 * d + 2 * slots - 1) / (2 * slots); }
 
-__global__ void k_score_classes(const i64* rp, i64 n, i32* cls) {
-    const i64 i = thread_item();
-    if (i >= n) return;
-    cls[i] = score_class(rp[i + 1] - rp[i]);
+// Both partitions of a plan in one pass each of counting and writing: the
+// order1 classes (src/header/ordering.h:17-19; ORD_CLS) and the scoring classes,
+// each stable by id.  Classes 0 .. ORD_CLS - 1 are the former, the others the
+// latter; counts[class * nb + tile].  Consecutive lanes take consecutive
+// vertices, and a vertex's place within its tile is the count of its class in
+// the (step, wave) runs before its own plus its rank among the lanes of its
+// class, found with a ballot per class bit.  As two partitions of three and
+// four kernels each over class arrays, 8 consecutive vertices per thread and a
+// block scan per class, a plan took 16 launches and 3 waits, now 3 and 1.
+constexpr int ORD_CLS = 3, PL_CLS = ORD_CLS + NCLS, PL_T = 256, PL_I = 8, PL_TILE = PL_T * PL_I, PL_W = PL_T / 64;
+__device__ __forceinline__ int order_class(i64 d) { return d < LARGE_CUTOFF ? 0 : (d < MASSIVE_CUTOFF ? 1 : 2); }
+__global__ void __launch_bounds__(PL_T) k_plan_count(const i64* __restrict__ rp, i64 n, i64 nb, i64* counts) {
+    __shared__ int cnt[PL_CLS];
+    const i64 b = block_id();
+    if (b >= nb) return;
+    if (threadIdx.x < PL_CLS) cnt[threadIdx.x] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < PL_I; k++) {
+        const i64 i = b * PL_TILE + k * PL_T + threadIdx.x;
+        if (i < n) {
+            const i64 d = rp[i + 1] - rp[i];
+            atomicAdd(&cnt[order_class(d)], 1);
+            atomicAdd(&cnt[ORD_CLS + score_class(d)], 1);
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < PL_CLS) counts[(i64)threadIdx.x * nb + b] = cnt[threadIdx.x];
 }
+// lanes of the wave whose 4-bit class equals this lane's
+__device__ __forceinline__ u64 same_class(int cls) {
+    u64 m = ~(u64)0;
+#pragma unroll
+    for (int bit = 0; bit < 4; bit++) {
+        const u64 s = __ballot((cls >> bit) & 1);
+        m &= ((cls >> bit) & 1) ? s : ~s;
+    }
+    return m;
+}
+// offs: exclusive scan of counts; host[0..PL_CLS] = class starts (the scoring
+// classes' from n on)
+__global__ void __launch_bounds__(PL_T) k_plan_write(const i64* __restrict__ rp, i64 n, i64 nb,
+                                                     const i64* __restrict__ offs, i32* __restrict__ o1,
+                                                     i32* __restrict__ list, i64* host) {
+    __shared__ int cnt[PL_I * PL_W][PL_CLS];  // class counts of the runs, then their prefix
+    const i64 b = block_id();
+    if (b >= nb) return;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    for (int q = threadIdx.x; q < PL_I * PL_W * PL_CLS; q += PL_T) cnt[q / PL_CLS][q % PL_CLS] = 0;
+    __syncthreads();
+    int c1[PL_I], c2[PL_I], r1[PL_I], r2[PL_I];
+    const u64 below = ((u64)1 << lane) - 1;
+#pragma unroll
+    for (int k = 0; k < PL_I; k++) {
+        const i64 i = b * PL_TILE + k * PL_T + threadIdx.x;
+        const bool in = i < n;
+        const i64 d = in ? rp[i + 1] - rp[i] : 0;
+        c1[k] = in ? order_class(d) : 15;
+        c2[k] = in ? score_class(d) : 15;
+        const u64 m1 = same_class(c1[k]), m2 = same_class(c2[k]);
+        r1[k] = __popcll(m1 & below);
+        r2[k] = __popcll(m2 & below);
+        if (in && r1[k] == 0) cnt[k * PL_W + wv][c1[k]] = __popcll(m1);
+        if (in && r2[k] == 0) cnt[k * PL_W + wv][ORD_CLS + c2[k]] = __popcll(m2);
+    }
+    __syncthreads();
+    if (threadIdx.x < PL_CLS) {
+        int run = 0;
+        for (int q = 0; q < PL_I * PL_W; q++) {
+            const int v = cnt[q][threadIdx.x];
+            cnt[q][threadIdx.x] = run;
+            run += v;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < PL_I; k++) {
+        const i64 i = b * PL_TILE + k * PL_T + threadIdx.x;
+        if (i >= n) continue;
+        o1[offs[(i64)c1[k] * nb + b] + cnt[k * PL_W + wv][c1[k]] + r1[k]] = (i32)i;
+        list[offs[(i64)(ORD_CLS + c2[k]) * nb + b] - n + cnt[k * PL_W + wv][ORD_CLS + c2[k]] + r2[k]] = (i32)i;
+    }
+    if (b == 0 && threadIdx.x <= PL_CLS) host[threadIdx.x] = offs[(i64)threadIdx.x * nb];
+}
+
 // Work of the large hubs: groups of NXCD consecutive hubs (sorted by degree, so
 // of similar size), each hub with as many blocks as the group's largest hub
 // has slices.  Block ids go round-robin over the XCDs, so with the blocks of a
@@ -155,12 +239,25 @@ void plan_level(Ctx& c, const DGraph& g, LevelPlan& p) {
     p.key = g.rp;
     p.n = g.n;
     p.epoch = c.knob_epoch;
-    make_orders(c, g, p.ord);
-    Buf<i32> cls(c, std::max<i64>(g.n, 1));
-    p.sc_list = Buf<i32>(c, std::max<i64>(g.n, 1));
-    k_score_classes<<<grid_items(g.n, 256), 256, 0, c.stream>>>(g.rp, g.n, cls);
-    PGGC_LAUNCH_CHECK();
-    partition_classes(c, cls, g.n, NCLS, p.sc_list, p.sc_start);
+    {
+        const int tk = c.kt_begin(KS_ORDER);
+        const i64 n = g.n, nb = ceil_div(std::max<i64>(n, 1), PL_TILE);
+        if (p.ord.o1.n < (size_t)n) p.ord.o1 = Buf<i32>(c, std::max<i64>(n, 1));
+        p.sc_list = Buf<i32>(c, std::max<i64>(n, 1));
+        Buf<i64> counts(c, PL_CLS * nb + 1);
+        k_plan_count<<<grid_blocks(nb), PL_T, 0, c.stream>>>(g.rp, n, nb, counts);
+        PGGC_LAUNCH_CHECK();
+        scan_i64(c, counts, counts, PL_CLS * nb);
+        k_plan_write<<<grid_blocks(nb), PL_T, 0, c.stream>>>(g.rp, n, nb, counts, p.ord.o1, p.sc_list,
+                                                             c.pinned_dev);
+        PGGC_LAUNCH_CHECK();
+        // row bounds read twice, ids written twice
+        c.kt_end(tk, 16.0 * (n + 1) + 8.0 * n);
+        c.sync();
+        p.ord.off_large = c.pinned[1];
+        p.ord.off_large2 = c.pinned[2];
+        for (int k = 0; k <= NCLS; k++) p.sc_start[k] = c.pinned[ORD_CLS + k] - n;
+    }
     // hub class by degree (stable: ties by id), so that the hubs scored in
     // LDS form a prefix; every hub is scored on its own, so the order within
     // the class does not change results
@@ -327,11 +424,8 @@ __device__ __forceinline__ NbRec load_rec(const RecView& rv, i32 v) {
     }
     return r;
 }
-__global__ void __launch_bounds__(256) k_rec_pack(i64 n, const i32* __restrict__ part, const i64* __restrict__ vol,
-                                                  const i32* __restrict__ cons, u64* __restrict__ r8,
-                                                  uint4* __restrict__ r16) {
-    const i64 i = thread_item();
-    if (i >= n) return;
+__device__ __forceinline__ void rec_pack(i64 i, const i32* part, const i64* vol, const i32* cons, u64* r8,
+                                         uint4* r16) {
     const i32 p = part[i];
     const u32 vf = __float_as_uint((float)vol[p]);
     if (r16) {
@@ -339,6 +433,12 @@ __global__ void __launch_bounds__(256) k_rec_pack(i64 n, const i32* __restrict__
     } else {
         r8[i] = (u64)(u32)p | ((u64)vf << 32);
     }
+}
+__global__ void __launch_bounds__(256) k_rec_pack(i64 n, const i32* __restrict__ part, const i64* __restrict__ vol,
+                                                  const i32* __restrict__ cons, u64* __restrict__ r8,
+                                                  uint4* __restrict__ r16) {
+    const i64 i = thread_item();
+    if (i < n) rec_pack(i, part, vol, cons, r8, r16);
 }
 
 // Lane exchange inside groups of G consecutive lanes.  DPP moves cover 16
@@ -941,16 +1041,16 @@ __global__ void __launch_bounds__(256) k_score_bytes(const i64* __restrict__ rp,
 }
 
 // alpha + beta * degree bytes per listed vertex (per candidate of the
-// afterburner, per mover of perform_moves) that is not NO_MOVE in dest (when
-// given), plus `extra` once
+// afterburner, per mover of perform_moves) that is not NO_MOVE in dest and is
+// marked in mvp (when given), plus `extra` once
 __global__ void __launch_bounds__(256) k_list_bytes(const i64* __restrict__ rp, const i32* __restrict__ list,
-                                                    const i32* __restrict__ dest, i64 k, i64 alpha, i64 beta,
-                                                    i64 extra, i64* acc) {
+                                                    const i32* __restrict__ dest, const u64* __restrict__ mvp, i64 k,
+                                                    i64 alpha, i64 beta, i64 extra, i64* acc) {
     const i64 x = thread_item();
     i64 b = 0;
     if (x < k) {
         const i32 i = list[x];
-        if (!dest || dest[i] != NO_MOVE) b = alpha + beta * (rp[i + 1] - rp[i]);
+        if ((!dest || dest[i] != NO_MOVE) && (!mvp || ((u32)mvp[i] >> 31))) b = alpha + beta * (rp[i + 1] - rp[i]);
     }
     if (x == 0) b += extra;
     b = block_sum_i64<256>(b);
@@ -1030,7 +1130,7 @@ static void launch_tables(Ctx& c, const LevelPlan& lp, const DGraph& g, WT W, co
 
 template <class LT>
 static void score_all(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, const i32* part, const i64* vol,
-                      const i32* cons, int raw, LT lam, float ratio, const ScoreOut& out) {
+                      const i32* cons, int raw, LT lam, float ratio, const ScoreOut& out, bool packed = false) {
     i32* dest = out.dest;
     // raw: every vertex a cluster of its own; 0: any clustering
     const i64* st = lp.sc_start;
@@ -1046,7 +1146,7 @@ static void score_all(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, co
                               g.rp, L, sb, dest, acct)));
         PGGC_LAUNCH_CHECK();
     }
-    if (g.n > 0) {
+    if (g.n > 0 && !packed) {
         if (cons && s.rec16.n < (size_t)g.n) s.rec16 = Buf<uint4>(c, s.cap);
         k_rec_pack<<<grid_items(g.n, 256), 256, 0, c.stream>>>(g.n, part, vol, cons, s.rec, cons ? s.rec16.p : nullptr);
         PGGC_LAUNCH_CHECK();
@@ -1159,6 +1259,17 @@ __device__ __forceinline__ float2 ab_terms(const AbInfo& q4, i32 v, i64 w, const
     return t;
 }
 
+// Direct sweeps (find_movers): a kept vertex is marked as a mover right away.
+struct AbMark {
+    u64* mvp;   // null: not marked here
+    i64* knew;  // counts the movers that need a new cluster
+    __device__ __forceinline__ void operator()(i32 i, const AbSelf& m) const {
+        if (!mvp) return;
+        mvp[i] = mvp_moved(m.p, m.best);
+        if (m.best == NEW_PART) atomicAdd((unsigned long long*)knew, 1ull);
+    }
+};
+
 // Degree below LARGE_CUTOFF: the terms are added in adjacency order.  The
 // gathers of the neighbours' records bound it, so AB_G lanes gather a
 // candidate's edges (AB_U in flight per lane) and leave the terms in LDS, and
@@ -1170,16 +1281,16 @@ constexpr int AB_G = 16, AB_U = 4, AB_PB = 256 / AB_G;
 template <class WT, class LT, class PT>
 __device__ __forceinline__ void ab_small(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
                                          const AbInfo* __restrict__ info, const i32* __restrict__ cand, i64 blk, i64 k,
-                                         LT lam, PT prio, i32* __restrict__ keep) {
+                                         LT lam, PT prio, i32* __restrict__ keep, const AbMark& mark) {
     __shared__ float2 term[AB_PB][LARGE_CUTOFF + 1];
     const int lane = threadIdx.x & (AB_G - 1), grp = threadIdx.x / AB_G;
     const i64 x = blk * AB_PB + grp;
     int d = 0;
-    float igain = 0.0f;
+    i32 i = 0;
+    AbSelf m = {0, 0, 0, 0.0f, 0.0f};
     if (x < k) {
-        const i32 i = cand[x];
-        const AbSelf m = ab_self(info, i, lam, prio);
-        igain = m.igain;
+        i = cand[x];
+        m = ab_self(info, i, lam, prio);
         const i64 s = rp[i];
         d = m.best == NO_MOVE ? -1 : (int)(rp[i + 1] - s);
         for (int jb = lane; jb < d; jb += AB_G * AB_U) {
@@ -1204,7 +1315,9 @@ __device__ __forceinline__ void ab_small(const i64* __restrict__ rp, const i32* 
             acc = acc + t.x;
             acc = acc + t.y;
         }
-        keep[x] = (d >= 0 && igain + acc >= 0.0f) ? 1 : 0;
+        const bool kept = d >= 0 && m.igain + acc >= 0.0f;
+        keep[x] = kept ? 1 : 0;
+        if (kept) mark(i, m);
     }
 }
 
@@ -1212,7 +1325,7 @@ __device__ __forceinline__ void ab_small(const i64* __restrict__ rp, const i32* 
 template <class WT, class LT, class PT>
 __device__ __forceinline__ void ab_wave(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
                                         const AbInfo* __restrict__ info, const i32* __restrict__ cand, i64 x, i64 k1,
-                                        LT lam, PT prio, i32* __restrict__ keep) {
+                                        LT lam, PT prio, i32* __restrict__ keep, const AbMark& mark) {
     const int lane = threadIdx.x & 63;
     if (x >= k1) return;
     const i32 i = cand[x];
@@ -1243,7 +1356,11 @@ __device__ __forceinline__ void ab_wave(const i64* __restrict__ rp, const i32* _
     xlane_fence(acc);
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) acc = acc + __shfl_down(acc, off);
-    if (lane == 0) keep[x] = (m.igain + acc >= 0.0f) ? 1 : 0;
+    if (lane == 0) {
+        const bool kept = m.igain + acc >= 0.0f;
+        keep[x] = kept ? 1 : 0;
+        if (kept) mark(i, m);
+    }
 }
 
 // both classes in one launch: list entries [0, k0) in the first b0 blocks
@@ -1251,17 +1368,19 @@ __device__ __forceinline__ void ab_wave(const i64* __restrict__ rp, const i32* _
 template <class WT, class LT, class PT>
 __global__ void __launch_bounds__(256) k_ab_lanes(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
                                                   const AbInfo* __restrict__ info, const i32* __restrict__ cand,
-                                                  i64 k0, i64 k1, i64 b0, LT lam, PT prio, i32* __restrict__ keep) {
+                                                  i64 k0, i64 k1, i64 b0, LT lam, PT prio, i32* __restrict__ keep,
+                                                  AbMark mark) {
     const i64 b = block_id();
-    if (b < b0) ab_small(rp, col, W, info, cand, b, k0, lam, prio, keep);
-    else ab_wave(rp, col, W, info, cand, k0 + (b - b0) * 4 + (threadIdx.x >> 6), k1, lam, prio, keep);
+    if (b < b0) ab_small(rp, col, W, info, cand, b, k0, lam, prio, keep, mark);
+    else ab_wave(rp, col, W, info, cand, k0 + (b - b0) * 4 + (threadIdx.x >> 6), k1, lam, prio, keep, mark);
 }
 
 // A 1024-thread block per candidate: 1024 strided partials and a halving tree.
 template <class WT, class LT, class PT>
 __global__ void __launch_bounds__(1024) k_ab_block(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
                                                    const AbInfo* __restrict__ info, const i32* __restrict__ cand,
-                                                   i64 k0, i64 k1, LT lam, PT prio, i32* __restrict__ keep) {
+                                                   i64 k0, i64 k1, LT lam, PT prio, i32* __restrict__ keep,
+                                                   AbMark mark) {
     __shared__ float sh[1024];
     const int t = threadIdx.x;
     const i64 x = k0 + block_id();
@@ -1302,7 +1421,11 @@ __global__ void __launch_bounds__(1024) k_ab_block(const i64* __restrict__ rp, c
         xlane_fence(acc);
 #pragma unroll
         for (int off = 32; off >= 1; off >>= 1) acc = acc + __shfl_down(acc, off);
-        if (t == 0) keep[x] = (m.igain + acc >= 0.0f) ? 1 : 0;
+        if (t == 0) {
+            const bool kept = m.igain + acc >= 0.0f;
+            keep[x] = kept ? 1 : 0;
+            if (kept) mark(i, m);
+        }
     }
 }
 
@@ -1345,10 +1468,11 @@ struct Movers {
     i64 cands;  // candidates
 };
 
-// cand: k candidates, or every vertex, in order1 order; b: class boundaries
+// The filter over cand (k candidates, or every vertex, in order1 order; b: class
+// boundaries): s.flag[x] = keep.
 template <class LT, class PT>
-static Movers afterburner(Ctx& c, MoveScratch& s, const DGraph& g, const i32* cand, i64 k, const i64* b, LT lam,
-                          PT prio, i32* moves, bool pack) {
+static void afterburner(Ctx& c, MoveScratch& s, const DGraph& g, const i32* cand, i64 k, const i64* b, LT lam,
+                        PT prio, bool pack, AbMark mark = {nullptr, nullptr}) {
     const int tk = c.kt_begin(KS_AFTERBURNER);
     if (pack) {
         k_ab_pack<<<grid_items(g.n, 256), 256, 0, c.stream>>>(g.n, s.gain, s.dest, s.part, g.vw, s.abi);
@@ -1358,10 +1482,10 @@ static Movers afterburner(Ctx& c, MoveScratch& s, const DGraph& g, const i32* ca
     PGGC_WDISPATCH(g, {
         if (nb0 + nb1 > 0)
             k_ab_lanes<<<grid_blocks(nb0 + nb1), 256, 0, c.stream>>>(g.rp, g.col, W, s.abi, cand, b[0], b[1], nb0, lam,
-                                                                     prio, s.flag);
+                                                                     prio, s.flag, mark);
         if (k > b[1])
             k_ab_block<<<grid_blocks(k - b[1]), 1024, 0, c.stream>>>(g.rp, g.col, W, s.abi, cand, b[1], k, lam,
-                                                                     prio, s.flag);
+                                                                     prio, s.flag, mark);
     });
     c.kt_end(tk, 0.0);
     PGGC_LAUNCH_CHECK();
@@ -1372,10 +1496,14 @@ static Movers afterburner(Ctx& c, MoveScratch& s, const DGraph& g, const i32* ca
         Buf<i64> acc(c, 1);
         fill_i64(c, acc, 1, 0);
         k_list_bytes<<<grid_items(std::max<i64>(k, 1), 256), 256, 0, c.stream>>>(
-            g.rp, cand, s.dest, k, 40, 20 + (g.wk == W_UNIT ? 0 : g.wk == W_I32 ? 4 : 8), pack ? 36 * g.n : 0, acc);
+            g.rp, cand, s.dest, nullptr, k, 40, 20 + (g.wk == W_UNIT ? 0 : g.wk == W_I32 ? 4 : 8), pack ? 36 * g.n : 0, acc);
         PGGC_LAUNCH_CHECK();
         acct_add(c, c.kt_counter(tk), acc);
     }
+}
+
+// the kept ones of cand, marked in mvp
+static Movers select_movers(Ctx& c, MoveScratch& s, const i32* cand, i64 k, i32* moves) {
     const i64* h = select_items(c, SelMoves{cand, s.flag, s.dest, s.part, moves, s.mvp}, k, SelBounds{0, 0},
                                 s.scal.p + SC_EXTRA);
     return Movers{h[0], h[3], h[4]};
@@ -1457,13 +1585,29 @@ static void set_new_cluster_ids(Ctx& c, MoveScratch& s, const DGraph& g, RefineD
 // v's cluster (k_mvp_init at the start of a call); a sweep marks its movers
 // (SelMoves, or k_mvp_moves once new cluster ids are known) and k_apply_moves settles them, so a sweep touches the movers'
 // words only, and an edge's uncut change reads one 8-byte word.
+__device__ __forceinline__ u64 mvp_settled(i32 p) { return (u64)(u32)p | ((u64)(u32)p << 32); }
 __global__ void __launch_bounds__(256) k_mvp_init(i64 n, const i32* __restrict__ part, u64* __restrict__ mvp,
                                                   i64* scal) {
     const i64 i = thread_item();
     if (i < SC_COUNT) scal[i] = 0;
-    if (i >= n) return;
-    const u64 p = (u64)(u32)part[i];
-    mvp[i] = p | (p << 32);
+    if (i < n) mvp[i] = mvp_settled(part[i]);
+}
+// The start of a local move: volumes and clusters copied, the vertices' words
+// settled, every vertex active, the scalars zero.
+__global__ void __launch_bounds__(256) k_move_begin(const i64* __restrict__ bvol, i64 L, i64* __restrict__ vol,
+                                                    const i32* __restrict__ bpart, i64 nfull, i32* __restrict__ part,
+                                                    i64 n, u64* __restrict__ mvp, i32* __restrict__ dest, i64* scal) {
+    const i64 x = thread_item();
+    if (x < SC_COUNT) scal[x] = 0;
+    if (x < L) vol[x] = bvol[x];
+    if (x < nfull) {
+        const i32 p = bpart[x];
+        part[x] = p;
+        if (x < n) {
+            mvp[x] = mvp_settled(p);
+            dest[x] = NULL_PART;
+        }
+    }
 }
 __global__ void __launch_bounds__(256) k_mvp_moves(const i32* __restrict__ moves, i64 k, const i32* __restrict__ part,
                                                    const i32* __restrict__ dest, u64* __restrict__ mvp) {
@@ -1513,15 +1657,17 @@ struct AccInst {
 // per block, and each thread has MV_U edges in flight.  As one thread per small
 // mover and one wave per mid-size one, in a kernel each for the two jobs, they
 // took 86 ms on R-MAT scale 20 (to stable), now 39 ms.
-// The list is in order1 order: the movers of degree >= LARGE_CUTOFF are a
-// suffix of at most nw entries, those >= MASSIVE_CUTOFF one of at most nb.
+// The list holds the movers, or in direct sweeps every vertex, in order1 order
+// (knew set: nothing is done when it counts any): those of degree >=
+// LARGE_CUTOFF are a suffix of at most nw entries, those >= MASSIVE_CUTOFF one of at most nb.
 constexpr int MV_G = 16, MV_U = 4;
 constexpr i64 MV_CHUNK = 8192;
 template <bool RESET, class WT, class AT>
 __global__ void __launch_bounds__(256) k_move_edges(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
                                                     const i32* __restrict__ moves, i64 k, i64 b1, i64 b2, i64 nw,
                                                     i64 nb, i64 cpm, const u64* __restrict__ mvp,
-                                                    i32* __restrict__ dest, AT at) {
+                                                    i32* __restrict__ dest, AT at, const i64* __restrict__ knew) {
+    if (knew && *knew != 0) return;  // kernel-uniform: the host takes the movers from here
     const i64 b = block_id();
     i64 x;         // list entry
     int lane, gs;  // this thread among the gs threads of the entry
@@ -1556,7 +1702,8 @@ __global__ void __launch_bounds__(256) k_move_edges(const i64* __restrict__ rp, 
         const i64 s0 = rp[i], d = rp[i + 1] - s0;
         const u64 me = mvp[i];
         const i32 oi = (i32)((u32)me & 0x7fffffffu), ni = (i32)(u32)(me >> 32);
-        if (d >= lo && d < hi && c0 < d) {
+        const bool moved = ((u32)me >> 31) != 0;
+        if (moved && d >= lo && d < hi && c0 < d) {
             const i64 e = s0 + (d < c0 + cl ? d : c0 + cl);
             for (i64 jb = s0 + c0 + lane; jb < e; jb += (i64)gs * MV_U) {
                 i32 v[MV_U];
@@ -1589,17 +1736,36 @@ __global__ void __launch_bounds__(256) k_move_edges(const i64* __restrict__ rp, 
 // then each distinct cluster gets one HBM atomic; the sums are exact
 // integers, so the order does not matter.  The movers' words and cached
 // destinations are settled for the next sweep.
+// In direct sweeps (info set) every vertex is looked at, k of them, and the
+// movers and candidates are counted.
 constexpr int AM_SLOTS = 1024;  // >= 2 keys per mover of a 256-thread block, at most half full
 __global__ void __launch_bounds__(256) k_apply_moves(const i32* __restrict__ moves, i64 k,
                                                      const i64* __restrict__ vw, u64* __restrict__ mvp,
-                                                     i32* __restrict__ part, i32* __restrict__ dest, i64* vol) {
+                                                     i32* __restrict__ part, i32* __restrict__ dest, i64* vol,
+                                                     const AbInfo* __restrict__ info, i64* scal) {
     __shared__ i32 lk[AM_SLOTS];
     __shared__ i64 lv[AM_SLOTS];
-    lds_agg_clear<256, AM_SLOTS>(lk, lv);
+    if (info && scal[SC_NEW] != 0) return;  // kernel-uniform
     const i64 x = thread_item();
+    i32 i = -1;
+    u64 q = 0;
     if (x < k) {
-        const i32 i = moves[x];
-        const u64 q = mvp[i];
+        i = moves ? moves[x] : (i32)x;
+        q = mvp[i];
+        if (((u32)q >> 31) == 0) i = -1;
+    }
+    if (info) {
+        const int km = __syncthreads_count(i >= 0);
+        const int kc = __syncthreads_count(x < k && info[x < k ? x : 0].dest != NO_MOVE);
+        if (threadIdx.x == 0) {
+            const i64 w = block_id() & (MV_SLOTS - 1);
+            if (km) atomicAdd((unsigned long long*)&scal[SC_KM + w], (unsigned long long)km);
+            if (kc) atomicAdd((unsigned long long*)&scal[SC_CAND + w], (unsigned long long)kc);
+        }
+        if (km == 0) return;  // block-uniform
+    }
+    lds_agg_clear<256, AM_SLOTS>(lk, lv);
+    if (i >= 0) {
         const i32 p = (i32)((u32)q & 0x7fffffffu);
         i32 b = (i32)(u32)(q >> 32);
         if (b >= 0) {  // unresolved NEW_PART cannot reach here (p_conn is 0 for singletons)
@@ -1610,7 +1776,7 @@ __global__ void __launch_bounds__(256) k_apply_moves(const i32* __restrict__ mov
         } else {
             b = p;
         }
-        mvp[i] = (u64)(u32)b | ((u64)(u32)b << 32);
+        mvp[i] = mvp_settled(b);
         dest[i] = NULL_PART;
     }
     __syncthreads();
@@ -1621,60 +1787,84 @@ __global__ void __launch_bounds__(256) k_apply_moves(const i32* __restrict__ mov
     }
 }
 
-// End of a sweep: the exact 128-bit sum of squared volumes and the uncut
-// change, stored to the host slots by the last block to finish (host[0] =
-// uncut change, host[1..2] = sum of squares high and low).  One launch instead of seven (fills, two reductions of two
-// kernels each, read-back): on small levels the sweep is bound by launches.
-__global__ void __launch_bounds__(256) k_finish(const i64* __restrict__ vol, i64 L, u64* part, i64* scal, i64* host) {
-    u64 lo = 0, hi = 0;
-    for (i64 x = (i64)blockIdx.x * 256 + threadIdx.x; x < L; x += (i64)gridDim.x * 256) {
-        const i64 v = vol[x];
-        const u64 a = (u64)(v < 0 ? -v : v);
-        const u64 plo = a * a;
-        lo += plo;
-        hi += __umul64hi(a, a) + (lo < plo ? 1 : 0);
-    }
-    __shared__ u64 slo[256], shi[256];
-    __shared__ int last;
-    auto tree = [&]() {
-        __syncthreads();
-        for (int o = 128; o > 0; o >>= 1) {
-            if ((int)threadIdx.x < o) {
-                const u64 a = slo[threadIdx.x], b = slo[threadIdx.x + o];
-                slo[threadIdx.x] = a + b;
-                shi[threadIdx.x] = shi[threadIdx.x] + shi[threadIdx.x + o] + (a + b < a ? 1 : 0);
-            }
-            __syncthreads();
-        }
-    };
-    slo[threadIdx.x] = lo;
-    shi[threadIdx.x] = hi;
-    tree();
-    if (threadIdx.x == 0) {
-        // agent-scope stores and loads: the blocks run on different XCDs
-        __hip_atomic_store(&part[2 * blockIdx.x], shi[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(&part[2 * blockIdx.x + 1], slo[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __threadfence();
-        last = atomicAdd((unsigned long long*)&scal[SC_TICKET], 1ull) == gridDim.x - 1;
-    }
+// End of a sweep: the exact 128-bit sum of squared volumes and the sums over
+// the slots, stored to the host slots by the last block to finish: host[0] =
+// uncut change, host[1..2] = sum of squares high and low, and in direct sweeps
+// host[3] = movers, host[4] = candidates, host[5] = movers that need a new
+// cluster.  rec / rec16 set: the vertices' records for the next sweep too.  One
+// launch instead of seven (fills, two reductions of two kernels each,
+// read-back): on small levels the sweep is bound by launches.
+struct Sq128 {
+    u64 hi, lo;
+};
+__device__ __forceinline__ Sq128 add_sq(Sq128 a, Sq128 b) {
+    const u64 lo = a.lo + b.lo;
+    return Sq128{a.hi + b.hi + (lo < a.lo ? 1 : 0), lo};
+}
+// over the block's 256 threads; thread 0 gets the result
+__device__ __forceinline__ Sq128 block_sq(Sq128 v) {
+    __shared__ Sq128 sh[4];
+    xlane_fence(v.hi);
+    xlane_fence(v.lo);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v = add_sq(v, Sq128{(u64)__shfl_xor(v.hi, o), (u64)__shfl_xor(v.lo, o)});
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
     __syncthreads();
-    if (!last) return;  // block-uniform
-    __threadfence();
+    if (threadIdx.x == 0)
+        for (int w = 1; w < 4; w++) v = add_sq(v, sh[w]);
+    __syncthreads();
+    return v;
+}
+__global__ void __launch_bounds__(256) k_finish(const i64* __restrict__ vol, i64 L, u64* part, i64* scal, i64* host,
+                                                i64 n, const i32* __restrict__ label, const i32* __restrict__ cons,
+                                                u64* __restrict__ rec, uint4* __restrict__ rec16) {
     const int t = threadIdx.x;
-    const bool in = t < (int)gridDim.x;  // gridDim.x <= FIN_BLOCKS
-    slo[t] = in ? __hip_atomic_load(&part[2 * t + 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
-    shi[t] = in ? __hip_atomic_load(&part[2 * t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
-    tree();
-    const u64 rlo = slo[0], rhi = shi[0];
-    __syncthreads();
-    const i64 du = block_sum_i64<256>(t < MV_SLOTS ? scal[SC_SLOTS + t] : 0);
-    if (t < MV_SLOTS) scal[SC_SLOTS + t] = 0;
-    if (t == 0) {
-        host[0] = du;
-        host[1] = (i64)rhi;
-        host[2] = (i64)rlo;
-        scal[SC_TICKET] = 0;
-        __threadfence_system();
+    for (i64 x = (i64)blockIdx.x * 256 + t; x < n; x += (i64)gridDim.x * 256)
+        rec_pack(x, label, vol, cons, rec, rec16);
+    Sq128 sq{0, 0};
+    for (i64 xb = (i64)blockIdx.x * 256; xb < L; xb += (i64)gridDim.x * 256) {  // block-uniform loop control
+        const i64 x = xb + t;
+        const i64 v = x < L ? vol[x] : 0;
+        const u64 a = (u64)(v < 0 ? -v : v);
+        sq = add_sq(sq, Sq128{__umul64hi(a, a), a * a});
+    }
+    sq = block_sq(sq);
+    if (gridDim.x > 1) {
+        __shared__ int last;
+        if (t == 0) {
+            // agent-scope stores and loads: the blocks run on different XCDs
+            __hip_atomic_store(&part[2 * blockIdx.x], sq.hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(&part[2 * blockIdx.x + 1], sq.lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __threadfence();
+            last = atomicAdd((unsigned long long*)&scal[SC_TICKET], 1ull) == gridDim.x - 1;
+        }
+        __syncthreads();
+        if (!last) return;  // block-uniform
+        __threadfence();
+        sq = Sq128{0, 0};
+        if (t < (int)gridDim.x)  // gridDim.x <= FIN_BLOCKS
+            sq = Sq128{__hip_atomic_load(&part[2 * t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
+                       __hip_atomic_load(&part[2 * t + 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)};
+        sq = block_sq(sq);
+    }
+    static_assert(MV_SLOTS == 64, "a wave sums each group of slots");
+    if (t < 64) {  // the first wave sums the slots and reports
+        i64 du = scal[SC_SLOTS + t], km = scal[SC_KM + t], kc = scal[SC_CAND + t];
+        scal[SC_SLOTS + t] = scal[SC_KM + t] = scal[SC_CAND + t] = 0;
+        const auto sum = [](i64 a, i64 b) { return a + b; };
+        du = group_reduce<64>(du, sum);
+        km = group_reduce<64>(km, sum);
+        kc = group_reduce<64>(kc, sum);
+        if (t == 0) {  // (the end of the kernel makes them visible to the host)
+            host[0] = du;
+            host[1] = (i64)sq.hi;
+            host[2] = (i64)sq.lo;
+            host[3] = km;
+            host[4] = kc;
+            host[5] = scal[SC_NEW];
+            scal[SC_NEW] = 0;
+            scal[SC_TICKET] = 0;
+        }
     }
 }
 
@@ -1683,43 +1873,58 @@ __global__ void __launch_bounds__(256) k_finish(const i64* __restrict__ vol, i64
 // MASSIVE_CUTOFF, which bound the movers of the last two classes.  The uncut
 // change goes to `at`.
 // reset: the movers' neighbours are scored again in the next sweep.  marked:
-// the movers' words are in mvp already.
+// the movers' words are in mvp already.  direct: moves lists every vertex.
 template <class AT>
 static void apply_moves_core(Ctx& c, MoveScratch& s, const LevelPlan& lp, const DGraph& g, i64* vol, const i32* moves,
-                             i64 k, bool marked, i64 n_large, i64 n_massive, bool reset, AT at) {
+                             i64 k, bool marked, i64 n_large, i64 n_massive, bool reset, AT at,
+                             bool direct = false) {
     const i64 nw = std::min(k, n_large);
     const i64 nb = std::min(k, n_massive);
-    const int tk = c.kt_begin(KS_MOVES);
     if (!marked) {
         k_mvp_moves<<<grid_items(k, 256), 256, 0, c.stream>>>(moves, k, s.part, s.dest, s.mvp);
         PGGC_LAUNCH_CHECK();
     }
+    Buf<i64> acct;
+    if (c.kt.on) {  // timing runs only
+        // per mover its word (written, read, settled), row bounds, cluster,
+        // destination, vertex weight and two volume updates; per mover edge
+        // the column, weight, the neighbour's word and its destination reset
+        const int wb = g.wk == W_UNIT ? 0 : g.wk == W_I32 ? 4 : 8;
+        acct = Buf<i64>(c, 1);
+        fill_i64(c, acct, 1, 0);
+        k_list_bytes<<<grid_items(std::max<i64>(k, 1), 256), 256, 0, c.stream>>>(
+            g.rp, moves, nullptr, s.mvp, k, 84, 12 + wb + (reset ? 4 : 0), 0, acct);
+        PGGC_LAUNCH_CHECK();
+    }
+    const int tk = c.kt_begin(KS_MOVES);
     const i64 cpm = nb > 0 ? ceil_div(lp.max_deg, MV_CHUNK) : 1;
+    const i64* knew = direct ? s.scal.p + SC_NEW : nullptr;
     const i64 b1 = ceil_div(k, 256 / MV_G), b2 = ceil_div(nw, 2), b3 = nb * cpm;
 #define PGGC_MOVE_EDGES(RS)                                                                                          \
     k_move_edges<RS><<<grid_blocks(b1 + b2 + b3), 256, 0, c.stream>>>(g.rp, g.col, W, moves, k, b1, b2, nw, nb, cpm,  \
-                                                                      s.mvp, s.dest, at)
+                                                                      s.mvp, s.dest, at, knew)
     PGGC_WDISPATCH(g, {
         if (reset) PGGC_MOVE_EDGES(true);
         else PGGC_MOVE_EDGES(false);
     });
 #undef PGGC_MOVE_EDGES
     PGGC_LAUNCH_CHECK();
-    k_apply_moves<<<grid_items(k, 256), 256, 0, c.stream>>>(moves, k, g.vw, s.mvp, s.part, s.dest, vol);
+    k_apply_moves<<<grid_items(k, 256), 256, 0, c.stream>>>(direct ? nullptr : moves, k, g.vw, s.mvp, s.part, s.dest, vol,
+                                                            direct ? s.abi.p : nullptr, s.scal);
     c.kt_end(tk, 0.0);
     PGGC_LAUNCH_CHECK();
-    if (tk >= 0) {  // timing runs only
-        // per mover its word (written, read, settled), row bounds, cluster,
-        // destination, vertex weight and two volume updates; per mover edge
-        // the column, weight, the neighbour's word and its destination reset
-        const int wb = g.wk == W_UNIT ? 0 : g.wk == W_I32 ? 4 : 8;
-        Buf<i64> acc(c, 1);
-        fill_i64(c, acc, 1, 0);
-        k_list_bytes<<<grid_items(std::max<i64>(k, 1), 256), 256, 0, c.stream>>>(
-            g.rp, moves, nullptr, k, 84, 12 + wb + (reset ? 4 : 0), 0, acc);
-        PGGC_LAUNCH_CHECK();
-        acct_add(c, c.kt_counter(tk), acc);
-    }
+    if (tk >= 0) acct_add(c, c.kt_counter(tk), acct);
+}
+
+// k_finish, and its results; the first n vertices' records when n > 0
+static const i64* finish_sweep(Ctx& c, MoveScratch& s, const RefineData& curr, i64 n, const i32* cons) {
+    const i64 L = curr.label_count;
+    if (n > 0 && cons && s.rec16.n < (size_t)n) s.rec16 = Buf<uint4>(c, s.cap);
+    k_finish<<<grid_for(std::max<i64>(std::max(L, n), 1), 256 * 4, FIN_BLOCKS), 256, 0, c.stream>>>(
+        curr.vol, L, s.sqpart, s.scal, c.pinned_dev, n, s.part, cons, s.rec, cons ? s.rec16.p : nullptr);
+    PGGC_LAUNCH_CHECK();
+    c.sync();
+    return c.pinned;
 }
 
 static void init_mvp(Ctx& c, MoveScratch& s, i64 n) {
@@ -1728,19 +1933,14 @@ static void init_mvp(Ctx& c, MoveScratch& s, i64 n) {
     PGGC_LAUNCH_CHECK();
 }
 
-static void perform_moves(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, RefineData& curr,
+static void perform_moves(Ctx& c, MoveScratch& s, const LevelPlan& lp, const DGraph& g, RefineData& curr,
                           const i32* moves, i64 k, bool marked, i64 n_large, i64 n_massive, bool& tables) {
     apply_moves_core(c, s, lp, g, curr.vol, moves, k, marked, n_large, n_massive, tables, AccOne{s.scal.p + SC_SLOTS});
     if (!tables) {
         tables = true;
         fill_i32(c, s.dest, g.n, NULL_PART);
     }
-    const i64 L = curr.label_count;
-    k_finish<<<grid_for(std::max<i64>(L, 1), 256 * 8, FIN_BLOCKS), 256, 0, c.stream>>>(curr.vol, L, s.sqpart, s.scal,
-                                                                                      c.pinned_dev);
-    PGGC_LAUNCH_CHECK();
-    c.sync();
-    const i64* h = c.pinned;
+    const i64* h = finish_sweep(c, s, curr, 0, nullptr);
     curr.uncut += h[0];
     curr.obj = objective_value(curr.uncut, curr.lambda, (u64)h[1], (u64)h[2]);
 }
@@ -1869,25 +2069,73 @@ static RefineData begin_curr(Ctx& c, const RefineData& best, Buf<i64>& cv, i64 n
     RefineData curr = best;
     curr.vol = cv;
     curr.cap = cap;
-    copy_state(c, curr, best);
     return curr;
 }
+static void move_begin(Ctx& c, MoveScratch& s, const RefineData& best, RefineData& curr, const i32* best_part, i64 n,
+                       i64 nfull) {
+    const i64 L = best.label_count;
+    if (L > curr.cap) throw Error(-4, "label capacity exceeded");
+    k_move_begin<<<grid_items(std::max<i64>(std::max(L, nfull), SC_COUNT), 256), 256, 0, c.stream>>>(
+        best.vol, L, curr.vol, best_part, nfull, s.part, n, s.mvp, s.dest, s.scal);
+    PGGC_LAUNCH_CHECK();
+}
 
-// The sweep's movers from its scored vertices.  Levels of at most
-// DIRECT_MAX vertices run the afterburner over all vertices and skip the
-// others, which saves a selection, its launches and a read-back; larger ones
-// list the candidates first, so that lanes are not spent on the others.
-// DIRECT
+// the sweep's movers from its scored vertices
 template <class LT, class PT>
 static Movers find_movers(Ctx& c, MoveScratch& s, const LevelPlan& lp, const DGraph& g, LT lam, PT prio, bool pack) {
     i64 b[2];
-    if (g.n <= DIRECT_MAX && !pack) {
-        b[0] = lp.ord.off_large;
-        b[1] = lp.ord.off_large2;
-        return afterburner(c, s, g, lp.ord.o1, g.n, b, lam, prio, s.moves, false);
-    }
     const i64 k = gather_candidates(c, lp, g, s.dest, s.cand, b);
-    return k > 0 ? afterburner(c, s, g, s.cand, k, b, lam, prio, s.moves, pack) : Movers{0, 0, 0};
+    if (k == 0) return Movers{0, 0, 0};
+    afterburner(c, s, g, s.cand, k, b, lam, prio, pack);
+    return select_movers(c, s, s.cand, k, s.moves);
+}
+
+// Filter and moves of a small level's sweep without lists and with one
+// read-back: the afterburner runs over all vertices and marks the movers, the
+// move kernels look at every vertex's mark, and the end of the sweep reports
+// the counts and packs the next sweep's records.  Levels of at most DIRECT_MAX
+// vertices and DIRECT_NNZ nonzeros: they are bound by launches and waits (a
+// sweep takes 7 launches and 1 wait; with lists 10 and 2, at first 34 and 5 or
+// 6).  Larger levels would spend lanes on the vertices that are no candidates
+// or do not move: the coarse level of R-MAT scale 20 (108,000 vertices, 30M
+// nonzeros) took 55 us per sweep in k_move_edges that way, with lists 36.
+// When movers need new cluster ids the move kernels leave everything as it is,
+// and the movers are selected, numbered and moved as on large levels.
+template <class LT, class PT>
+static Movers direct_sweep(Ctx& c, MoveScratch& s, const LevelPlan& lp, const DGraph& g, RefineData& curr, LT lam,
+                           PT prio, bool first, i32* cons, const i32* ids, i64 nfull, bool& tables, bool& fresh,
+                           bool& packed) {
+    const i64 n = g.n, n_large = n - lp.ord.off_large, n_massive = n - lp.ord.off_large2;
+    const i64 b[2] = {lp.ord.off_large, lp.ord.off_large2};
+    const i32* o1 = lp.ord.o1;
+    afterburner(c, s, g, o1, n, b, lam, prio, false, AbMark{s.mvp, s.scal.p + SC_NEW});
+    apply_moves_core(c, s, lp, g, curr.vol, o1, n, true, n_large, n_massive, tables, AccOne{s.scal.p + SC_SLOTS}, true);
+    const i64* h = finish_sweep(c, s, curr, n, cons);
+    Movers mv{h[3], h[5], h[4]};
+    if (mv.knew > 0) {
+        mv = select_movers(c, s, o1, n, s.moves);
+        // (the first sweep of an initial call gives no new ids)
+        if (!first) set_new_cluster_ids(c, s, g, curr, s.moves, mv.k, cons, ids, nfull);
+        fresh = !tables;
+        perform_moves(c, s, lp, g, curr, s.moves, mv.k, false, n_large, n_massive, tables);
+        return mv;
+    }
+    packed = true;
+    if (mv.k == 0) return mv;
+    curr.uncut += h[0];
+    curr.obj = objective_value(curr.uncut, curr.lambda, (u64)h[1], (u64)h[2]);
+    fresh = !tables;
+    if (!tables) {
+        tables = true;
+        fill_i32(c, s.dest, n, NULL_PART);
+    }
+    return mv;
+}
+
+static void sweep_note(const Ctx& c, i64 n, int iter, const Movers& mv, const RefineData& curr) {
+    if (c.verbose < 3) return;
+    fprintf(stderr, "sweep n=%lld it=%d cands=%lld moves=%lld labels=%d uncut=%lld obj=%.17g\n", (long long)n, iter,
+            (long long)mv.cands, (long long)mv.k, curr.label_count, (long long)curr.uncut, curr.obj);
 }
 
 template <class PT>
@@ -1917,9 +2165,7 @@ static void local_move_t(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g,
     c.mem_note("local move: plan ready");
     Buf<i64> cv;
     RefineData curr = begin_curr(c, best, cv, nfull);
-    copy_dev(c, s.part, best_part, nfull * sizeof(i32));
-    init_mvp(c, s, n);
-    fill_i32(c, s.dest, n, NULL_PART);
+    move_begin(c, s, best, curr, best_part, n, nfull);
     bool tables = !is_initial;
     const float ratios[2] = {0.75f, 0.25f};
     const int limits[2] = {4, 2};
@@ -1940,7 +2186,8 @@ static void local_move_t(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g,
     if (G) gnn_begin(c, *G, n, train);
     i64 kprev = n;
     i64 npred = 0;  // predicted sweeps in this call
-    bool fresh = false;  // every vertex was made active by the last sweep
+    bool fresh = false;   // every vertex was made active by the last sweep
+    bool packed = false;  // the last sweep packed this one's records
     for (int x = 0; x < 2; x++) {
         const float fr = SA ? ratios[x] : 0.0f;
         for (int cnt = 0; cnt < limits[x]; cnt++) {
@@ -1957,7 +2204,22 @@ static void local_move_t(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g,
             }
             tr.begin(s.dest, iter == 1 && !use, fresh);
             fresh = false;
-            score_all(c, s, lp, g, s.part, curr.vol, ccons, tables ? 0 : raw_mode, lam, fr, so);
+            score_all(c, s, lp, g, s.part, curr.vol, ccons, tables ? 0 : raw_mode, lam, fr, so, packed);
+            packed = false;
+            if (n <= DIRECT_MAX && g.nnz <= DIRECT_NNZ && !G && n > 0) {
+                const Movers mv = direct_sweep(c, s, lp, g, curr, lam, prio, is_initial && iter == 1,
+                                               constrained ? cons : nullptr, ids, nfull, tables, fresh, packed);
+                if (stats) {
+                    stats->sweeps++;
+                    stats->cands += mv.cands;
+                    stats->moves += mv.k;
+                }
+                sweep_note(c, nfull, iter, mv, curr);
+                if (mv.k > 0 && curr.obj > best.obj) copy_best(c, best, curr, best_part, s.part, n);
+                tr.end(mv.cands, mv.k);
+                if (mv.k == 0) break;
+                continue;
+            }
             Movers mv = find_movers(c, s, lp, g, lam, prio, so.info == nullptr);
             if (mv.k == 0 && G && gnn_restore(c, *G, n, s.dest)) {
                 // nothing to move among the vertices let through: score the
@@ -1988,10 +2250,7 @@ static void local_move_t(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g,
             fresh = !tables;
             perform_moves(c, s, lp, g, curr, s.moves, km, !fresh_ids, g.n - lp.ord.off_large, g.n - lp.ord.off_large2, tables);
             if (stats) stats->moves += km;
-            if (c.verbose >= 3)
-                fprintf(stderr, "sweep n=%lld it=%d cands=%lld moves=%lld labels=%d uncut=%lld obj=%.17g\n",
-                        (long long)n, iter, (long long)k, (long long)km, curr.label_count, (long long)curr.uncut,
-                        curr.obj);
+            sweep_note(c, nfull, iter, mv, curr);
             if (curr.obj > best.obj) copy_best(c, best, curr, best_part, s.part, n);
             tr.end(k, km);
         }
@@ -2070,9 +2329,7 @@ void local_move_strict(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, i
     plan_level(c, g, lp);
     Buf<i64> cv;
     RefineData curr = begin_curr(c, best, cv, n);
-    copy_dev(c, s.part, best_part, n * sizeof(i32));
-    init_mvp(c, s, n);
-    fill_i32(c, s.dest, n, NULL_PART);
+    move_begin(c, s, best, curr, best_part, n, n);
     bool tables = !is_initial;
     const i32* ccons = constrained ? cons : nullptr;
     Buf<float> sg(c, std::max<i64>(n, 1));
@@ -2135,7 +2392,8 @@ i64 sweep_once(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, const i32
     *ncand = k;
     i64 km = 0;
     if (k > 0) {
-        km = afterburner(c, s, g, s.cand, k, b, LamOne{lam}, PrioOne{}, moves_out, true).k;
+        afterburner(c, s, g, s.cand, k, b, LamOne{lam}, PrioOne{}, true);
+        km = select_movers(c, s, s.cand, k, moves_out).k;
     }
     copy_dev(c, dest, s.dest, n * sizeof(i32));
     copy_dev(c, gain, s.gain, n * sizeof(float));
@@ -2469,7 +2727,10 @@ void local_move_batch(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, co
         i64 b[2];
         const i64 kc = gather_candidates(c, lp, g, s.dest, s.cand, b);
         Movers mv{0, 0, 0};
-        if (kc > 0) mv = afterburner(c, s, g, s.cand, kc, b, lam, prio, s.moves, false);
+        if (kc > 0) {
+            afterburner(c, s, g, s.cand, kc, b, lam, prio, false);
+            mv = select_movers(c, s, s.cand, kc, s.moves);
+        }
         const i64 km = mv.k;
         fill_i64(c, cnt2, 2 * K, 0);
         if (kc > 0) k_inst_count<<<grid_items(kc, 256), 256, 0, c.stream>>>(s.cand, kc, bl.inst, cnt2);

@@ -181,9 +181,12 @@ void fill_i64(Ctx& c, i64* p, i64 n, i64 v) {
 // device-to-device copy as a kernel on the context stream (16-byte words
 // when both ends are 16-byte aligned, else 4-byte words; every copy in the
 // library is a multiple of 4 bytes)
-__global__ void k_copy16(const uint4* __restrict__ src, uint4* __restrict__ dst, i64 n) {
+// (the last thread also copies a tail of up to 12 bytes)
+__global__ void k_copy16(const uint4* __restrict__ src, uint4* __restrict__ dst, i64 n, int tail) {
     const i64 i = thread_item();
     if (i < n) dst[i] = src[i];
+    if (i == n)
+        for (int q = 0; q < tail; q++) ((u32*)(dst + n))[q] = ((const u32*)(src + n))[q];
 }
 __global__ void k_copy4(const u32* __restrict__ src, u32* __restrict__ dst, i64 n) {
     const i64 i = thread_item();
@@ -194,17 +197,10 @@ void copy_dev(Ctx& c, void* dst, const void* src, size_t bytes) {
     if (bytes % 4 != 0 || ((uintptr_t)dst | (uintptr_t)src) % 4 != 0)
         throw Error(-5, "copy_dev: size and addresses must be multiples of 4 bytes");
     if (((uintptr_t)dst | (uintptr_t)src) % 16 == 0) {
-        // 16-byte words for the bulk, 4-byte words for a tail of up to 12 bytes
         const i64 n16 = (i64)(bytes / 16);
-        if (n16 > 0) {
-            k_copy16<<<grid_items(n16, 256), 256, 0, c.stream>>>((const uint4*)src, (uint4*)dst, n16);
-            PGGC_LAUNCH_CHECK();
-        }
-        const i64 n4 = (i64)(bytes % 16) / 4;
-        if (n4 > 0) {
-            k_copy4<<<1, 64, 0, c.stream>>>((const u32*)src + 4 * n16, (u32*)dst + 4 * n16, n4);
-            PGGC_LAUNCH_CHECK();
-        }
+        k_copy16<<<grid_items(n16 + 1, 256), 256, 0, c.stream>>>((const uint4*)src, (uint4*)dst, n16,
+                                                                 (int)(bytes % 16) / 4);
+        PGGC_LAUNCH_CHECK();
         return;
     }
     const i64 n = (i64)(bytes / 4);
