@@ -211,7 +211,6 @@ static void contract_level(Ctx& c, const DGraph& g, const i32* map, i64 nc, Owne
         renum_gather(c, *rn, map, rn->part);
         contract(c, rn->g, rn->part, nc, og);
     }
-    narrow_weights(c, g, og);
 }
 
 // louvain_part<constrained> (src/clustering_methods.cpp:139-222)
@@ -988,7 +987,7 @@ int pggc_contract(pggc_ctx* ctx, const pggc_graph* gg, const int32_t* vcmap, int
         if (nc < 0) throw Error(PGGC_EINVAL, "negative cluster count");
         Ctx& c = ctx->c;
         OwnedGraph og;
-        contract(c, g, vcmap, nc, og);
+        contract(c, g, vcmap, nc, og, true);
         *nnz_out = og.nnz;
         copy_dev(c, out_rp, og.rp, (nc + 1) * sizeof(i64));
         if (og.nnz > cap) {
@@ -1091,6 +1090,7 @@ int pggc_cluster(pggc_ctx* ctx, const pggc_graph* gg, int algo, int objective, d
             g.wk = W_UNIT;
         }
         Ctx& c = ctx->c;
+        if (g.wk != W_UNIT && g.nnz > 0) g.wmax = max_weight(c, g);  // read by every plan and contraction
         c.seed = seed;
         c.draws = 0;
         Buf<i64> vol(c, g.n + 1);

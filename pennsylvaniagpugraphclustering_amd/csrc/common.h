@@ -72,7 +72,8 @@ struct DGraph {
     const void* w = nullptr;   // weights [nnz] (null when W_UNIT)
     int wk = W_UNIT;
     const i64* vw = nullptr;   // vertex weights [n]
-    bool wsmall = false;       // all weights together are known to sum to less than 2^32
+    bool wsmall = false;       // all weights together are known to sum to less than 2^31
+    u64 wmax = 0;              // largest weight as an unsigned value, 0 when not known
 };
 
 #define PGGC_WDISPATCH(G, ...)                               \

@@ -14,6 +14,7 @@ struct OwnedGraph {
     Buf<i64> vw;
     i64 n = 0, nnz = 0;
     bool wsmall = false;  // DGraph::wsmall
+    u64 wmax = 0;         // DGraph::wmax
     DGraph view() const {
         DGraph g;
         g.n = n;
@@ -29,11 +30,13 @@ struct OwnedGraph {
         }
         g.vw = vw.p;
         g.wsmall = wsmall;
+        g.wmax = wmax;
         return g;
     }
 };
 
 // Stable degree bucketing (src/ordering.cpp:131-164).
+__device__ __forceinline__ int order_class(i64 d) { return d < LARGE_CUTOFF ? 0 : (d < MASSIVE_CUTOFF ? 1 : 2); }
 struct Orders {
     Buf<i32> o1, o2;
     i64 off_large = 0, off_large2 = 0, off_mid = 0, off_mid2 = 0;
@@ -47,16 +50,13 @@ void evaluate(Ctx& c, const DGraph& g, const i32* labels, i64 L, i64* vol, i64* 
 // out[i] = sum of w(i,j) over neighbours j with labels[j] == labels[i].
 void own_weight(Ctx& c, const DGraph& g, const i32* labels, i64* out);
 
-// Contraction (src/contract.cpp:234-336) with sorted coarse rows.
-void contract(Ctx& c, const DGraph& g, const i32* vcmap, i64 nc, OwnedGraph& out);
-
-// Replaces g's int64 coarse weights by int32 ones when every weight fits:
-// always when the level it was contracted from has unit weights and fewer
-// than 2^31 nonzeros (a coarse weight then counts fine edges), else after a
-// max reduction.  The values, and so every result, are unchanged; the
-// sweeps read 4 instead of 8 weight bytes per edge and the level holds 8
-// instead of 12 bytes per nonzero.
-void narrow_weights(Ctx& c, const DGraph& fine, OwnedGraph& g);
+// Contraction (src/contract.cpp:234-336) with sorted coarse rows.  The coarse
+// weights are int32 when every one fits (the values, and so every result, are
+// the same; the sweeps read 4 instead of 8 weight bytes per edge and the level
+// holds 8 instead of 12 bytes per nonzero) and int64 otherwise, or always with
+// want64: when the finer level's weights sum to less than 2^31 they are written
+// as int32 at once, else after a max reduction.
+void contract(Ctx& c, const DGraph& g, const i32* vcmap, i64 nc, OwnedGraph& out, bool want64 = false);
 
 // largest weight of g as an unsigned value (a negative weight is huge); g.nnz > 0
 u64 max_weight(Ctx& c, const DGraph& g);

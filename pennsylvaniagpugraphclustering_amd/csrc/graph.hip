@@ -6,112 +6,39 @@
 #include "device.h"
 #include "graph.h"
 #include "hash.h"
+#include "select.h"
 
 namespace pggc {
 
-// ------------------------------------------------------ stable K-way partition
-constexpr int PT = 256, PI = 8, PTILE = PT * PI;
-
-template <int K>
-__global__ void __launch_bounds__(PT) k_part_count(const i32* cls, i64 n, i64* counts, i64 nb) {
-    i64 base = (i64)blockIdx.x * PTILE + (i64)threadIdx.x * PI;
-    i64 c[K];
-#pragma unroll
-    for (int k = 0; k < K; k++) c[k] = 0;
-#pragma unroll
-    for (int q = 0; q < PI; q++) {
-        i64 x = base + q;
-        if (x < n) {
-            int k = cls[x];
-#pragma unroll
-            for (int kk = 0; kk < K; kk++) c[kk] += (k == kk);
-        }
-    }
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-        i64 s = block_sum_i64<PT>(c[k]);
-        if (threadIdx.x == 0) counts[(i64)k * nb + blockIdx.x] = s;
-    }
-}
-
-template <int K>
-__global__ void __launch_bounds__(PT) k_part_write(const i32* cls, i64 n, const i64* offs, i64 nb, i32* out) {
-    i64 base = (i64)blockIdx.x * PTILE + (i64)threadIdx.x * PI;
-    int ck[PI];
-    i64 c[K];
-#pragma unroll
-    for (int k = 0; k < K; k++) c[k] = 0;
-#pragma unroll
-    for (int q = 0; q < PI; q++) {
-        i64 x = base + q;
-        ck[q] = x < n ? cls[x] : -1;
-#pragma unroll
-        for (int kk = 0; kk < K; kk++) c[kk] += (ck[q] == kk);
-    }
-    i64 pos[K];
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-        i64 tot;
-        pos[k] = block_excl_scan_i64(c[k], &tot) + offs[(i64)k * nb + blockIdx.x];
-    }
-#pragma unroll
-    for (int q = 0; q < PI; q++) {
-#pragma unroll
-        for (int kk = 0; kk < K; kk++)
-            if (ck[q] == kk) out[pos[kk]++] = (i32)(base + q);
-    }
-}
-
-__global__ void k_gather_starts(const i64* offs, i64 nb, int K, i64* starts) {
-    int k = threadIdx.x;
-    if (k <= K) starts[k] = offs[(i64)k * nb];
-}
-
-template <int K>
-static void partition_k(Ctx& c, const i32* cls, i64 n, i32* out, i64* starts) {
-    i64 nb = ceil_div(std::max<i64>(n, 1), PTILE);
-    Buf<i64> counts(c, K * nb + 1);
-    k_part_count<K><<<(int)nb, PT, 0, c.stream>>>(cls, n, counts, nb);
-    PGGC_LAUNCH_CHECK();
-    scan_i64(c, counts, counts, K * nb);
-    k_part_write<K><<<(int)nb, PT, 0, c.stream>>>(cls, n, counts, nb, out);
-    PGGC_LAUNCH_CHECK();
-    Buf<i64> st(c, K + 1);
-    k_gather_starts<<<1, 64, 0, c.stream>>>(counts, nb, K, st);
-    PGGC_LAUNCH_CHECK();
-    const i64* h = c.read(st, K + 1);
-    for (int k = 0; k <= K; k++) starts[k] = h[k];
-}
-
 // ------------------------------------------------------------------ orderings
-__global__ void k_order_classes(const i64* rp, i64 n, i32* c1, i32* c2) {
-    const i64 i = thread_item();
-    if (i >= n) return;
-    i64 d = rp[i + 1] - rp[i];
-    c1[i] = d < LARGE_CUTOFF ? 0 : (d < MASSIVE_CUTOFF ? 1 : 2);
-    c2[i] = d < MID_CUTOFF ? 0 : (d < MASSIVE_CUTOFF ? 1 : 2);
-}
+struct Order1 {
+    const i64* rp;
+    __device__ __forceinline__ int operator()(i64 i) const { return order_class(rp[i + 1] - rp[i]); }
+};
+struct Order2 {
+    const i64* rp;
+    __device__ __forceinline__ int operator()(i64 i) const {
+        const i64 d = rp[i + 1] - rp[i];
+        return d < MID_CUTOFF ? 0 : (d < MASSIVE_CUTOFF ? 1 : 2);
+    }
+};
 
 void make_orders(Ctx& c, const DGraph& g, Orders& o) {
     i64 n = g.n;
-    // row bounds and two class bytes per vertex read, then per partition
-    // the classes read twice (count, write) and the ids written
+    // per partition the row bounds read twice and the ids written
     const int tk = c.kt_begin(KS_ORDER);
-    if (o.o1.n < (size_t)n) {
+    if (o.o1.n < (size_t)n || !o.o2.p) {
         o.o1 = Buf<i32>(c, std::max<i64>(n, 1));
         o.o2 = Buf<i32>(c, std::max<i64>(n, 1));
     }
-    Buf<i32> c1(c, std::max<i64>(n, 1)), c2(c, std::max<i64>(n, 1));
-    k_order_classes<<<grid_items(n, 256), 256, 0, c.stream>>>(g.rp, n, c1, c2);
-    PGGC_LAUNCH_CHECK();
     i64 s1[4], s2[4];
-    partition_k<3>(c, c1, n, o.o1, s1);
-    partition_k<3>(c, c2, n, o.o2, s2);
+    class_partition(c, Order1{g.rp}, n, 3, o.o1, s1);
+    class_partition(c, Order2{g.rp}, n, 3, o.o2, s2);
     o.off_large = s1[1];
     o.off_large2 = s1[2];
     o.off_mid = s2[1];
     o.off_mid2 = s2[2];
-    c.kt_end(tk, 8.0 * (n + 1) + 8.0 * n + 2.0 * 12.0 * n);
+    c.kt_end(tk, 2.0 * (16.0 * (n + 1) + 4.0 * n));
 }
 
 // ------------------------------------------------- edge-chunk row reductions
@@ -250,10 +177,12 @@ __global__ void __launch_bounds__(256) k_ccount(const i64* rp, const i32* vcmap,
 }
 
 // member lists: a block's vertices take ranks per coarse id in LDS, each
-// distinct id reserves its run of the list with one HBM atomic, and every
-// vertex writes at run start + rank (the order inside a list is free: the
-// merges that read it are order-independent)
-__global__ void __launch_bounds__(256) k_cscatter(const i32* vcmap, i64 n, i64* pos, i32* members) {
+// distinct id reserves its run of the list with one HBM atomic (left counts the
+// members not placed yet down from the member counts), and every vertex writes
+// at run start + rank (the order inside a list is free: the merges that read it
+// are order-independent)
+__global__ void __launch_bounds__(256) k_cscatter(const i32* vcmap, i64 n, const i64* __restrict__ mstart, i64* left,
+                                                  i32* members) {
     __shared__ i32 lk[CC_SLOTS], lc[CC_SLOTS];
     __shared__ i64 lb[CC_SLOTS];
     for (int q = threadIdx.x; q < CC_SLOTS; q += 256) {
@@ -276,22 +205,24 @@ __global__ void __launch_bounds__(256) k_cscatter(const i32* vcmap, i64 n, i64* 
     }
     __syncthreads();
     for (int q = threadIdx.x; q < CC_SLOTS; q += 256)
-        if (lk[q] != EMPTY_KEY) lb[q] = (i64)atomicAdd((unsigned long long*)&pos[lk[q]], (unsigned long long)lc[q]);
+        if (lk[q] != EMPTY_KEY)
+            lb[q] = mstart[lk[q]] +
+                    (i64)atomicAdd((unsigned long long*)&left[lk[q]], (unsigned long long)-(i64)lc[q]) - lc[q];
     __syncthreads();
     if (i < n) members[lb[h] + r] = (i32)i;
 }
 
-constexpr i64 C_SMALL = 256;   // bound <= C_SMALL: 64-thread block, 512-slot LDS table
-constexpr i64 C_HALF = 1024;   // bound <= C_HALF: 256-thread block, 2048-slot LDS table
-constexpr i64 C_MID = 2048;    // bound <= C_MID: 256-thread block, 4096-slot LDS table
-
-// classes: 0..2 LDS merge (small, half, mid), 3 big rows, 4 empty rows
-__global__ void k_cclass(const i64* bound, i64 nc, i32* cls) {
-    const i64 u = thread_item();
-    if (u >= nc) return;
-    i64 b = bound[u];
-    cls[u] = b == 0 ? 4 : (b <= C_SMALL ? 0 : (b <= C_HALF ? 1 : (b <= C_MID ? 2 : 3)));
-}
+// Merge classes by bound (the summed degrees of a row's members): LDS tables
+// for bounds up to C_BOUND[q], then big rows and empty ones.
+constexpr int C_BIG = 5, C_EMPTY = 6, C_CLS = 7;
+constexpr i64 C_TOP = 8192;  // largest bound merged in LDS
+struct MergeClass {
+    const i64* bound;
+    __device__ __forceinline__ int operator()(i64 u) const {
+        const i64 b = bound[u];
+        return b == 0 ? C_EMPTY : b <= 256 ? 0 : b <= 1024 ? 1 : b <= 2048 ? 2 : b <= 4096 ? 3 : b <= C_TOP ? 4 : C_BIG;
+    }
+};
 
 __host__ __device__ __forceinline__ i64 table_slots(i64 bound, i64 nc) {
     i64 cap = bound < nc ? bound : nc;
@@ -306,157 +237,241 @@ __global__ void k_goff_sizes(const i32* list, i64 m, const i64* bound, i64 nc, i
     sz[x] = table_slots(bound[list[x]], nc);
 }
 
-// One block per coarse vertex: hash-merge the members' edges by coarse
-// neighbour, then write the distinct (neighbour, weight) pairs to the
-// temporary row at toff[u] (sorted when the table lives in LDS).
-template <int BS, int SLOTS, bool GLOBAL, class WT>
-__global__ void __launch_bounds__(BS) k_cagg(const i64* rp, const i32* col, WT W, const i32* vcmap, i64 nc,
-                                              const i32* list, i64 nlist, const i64* mstart, const i32* members,
-                                              const i64* bound, i32* gkeys, i64* gvals, const i64* goff,
-                                              const i64* toff, i32* tcol, i64* tw, i64* ccnt) {
-    __shared__ i32 skeys[GLOBAL ? 1 : SLOTS];
-    __shared__ i64 svals[GLOBAL ? 1 : SLOTS];
-    __shared__ i64 pre[BS];
+// the wave's smallest lo and largest hi, in every lane
+__device__ __forceinline__ void wave_min_max(i32& lo, i32& hi) {
+    xlane_fence(lo);
+    xlane_fence(hi);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        const i32 a = __shfl_xor(lo, o), b = __shfl_xor(hi, o);
+        lo = a < lo ? a : lo;
+        hi = b > hi ? b : hi;
+    }
+}
+// ascending bitonic sort of the first n keys in LDS (room for the next power
+// of two); every thread of the block calls it
+template <int BS>
+__device__ __forceinline__ void lds_sort_keys(i32* k, int n) {
+    int P = 2;
+    while (P < n) P <<= 1;
+    for (int q = n + threadIdx.x; q < P; q += BS) k[q] = 0x7fffffff;
+    __syncthreads();
+    for (int len = 2; len <= P; len <<= 1)
+        for (int o = len >> 1; o > 0; o >>= 1) {
+            for (int q = threadIdx.x; q < P / 2; q += BS) {
+                const int i = (q / o) * 2 * o + (q % o), j = i + o;
+                const bool up = (i & len) == 0;
+                const i32 a = k[i], b = k[j];
+                if ((a > b) == up) {
+                    k[i] = b;
+                    k[j] = a;
+                }
+            }
+            __syncthreads();
+        }
+}
+constexpr i32 C_FAT = 96;  // largest bucket that is ranked by comparing every pair of its keys
+
+// One block per coarse vertex of bound at most D: hash-merge the members' edges
+// by coarse neighbour in LDS, then write the distinct (neighbour, weight) pairs,
+// sorted by neighbour, to the temporary row at toff[u].
+//
+// The gathers of the neighbours' coarse ids bound the merge, so each thread has
+// CR edges in flight; the member that holds an edge is a binary search over the
+// members' degree prefix in LDS.  AT: u32 when every row sum of bound C_TOP fits
+// 32 bits, else i64 (the same sums).  The sort: the distinct keys are counted
+// into D buckets of equal id ranges between their smallest and largest, moved to
+// their bucket, and ranked among the keys of their bucket (one or two on
+// average; a row with a bucket of more than C_FAT keys, ids that bunch within
+// their range, is sorted instead, and the ranks are searched).  R-MAT scale 22
+// into 65,536 random clusters: rows of bounds up to 2048 took 4.2 ms with one
+// gather in flight, 64-bit sums and a bitonic sort of the whole table (66
+// barriers for 2,048 slots); rows up to 8192 take 2.05 ms now, and the rows
+// above, which alone are merged in HBM and sorted there, 1.5 + 1.6 ms (from 4.6
+// + 3.5, and 14.8 -> 7.1 ms for the whole call).
+template <int BS, int D, int SLOTS, class AT, class TT, class WT>
+__global__ void __launch_bounds__(BS) k_cagg(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
+                                              const i32* __restrict__ vcmap, i64 nc, const i32* __restrict__ list,
+                                              i64 nlist, const i64* __restrict__ mstart,
+                                              const i32* __restrict__ members, const i64* __restrict__ bound,
+                                              const i64* __restrict__ toff, i32* __restrict__ tcol,
+                                              TT* __restrict__ tw, i64* __restrict__ ccnt) {
+    static_assert(SLOTS > D, "the table holds every key and the bucket starts");
+    __shared__ i32 keys[SLOTS];  // the table's keys, then the keys in bucket order
+    __shared__ AT vals[SLOTS];   // the table's sums, then the bucket starts
+    __shared__ i32 pre[BS];
     __shared__ i64 rs[BS];
-    __shared__ int s_cnt;
+    __shared__ i32 s_min, s_max, s_fat;
     const int t = threadIdx.x;
     const i64 li = block_id();
     if (li >= nlist) return;
-    {
-        const i32 u = list[li];
-        const i64 S = table_slots(bound[u], nc);
-        const u32 mask = (u32)(S - 1);
-        i32* keys = GLOBAL ? gkeys + goff[li] : skeys;
-        i64* vals = GLOBAL ? gvals + goff[li] : svals;
-        for (i64 s = t; s < S; s += BS) {
-            keys[s] = EMPTY_KEY;
-            vals[s] = 0;
+    if (t == 0) {
+        s_min = 0x7fffffff;
+        s_max = -1;
+        s_fat = 0;
+    }
+    const i32 u = list[li];
+    const i64 cap = bound[u] < nc ? bound[u] : nc;
+    int S = 2;
+    while (S < 2 * cap) S <<= 1;
+    S = S < SLOTS ? S : SLOTS;
+    for (int s = t; s < S; s += BS) {
+        keys[s] = EMPTY_KEY;
+        vals[s] = 0;
+    }
+    __syncthreads();
+    const i64 m0 = mstart[u], m1 = mstart[u + 1];
+    for (i64 mb = m0; mb < m1; mb += BS) {
+        const i64 mi = mb + t;
+        i64 d = 0, st = 0;
+        if (mi < m1) {
+            const i32 v = members[mi];
+            st = rp[v];
+            d = rp[v + 1] - st;
         }
-        if (t == 0) s_cnt = 0;
+        i64 tot;
+        const i64 ex = block_excl_scan_i64(d, &tot);
+        pre[t] = (i32)ex;
+        rs[t] = st;
         __syncthreads();
-        const i64 m0 = mstart[u], m1 = mstart[u + 1];
-        for (i64 mb = m0; mb < m1; mb += BS) {
-            i64 mi = mb + t;
-            i64 d = 0, st = 0;
-            if (mi < m1) {
-                i32 v = members[mi];
-                st = rp[v];
-                d = rp[v + 1] - st;
-            }
-            i64 tot;
-            i64 ex = block_excl_scan_i64(d, &tot);
-            pre[t] = ex;
-            rs[t] = st;
-            __syncthreads();
-            // groups of CR edges per thread: locate and gather all of them
-            // (independent loads in flight together), then insert
-            constexpr int CR = 4;
-            for (i64 eb = 0; eb < tot; eb += (i64)BS * CR) {  // block-uniform loop control
-                i32 cv[CR];
-                i64 cw[CR];
+        const int nm = (int)(m1 - mb < BS ? m1 - mb : BS);
+        constexpr int CR = 4;
+        for (i64 eb = 0; eb < tot; eb += (i64)BS * CR) {  // block-uniform loop control
+            i32 cv[CR];
+            i64 j[CR];
 #pragma unroll
-                for (int r = 0; r < CR; r++) {
-                    const i64 e = eb + (i64)r * BS + t;
-                    cv[r] = u;  // no entry
-                    cw[r] = 0;
-                    if (e < tot) {
-                        int lo = 0, hi = BS;
-                        while (hi - lo > 1) {
-                            int md = (lo + hi) >> 1;
-                            if (pre[md] <= e) lo = md;
-                            else hi = md;
-                        }
-                        const i64 j = rs[lo] + (e - pre[lo]);
-                        cv[r] = vcmap[col[j]];
-                        cw[r] = W(j);
+            for (int r = 0; r < CR; r++) {
+                const i32 e = (i32)eb + r * BS + t;
+                j[r] = -1;
+                if (e < tot) {
+                    int lo = 0, hi = nm;
+                    while (hi - lo > 1) {
+                        const int md = (lo + hi) >> 1;
+                        if (pre[md] <= e) lo = md;
+                        else hi = md;
                     }
+                    j[r] = rs[lo] + (e - pre[lo]);
                 }
+            }
 #pragma unroll
-                for (int r = 0; r < CR; r++) {
-                    if (cv[r] == u) continue;
-                    if (GLOBAL) table_add_global(keys, vals, mask, cv[r], cw[r]);
-                    else table_add_lds(keys, vals, mask, cv[r], cw[r]);
-                }
-            }
-            __syncthreads();
-        }
-        if (!GLOBAL) {
-            // Sort only the distinct entries: move them to the front of the
-            // table (through registers, so no second LDS buffer), then rank
-            // them directly when one block's threads suffice (keys are
-            // distinct) or bitonic-sort the next power of two above them.
-            constexpr int R = SLOTS / BS;
-            i32 ek[R];
-            i64 ev[R];
+            for (int r = 0; r < CR; r++) cv[r] = j[r] >= 0 ? col[j[r]] : -1;
 #pragma unroll
-            for (int r = 0; r < R; r++) {
-                const i64 q = t + (i64)r * BS;
-                ek[r] = q < S ? keys[q] : EMPTY_KEY;
-                ev[r] = q < S ? vals[q] : 0;
-            }
-            __syncthreads();
+            for (int r = 0; r < CR; r++) cv[r] = cv[r] >= 0 ? vcmap[cv[r]] : u;
 #pragma unroll
-            for (int r = 0; r < R; r++) {
-                if (ek[r] != EMPTY_KEY) {
-                    const int pos = atomicAdd(&s_cnt, 1);
-                    keys[pos] = ek[r];
-                    vals[pos] = ev[r];
+            for (int r = 0; r < CR; r++) {
+                if (cv[r] == u) continue;  // inside the cluster, or no entry
+                const AT w = (AT)W(j[r]);
+                u32 h = __umulhi((u32)cv[r] * 0x9E3779B1u, (u32)S);
+                while (true) {  // fewer keys than slots: an empty slot is always found
+                    const i32 old = atomicCAS(&keys[h], EMPTY_KEY, cv[r]);
+                    if (old == EMPTY_KEY || old == cv[r]) break;
+                    h = h + 1 < (u32)S ? h + 1 : 0;
                 }
+                if (sizeof(AT) == 4) atomicAdd((u32*)&vals[h], (u32)w);
+                else atomicAdd((unsigned long long*)&vals[h], (unsigned long long)w);
             }
-            __syncthreads();
-            const int c = s_cnt;
-            const i64 base = toff[u];
-            if (c <= BS) {
-                if (t < c) {
-                    const i32 mk = keys[t];
-                    int rank = 0;
-                    for (int j = 0; j < c; j++) rank += keys[j] < mk ? 1 : 0;
-                    tcol[base + rank] = mk;
-                    tw[base + rank] = vals[t];
-                }
-            } else {
-                int P = 1;
-                while (P < c) P <<= 1;  // P <= S: the table has at least twice the distinct keys
-                for (int q = c + t; q < P; q += BS) {
-                    keys[q] = 0x7fffffff;
-                    vals[q] = 0;
-                }
-                __syncthreads();
-                bitonic_sort_lds<BS>(keys, vals, P);
-                for (int q = t; q < c; q += BS) {
-                    tcol[base + q] = keys[q];
-                    tw[base + q] = vals[q];
-                }
-            }
-            if (t == 0) ccnt[u] = c;
-        } else {
-            __threadfence();
-            __syncthreads();
-            i64 base = toff[u];
-            for (i64 s = t; s < S; s += BS) {
-                i32 k = __hip_atomic_load(&keys[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (k != EMPTY_KEY) {
-                    int p = atomicAdd(&s_cnt, 1);
-                    tcol[base + p] = k;
-                    tw[base + p] = __hip_atomic_load(&vals[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                }
-            }
-            __syncthreads();
-            if (t == 0) ccnt[u] = s_cnt;
         }
         __syncthreads();
     }
+    // the distinct entries in registers, their smallest and largest key
+    constexpr int R = (SLOTS + BS - 1) / BS;
+    i32 ek[R];
+    AT ev[R];
+    i32 kmin = 0x7fffffff, kmax = -1;
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const int q = t + r * BS;
+        ek[r] = q < S ? keys[q] : EMPTY_KEY;
+        ev[r] = q < S ? vals[q] : 0;
+        if (ek[r] != EMPTY_KEY) {
+            kmin = ek[r] < kmin ? ek[r] : kmin;
+            kmax = ek[r] > kmax ? ek[r] : kmax;
+        }
+    }
+    wave_min_max(kmin, kmax);
+    if ((t & 63) == 0) {
+        atomicMin(&s_min, kmin);
+        atomicMax(&s_max, kmax);
+    }
+    __syncthreads();
+    kmin = s_min;
+    kmax = s_max;
+    if (kmax < 0) {  // no coarse neighbour (block-uniform)
+        if (t == 0) ccnt[u] = 0;
+        return;
+    }
+    u32* hist = (u32*)vals;
+    for (int q = t; q < D; q += BS) hist[q] = 0;
+    __syncthreads();
+    // bucket of key k: (k - kmin) * scale >> 32, below D and monotone in k
+    const u64 scale = ((u64)D << 32) / (u64)((i64)kmax - kmin + 1);
+    u32 eb_[R], ep[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        eb_[r] = ep[r] = 0;
+        if (ek[r] == EMPTY_KEY) continue;
+        eb_[r] = (u32)(((u64)(u32)(ek[r] - kmin) * scale) >> 32);
+        ep[r] = atomicAdd(&hist[eb_[r]], 1u);
+    }
+    __syncthreads();
+    // exclusive scan of the bucket counts, D / BS consecutive ones per thread
+    constexpr int HB = D / BS;
+    u32 hc[HB];
+    i64 mine = 0;
+    i32 none = 0, fat = 0;
+#pragma unroll
+    for (int q = 0; q < HB; q++) {
+        hc[q] = hist[t * HB + q];
+        mine += hc[q];
+        fat = (i32)hc[q] > fat ? (i32)hc[q] : fat;
+    }
+    wave_min_max(none, fat);
+    if ((t & 63) == 0) atomicMax(&s_fat, fat);
+    i64 c;
+    u32 run = (u32)block_excl_scan_i64(mine, &c);
+#pragma unroll
+    for (int q = 0; q < HB; q++) {
+        hist[t * HB + q] = run;
+        run += hc[q];
+    }
+    if (t == 0) hist[D] = (u32)c;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; r++)
+        if (ek[r] != EMPTY_KEY) keys[hist[eb_[r]] + ep[r]] = ek[r];
+    __syncthreads();
+    const bool crowded = s_fat > C_FAT;  // block-uniform
+    if (crowded) lds_sort_keys<BS>(keys, (int)c);
+    const i64 base = toff[u];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        if (ek[r] == EMPTY_KEY) continue;
+        const u32 b0 = hist[eb_[r]], b1 = hist[eb_[r] + 1];
+        u32 rank = b0;
+        if (crowded) {
+            u32 hi = b1;
+            while (hi - rank > 1) {
+                const u32 md = (rank + hi) >> 1;
+                if (keys[md] <= ek[r]) rank = md;
+                else hi = md;
+            }
+        } else {
+            for (u32 q = b0; q < b1; q++) rank += keys[q] < ek[r] ? 1 : 0;
+        }
+        tcol[base + rank] = ek[r];
+        tw[base + rank] = (TT)ev[r];
+    }
+    if (t == 0) ccnt[u] = c;
 }
 
-// Big coarse rows (bound > C_MID): the flattened member-edge range of each
+// Big coarse rows (bound > C_TOP): the flattened member-edge range of each
 // such row is split into work items of BCH_E edges, each item a block that
 // merges its edges in LDS and then inserts the distinct pairs into the row's
 // HBM hash table; a second pass splits each table into slot items of BCH_S
 // slots and compacts the occupied slots.
-constexpr int BCH_E = 1024;      // member edges per insert item (4 per thread)
+constexpr int BCH_E = 2048;      // member edges per insert item (8 per thread)
 constexpr int BCH_S = 4096;      // table slots per extract item (16 per thread)
 constexpr int BLDS = 2 * BCH_E;  // LDS pre-aggregation slots
-
 __global__ void k_member_degs(const i32* members, const i64* rp, i64 n, i64* mdp) {
     const i64 k = thread_item();
     if (k >= n) return;
@@ -471,37 +486,83 @@ __global__ void k_items(const i32* list, i64 m, const i64* bound, const i64* gof
     items[x] = (len + per - 1) / per;
 }
 
-template <class WT>
-__global__ void __launch_bounds__(256) k_cbig_insert(const i64* rp, const i32* col, WT W, const i32* vcmap,
-                                                      const i32* members, const i64* mstart, const i64* mdp,
-                                                      const i32* big, i64 nbig, const i64* items, const i64* goff,
-                                                      i32* gkeys, i64* gvals, u64* gtab) {
-    // big, items and goff point at a batch of rows: items[0] and goff[0] are
-    // the batch's first work item and first table slot
+// row of every work item of the big rows: a block per row
+__global__ void __launch_bounds__(256) k_item_rows(const i64* __restrict__ items, i64 m, i32* __restrict__ row) {
+    const i64 x = block_id();
+    if (x >= m) return;
+    for (i64 b = items[x] + threadIdx.x; b < items[x + 1]; b += 256) row[b] = (i32)x;
+}
+
+// An item's threads take EPI consecutive edges each: the member that holds the
+// first one is searched between the members of the item's first and last edge,
+// and columns and coarse ids are gathered EPI at a time.  AT as in k_cagg for
+// the sums of an item.  The gathers and the inserts bound it: 6.2 ms for the
+// rows above 8192 of R-MAT scale 24's first level (13.1 ms for those above 2048
+// with the member searched in the whole list by every thread, one gather in
+// flight and 1024-edge items).
+template <class AT, class WT>
+__global__ void __launch_bounds__(256) k_cbig_insert(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
+                                                      const i32* __restrict__ vcmap, const i32* __restrict__ members,
+                                                      const i64* __restrict__ mstart, const i64* __restrict__ mdp,
+                                                      const i32* __restrict__ big, i64 r0, i64 nbig,
+                                                      const i32* __restrict__ row, const i64* __restrict__ items,
+                                                      const i64* __restrict__ goff, i32* gkeys, i64* gvals, u64* gtab) {
+    // a batch of rows, from row r0 on: big, items and goff point at its first
+    // row, items[0] and goff[0] are its first work item and first table slot
+    __shared__ i32 lk[BLDS];
+    __shared__ AT lv[BLDS];
+    __shared__ i64 s_k[2];
     const i64 b = block_id() + items[0];
     if (b >= items[nbig]) return;
-    const i64 ui = upper_row(items, 0, nbig, b);
+    const int t = threadIdx.x;
+    const i64 ui = (i64)row[b] - r0;
     const i32 u = big[ui];
     const i64 m0 = mstart[u], m1 = mstart[u + 1];
     const i64 e_lo = mdp[m0] + (b - items[ui]) * BCH_E;
     const i64 e_end = mdp[m1];
     const i64 e_hi = e_lo + BCH_E < e_end ? e_lo + BCH_E : e_end;
-    __shared__ i32 lk[BLDS];
-    __shared__ i64 lv[BLDS];
-    lds_agg_clear<256, BLDS>(lk, lv);
+    for (int q = t; q < BLDS; q += 256) {
+        lk[q] = EMPTY_KEY;
+        lv[q] = 0;
+    }
+    if (t < 2) s_k[t] = upper_row(mdp, m0, m1, t == 0 ? e_lo : e_hi - 1);
+    __syncthreads();
     constexpr int EPI = BCH_E / 256;
-    const i64 e0 = e_lo + (i64)threadIdx.x * EPI;
+    const i64 e0 = e_lo + (i64)t * EPI;
     if (e0 < e_hi) {
-        i64 k = upper_row(mdp, m0, m1, e0);
+        i64 k = upper_row(mdp, s_k[0], s_k[1] + 1, e0);
         i64 nxt = mdp[k + 1];
+        i64 shift = rp[members[k]] - mdp[k];
+        i64 j[EPI];
+        i32 cv[EPI];
+#pragma unroll
         for (int q = 0; q < EPI; q++) {
             const i64 e = e0 + q;
-            if (e >= e_hi) break;
-            if (e >= nxt) k = advance_row(mdp, k, m1, e, nxt);
-            const i32 v = members[k];
-            const i64 j = rp[v] + (e - mdp[k]);
-            const i32 cv = vcmap[col[j]];
-            if (cv != u) table_add_lds(lk, lv, BLDS - 1, cv, W(j));
+            j[q] = -1;
+            if (e < e_hi) {
+                if (e >= nxt) {
+                    k = advance_row(mdp, k, s_k[1] + 1, e, nxt);
+                    shift = rp[members[k]] - mdp[k];
+                }
+                j[q] = shift + e;
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < EPI; q++) cv[q] = j[q] >= 0 ? col[j[q]] : -1;
+#pragma unroll
+        for (int q = 0; q < EPI; q++) cv[q] = cv[q] >= 0 ? vcmap[cv[q]] : u;
+#pragma unroll
+        for (int q = 0; q < EPI; q++) {
+            if (cv[q] == u) continue;
+            const AT w = (AT)W(j[q]);
+            u32 h = slot_hash(cv[q], BLDS - 1);
+            while (true) {  // at most BLDS / 2 keys
+                const i32 old = atomicCAS(&lk[h], EMPTY_KEY, cv[q]);
+                if (old == EMPTY_KEY || old == cv[q]) break;
+                h = (h + 1) & (BLDS - 1);
+            }
+            if (sizeof(AT) == 4) atomicAdd((u32*)&lv[h], (u32)w);
+            else atomicAdd((unsigned long long*)&lv[h], (unsigned long long)w);
         }
     }
     const u32 gmask = (u32)(goff[ui + 1] - goff[ui] - 1);
@@ -511,9 +572,10 @@ __global__ void __launch_bounds__(256) k_cbig_insert(const i64* rp, const i32* c
 }
 
 // gtab non-null: packed tables (key << 32 | weight), else gkeys / gvals
+template <class TT>
 __global__ void __launch_bounds__(256) k_cbig_extract(const i32* big, i64 nbig, const i64* items, const i64* goff,
                                                        const i32* gkeys, const i64* gvals, const u64* gtab,
-                                                       const i64* toff, i32* tcol, i64* tw, i64* ccnt) {
+                                                       const i64* toff, i32* tcol, TT* tw, i64* ccnt) {
     __shared__ int s_cnt;
     __shared__ i64 s_base;
     // a batch of rows, as in k_cbig_insert; slot sl lives at sl - g0
@@ -549,7 +611,7 @@ __global__ void __launch_bounds__(256) k_cbig_extract(const i32* big, i64 nbig, 
         if (pos[q] >= 0) {
             const i64 sl = s_lo + threadIdx.x + (i64)q * 256;
             tcol[base + pos[q]] = kk[q];
-            tw[base + pos[q]] = gtab ? (i64)(gtab[sl - g0] & 0xffffffffull) : gvals[sl - g0];
+            tw[base + pos[q]] = (TT)(gtab ? (i64)(gtab[sl - g0] & 0xffffffffull) : gvals[sl - g0]);
         }
     }
 }
@@ -561,8 +623,9 @@ __global__ void __launch_bounds__(256) k_cbig_extract(const i32* big, i64 nbig, 
 // the chunk start clamped to [0, EC]; a chunk spanning more than EC rows (runs
 // of empty rows) searches the row pointers in global memory instead.  The
 // search interval carries over between steps since entries only move right.
+template <class TT, class OT>
 __global__ void __launch_bounds__(EB) k_crow_copy(const i64* crp, i64 nc, i64 nnzc, const i64* toff, const i32* tcol,
-                                                   const i64* tw, i32* ocol, i64* ow) {
+                                                   const TT* tw, i32* ocol, OT* ow) {
     __shared__ i32 s_st[EC + 1];
     ChunkRows cr;
     chunk_rows(crp, nc, nnzc, cr);
@@ -595,7 +658,7 @@ __global__ void __launch_bounds__(EB) k_crow_copy(const i64* crp, i64 nc, i64 nn
         }
         const i64 src = toff[r] + (j - crp[r]);
         ocol[j] = tcol[src];
-        ow[j] = tw[src];
+        ow[j] = (OT)tw[src];
     }
 }
 
@@ -609,8 +672,9 @@ __global__ void k_big_count(const i32* list, i64 m, const i64* crp, i64* cnt) {
 }
 // key = (big row index in the batch << cb) | column (columns < 2^cb), so the
 // radix sort needs only cb + bits(rows in the batch) bits
+template <class OT>
 __global__ void k_big_flatten(const i32* list, i64 m, const i64* crp, const i64* boff, const i32* ocol,
-                              const i64* ow, int cb, u64* key, i64* val, i64* target) {
+                              const OT* ow, int cb, u64* key, OT* val, i64* target) {
     const i64 x = block_id();
     if (x >= m) return;
     {
@@ -626,8 +690,9 @@ __global__ void k_big_flatten(const i32* list, i64 m, const i64* crp, const i64*
 }
 // the f-th smallest key of the batch goes to the f-th position of its rows
 // in row order (rows keep their order and their lengths through the sort)
-__global__ void k_big_scatter(const u64* key, const i64* target, i64 E, const i64* wsorted, int cb, i32* ocol,
-                              i64* ow) {
+template <class OT>
+__global__ void k_big_scatter(const u64* key, const i64* target, i64 E, const OT* wsorted, int cb, i32* ocol,
+                              OT* ow) {
     const u64 mask = ((u64)1 << cb) - 1;
     for (i64 f = (i64)blockIdx.x * blockDim.x + threadIdx.x; f < E; f += (i64)gridDim.x * blockDim.x) {
         i64 j = target[f];
@@ -703,72 +768,66 @@ u64 max_weight(Ctx& c, const DGraph& g) {
     return (u64)c.read1((const i64*)mx.p);
 }
 
-void narrow_weights(Ctx& c, const DGraph& fine, OwnedGraph& g) {
-    if (g.nnz == 0 || !g.w.p) return;
-    bool fits = fine.wk == W_UNIT && fine.nnz < ((i64)1 << 31);
-    if (!fits) {
-        fits = max_weight(c, g.view()) <= 0x7fffffffull;
-    }
-    if (!fits) return;
+// int64 coarse weights replaced by int32 ones when every one fits
+static void narrow_weights(Ctx& c, OwnedGraph& g) {
+    if (g.nnz == 0) return;
+    g.wmax = max_weight(c, g.view());
+    if (g.wmax > 0x7fffffffull) return;
     g.w32 = Buf<i32>(c, g.nnz);
     k_narrow<<<grid_for(g.nnz, 256 * 8, 8192), 256, 0, c.stream>>>(g.w, g.nnz, g.w32);
     PGGC_LAUNCH_CHECK();
     g.w.reset();
 }
 
-void contract(Ctx& c, const DGraph& g, const i32* vcmap, i64 nc, OwnedGraph& out) {
+// AT: sums of rows merged in LDS; TT: staged weights; OT: weights written to
+// `ow` (out.w or out.w32, allocated here)
+template <class AT, class TT, class OT>
+static void contract_t(Ctx& c, const DGraph& g, const i32* vcmap, i64 nc, OwnedGraph& out, Buf<OT>& ow) {
     const i64 n = g.n;
-    Buf<i64> cnt(c, nc + 1), bound(c, nc + 1), mstart(c, nc + 1), toff(c, nc + 1), pos(c, nc + 1);
+    // member counts, bounds and coarse degrees, zeroed by one launch
+    Buf<i64> zero(c, 3 * (nc + 1)), mstart(c, nc + 1), toff(c, nc + 1);
+    i64 *cnt = zero.p, *bound = cnt + nc + 1, *ccnt = bound + nc + 1;
     Buf<i32> members(c, std::max<i64>(n, 1));
-    fill_i64(c, cnt, nc + 1, 0);
-    fill_i64(c, bound, nc + 1, 0);
+    fill_i64(c, zero, 3 * (nc + 1), 0);
     k_ccount<<<grid_items(n, 256), 256, 0, c.stream>>>(g.rp, vcmap, n, cnt, bound);
     PGGC_LAUNCH_CHECK();
     scan_i64(c, cnt, mstart, nc);
     scan_i64(c, bound, toff, nc);
-    copy_dev(c, pos, mstart, nc * sizeof(i64));
-    k_cscatter<<<grid_items(n, 256), 256, 0, c.stream>>>(vcmap, n, pos, members);
+    k_cscatter<<<grid_items(n, 256), 256, 0, c.stream>>>(vcmap, n, mstart, cnt, members);
     PGGC_LAUNCH_CHECK();
-    const i64 tb = c.read1(toff.p + nc);
     c.mem_note("contract: before row staging");
-    Buf<i32> tcol(c, std::max<i64>(tb, 1));
-    Buf<i64> tw(c, std::max<i64>(tb, 1));
-    Buf<i64> ccnt(c, nc + 1);
-    Buf<i32> cls(c, std::max<i64>(nc, 1)), list(c, std::max<i64>(nc, 1));
-    k_cclass<<<grid_items(nc, 256), 256, 0, c.stream>>>(bound, nc, cls);
-    PGGC_LAUNCH_CHECK();
-    i64 st[6];
-    partition_k<5>(c, cls, nc, list, st);
-    fill_i64(c, ccnt, nc + 1, 0);
-    const i64 n0 = st[1] - st[0], n1 = st[2] - st[1], n1b = st[3] - st[2], n2 = st[4] - st[3];
+    Buf<i32> tcol(c, std::max<i64>(g.nnz, 1));  // (the bounds add up to nnz)
+    Buf<TT> tw(c, std::max<i64>(g.nnz, 1));
+    Buf<i32> list(c, std::max<i64>(nc, 1));
+    i64 st[C_CLS + 1];
+    class_partition(c, MergeClass{bound}, nc, C_CLS, list, st);
     int tk = c.kt_begin(KS_CONTRACT_AGG);
+#define PGGC_CAGG(q, BS, D, SLOTS)                                                                                    \
+    if (st[q + 1] > st[q])                                                                                            \
+    k_cagg<BS, D, SLOTS, AT, TT><<<grid_blocks(st[q + 1] - st[q]), BS, 0, c.stream>>>(                                \
+        g.rp, g.col, W, vcmap, nc, list.p + st[q], st[q + 1] - st[q], mstart, members, bound, toff, tcol, tw, ccnt)
     PGGC_WDISPATCH(g, {
-        if (n0 > 0)
-            k_cagg<64, 512, false><<<grid_blocks(n0), 64, 0, c.stream>>>(
-                g.rp, g.col, W, vcmap, nc, list.p + st[0], n0, mstart, members, bound, nullptr, nullptr, nullptr,
-                toff, tcol, tw, ccnt);
-        if (n1 > 0)
-            k_cagg<256, 2048, false><<<grid_blocks(n1), 256, 0, c.stream>>>(
-                g.rp, g.col, W, vcmap, nc, list.p + st[1], n1, mstart, members, bound, nullptr, nullptr, nullptr,
-                toff, tcol, tw, ccnt);
-        if (n1b > 0)
-            k_cagg<256, 4096, false><<<grid_blocks(n1b), 256, 0, c.stream>>>(
-                g.rp, g.col, W, vcmap, nc, list.p + st[2], n1b, mstart, members, bound, nullptr, nullptr, nullptr,
-                toff, tcol, tw, ccnt);
+        PGGC_CAGG(0, 64, 256, 512);
+        PGGC_CAGG(1, 256, 1024, 2048);
+        PGGC_CAGG(2, 256, 2048, 4096);
+        PGGC_CAGG(3, 512, 4096, 8192);
+        PGGC_CAGG(4, 1024, 8192, 9600);
     });
+#undef PGGC_CAGG
     c.kt_end(tk, 0.0);
     PGGC_LAUNCH_CHECK();
     const int wb = g.wk == W_UNIT ? 0 : g.wk == W_I32 ? 4 : 8;
-    contract_bytes(c, tk, list.p + st[0], n0 + n1 + n1b, mstart, bound, ccnt, wb);
+    contract_bytes(c, tk, list.p, st[C_BIG], mstart, bound, ccnt, wb);
+    const i64 n2 = st[C_BIG + 1] - st[C_BIG];
+    const i32* big = list.p + st[C_BIG];
     if (n2 > 0) {
-        const i32* big = list.p + st[3];
         Buf<i64> goff(c, n2 + 1), items(c, n2 + 1), items2(c, n2 + 1), mdp(c, n + 1);
         k_goff_sizes<<<grid_items(n2, 256), 256, 0, c.stream>>>(big, n2, bound, nc, goff);
         PGGC_LAUNCH_CHECK();
         scan_i64(c, goff, goff, n2);
         // packed tables (one CAS per new key) when every coarse weight fits
-        // 32 bits: with unit weights a coarse weight counts fine edges
-        const bool packed = g.wk == W_UNIT && g.nnz < ((i64)1 << 32) - 1;
+        // 32 bits
+        const bool packed = sizeof(TT) == 4;
         k_member_degs<<<grid_items(n, 256), 256, 0, c.stream>>>(members, g.rp, n, mdp);
         PGGC_LAUNCH_CHECK();
         scan_i64(c, mdp, mdp, n);
@@ -786,6 +845,9 @@ void contract(Ctx& c, const DGraph& g, const i32* vcmap, i64 nc, OwnedGraph& out
         download_i64(c, hg, goff, n2 + 1);
         download_i64(c, hi, items, n2 + 1);
         download_i64(c, hi2, items2, n2 + 1);
+        Buf<i32> row(c, std::max<i64>(hi[n2], 1));
+        k_item_rows<<<grid_blocks(n2), 256, 0, c.stream>>>(items, n2, row);
+        PGGC_LAUNCH_CHECK();
         i64 gmax = 0;
         const std::vector<i64> cuts = batch_cuts(hg, slot_cap, &gmax);
         Buf<i32> gkeys(c, packed ? 1 : gmax);
@@ -804,15 +866,15 @@ void contract(Ctx& c, const DGraph& g, const i32* vcmap, i64 nc, OwnedGraph& out
             }
             const i64 I = hi[r1] - hi[r0];
             if (I > 0) {
-                PGGC_WDISPATCH(g, (k_cbig_insert<<<grid_blocks(I), 256, 0, c.stream>>>(
-                                      g.rp, g.col, W, vcmap, members, mstart, mdp, big + r0, r1 - r0, items.p + r0,
-                                      goff.p + r0, gkeys, gvals, gt)));
+                PGGC_WDISPATCH(g, (k_cbig_insert<AT><<<grid_blocks(I), 256, 0, c.stream>>>(
+                                      g.rp, g.col, W, vcmap, members, mstart, mdp, big + r0, r0, r1 - r0, row,
+                                      items.p + r0, goff.p + r0, gkeys, gvals, gt)));
                 PGGC_LAUNCH_CHECK();
             }
             const i64 I2 = hi2[r1] - hi2[r0];
             if (I2 > 0) {
                 k_cbig_extract<<<grid_blocks(I2), 256, 0, c.stream>>>(big + r0, r1 - r0, items2.p + r0, goff.p + r0,
-                                                                      gkeys, gvals, gt, toff, tcol, tw, ccnt);
+                                                                      gkeys, gvals, gt, toff, tcol, tw.p, ccnt);
                 PGGC_LAUNCH_CHECK();
             }
         }
@@ -821,19 +883,19 @@ void contract(Ctx& c, const DGraph& g, const i32* vcmap, i64 nc, OwnedGraph& out
     }
     out.n = nc;
     // (a coarse graph's weights sum to at most the finer level's)
-    out.wsmall = g.wsmall || (g.wk == W_UNIT && g.nnz < ((i64)1 << 32));
+    out.wsmall = sizeof(TT) == 4;
     out.rp = Buf<i64>(c, nc + 1);
     scan_i64(c, ccnt, out.rp, nc);
     out.nnz = c.read1(out.rp.p + nc);
     out.col = Buf<i32>(c, std::max<i64>(out.nnz, 1));
-    out.w = Buf<i64>(c, std::max<i64>(out.nnz, 1));
+    ow = Buf<OT>(c, std::max<i64>(out.nnz, 1));
     if (out.nnz > 0) {
         // algorithmic bytes: coarse offsets, row starts in the temporary rows,
         // (column, weight) read and written once
-        const double bytes = 16.0 * (nc + 1) + 24.0 * out.nnz;
+        const double bytes = 16.0 * (nc + 1) + (8.0 + sizeof(TT) + sizeof(OT)) * out.nnz;
         const int tkc = c.kt_begin(KS_CONTRACT_COPY);
-        k_crow_copy<<<(int)ceil_div(out.nnz, EC), EB, 0, c.stream>>>(out.rp, nc, out.nnz, toff, tcol, tw, out.col,
-                                                                   out.w);
+        k_crow_copy<<<(int)ceil_div(out.nnz, EC), EB, 0, c.stream>>>(out.rp, nc, out.nnz, toff, tcol, tw.p, out.col,
+                                                                   ow.p);
         c.kt_end(tkc, bytes);
         PGGC_LAUNCH_CHECK();
     }
@@ -844,7 +906,6 @@ void contract(Ctx& c, const DGraph& g, const i32* vcmap, i64 nc, OwnedGraph& out
         // column, in batches of at most c.contract_batch / 4 entries (a
         // larger row is a batch of its own)
         const i64 sort_cap = std::max<i64>(c.contract_batch / 4, 1);
-        const i32* big = list.p + st[3];
         Buf<i64> boff(c, n2 + 1);
         k_big_count<<<grid_items(n2, 256), 256, 0, c.stream>>>(big, n2, out.rp, boff);
         PGGC_LAUNCH_CHECK();
@@ -855,22 +916,42 @@ void contract(Ctx& c, const DGraph& g, const i32* vcmap, i64 nc, OwnedGraph& out
         const std::vector<i64> cuts = batch_cuts(hb, sort_cap, &emax);
         if (emax > 0) {
             Buf<u64> key(c, emax);
-            Buf<i64> val(c, emax), target(c, emax);
+            Buf<OT> val(c, emax);
+            Buf<i64> target(c, emax);
             const int cb = bits_for(nc - 1);
             for (size_t q = 0; q + 1 < cuts.size(); q++) {
                 const i64 r0 = cuts[q], r1 = cuts[q + 1], E = hb[r1] - hb[r0];
                 if (E == 0) continue;
                 k_big_flatten<<<grid_blocks(r1 - r0), 256, 0, c.stream>>>(big + r0, r1 - r0, out.rp, boff.p + r0,
-                                                                          out.col, out.w, cb, key, val, target);
+                                                                          out.col, ow.p, cb, key, val.p, target);
                 PGGC_LAUNCH_CHECK();
-                radix_sort_pairs(c, key, val, E, cb + bits_for(r1 - r0));
-                k_big_scatter<<<grid_for(E, 256 * 4, 8192), 256, 0, c.stream>>>(key, target, E, val, cb, out.col,
-                                                                                out.w);
+                radix_sort_pairs(c, key, val.p, E, cb + bits_for(r1 - r0));
+                k_big_scatter<<<grid_for(E, 256 * 4, 8192), 256, 0, c.stream>>>(key, target, E, val.p, cb, out.col,
+                                                                                ow.p);
                 PGGC_LAUNCH_CHECK();
             }
         }
     }
-    (void)n1;
+}
+
+void contract(Ctx& c, const DGraph& g, const i32* vcmap, i64 nc, OwnedGraph& out, bool want64) {
+    // all weights together below 2^31: every coarse weight and sum fits 32 bits
+    const u64 top = (u64)1 << 31;
+    const bool small = g.wsmall || (g.wk == W_UNIT ? (u64)g.nnz < top
+                                                   : g.wmax > 0 && g.wmax < top && (u64)g.nnz * g.wmax < top);
+    if (small && !want64) {
+        contract_t<u32, i32>(c, g, vcmap, nc, out, out.w32);
+        return;
+    }
+    if (small) {
+        contract_t<u32, i32>(c, g, vcmap, nc, out, out.w);
+    } else {
+        // 32-bit sums in LDS when the weights are small enough for C_TOP of them
+        const u64 mx = g.wk == W_UNIT ? 1 : g.wmax ? g.wmax : g.nnz > 0 ? max_weight(c, g) : 1;
+        if (mx <= 0xffffffffull / C_TOP) contract_t<u32, i64>(c, g, vcmap, nc, out, out.w);
+        else contract_t<i64, i64>(c, g, vcmap, nc, out, out.w);
+        if (!want64) narrow_weights(c, out);
+    }
 }
 
 }  // namespace pggc

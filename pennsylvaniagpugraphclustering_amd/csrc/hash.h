@@ -1,5 +1,5 @@
 // Open-addressing (linear probing) cluster-id -> int64 weight tables in LDS or
-// HBM, and an in-LDS bitonic sort of (key, value) pairs.
+// HBM.
 #pragma once
 #include "common.h"
 
@@ -69,12 +69,12 @@ __device__ __forceinline__ void lds_agg_clear(i32* lk, i64* lv) {
     }
     __syncthreads();
 }
-template <int BS, int LSLOTS>
-__device__ __forceinline__ void lds_agg_flush(const i32* lk, const i64* lv, i32* gkeys, i64* gvals, u32 gmask) {
+template <int BS, int LSLOTS, class AT>
+__device__ __forceinline__ void lds_agg_flush(const i32* lk, const AT* lv, i32* gkeys, i64* gvals, u32 gmask) {
     __syncthreads();
     for (int q = threadIdx.x; q < LSLOTS; q += BS) {
         const i32 key = lk[q];
-        const i64 w = lv[q];
+        const i64 w = (i64)lv[q];
         if (key != EMPTY_KEY) table_add_global(gkeys, gvals, gmask, key, w);
     }
 }
@@ -83,8 +83,8 @@ __device__ __forceinline__ void lds_agg_flush(const i32* lk, const i64* lv, i32*
 // together; a key new to the table then costs one atomic), then adds to the
 // slots that turned out to hold the key already (no-return atomics); only
 // keys that meet another key fall back to probing.
-template <int BS, int LSLOTS>
-__device__ __forceinline__ void lds_agg_flush_packed(const i32* lk, const i64* lv, u64* tab, u32 gmask) {
+template <int BS, int LSLOTS, class AT>
+__device__ __forceinline__ void lds_agg_flush_packed(const i32* lk, const AT* lv, u64* tab, u32 gmask) {
     __syncthreads();
     constexpr int R = LSLOTS / BS;
     i32 key[R];
@@ -106,31 +106,6 @@ __device__ __forceinline__ void lds_agg_flush_packed(const i32* lk, const i64* l
         if (key[r] == EMPTY_KEY || cur[r] == PEMPTY) continue;  // done, or the CAS claimed the slot
         if ((u32)(cur[r] >> 32) == (u32)key[r]) atomicAdd((unsigned long long*)&tab[h[r]], (unsigned long long)w[r]);
         else ptable_add_from(tab, gmask, key[r], w[r], (h[r] + 1) & gmask);
-    }
-}
-
-// Ascending bitonic sort of S (power of two) pairs held in LDS by a block of
-// BS threads.  Must be called by every thread of the block.
-template <int BS>
-__device__ __forceinline__ void bitonic_sort_lds(i32* keys, i64* vals, int S) {
-    for (int k = 2; k <= S; k <<= 1) {
-        for (int j = k >> 1; j > 0; j >>= 1) {
-            for (int i = threadIdx.x; i < S; i += BS) {
-                int ixj = i ^ j;
-                if (ixj > i) {
-                    bool up = (i & k) == 0;
-                    i32 a = keys[i], b = keys[ixj];
-                    if ((a > b) == up) {
-                        keys[i] = b;
-                        keys[ixj] = a;
-                        i64 t = vals[i];
-                        vals[i] = vals[ixj];
-                        vals[ixj] = t;
-                    }
-                }
-            }
-            __syncthreads();
-        }
     }
 }
 

@@ -107,7 +107,6 @@ __host__ __device__ __forceinline__ i64 hub_slices(i64 d, int slots) { return (3
 // four kernels each over class arrays, 8 consecutive vertices per thread and a
 // block scan per class, a plan took 16 launches and 3 waits, now 3 and 1.
 constexpr int ORD_CLS = 3, PL_CLS = ORD_CLS + NCLS, PL_T = 256, PL_I = 8, PL_TILE = PL_T * PL_I, PL_W = PL_T / 64;
-__device__ __forceinline__ int order_class(i64 d) { return d < LARGE_CUTOFF ? 0 : (d < MASSIVE_CUTOFF ? 1 : 2); }
 __global__ void __launch_bounds__(PL_T) k_plan_count(const i64* __restrict__ rp, i64 n, i64 nb, i64* counts) {
     __shared__ int cnt[PL_CLS];
     const i64 b = block_id();
@@ -125,16 +124,6 @@ __global__ void __launch_bounds__(PL_T) k_plan_count(const i64* __restrict__ rp,
     }
     __syncthreads();
     if (threadIdx.x < PL_CLS) counts[(i64)threadIdx.x * nb + b] = cnt[threadIdx.x];
-}
-// lanes of the wave whose 4-bit class equals this lane's
-__device__ __forceinline__ u64 same_class(int cls) {
-    u64 m = ~(u64)0;
-#pragma unroll
-    for (int bit = 0; bit < 4; bit++) {
-        const u64 s = __ballot((cls >> bit) & 1);
-        m &= ((cls >> bit) & 1) ? s : ~s;
-    }
-    return m;
 }
 // offs: exclusive scan of counts; host[0..PL_CLS] = class starts (the scoring
 // classes' from n on)
@@ -284,7 +273,7 @@ void plan_level(Ctx& c, const DGraph& g, LevelPlan& p) {
     // weights small enough for the degrees
     p.agg32 = p.hub32 = g.wk == W_UNIT || g.wsmall;
     if (!p.agg32 && g.nnz > 0) {
-        const u64 mx = max_weight(c, g);
+        const u64 mx = g.wmax ? g.wmax : max_weight(c, g);
         p.agg32 = mx <= 0xffffffffull / HUB_LDS_BOUND;
         p.hub32 = mx <= 0xffffffffull / (u64)std::max(p.max_deg, HUB_LDS_BOUND);
     }

@@ -176,6 +176,7 @@ bool renum_build(Ctx& c, const DGraph& top, Renum& r, bool force) {
     g.wk = top.wk;
     g.vw = r.vw;
     g.wsmall = top.wsmall;
+    g.wmax = top.wmax;
     if (nnz > 0) {
         const int grid = (int)ceil_div(nnz, EC);
         if (top.wk == W_I32) {

@@ -177,4 +177,83 @@ inline i64 compact_flags(Ctx& c, const i32* flag, const i32* src, i64 n, i32* ou
     return select_items(c, SelFlags{flag, src, out}, n)[0];
 }
 
+// Stable partition of [0, n) by class: out receives the items grouped by
+// f(x) in [0, K) (K <= 15), and starts[0..K] the class boundaries (waits).
+// Tiles and runs as in the selections; an item's rank among the lanes of its
+// class comes from a ballot per class bit.
+constexpr int CLS_MAX = 15;
+// lanes of the wave whose 4-bit class equals this lane's
+__device__ __forceinline__ u64 same_class(int cls) {
+    u64 m = ~(u64)0;
+#pragma unroll
+    for (int bit = 0; bit < 4; bit++) {
+        const u64 s = __ballot((cls >> bit) & 1);
+        m &= ((cls >> bit) & 1) ? s : ~s;
+    }
+    return m;
+}
+template <class F>
+__global__ void __launch_bounds__(SEL_T) k_cls_count(F f, i64 n, i64 nb, int K, i64* counts) {
+    __shared__ int cnt[CLS_MAX];
+    const i64 b = block_id();
+    if (b >= nb) return;
+    if (threadIdx.x < CLS_MAX) cnt[threadIdx.x] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < SEL_I; k++) {
+        const i64 x = b * SEL_TILE + k * SEL_T + threadIdx.x;
+        if (x < n) atomicAdd(&cnt[f(x)], 1);
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < K) counts[(i64)threadIdx.x * nb + b] = cnt[threadIdx.x];
+}
+template <class F>
+__global__ void __launch_bounds__(SEL_T) k_cls_write(F f, i64 n, i64 nb, int K, const i64* __restrict__ offs,
+                                                     i32* __restrict__ out, i64* host) {
+    __shared__ int cnt[SEL_I * SEL_W][CLS_MAX + 1];  // class counts of the runs, then their prefix
+    const i64 b = block_id();
+    if (b >= nb) return;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    for (int q = threadIdx.x; q < SEL_I * SEL_W * (CLS_MAX + 1); q += SEL_T) cnt[q / (CLS_MAX + 1)][q % (CLS_MAX + 1)] = 0;
+    __syncthreads();
+    int cl[SEL_I], rk[SEL_I];
+#pragma unroll
+    for (int k = 0; k < SEL_I; k++) {
+        const i64 x = b * SEL_TILE + k * SEL_T + threadIdx.x;
+        cl[k] = x < n ? f(x) : CLS_MAX;
+        const u64 m = same_class(cl[k]);
+        rk[k] = __popcll(m & (((u64)1 << lane) - 1));
+        if (rk[k] == 0) cnt[k * SEL_W + wv][cl[k]] = __popcll(m);
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < K) {
+        int run = 0;
+        for (int q = 0; q < SEL_I * SEL_W; q++) {
+            const int v = cnt[q][threadIdx.x];
+            cnt[q][threadIdx.x] = run;
+            run += v;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < SEL_I; k++) {
+        const i64 x = b * SEL_TILE + k * SEL_T + threadIdx.x;
+        if (x < n) out[offs[(i64)cl[k] * nb + b] + cnt[k * SEL_W + wv][cl[k]] + rk[k]] = (i32)x;
+    }
+    if (b == 0 && (int)threadIdx.x <= K) host[threadIdx.x] = offs[(i64)threadIdx.x * nb];
+}
+template <class F>
+void class_partition(Ctx& c, const F& f, i64 n, int K, i32* out, i64* starts) {
+    if (K > CLS_MAX) throw Error(-5, "class_partition: too many classes");
+    const i64 nb = ceil_div(n > 0 ? n : 1, SEL_TILE);
+    Buf<i64> counts(c, K * nb + 1);
+    k_cls_count<<<grid_blocks(nb), SEL_T, 0, c.stream>>>(f, n, nb, K, counts);
+    PGGC_LAUNCH_CHECK();
+    scan_i64(c, counts, counts, K * nb);
+    k_cls_write<<<grid_blocks(nb), SEL_T, 0, c.stream>>>(f, n, nb, K, counts, out, c.pinned_dev);
+    PGGC_LAUNCH_CHECK();
+    c.sync();
+    for (int k = 0; k <= K; k++) starts[k] = c.pinned[k];
+}
+
 }  // namespace pggc

@@ -1,0 +1,55 @@
+"""Contraction at the edges of its row classes: coarse rows whose bound (the
+summed degrees of their members) is one below, at and one above the sizes of
+the tables in LDS, with spread and with bunched neighbour ids, unit, small and
+31-bit weights, against the oracle, bit for bit."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from pennsylvaniagpugraphclustering_amd import graphs
+
+pytestmark = pytest.mark.gpu
+
+DEGREES = [1, 63, 255, 256, 257, 1023, 1024, 1025, 2047, 2048, 2049, 4095, 4096, 4097, 8191, 8192, 8193, 20000]
+LEAVES = 50000
+
+
+def stars(kind, weights, seed):
+    """One star per degree over shared leaves; leaf 0 belongs to every star,
+    so a bunched star's other leaves fall into one sliver of its id range."""
+    rng = np.random.default_rng(seed)
+    src, dst = [], []
+    for k, d in enumerate(DEGREES):
+        if kind == "spread":
+            leaves = rng.permutation(LEAVES)[:d]
+        else:
+            leaves = np.concatenate([[0], LEAVES - 1 - np.arange(d - 1)])
+        src.append(np.full(d, LEAVES + k))
+        dst.append(leaves)
+    src, dst = np.concatenate(src), np.concatenate(dst)
+    w = None if weights is None else rng.integers(weights[0], weights[1], src.size, endpoint=True)
+    return graphs.from_edges(LEAVES + len(DEGREES), src, dst, w)
+
+
+@pytest.mark.parametrize("weights", [None, (1, 50), (2 ** 30, 2 ** 31 - 1)])
+@pytest.mark.parametrize("kind", ["spread", "bunched"])
+@pytest.mark.parametrize("leaf_groups", [0, 700])
+def test_rows_at_table_sizes(gpu_ctx, kind, weights, leaf_groups):
+    """leaf_groups 0: every vertex stays alone (each star's row is its bound
+    long); otherwise the leaves fall into that many clusters, whose rows merge
+    the stars' edges from many members."""
+    from pennsylvaniagpugraphclustering_amd import clustering as C
+    g = stars(kind, weights, 3)
+    vc = np.arange(g.n, dtype=np.int32)
+    nc = g.n
+    if leaf_groups:
+        vc[:LEAVES] = np.random.default_rng(4).integers(0, leaf_groups, LEAVES)
+        vc[LEAVES:] = leaf_groups + np.arange(len(DEGREES))
+        nc = leaf_groups + len(DEGREES)
+    print(f"contract stars {kind} w={weights} groups={leaf_groups}", flush=True)
+    dg = C.DeviceGraph.from_csr(g, "Mod" if weights is None else "WMod")
+    rp, col, w = C.build_coarse_graph(dg, vc, nc)
+    rrp, rcol, rw = O.contract(g.rp, g.col, g.w, vc, nc)
+    assert np.array_equal(rp.cpu().numpy(), rrp)
+    assert np.array_equal(col.cpu().numpy(), rcol)
+    assert np.array_equal(w.cpu().numpy(), rw)
