@@ -47,15 +47,18 @@ struct Error : std::runtime_error {
 // Edge-weight accessors: unit (uniform graphs), int32 (input graphs) and
 // int64 (coarse graphs, whose summed weights can exceed int32).
 struct WUnit {
+    using value = signed char;  // an edge's weight as stored
     static constexpr int bytes = 0;  // weight bytes read per edge
     __device__ __forceinline__ i64 operator()(i64) const { return 1; }
 };
 struct W32 {
+    using value = i32;
     static constexpr int bytes = 4;
     const i32* p;
     __device__ __forceinline__ i64 operator()(i64 j) const { return p[j]; }
 };
 struct W64 {
+    using value = i64;
     static constexpr int bytes = 8;
     const i64* p;
     __device__ __forceinline__ i64 operator()(i64 j) const { return p[j]; }

@@ -133,16 +133,33 @@ __device__ __forceinline__ i64 advance_row(const i64* rp, i64 r, i64 rhi, i64 j,
 // monotone row pointer (per-row partial sums then go out with atomics).
 constexpr int EB = 256, EPT = 16, EC = EB * EPT;
 
+// upper_row searched by a whole wave, 64 probes a step: 4 dependent loads
+// instead of 23 for 8M rows (rp[lo] <= j on entry)
+__device__ __forceinline__ i64 wave_upper_row(const i64* rp, i64 lo, i64 hi, i64 j) {
+    const int lane = threadIdx.x & 63;
+    while (hi - lo > 1) {  // wave-uniform loop control
+        const i64 step = (hi - lo + 63) / 64, p = lo + lane * step;
+        i32 in = p < hi && rp[p] <= j ? 1 : 0;  // true for a prefix of the lanes, lane 0 among them
+        xlane_fence(in);
+        const i64 k = 63 - __clzll((long long)__ballot(in != 0));
+        lo += k * step;
+        hi = lo + step < hi ? lo + step : hi;
+    }
+    return lo;
+}
+
 struct ChunkRows {
     i64 eb, ee, rlo, rhi;
 };
+template <int E = EC>
 __device__ __forceinline__ void chunk_rows(const i64* rp, i64 n, i64 nnz, ChunkRows& cr) {
     __shared__ i64 s_lo, s_hi;
-    cr.eb = (i64)blockIdx.x * EC;
-    cr.ee = cr.eb + EC < nnz ? cr.eb + EC : nnz;
-    if (threadIdx.x == 0) {
-        s_lo = upper_row(rp, 0, n, cr.eb);
-        s_hi = upper_row(rp, 0, n, cr.ee - 1) + 1;
+    cr.eb = (i64)blockIdx.x * E;
+    cr.ee = cr.eb + E < nnz ? cr.eb + E : nnz;
+    if (threadIdx.x < 128) {  // one end per wave
+        const i64 r = wave_upper_row(rp, 0, n, threadIdx.x < 64 ? cr.eb : cr.ee - 1);
+        if (threadIdx.x == 0) s_lo = r;
+        if (threadIdx.x == 64) s_hi = r + 1;
     }
     __syncthreads();
     cr.rlo = s_lo;

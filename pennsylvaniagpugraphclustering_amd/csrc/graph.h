@@ -2,6 +2,7 @@
 // contraction, and the device-resident coarse graph type.
 #pragma once
 #include "ctx.h"
+#include "device.h"
 
 namespace pggc {
 
@@ -36,6 +37,77 @@ struct OwnedGraph {
 };
 
 // Stable degree bucketing (src/ordering.cpp:131-164).
+// out[r] += the weights of row r's edges whose neighbour passes Pass()(key[r],
+// key[neighbour]); out is zeroed by the caller, sums are exact integers.
+//
+// A block takes RS_E consecutive edges.  The gathers of the neighbours' keys
+// bound it: columns, weights and keys are loaded by consecutive lanes, RS_T of
+// each in flight per thread, and staged in LDS; every thread then walks RS_T
+// consecutive edges with a row pointer.  Row sums meet in LDS, where a row that lies
+// within the chunk is written with a plain store (rows cut by the chunk's ends,
+// and chunks of more than RS_R rows, add with atomics).  With each thread
+// loading its own consecutive edges and one atomic per thread and row, the weights of
+// the own clusters of an LFR graph (8.4M vertices, 160M nonzeros) took 4.6 ms;
+// 2.65 now.
+constexpr int RS_T = 8, RS_E = 256 * RS_T, RS_R = 1024;
+template <class Pass, class KT, class WT>
+__global__ void __launch_bounds__(256) k_row_sums(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
+                                                  const KT* __restrict__ key, i64 n, i64 nnz, i64* out) {
+    __shared__ KT sk[RS_E + RS_E / RS_T];  // one pad per thread: its entries start in a bank of their own
+    __shared__ typename WT::value sw[RS_E + RS_E / RS_T];
+    __shared__ i64 acc[RS_R];
+    ChunkRows cr;
+    chunk_rows<RS_E>(rp, n, nnz, cr);
+    const int t = threadIdx.x;
+    const i64 nr = cr.rhi - cr.rlo;
+    const bool local = nr <= RS_R;
+    i32 v[RS_T];
+#pragma unroll
+    for (int q = 0; q < RS_T; q++) {
+        const i64 j = cr.eb + q * 256 + t;
+        v[q] = j < cr.ee ? col[j] : 0;
+    }
+#pragma unroll
+    for (int q = 0; q < RS_T; q++) {
+        const int o = q * 256 + t;
+        const i64 j = cr.eb + o;
+        sk[o + o / RS_T] = key[v[q]];
+        if (WT::bytes) sw[o + o / RS_T] = j < cr.ee ? (typename WT::value)W(j) : 0;
+    }
+    for (int q = t; q < (local ? (int)nr : 0); q += 256) acc[q] = 0;
+    __syncthreads();
+    const i64 j0 = cr.eb + (i64)t * RS_T;
+    if (j0 < cr.ee) {
+        i64 r = upper_row(rp, cr.rlo, cr.rhi, j0);
+        i64 nxt = rp[r + 1];
+        KT mine = key[r];
+        i64 a = 0;
+#pragma unroll
+        for (int q = 0; q < RS_T; q++) {
+            const i64 j = j0 + q;
+            if (j >= cr.ee) break;
+            if (j >= nxt) {
+                if (a) atomicAdd((unsigned long long*)(local ? &acc[r - cr.rlo] : &out[r]), (unsigned long long)a);
+                a = 0;
+                r = advance_row(rp, r, cr.rhi, j, nxt);
+                mine = key[r];
+            }
+            const int o = t * (RS_T + 1) + q;
+            if (Pass()(mine, sk[o])) a += WT::bytes ? (i64)sw[o] : 1;
+        }
+        if (a) atomicAdd((unsigned long long*)(local ? &acc[r - cr.rlo] : &out[r]), (unsigned long long)a);
+    }
+    if (!local) return;  // block-uniform
+    __syncthreads();
+    for (int q = t; q < (int)nr; q += 256) {
+        const i64 a = acc[q];
+        if (a == 0) continue;
+        // only the first and the last row can reach beyond the chunk
+        if (q == 0 || q == (int)nr - 1) atomicAdd((unsigned long long*)&out[cr.rlo + q], (unsigned long long)a);
+        else out[cr.rlo + q] = a;
+    }
+}
+
 __device__ __forceinline__ int order_class(i64 d) { return d < LARGE_CUTOFF ? 0 : (d < MASSIVE_CUTOFF ? 1 : 2); }
 struct Orders {
     Buf<i32> o1, o2;

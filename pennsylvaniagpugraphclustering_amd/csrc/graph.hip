@@ -94,36 +94,14 @@ void evaluate(Ctx& c, const DGraph& g, const i32* labels, i64 L, i64* vol, i64* 
     }
 }
 
-template <class WT>
-__global__ void __launch_bounds__(EB) k_own_weight(const i64* rp, const i32* col, WT W, const i32* lab, i64 n,
-                                                    i64 nnz, i64* out) {
-    ChunkRows cr;
-    chunk_rows(rp, n, nnz, cr);
-    i64 j0 = cr.eb + (i64)threadIdx.x * EPT;
-    if (j0 >= cr.ee) return;
-    i64 r = upper_row(rp, cr.rlo, cr.rhi, j0);
-    i64 nxt = rp[r + 1];
-    i32 lr = lab[r];
-    i64 acc = 0;
-    for (int k = 0; k < EPT; k++) {
-        i64 j = j0 + k;
-        if (j >= cr.ee) break;
-        if (j >= nxt) {
-            if (acc) atomicAdd((unsigned long long*)&out[r], (unsigned long long)acc);
-            acc = 0;
-            r = advance_row(rp, r, cr.rhi, j, nxt);
-            lr = lab[r];
-        }
-        if (lab[col[j]] == lr) acc += W(j);
-    }
-    if (acc) atomicAdd((unsigned long long*)&out[r], (unsigned long long)acc);
-}
-
+struct SameLabel {
+    __device__ __forceinline__ bool operator()(i32 mine, i32 other) const { return mine == other; }
+};
 void own_weight(Ctx& c, const DGraph& g, const i32* labels, i64* out) {
     fill_i64(c, out, g.n, 0);
     if (g.nnz == 0) return;
-    PGGC_WDISPATCH(g, (k_own_weight<<<(int)ceil_div(g.nnz, EC), EB, 0, c.stream>>>(g.rp, g.col, W, labels, g.n,
-                                                                                   g.nnz, out)));
+    PGGC_WDISPATCH(g, (k_row_sums<SameLabel><<<(int)ceil_div(g.nnz, RS_E), 256, 0, c.stream>>>(g.rp, g.col, W, labels,
+                                                                                              g.n, g.nnz, out)));
     PGGC_LAUNCH_CHECK();
 }
 
