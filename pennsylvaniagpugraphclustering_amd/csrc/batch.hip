@@ -102,8 +102,8 @@ static std::vector<i64> read_offsets(Ctx& c, const i64* rp, const BatchLevel& bl
     k_at_offsets<<<grid_items(K1, 256), 256, 0, c.stream>>>(K1, rp, bl.dvoff, d);
     PGGC_LAUNCH_CHECK();
     std::vector<i64> e(K1);
-    PGGC_HIP(hipMemcpyAsync(e.data(), d.p, K1 * sizeof(i64), hipMemcpyDeviceToHost, c.stream));
-    c.sync();
+    const Fetch f = fetch(e, d.p, K1);
+    copy_d2h(c, &f, 1);
     return e;
 }
 

@@ -56,9 +56,12 @@ struct Ctx {
     size_t bytes_live = 0, bytes_cached = 0;
     i64* pinned = nullptr;      // 64 pinned int64 readback slots
     i64* pinned_dev = nullptr;  // the same slots as seen from the device
-    void* stage = nullptr;      // pinned coherent staging area for uploads
-    void* stage_dev = nullptr;
-    size_t stage_cap = 0;
+    // pinned coherent staging area for small copies between host and device: a
+    // copy takes the next bytes of it and needs no wait of its own; a wait for the
+    // stream frees all of it
+    char* stage = nullptr;
+    char* stage_dev = nullptr;  // the same bytes as seen from the device
+    size_t stage_cap = 0, stage_off = 0;
     u64 seed = 0;           // leidenR seed stream
     u64 draws = 0;
     int verbose = 0;        // >0: per-iteration progress lines on stderr; >=2: memory by stage
@@ -111,7 +114,12 @@ struct Ctx {
     size_t cache_keep = 0;
     size_t mem_total = 0;  // of the device
     void trim_large();
-    void sync() { PGGC_HIP(hipStreamSynchronize(stream)); }
+    void sync() {
+        PGGC_HIP(hipStreamSynchronize(stream));
+        stage_off = 0;
+    }
+    // `bytes` of the staging area (waits when it is full)
+    char* stage_take(size_t bytes, char** dev);
     // copy `count` int64 device values to the pinned slots and wait
     const i64* read(const i64* dev, int count);
     i64 read1(const i64* dev) { return read(dev, 1)[0]; }
@@ -171,7 +179,21 @@ void copy_dev(Ctx& c, void* dst, const void* src, size_t bytes);  // on c.stream
 // host -> device copy, done when it returns: the bytes go through a pinned
 // coherent staging area and a copy kernel on the stream, so later kernels
 // read them through the same cache path as data written by kernels
+// Host to device in stream order; src may be changed at once.
 void copy_h2d(Ctx& c, void* dst, const void* src, size_t bytes);
+// Device to host, for several arrays with one wait: count values of each src
+// into dst.
+struct Fetch {
+    void* dst;
+    const void* src;
+    size_t bytes;
+};
+void copy_d2h(Ctx& c, const Fetch* f, int nf);
+template <class T>
+inline Fetch fetch(std::vector<T>& dst, const T* src, size_t count) {
+    dst.resize(count);
+    return Fetch{dst.data(), src, count * sizeof(T)};
+}
 // out[0..n] = exclusive scan of in[0..n); out[n] = total.  in may alias out.
 void scan_i64(Ctx& c, const i64* in, i64* out, i64 n);
 void scan_i32_to_i64(Ctx& c, const i32* in, i64* out, i64 n);

@@ -691,6 +691,7 @@ void Gnn::set_params(Ctx& c, const float* host) {
     for (int k = 0; k < GNN_IN * GNN_HID; k++) wb[k] = bf16_rne(host[GP_W1 + k]);
     copy_h2d(c, prm.p, host, GNN_P * sizeof(float));
     copy_h2d(c, w1b.p, wb.data(), wb.size() * sizeof(u16));
+    c.sync();  // (other streams may read them)
     fill_i32(c, (i32*)m1.p, GNN_P, 0);
     fill_i32(c, (i32*)m2.p, GNN_P, 0);
     c.sync();

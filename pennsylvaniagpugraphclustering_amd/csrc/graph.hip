@@ -707,12 +707,6 @@ static void contract_bytes(Ctx& c, int tk, const i32* list, i64 m, const i64* ms
 }
 
 
-static void download_i64(Ctx& c, std::vector<i64>& dst, const i64* src, i64 count) {
-    dst.resize((size_t)count);
-    c.sync();
-    PGGC_HIP(hipMemcpy(dst.data(), src, (size_t)count * sizeof(i64), hipMemcpyDeviceToHost));
-}
-
 static int bits_for(i64 v) {
     int b = 0;
     while (b < 62 && ((i64)1 << b) <= v) b++;
@@ -820,9 +814,8 @@ static void contract_t(Ctx& c, const DGraph& g, const i32* vcmap, i64 nc, OwnedG
         // memory stays bounded on graphs of billions of edges
         const i64 slot_cap = std::max<i64>(c.contract_batch, 1);
         std::vector<i64> hg, hi, hi2;
-        download_i64(c, hg, goff, n2 + 1);
-        download_i64(c, hi, items, n2 + 1);
-        download_i64(c, hi2, items2, n2 + 1);
+        const Fetch f[3] = {fetch(hg, goff.p, n2 + 1), fetch(hi, items.p, n2 + 1), fetch(hi2, items2.p, n2 + 1)};
+        copy_d2h(c, f, 3);
         Buf<i32> row(c, std::max<i64>(hi[n2], 1));
         k_item_rows<<<grid_blocks(n2), 256, 0, c.stream>>>(items, n2, row);
         PGGC_LAUNCH_CHECK();
@@ -889,7 +882,8 @@ static void contract_t(Ctx& c, const DGraph& g, const i32* vcmap, i64 nc, OwnedG
         PGGC_LAUNCH_CHECK();
         scan_i64(c, boff, boff, n2);
         std::vector<i64> hb;
-        download_i64(c, hb, boff, n2 + 1);
+        const Fetch f = fetch(hb, boff.p, n2 + 1);
+        copy_d2h(c, &f, 1);
         i64 emax = 0;
         const std::vector<i64> cuts = batch_cuts(hb, sort_cap, &emax);
         if (emax > 0) {

@@ -2427,10 +2427,8 @@ static void upload(Ctx& c, T* dst, const std::vector<T>& src) {
 }
 template <class T>
 static void download(Ctx& c, std::vector<T>& dst, const T* src, size_t count) {
-    dst.resize(count);
-    if (count == 0) return;
-    PGGC_HIP(hipMemcpyAsync(dst.data(), src, count * sizeof(T), hipMemcpyDeviceToHost, c.stream));
-    c.sync();
+    const Fetch f = fetch(dst, src, count);
+    copy_d2h(c, &f, 1);
 }
 
 // Per-instance sums.  A list holds long runs of one instance (instances own
@@ -2604,8 +2602,8 @@ static void set_new_cluster_ids_batch(Ctx& c, MoveScratch& s, const DGraph& g, c
         radix_sort_pairs(c, keys, s.tmp.p, KN, bits);
     }
     std::vector<i64> ha, hk;
-    download(c, ha, acnt.p, K);
-    download(c, hk, kcnt.p, K);
+    const Fetch f[2] = {fetch(ha, acnt.p, K), fetch(hk, kcnt.p, K)};
+    copy_d2h(c, f, 2);
     std::vector<i64> us(K), ns(K);
     i64 u0 = 0, n0 = 0;
     for (i64 q = 0; q < K; q++) {
@@ -2755,8 +2753,8 @@ void local_move_batch(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, co
             upload(c, imp.p, himp);
             k_inst_sumsq<<<grid_blocks(K), 256, 0, c.stream>>>(cvol, best.dloff, Ld, imp, K, sq);
             PGGC_LAUNCH_CHECK();
-            download(c, hacc, acc.p, K);
-            download(c, hsq, sq.p, 2 * K);
+            const Fetch f[2] = {fetch(hacc, acc.p, K), fetch(hsq, sq.p, 2 * K)};
+            copy_d2h(c, f, 2);
             bool anyimp = false;
             for (i64 q = 0; q < K; q++) {
                 const bool moved = himp[q] != 0;
