@@ -74,10 +74,13 @@ __host__ __device__ __forceinline__ int score_class(i64 d) {
 }
 // small levels, bound by launches (direct_sweep)
 constexpr i64 DIRECT_MAX = (i64)1 << 18, DIRECT_NNZ = (i64)1 << 22;
-// Level of at most this many rows in the LDS-table classes: one launch for all
-// (the chip holds 5 of its 256-thread blocks per CU, 1,280 at once, so two
-// rounds of blocks cost less than the four launches saved).
-constexpr i64 TABLE_ONE_LAUNCH = 2048;
+// Level of at most this many rows of degree 65 to 2048: one launch for their
+// five classes (the chip holds 5 of its 256-thread blocks per CU, 1,280 at once; a
+// class of its own takes 5 to 9 us of a launch's latency however few its rows).
+// At 2,048 rows, and only without longer ones, a CPM run of 30,011 vertices took 2.94
+// ms, 2.70 now, weighted pLeiden+ on R-MAT scale 17 28.7, 27.3 now; at the 12,000 to
+// 200,000 rows of R-MAT scale 22's levels the classes' own widths are better.
+constexpr i64 TABLE_ONE_LAUNCH = 8192;
 // LDS table of a vertex of degree d: the power of two >= spe * d slots, at most
 // `most`
 __host__ __device__ __forceinline__ int tslots(i64 d, int spe, int most) {
@@ -1095,12 +1098,11 @@ static void launch_groups(Ctx& c, const DGraph& g, WT W, const ScoreArgs<LT>& a,
 template <class AT, class WT, class LT>
 static void launch_tables(Ctx& c, const LevelPlan& lp, const DGraph& g, WT W, const ScoreArgs<LT>& a) {
     const i64* st = lp.sc_start;
-    // few rows: one launch for all classes (the widest block), as launches
-    // then cost more than the lower occupancy
-    if (lp.hub0 - st[CL_TABLE] <= TABLE_ONE_LAUNCH && lp.hub0 == st[CL_HUB]) {
-        launch_table<AT, 256, 2048, 4096, 2>(c, g, W, a, st[CL_TABLE], st[CL_HUB]);
-        return;
-    }
+    const bool one = st[CL_HUB] - st[CL_TABLE] <= TABLE_ONE_LAUNCH;
+    if (one) launch_table<AT, 256, 2048, 4096, 2>(c, g, W, a, st[CL_TABLE], st[CL_HUB]);
+    launch_table<AT, 1024, HUB_HALF, 8192, 2>(c, g, W, a, st[CL_HUB], st[CL_HUB] + lp.nhalf);
+    launch_table<AT, 1024, HUB_LDS_BOUND, HUB_LDS_SLOTS, 2>(c, g, W, a, st[CL_HUB] + lp.nhalf, lp.hub0);
+    if (one) return;
     // LDS tables sized for the class, so the many low-degree rows keep more
     // waves resident per CU; threads per vertex and slots per edge are knobs
     launch_table_class<AT, 128>(c, g, W, a, st[5], st[6]);
@@ -1113,8 +1115,6 @@ static void launch_tables(Ctx& c, const LevelPlan& lp, const DGraph& g, WT W, co
         launch_table<AT, 256, 1024, 4096, 4>(c, g, W, a, st[8], st[9]);
         launch_table<AT, 512, 2048, 8192, 4>(c, g, W, a, st[9], st[10]);
     }
-    launch_table<AT, 1024, HUB_HALF, 8192, 2>(c, g, W, a, st[CL_HUB], st[CL_HUB] + lp.nhalf);
-    launch_table<AT, 1024, HUB_LDS_BOUND, HUB_LDS_SLOTS, 2>(c, g, W, a, st[CL_HUB] + lp.nhalf, lp.hub0);
 }
 
 template <class LT>
