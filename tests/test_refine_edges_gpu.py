@@ -31,14 +31,11 @@ def edge_graph(gap, wmax):
     return graphs.from_edges(n, ids[src], ids[dst], w)
 
 
-@pytest.mark.parametrize("wide", [False, True])
-@pytest.mark.parametrize("wmax", [None, 30])
+@pytest.mark.parametrize("wmax,wide", [(None, False), (30, False), (30, True)])
 @pytest.mark.parametrize("gap", [1, 40])
 def test_refine_at_tile_edges(gpu_ctx, gap, wmax, wide):
     from pennsylvaniagpugraphclustering_amd import clustering as C
     from tests.test_gpu_parity import dgraph, npy, weights_for
-    if wide and wmax is None:
-        pytest.skip("unit weights have one width")
     g = edge_graph(gap, wmax)
     obj = "Mod" if wmax is None else "WMod"
     w = weights_for(g, obj)
