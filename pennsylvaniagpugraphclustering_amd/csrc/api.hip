@@ -170,22 +170,26 @@ constexpr int LEIDEN_MAX_STALLS = 8;
 // pays (renum_build) or the call makes several top-level passes (reuse) with
 // it at 2 (the default), never at 0 or with the active-set predictor on, whose
 // features follow the vertex order.
+// Copies that no knob or reuse asks for hold at most RN_MEM of the device's
+// memory: a top level's copy, and those of a run's coarse levels together.  On
+// graphs of billions of edges the finer levels go without, as their hierarchy
+// takes most of the memory.
+constexpr double RN_MEM = 1.0 / 16;
+static double renum_bytes(const DGraph& g) { return 32.0 * g.n + (g.wk == W_I64 ? 12.0 : 8.0) * g.nnz; }
 static Renum* top_renum(Ctx& c, MoveScratch& ms, const DGraph& g, Renum& r, bool reuse) {
     if (c.renumber == 0 || (ms.gnn && ms.gnn->cfg.mode != GNN_OFF)) return nullptr;
-    return renum_build(c, g, r, c.renumber == 1 || reuse) ? &r : nullptr;
+    const bool force = c.renumber == 1 || reuse;
+    if (!force && renum_bytes(g) > RN_MEM * (double)c.mem_total) return nullptr;
+    return renum_build(c, g, r, force) ? &r : nullptr;
 }
-// The same for a coarse level, built once and kept for the way back up.  The
-// copies of a run hold at most RN_MEM of the device's memory together: on
-// graphs of billions of edges the finer levels go without.
-constexpr double RN_MEM = 1.0 / 8;
+// The same for a coarse level, built once and kept for the way back up.
 static Renum* coarse_renum(Ctx& c, MoveScratch& ms, std::vector<Level>& levels, size_t li) {
     Level& l = levels[li];
     if (c.renumber == 0 || (ms.gnn && ms.gnn->cfg.mode != GNN_OFF)) return nullptr;
     if (!l.rn) {
-        auto bytes = [](const DGraph& g) { return 32.0 * g.n + (g.wk == W_I64 ? 12.0 : 8.0) * g.nnz; };
-        double held = bytes(l.g);
+        double held = renum_bytes(l.g);
         for (size_t k = 0; k < li; k++)
-            if (levels[k].rn && levels[k].rn->copied) held += bytes(levels[k].g);
+            if (levels[k].rn && levels[k].rn->copied) held += renum_bytes(levels[k].g);
         l.rn.reset(new Renum());
         if (held <= RN_MEM * (double)c.mem_total) renum_build(c, l.g, *l.rn, c.renumber == 1);
     }
