@@ -991,16 +991,13 @@ int pggc_contract(pggc_ctx* ctx, const pggc_graph* gg, const int32_t* vcmap, int
         if (nc < 0) throw Error(PGGC_EINVAL, "negative cluster count");
         Ctx& c = ctx->c;
         OwnedGraph og;
-        contract(c, g, vcmap, nc, og, true);
+        const ContractTo to{out_col, out_w, cap};
+        contract(c, g, vcmap, nc, og, &to);
         *nnz_out = og.nnz;
         copy_dev(c, out_rp, og.rp, (nc + 1) * sizeof(i64));
         if (og.nnz > cap) {
             c.sync();
             throw Error(PGGC_ECAPACITY, "coarse nnz exceeds output capacity");
-        }
-        if (og.nnz > 0) {
-            copy_dev(c, out_col, og.col, og.nnz * sizeof(i32));
-            copy_dev(c, out_w, og.w, og.nnz * sizeof(i64));
         }
         c.sync();
     });

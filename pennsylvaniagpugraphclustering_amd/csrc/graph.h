@@ -126,9 +126,17 @@ void own_weight(Ctx& c, const DGraph& g, const i32* labels, i64* out);
 // weights are int32 when every one fits (the values, and so every result, are
 // the same; the sweeps read 4 instead of 8 weight bytes per edge and the level
 // holds 8 instead of 12 bytes per nonzero) and int64 otherwise, or always with
-// want64: when the finer level's weights sum to less than 2^31 they are written
+// `to`: when the finer level's weights sum to less than 2^31 they are written
 // as int32 at once, else after a max reduction.
-void contract(Ctx& c, const DGraph& g, const i32* vcmap, i64 nc, OwnedGraph& out, bool want64 = false);
+// With `to` the columns and int64 weights go to the caller's arrays instead of
+// out's (nothing is written there when they do not fit cap); the copy from out's
+// took 0.4 of 7.0 ms for 100M coarse nonzeros.
+struct ContractTo {
+    i32* col;
+    i64* w;
+    i64 cap;
+};
+void contract(Ctx& c, const DGraph& g, const i32* vcmap, i64 nc, OwnedGraph& out, const ContractTo* to = nullptr);
 
 // largest weight of g as an unsigned value (a negative weight is huge); g.nnz > 0
 u64 max_weight(Ctx& c, const DGraph& g);

@@ -266,7 +266,7 @@ constexpr i32 C_FAT = 96;  // largest bucket that is ranked by comparing every p
 // gather in flight, 64-bit sums and a bitonic sort of the whole table (66
 // barriers for 2,048 slots); rows up to 8192 take 2.05 ms now, and the rows
 // above, which alone are merged in HBM and sorted there, 1.5 + 1.6 ms (from 4.6
-// + 3.5, and 14.8 -> 7.1 ms for the whole call).
+// + 3.5, and 14.8 -> 6.6 ms for the whole call).
 template <int BS, int D, int SLOTS, class AT, class TT, class WT>
 __global__ void __launch_bounds__(BS) k_cagg(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
                                               const i32* __restrict__ vcmap, i64 nc, const i32* __restrict__ list,
@@ -752,9 +752,10 @@ static void narrow_weights(Ctx& c, OwnedGraph& g) {
 }
 
 // AT: sums of rows merged in LDS; TT: staged weights; OT: weights written to
-// `ow` (out.w or out.w32, allocated here)
+// `ow` (out.w or out.w32, allocated here), or int64 ones to the caller's arrays
 template <class AT, class TT, class OT>
-static void contract_t(Ctx& c, const DGraph& g, const i32* vcmap, i64 nc, OwnedGraph& out, Buf<OT>& ow) {
+static void contract_t(Ctx& c, const DGraph& g, const i32* vcmap, i64 nc, OwnedGraph& out, Buf<OT>& ow,
+                       const ContractTo* to) {
     const i64 n = g.n;
     // member counts, bounds and coarse degrees, zeroed by one launch
     Buf<i64> zero(c, 3 * (nc + 1)), mstart(c, nc + 1), toff(c, nc + 1);
@@ -858,15 +859,25 @@ static void contract_t(Ctx& c, const DGraph& g, const i32* vcmap, i64 nc, OwnedG
     out.rp = Buf<i64>(c, nc + 1);
     scan_i64(c, ccnt, out.rp, nc);
     out.nnz = c.read1(out.rp.p + nc);
-    out.col = Buf<i32>(c, std::max<i64>(out.nnz, 1));
-    ow = Buf<OT>(c, std::max<i64>(out.nnz, 1));
+    i32* ocol;
+    OT* owt;
+    if (to) {
+        if (out.nnz > to->cap) return;
+        ocol = to->col;
+        owt = (OT*)(void*)to->w;  // (OT is i64)
+    } else {
+        out.col = Buf<i32>(c, std::max<i64>(out.nnz, 1));
+        ow = Buf<OT>(c, std::max<i64>(out.nnz, 1));
+        ocol = out.col;
+        owt = ow;
+    }
     if (out.nnz > 0) {
         // algorithmic bytes: coarse offsets, row starts in the temporary rows,
         // (column, weight) read and written once
         const double bytes = 16.0 * (nc + 1) + (8.0 + sizeof(TT) + sizeof(OT)) * out.nnz;
         const int tkc = c.kt_begin(KS_CONTRACT_COPY);
-        k_crow_copy<<<(int)ceil_div(out.nnz, EC), EB, 0, c.stream>>>(out.rp, nc, out.nnz, toff, tcol, tw.p, out.col,
-                                                                   ow.p);
+        k_crow_copy<<<(int)ceil_div(out.nnz, EC), EB, 0, c.stream>>>(out.rp, nc, out.nnz, toff, tcol, tw.p, ocol,
+                                                                   owt);
         c.kt_end(tkc, bytes);
         PGGC_LAUNCH_CHECK();
     }
@@ -895,34 +906,34 @@ static void contract_t(Ctx& c, const DGraph& g, const i32* vcmap, i64 nc, OwnedG
                 const i64 r0 = cuts[q], r1 = cuts[q + 1], E = hb[r1] - hb[r0];
                 if (E == 0) continue;
                 k_big_flatten<<<grid_blocks(r1 - r0), 256, 0, c.stream>>>(big + r0, r1 - r0, out.rp, boff.p + r0,
-                                                                          out.col, ow.p, cb, key, val.p, target);
+                                                                          ocol, owt, cb, key, val.p, target);
                 PGGC_LAUNCH_CHECK();
                 radix_sort_pairs(c, key, val.p, E, cb + bits_for(r1 - r0));
-                k_big_scatter<<<grid_for(E, 256 * 4, 8192), 256, 0, c.stream>>>(key, target, E, val.p, cb, out.col,
-                                                                                ow.p);
+                k_big_scatter<<<grid_for(E, 256 * 4, 8192), 256, 0, c.stream>>>(key, target, E, val.p, cb, ocol,
+                                                                                owt);
                 PGGC_LAUNCH_CHECK();
             }
         }
     }
 }
 
-void contract(Ctx& c, const DGraph& g, const i32* vcmap, i64 nc, OwnedGraph& out, bool want64) {
+void contract(Ctx& c, const DGraph& g, const i32* vcmap, i64 nc, OwnedGraph& out, const ContractTo* to) {
     // all weights together below 2^31: every coarse weight and sum fits 32 bits
     const u64 top = (u64)1 << 31;
     const bool small = g.wsmall || (g.wk == W_UNIT ? (u64)g.nnz < top
                                                    : g.wmax > 0 && g.wmax < top && (u64)g.nnz * g.wmax < top);
-    if (small && !want64) {
-        contract_t<u32, i32>(c, g, vcmap, nc, out, out.w32);
+    if (small && !to) {
+        contract_t<u32, i32>(c, g, vcmap, nc, out, out.w32, nullptr);
         return;
     }
     if (small) {
-        contract_t<u32, i32>(c, g, vcmap, nc, out, out.w);
+        contract_t<u32, i32>(c, g, vcmap, nc, out, out.w, to);
     } else {
         // 32-bit sums in LDS when the weights are small enough for C_TOP of them
         const u64 mx = g.wk == W_UNIT ? 1 : g.wmax ? g.wmax : g.nnz > 0 ? max_weight(c, g) : 1;
-        if (mx <= 0xffffffffull / C_TOP) contract_t<u32, i64>(c, g, vcmap, nc, out, out.w);
-        else contract_t<i64, i64>(c, g, vcmap, nc, out, out.w);
-        if (!want64) narrow_weights(c, out);
+        if (mx <= 0xffffffffull / C_TOP) contract_t<u32, i64>(c, g, vcmap, nc, out, out.w, to);
+        else contract_t<i64, i64>(c, g, vcmap, nc, out, out.w, to);
+        if (!to) narrow_weights(c, out);
     }
 }
 
