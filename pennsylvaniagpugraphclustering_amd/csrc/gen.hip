@@ -105,6 +105,7 @@ __device__ __forceinline__ bool uniq_flag(const u64* keys, i64 x, u64 invalid) {
 
 __global__ void __launch_bounds__(UT) k_uniq_sums(const u64* __restrict__ keys, i64 m, u64 invalid, i64* bsum) {
     const i64 base = block_id() * UTILE;
+    if (base >= m) return;  // a padded grid has more blocks than tiles
     i64 s = 0;
     for (int k = 0; k < UI; k++) {
         const i64 x = base + (i64)k * UT + threadIdx.x;
@@ -124,6 +125,7 @@ __global__ void __launch_bounds__(UT) k_uniq_write(const u64* __restrict__ keys,
     constexpr int NW = UT / 64;
     __shared__ int cnt[UI * NW];
     const i64 base = block_id() * UTILE;
+    if (base >= m) return;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     u64 bal[UI];
 #pragma unroll

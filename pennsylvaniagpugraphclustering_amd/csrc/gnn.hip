@@ -71,6 +71,7 @@ __global__ void __launch_bounds__(256) k_gnn_pack(i64 n, const i64* __restrict__
                                                   const i32* __restrict__ dest, const float* __restrict__ gain,
                                                   const i32* __restrict__ stamp, i32 cur, int first,
                                                   u64* __restrict__ pk, i64* __restrict__ blk) {
+    if (block_id() * 256 >= n) return;  // a padded grid has more blocks than blk has entries
     const i64 i = thread_item();
     i64 a = 0;
     if (i < n) {
@@ -89,6 +90,7 @@ __global__ void __launch_bounds__(256) k_gnn_pack(i64 n, const i64* __restrict__
 
 // blk[block] = vertices with flag[i] == v (v != 0) or, for v == 0, flag[i] != 0
 __global__ void __launch_bounds__(256) k_gnn_count(i64 n, const i32* __restrict__ flag, i32 v, i64* __restrict__ blk) {
+    if (block_id() * 256 >= n) return;
     const i64 i = thread_item();
     const i64 a = (i < n && (v ? flag[i] == v : flag[i] != 0)) ? 1 : 0;
     const i64 s = block_sum_i64<256>(a);
@@ -627,6 +629,7 @@ __global__ void k_gnn_stamp(const i32* moves, i64 k, i32* stamp, i32 cur) {
 }
 
 __global__ void __launch_bounds__(256) k_gnn_restore(i64 n, i32* pruned, i32* dest, i64* blk) {
+    if (block_id() * 256 >= n) return;
     const i64 i = thread_item();
     i64 a = 0;
     if (i < n && pruned[i]) {
