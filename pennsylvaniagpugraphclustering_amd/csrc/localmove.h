@@ -46,13 +46,14 @@ struct LevelPlan {
     i64 sc_start[NCLS + 1] = {0};
     // hubs (the class above 2048, sorted by degree): the first nlds of them
     // (degree <= 8192; the first nhalf <= 4096) are scored from LDS tables like
-    // the smaller classes, the others (from list entry hub0 on) by one block
-    // per slice of their clusters' hash range: hub_groups is the slice prefix
-    // over groups of 8 hubs, hub_blocks the grid, hub_eoff the prefix of their
-    // degrees (hub_edges in all).  hub_pv and hub_best are zero between sweeps.
-    Buf<i64> hub_groups, hub_pv, hub_eoff;
+    // the smaller classes, the others (from list entry hub0 on) in chunks of
+    // their edges and slices of their clusters' hash range: hub_pre holds the
+    // prefixes of their edges, chunks and bucket starts and of the slices of
+    // groups of 8 hubs (k_hub_sizes; hub_edges, hub_chunks, hub_starts and
+    // hub_blocks in all).  hub_pv and hub_best are zero between sweeps.
+    Buf<i64> hub_pre, hub_pv;
     Buf<u64> hub_best;
-    i64 hub_blocks = 0, hub_edges = 0, nhalf = 0;
+    i64 hub_blocks = 0, hub_edges = 0, hub_chunks = 0, hub_starts = 0, nhalf = 0;
     bool hub32 = false;   // their row sums fit 32 bits
     u64 epoch = ~(u64)0;
     i64 nlds = 0, hub0 = 0, nhub = 0;
@@ -80,12 +81,18 @@ struct MoveScratch {
     Buf<u64> mvp;  // per vertex: cluster | moved << 31, and the cluster after this sweep's moves
     Buf<u64> rec;     // per vertex: cluster and its volume as fp32 (scoring)
     Buf<uint4> rec16; // the same with the cluster's constraint value, when there is one
-    Buf<u64> hub_kv;  // the large hubs' gathered records, while a local move runs
+    // the large hubs' gathered entries, while a local move runs: cluster and
+    // volume, weight (32 or 64 bits), and the bucket starts of every chunk
+    Buf<u64> hub_kv;
+    Buf<u32> hub_kw;
+    Buf<unsigned short> hub_st;
     Buf<u64> sqpart;  // partial sums of k_finish
     Buf<i32> part, dest, cand, moves, flag, tmp, tmp2;
     Buf<float> gain;
     Buf<i64> prio, scal;
     void ensure(Ctx& c, i64 n);
+    void ensure_hubs(Ctx& c, const LevelPlan& lp);
+    void drop_hubs();
 };
 
 void plan_level(Ctx& c, const DGraph& g, LevelPlan& p);

@@ -67,6 +67,28 @@ void MoveScratch::ensure(Ctx& c, i64 n) {
     sqpart = Buf<u64>(c, 2 * FIN_BLOCKS);
 }
 
+// the large hubs' gathered entries
+void MoveScratch::ensure_hubs(Ctx& c, const LevelPlan& lp) {
+    if (hub_kv.n < (size_t)lp.hub_edges) {
+        hub_kv.reset();
+        hub_kv = Buf<u64>(c, lp.hub_edges);
+    }
+    const size_t words = lp.hub32 ? lp.hub_edges : 2 * lp.hub_edges;
+    if (hub_kw.n < words) {
+        hub_kw.reset();
+        hub_kw = Buf<u32>(c, words);
+    }
+    if (hub_st.n < (size_t)lp.hub_starts) {
+        hub_st.reset();
+        hub_st = Buf<unsigned short>(c, lp.hub_starts);
+    }
+}
+void MoveScratch::drop_hubs() {
+    hub_kv.reset();
+    hub_kw.reset();
+    hub_st.reset();
+}
+
 // ------------------------------------------------------------- level plan
 __host__ __device__ __forceinline__ int score_class(i64 d) {
     return d <= 4 ? 0 : d <= 8 ? 1 : d <= 16 ? 2 : d <= 32 ? 3 : d <= 64 ? 4 : d <= 128 ? 5 : d <= 256 ? 6
@@ -99,6 +121,13 @@ constexpr int HUB_LDS_SLOTS = 10112;
 // slices of a hub: 1.5 slots per edge, so a slice is at most 2/3 full on average
 constexpr int HUB_SLOTS32 = 12288, HUB_SLOTS64 = 8192;
 __host__ __device__ __forceinline__ i64 hub_slices(i64 d, int slots) { return (3 * d + 2 * slots - 1) / (2 * slots); }
+// Their edges are gathered in chunks of HUB_E, merged in an LDS table of HUB_GS
+// slots (2/3 full at most; two blocks per CU with 32-bit sums) and left grouped
+// by bucket: a slice, or several slices of a hub that has more than HUB_BUCKETS
+constexpr int HUB_E = 4096, HUB_GS = 6144, HUB_BUCKETS = 1024;
+__host__ __device__ __forceinline__ i64 hub_chunks(i64 d) { return (d + HUB_E - 1) / HUB_E; }
+__host__ __device__ __forceinline__ i64 hub_per(i64 ns) { return (ns + HUB_BUCKETS - 1) / HUB_BUCKETS; }
+__host__ __device__ __forceinline__ i64 hub_nb(i64 ns) { return (ns + hub_per(ns) - 1) / hub_per(ns); }
 
 // Both partitions of a plan in one pass each of counting and writing: the
 // order1 classes (src/header/ordering.h:17-19; ORD_CLS) and the scoring classes,
@@ -180,28 +209,44 @@ __global__ void __launch_bounds__(PL_T) k_plan_write(const i64* __restrict__ rp,
 // group interleaved all slices of one hub run on one XCD and read the hub's
 // edges and records through its L2.
 constexpr int NXCD = 8;
-__global__ void k_hub_groups(const i64* rp, const i32* hubs, i64 m, int slots, i64* gs) {
-    const i64 g = thread_item();
-    if (g >= (m + NXCD - 1) / NXCD) return;
-    const i64 last = (g + 1) * NXCD < m ? (g + 1) * NXCD - 1 : m - 1;
-    const i32 i = hubs[last];
-    gs[g] = hub_slices(rp[i + 1] - rp[i], slots);
-}
-// block -> hub and slice; false for padding.  The largest hubs come first.
-__global__ void k_hub_degrees(const i64* rp, const i32* hubs, i64 m, i64* deg) {
+// sizes whose exclusive scan is LevelPlan::hub_pre: per hub its edges, its
+// chunks and the bucket starts of its chunks, and the slices per group of hubs
+__global__ void k_hub_sizes(const i64* rp, const i32* hubs, i64 m, int slots, i64* sz) {
     const i64 x = thread_item();
-    if (x >= m) return;
-    deg[x] = rp[hubs[x] + 1] - rp[hubs[x]];
+    const i64 ng = (m + NXCD - 1) / NXCD;
+    if (x < m) {
+        const i64 d = rp[hubs[x] + 1] - rp[hubs[x]];
+        sz[x] = d;
+        sz[m + x] = hub_chunks(d);
+        sz[2 * m + x] = hub_chunks(d) * (hub_nb(hub_slices(d, slots)) + 1);
+    }
+    if (x < ng) {
+        const i64 last = (x + 1) * NXCD < m ? (x + 1) * NXCD - 1 : m - 1;
+        const i32 i = hubs[last];
+        sz[3 * m + x] = hub_slices(rp[i + 1] - rp[i], slots);
+    }
 }
-__device__ __forceinline__ bool hub_block(const i64* gpre, i64 ng, i64 m, i64 bid, i64 nblk, i64& h, i64& sl) {
-    if (bid >= nblk) return false;
-    const i64 b = nblk - 1 - bid;
-    const i64 q = b / NXCD;
-    const i64 g = upper_row(gpre, 0, ng, q);
-    h = g * NXCD + b % NXCD;
-    sl = q - gpre[g];
-    return h < m;
-}
+// The scanned sizes of a level's m hubs: rows of hub_pre, each relative to its
+// first entry.
+struct HubView {
+    const i32* hubs;
+    const i64* pre;
+    i64 m, ng, nblk;
+    __device__ __forceinline__ i64 edge0(i64 h) const { return pre[h]; }
+    __device__ __forceinline__ i64 chunk0(i64 h) const { return pre[m + h] - pre[m]; }
+    __device__ __forceinline__ i64 start0(i64 h) const { return pre[2 * m + h] - pre[2 * m]; }
+    // block -> hub and slice; false for padding.  The largest hubs come first.
+    __device__ __forceinline__ bool slice(i64 bid, i64& h, i64& sl) const {
+        if (bid >= nblk) return false;
+        const i64* g0 = pre + 3 * m;
+        const i64 b = nblk - 1 - bid;
+        const i64 q = b / NXCD + g0[0];
+        const i64 g = upper_row(g0, 0, ng, q);
+        h = g * NXCD + b % NXCD;
+        sl = q - g0[g];
+        return h < m;
+    }
+};
 
 __global__ void k_hub_deg_keys(const i64* rp, const i32* list, i64 m, u64* keys, i32* vals) {
     const i64 x = thread_item();
@@ -284,22 +329,25 @@ void plan_level(Ctx& c, const DGraph& g, LevelPlan& p) {
     p.nhub = nh - p.nlds;
     p.hub_blocks = 0;
     if (p.nhub > 0) {
-        const i64 ng = ceil_div(p.nhub, NXCD);
-        p.hub_groups = Buf<i64>(c, ng + 1);
-        p.hub_pv = Buf<i64>(c, p.nhub);
-        p.hub_best = Buf<u64>(c, p.nhub);
-        k_hub_groups<<<grid_items(ng, 256), 256, 0, c.stream>>>(g.rp, p.sc_list.p + p.hub0, p.nhub,
-                                                                p.hub32 ? HUB_SLOTS32 : HUB_SLOTS64, p.hub_groups);
+        const i64 m = p.nhub, ng = ceil_div(m, NXCD), np = 3 * m + ng;
+        p.hub_pre = Buf<i64>(c, np + 1);
+        p.hub_pv = Buf<i64>(c, m);
+        p.hub_best = Buf<u64>(c, m);
+        k_hub_sizes<<<grid_items(m, 256), 256, 0, c.stream>>>(g.rp, p.sc_list.p + p.hub0, m,
+                                                              p.hub32 ? HUB_SLOTS32 : HUB_SLOTS64, p.hub_pre);
         PGGC_LAUNCH_CHECK();
-        scan_i64(c, p.hub_groups, p.hub_groups, ng);
-        p.hub_eoff = Buf<i64>(c, p.nhub + 1);
-        k_hub_degrees<<<grid_items(p.nhub, 256), 256, 0, c.stream>>>(g.rp, p.sc_list.p + p.hub0, p.nhub, p.hub_eoff);
-        PGGC_LAUNCH_CHECK();
-        scan_i64(c, p.hub_eoff, p.hub_eoff, p.nhub);
-        fill_i64(c, (i64*)p.hub_best.p, p.nhub, 0);  // zero between sweeps (k_hub_decide)
-        fill_i64(c, p.hub_pv, p.nhub, 0);
-        p.hub_blocks = c.read1(p.hub_groups.p + ng) * NXCD;
-        p.hub_edges = c.read1(p.hub_eoff.p + p.nhub);
+        scan_i64(c, p.hub_pre, p.hub_pre, np);
+        fill_i64(c, (i64*)p.hub_best.p, m, 0);  // zero between sweeps (k_hub_decide)
+        fill_i64(c, p.hub_pv, m, 0);
+        i64 e[4];
+        const i64 at[4] = {m, 2 * m, 3 * m, np};
+        Fetch f[4];
+        for (int k = 0; k < 4; k++) f[k] = Fetch{&e[k], p.hub_pre.p + at[k], sizeof(i64)};
+        copy_d2h(c, f, 4);
+        p.hub_edges = e[0];
+        p.hub_chunks = e[1] - e[0];
+        p.hub_starts = e[2] - e[1];
+        p.hub_blocks = (e[3] - e[2]) * NXCD;
     }
 }
 
@@ -780,25 +828,25 @@ __global__ void __launch_bounds__(BS) k_score_raw(const i64* __restrict__ rp, co
     if (threadIdx.x == 0) decide(i, p_conn, bk, p, wi, out);
 }
 
-// Hubs of degree above HUB_LDS_BOUND: a block per slice of a hub's hash range
-// (hub_block), folded into hub_best with atomicMax.
+// Hubs of degree above HUB_LDS_BOUND.
 //
-// First the hubs' edges are gathered: k_hub_gather leaves the (cluster, volume)
-// record of every edge at hub_eoff[h] + edge, so that each edge costs one
-// random access, and sums the own-cluster weights, which the candidates'
-// threshold needs (own edges and edges that the constraint rules out are left
-// empty).  A slice block then streams all of its hub's records (the slices of
-// one hub share an XCD's L2), keeps the clusters whose hash falls in its slice
-// in an LDS table with their weight and volume, and takes the best candidate
-// from the table.  Nothing but the best candidate leaves the chip.  LDS limits
-// it to one 1024-thread block per CU.  With tables in HBM, built slice by slice
-// and kept current from the movers, the same scoring wrote and listed 1.5-3
-// slots per edge, gathered a volume per cluster, and the updates were a chain of
-// dependent atomics per mover edge: scoring all degrees above
-// 2048 and the updates took about 200 ms on R-MAT scale 24 (two passes), now 135
-// (78 here: 64M edges gathered in 0.6 ms and streamed 5.7 times each in 1.2 ms a
-// sweep, 57 in the LDS tables of the degrees up to 8192).  Without the gather
-// pass, each slice reading records at random, a sweep took 3.0 ms.
+// k_hub_gather takes a chunk of HUB_E edges per block: it gathers the neighbours'
+// records, so that each edge costs one random access, sums the own-cluster
+// weights, which the candidates' threshold needs, merges the others by cluster in
+// LDS, and writes the distinct (cluster, volume, weight) entries grouped by the
+// bucket of their cluster's hash, with the buckets' starts.  k_hub_score takes a
+// slice of a hub's hash range per block: it reads its bucket's run of every
+// chunk (the slices of one hub share an XCD's L2), adds the weights per cluster
+// in an LDS table and takes the best candidate from it.  Nothing but the best
+// candidate leaves the chip.  Each entry is read once, or once per slice of its
+// bucket, and a cluster that most of the edges lead to is merged by the chunks
+// that meet it, so the work grows with the degree.
+// The random record gathers and the LDS atomics bound them.  R-MAT scale 24 (two
+// passes, 64M hub edges): 0.59 + 0.47 ms a sweep, 47 ms in all; with records left
+// in edge order, so that every slice of a hub read all of them (5.7 times each),
+// 0.6 + 1.2 ms and 78 ms, and time that grew with the square of the degree: one
+// hub of 2^20, 2^22 or 2^24 edges took 0.28, 2.8 or 33.8 ms a sweep, now 0.042,
+// 0.087 and 0.30.  Each slice gathering at random: 3.0 ms at scale 24.
 //
 // The hash is a bijection of the 32-bit id, split by range: a slice whose keys
 // do not fit (never seen with 1.5 slots per edge) is done again in 2, 4, ...
@@ -811,76 +859,133 @@ __device__ __forceinline__ u32 mix32(u32 x) {  // the finalizer of MurmurHash3
     x ^= x >> 16;
     return x;
 }
-// the share [j_lo, j_hi) of a hub's edges that block sl of ns handles
-__device__ __forceinline__ void hub_share(i64 s, i64 e, i64 ns, i64 sl, i64& j_lo, i64& j_hi) {
-    const i64 share = (e - s + ns - 1) / ns;
-    j_lo = s + sl * share;
-    j_hi = j_lo + share < e ? j_lo + share : e;
-}
-template <int SL, class WT>
-__global__ void __launch_bounds__(256) k_hub_gather(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
-                                                    const i32* __restrict__ hubs, i64 m, const i64* __restrict__ gpre,
-                                                    i64 ng, i64 nblk, const i64* __restrict__ eoff,
-                                                    const i32* __restrict__ part, RecView rv,
-                                                    const i32* __restrict__ cons, const i32* __restrict__ dest,
-                                                    u64* __restrict__ kv, i64* hub_pv) {
-    i64 h, sl;
-    if (!hub_block(gpre, ng, m, block_id(), nblk, h, sl)) return;
-    const i32 i = hubs[h];
+constexpr int HUB_GT = 512;
+template <int SL, class AT, class WT>
+__global__ void __launch_bounds__(HUB_GT) k_hub_gather(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
+                                                       HubView hv, const i32* __restrict__ part, RecView rv,
+                                                       const i32* __restrict__ cons, const i32* __restrict__ dest,
+                                                       u64* __restrict__ kv, AT* __restrict__ kw,
+                                                       unsigned short* __restrict__ starts, i64* hub_pv) {
+    __shared__ i32 lk[HUB_GS];
+    __shared__ AT lv[HUB_GS];
+    __shared__ float lf[HUB_GS];
+    __shared__ u32 hist[HUB_BUCKETS];
+    const i64 b = block_id();
+    if (b >= hv.chunk0(hv.m)) return;
+    const i64 h = upper_row(hv.pre + hv.m, 0, hv.m, b + hv.pre[hv.m]);
+    const i32 i = hv.hubs[h];
     if (dest[i] == NO_MOVE) return;
-    const i64 s = rp[i], e = rp[i + 1];
-    const i64 ns = hub_slices(e - s, SL);
-    if (sl >= ns) return;
-    i64 j_lo, j_hi;
-    hub_share(s, e, ns, sl, j_lo, j_hi);
+    const int t = threadIdx.x;
+    const i64 s = rp[i], d = rp[i + 1] - s, c = b - hv.chunk0(h);
+    const i64 j0 = s + c * HUB_E;
+    const int n = (int)(d - c * HUB_E < HUB_E ? d - c * HUB_E : HUB_E);
+    const i64 ns = hub_slices(d, SL);
+    const u32 per = (u32)hub_per(ns);
+    const int nb = (int)hub_nb(ns);
     const i32 p = part[i];
     const i32 cp = cons ? cons[p] : 0;
-    u64* out = kv + eoff[h];
-    const int t = threadIdx.x;
-    i64 own = 0;
-    constexpr int U = 8;  // edges in flight per thread
-    for (i64 jb = j_lo; jb < j_hi; jb += 256 * U) {  // block-uniform loop control
-        i32 v[U];
-        NbRec r[U];
+    constexpr int U = HUB_E / HUB_GT;  // edges in flight per thread
+    i32 v[U];
+    NbRec r[U];
+    AT w[U];
 #pragma unroll
-        for (int u = 0; u < U; u++) v[u] = jb + u * 256 + t < j_hi ? col[jb + u * 256 + t] : -1;
+    for (int u = 0; u < U; u++) v[u] = u * HUB_GT + t < n ? col[j0 + u * HUB_GT + t] : -1;
 #pragma unroll
-        for (int u = 0; u < U; u++)
-            if (v[u] >= 0) r[u] = load_rec(rv, v[u]);
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            if (v[u] < 0) continue;
-            const i64 j = jb + u * 256 + t;
-            if (r[u].part == p) own += W(j);
-            const i32 key = (r[u].part == p || r[u].cons != cp) ? EMPTY_KEY : r[u].part;
-            out[j - s] = (u64)(u32)key | ((u64)__float_as_uint(r[u].volf) << 32);
+    for (int u = 0; u < U; u++) {
+        w[u] = 0;
+        r[u].part = p;
+        if (v[u] >= 0) {
+            r[u] = load_rec(rv, v[u]);
+            w[u] = (AT)W(j0 + u * HUB_GT + t);
         }
     }
-    own = block_sum_i64<256>(own);
+    for (int q = t; q < HUB_GS; q += HUB_GT) {
+        lk[q] = EMPTY_KEY;
+        lv[q] = 0;
+    }
+    for (int q = t; q < HUB_BUCKETS; q += HUB_GT) hist[q] = 0;
+    AT own = 0;
+#pragma unroll
+    for (int u = 0; u < U; u++) own += r[u].part == p ? w[u] : (AT)0;
+    own = block_reduce<HUB_GT>(own, [](AT x, AT y) { return x + y; });
     if (t == 0 && own) atomicAdd((unsigned long long*)&hub_pv[h], (unsigned long long)own);
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        if (r[u].part == p || r[u].cons != cp) continue;
+        const u32 q = table_add_slot(lk, lv, (u32)HUB_GS, r[u].part, w[u]);
+        lf[q] = r[u].volf;  // (the same value whoever stores it)
+    }
+    __syncthreads();
+    constexpr int R = HUB_GS / HUB_GT;
+    u32 bu[R], rk[R];
+#pragma unroll
+    for (int q = 0; q < R; q++) {
+        const i32 key = lk[t + q * HUB_GT];
+        bu[q] = ~0u;
+        rk[q] = 0;
+        if (key == EMPTY_KEY) continue;
+        const u32 sl = (u32)(((u64)mix32((u32)key) * (u64)ns) >> 32);
+        bu[q] = per == 1 ? sl : sl / per;
+        rk[q] = atomicAdd(&hist[bu[q]], 1u);
+    }
+    __syncthreads();
+    constexpr int HB = HUB_BUCKETS / HUB_GT;
+    u32 hc[HB];
+    i64 mine = 0, total;
+#pragma unroll
+    for (int q = 0; q < HB; q++) {
+        hc[q] = hist[t * HB + q];
+        mine += hc[q];
+    }
+    u32 run = (u32)block_excl_scan_i64(mine, &total);
+    unsigned short* st = starts + hv.start0(h) + c * (nb + 1);
+#pragma unroll
+    for (int q = 0; q < HB; q++) {
+        hist[t * HB + q] = run;
+        if (t * HB + q < nb) st[t * HB + q] = (unsigned short)run;
+        run += hc[q];
+    }
+    if (t == 0) st[nb] = (unsigned short)total;
+    __syncthreads();
+    const i64 o = hv.edge0(h) + c * HUB_E;
+#pragma unroll
+    for (int q = 0; q < R; q++) {
+        if (bu[q] == ~0u) continue;
+        const int sl = t + q * HUB_GT;
+        const i64 x = o + hist[bu[q]] + rk[q];
+        kv[x] = (u64)(u32)lk[sl] | ((u64)__float_as_uint(lf[sl]) << 32);
+        kw[x] = lv[sl];
+    }
 }
 
-template <int SL, int BS, class AT, class WT, class LT>
-__global__ void __launch_bounds__(BS) k_hub_score(const i64* __restrict__ rp, WT W, const i64* __restrict__ vw,
-                                                  const i32* __restrict__ hubs, i64 m, const i64* __restrict__ gpre,
-                                                  i64 ng, i64 nblk, const i64* __restrict__ eoff,
+template <int SL, int BS, class AT, class LT>
+__global__ void __launch_bounds__(BS) k_hub_score(const i64* __restrict__ rp, const i64* __restrict__ vw, HubView hv,
                                                   const i32* __restrict__ part, const i64* __restrict__ vol, LT lam,
                                                   float ratio, const i32* __restrict__ dest,
-                                                  const u64* __restrict__ kv, const i64* __restrict__ hub_pv,
-                                                  u64* hub_best) {
+                                                  const u64* __restrict__ kv, const AT* __restrict__ kw,
+                                                  const unsigned short* __restrict__ starts,
+                                                  const i64* __restrict__ hub_pv, u64* hub_best) {
     __shared__ i32 lk[SL];
     __shared__ AT lv[SL];
     __shared__ float lf[SL];
     __shared__ int full;
     i64 h, sl;
-    if (!hub_block(gpre, ng, m, block_id(), nblk, h, sl)) return;
-    const i32 i = hubs[h];
+    if (!hv.slice(block_id(), h, sl)) return;
+    const i32 i = hv.hubs[h];
     if (dest[i] == NO_MOVE) return;
-    const i64 s = rp[i], d = rp[i + 1] - s;
+    const i64 d = rp[i + 1] - rp[i];
     const i64 ns = hub_slices(d, SL);
     if (sl >= ns) return;
     const int t = threadIdx.x;
-    const u64* in = kv + eoff[h];
+    const i64 nch = hub_chunks(d), per = hub_per(ns), nb = hub_nb(ns);
+    const unsigned short* st = starts + hv.start0(h) + sl / per;
+    const u64* in = kv + hv.edge0(h);
+    const AT* iw = kw + hv.edge0(h);
+    // as many lanes per chunk as its run is long on average
+    int lg = 2;
+    while (lg < 10 && ((i64)2 << lg) * nb <= HUB_E) lg++;
+    const int lane = t & ((1 << lg) - 1), G = 1 << lg;
     float multi, p_conn, b;
     own_terms(hub_pv[h], vol[part[i]], vw[i], lam(i), lam.rt(i, ratio), multi, p_conn, b);
     u64 bk = 0;
@@ -896,35 +1001,55 @@ __global__ void __launch_bounds__(BS) k_hub_score(const i64* __restrict__ rp, WT
             if (t == 0) full = 0;
             __syncthreads();
             bool ok = true;
-            constexpr int U = 8;  // records in flight per thread
-            for (i64 xb = 0; xb < d; xb += (i64)BS * U) {  // block-uniform loop control
-                u64 r[U];
-#pragma unroll
-                for (int u = 0; u < U; u++) {
-                    const i64 x = xb + (i64)u * BS + t;
-                    r[u] = x < d ? in[x] : (u64)(u32)EMPTY_KEY;
-                }
-#pragma unroll
-                for (int u = 0; u < U; u++) {
-                    const i32 key = (i32)(u32)r[u];
-                    if (key == EMPTY_KEY) continue;
-                    const u64 y = (u64)mix32((u32)key) * total;
-                    if ((y >> 32) != want) continue;
-                    const i64 w = W(s + xb + (i64)u * BS + t);
-                    u32 q = __umulhi((u32)y, (u32)SL);
-                    int probe = 0;
-                    for (; probe < SL; probe++) {
-                        const i32 old = atomicCAS(&lk[q], EMPTY_KEY, key);
-                        if (old == EMPTY_KEY) lf[q] = __uint_as_float((u32)(r[u] >> 32));
-                        if (old == EMPTY_KEY || old == key) {
-                            if (sizeof(AT) == 4) atomicAdd((u32*)&lv[q], (u32)w);
-                            else atomicAdd((unsigned long long*)&lv[q], (unsigned long long)w);
-                            break;
-                        }
-                        q = q + 1 < (u32)SL ? q + 1 : 0;
+            auto add = [&](u64 rec, AT w) {
+                const i32 key = (i32)(u32)rec;
+                const u64 y = (u64)mix32((u32)key) * total;
+                if ((y >> 32) != want) return;  // of another slice of the bucket, or part
+                u32 q = __umulhi((u32)y, (u32)SL);
+                int probe = 0;
+                for (; probe < SL; probe++) {
+                    const i32 old = atomicCAS(&lk[q], EMPTY_KEY, key);
+                    if (old == EMPTY_KEY) lf[q] = __uint_as_float((u32)(rec >> 32));
+                    if (old == EMPTY_KEY || old == key) {
+                        if (sizeof(AT) == 4) atomicAdd((u32*)&lv[q], (u32)w);
+                        else atomicAdd((unsigned long long*)&lv[q], (unsigned long long)w);
+                        break;
                     }
-                    ok = ok && probe < SL;
+                    q = q + 1 < (u32)SL ? q + 1 : 0;
                 }
+                ok = ok && probe < SL;
+            };
+            constexpr int U = 4;  // chunks in flight per lane group
+            const i64 step = BS >> lg;
+            for (i64 cb = 0; cb < nch; cb += step * U) {  // block-uniform loop control
+                i64 x[U], e[U];
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const i64 c = cb + u * step + (t >> lg);
+                    x[u] = e[u] = 0;
+                    if (c < nch) {
+                        const unsigned short* q = st + c * (nb + 1);
+                        x[u] = c * HUB_E + q[0] + lane;
+                        e[u] = c * HUB_E + q[1];
+                    }
+                }
+                u64 r[U];
+                AT w[U];
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    r[u] = (u64)(u32)EMPTY_KEY;
+                    w[u] = 0;
+                    if (x[u] < e[u]) {
+                        r[u] = in[x[u]];
+                        w[u] = iw[x[u]];
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < U; u++)
+                    if (x[u] < e[u]) add(r[u], w[u]);
+#pragma unroll
+                for (int u = 0; u < U; u++)
+                    for (i64 y = x[u] + G; y < e[u]; y += G) add(in[y], iw[y]);
             }
             if (!ok) full = 1;
             __syncthreads();
@@ -953,23 +1078,22 @@ __global__ void __launch_bounds__(BS) k_hub_score(const i64* __restrict__ rp, WT
     if (t == 0 && bk) atomicMax((unsigned long long*)&hub_best[h], (unsigned long long)bk);
 }
 
-// raw sweep: the same blocks, each with an equal share of the hub's edges
+// raw sweep: a block per slice again, each with an equal share of the hub's edges
 template <int SL, class WT, class LT>
 __global__ void __launch_bounds__(256) k_hub_raw(const i64* __restrict__ rp, const i32* __restrict__ col, WT W,
-                                                 const i64* __restrict__ vw, const i32* __restrict__ hubs, i64 m,
-                                                 const i64* __restrict__ gpre, i64 ng, i64 nblk,
+                                                 const i64* __restrict__ vw, HubView hv,
                                                  const i32* __restrict__ part, const i64* __restrict__ vol,
                                                  RecView rv, const i32* __restrict__ cons, LT lam, float ratio,
                                                  const i32* __restrict__ dest, u64* hub_best) {
     i64 h, sl;
-    if (!hub_block(gpre, ng, m, block_id(), nblk, h, sl)) return;
-    const i32 i = hubs[h];
+    if (!hv.slice(block_id(), h, sl)) return;
+    const i32 i = hv.hubs[h];
     if (dest[i] == NO_MOVE) return;
     const i64 s = rp[i], e = rp[i + 1];
     const i64 ns = hub_slices(e - s, SL);
     if (sl >= ns) return;
-    i64 j_lo, j_hi;
-    hub_share(s, e, ns, sl, j_lo, j_hi);
+    const i64 share = (e - s + ns - 1) / ns;
+    const i64 j_lo = s + sl * share, j_hi = j_lo + share < e ? j_lo + share : e;
     const i32 p = part[i];
     const i32 cp = cons ? cons[p] : 0;
     float multi, p_conn, bth;
@@ -1140,18 +1264,16 @@ static void score_all(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, co
         k_rec_pack<<<grid_items(g.n, 256), 256, 0, c.stream>>>(g.n, part, vol, cons, s.rec, cons ? s.rec16.p : nullptr);
         PGGC_LAUNCH_CHECK();
     }
-#define PGGC_HUB_RAW(SL)                                                                                              \
-    k_hub_raw<SL><<<grid_blocks(lp.hub_blocks), 256, 0, c.stream>>>(g.rp, g.col, W, g.vw, hubs, m, lp.hub_groups, ng, \
-                                                                    lp.hub_blocks, part, vol, a.rv, cons, lam, ratio, \
-                                                                    dest, lp.hub_best)
-#define PGGC_HUB(SL, AT)                                                                                              \
-    do {                                                                                                              \
-        k_hub_gather<SL><<<grid_blocks(lp.hub_blocks), 256, 0, c.stream>>>(                                           \
-            g.rp, g.col, W, hubs, m, lp.hub_groups, ng, lp.hub_blocks, lp.hub_eoff, part, a.rv, cons, dest, s.hub_kv, \
-            lp.hub_pv);                                                                                               \
-        k_hub_score<SL, 1024, AT><<<grid_blocks(lp.hub_blocks), 1024, 0, c.stream>>>(                                 \
-            g.rp, W, g.vw, hubs, m, lp.hub_groups, ng, lp.hub_blocks, lp.hub_eoff, part, vol, lam, ratio, dest,       \
-            s.hub_kv, lp.hub_pv, lp.hub_best);                                                                        \
+#define PGGC_HUB_RAW(SL)                                                                                             \
+    k_hub_raw<SL><<<grid_blocks(lp.hub_blocks), 256, 0, c.stream>>>(g.rp, g.col, W, g.vw, hv, part, vol, a.rv, cons, \
+                                                                    lam, ratio, dest, lp.hub_best)
+#define PGGC_HUB(SL, AT)                                                                                             \
+    do {                                                                                                             \
+        AT* kw = (AT*)(void*)s.hub_kw.p;                                                                             \
+        k_hub_gather<SL, AT><<<grid_blocks(lp.hub_chunks), HUB_GT, 0, c.stream>>>(                                   \
+            g.rp, g.col, W, hv, part, a.rv, cons, dest, s.hub_kv, kw, s.hub_st, lp.hub_pv);                          \
+        k_hub_score<SL, 1024, AT><<<grid_blocks(lp.hub_blocks), 1024, 0, c.stream>>>(                                \
+            g.rp, g.vw, hv, part, vol, lam, ratio, dest, s.hub_kv, kw, s.hub_st, lp.hub_pv, lp.hub_best);            \
     } while (0)
     const ScoreArgs<LT> a{L, part, vol, RecView{s.rec.p, cons ? s.rec16.p : nullptr}, cons, lam, ratio, out};
     PGGC_WDISPATCH(g, {
@@ -1179,18 +1301,14 @@ static void score_all(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, co
         c.kt_end(tk, 0.0);
         if (tk >= 0) acct_add(c, c.kt_counter(tk), acct.p + 1);
         if ((m = lp.nhub) > 0) {
-            const i32* hubs = L + lp.hub0;
+            const HubView hv{L + lp.hub0, lp.hub_pre, m, ceil_div(m, NXCD), lp.hub_blocks};
+            if (!raw) s.ensure_hubs(c, lp);
             tk = c.kt_begin(KS_SCORE_HUB);
-            const i64 ng = ceil_div(m, NXCD);
-            if (!raw && s.hub_kv.n < (size_t)lp.hub_edges) {
-                s.hub_kv.reset();
-                s.hub_kv = Buf<u64>(c, lp.hub_edges);
-            }
             if (raw && lp.hub32) PGGC_HUB_RAW(HUB_SLOTS32);
             else if (raw) PGGC_HUB_RAW(HUB_SLOTS64);
             else if (lp.hub32) PGGC_HUB(HUB_SLOTS32, u32);
             else PGGC_HUB(HUB_SLOTS64, A64);
-            k_hub_decide<<<grid_items(m, 256), 256, 0, c.stream>>>(hubs, m, part, g.vw, vol, lam, ratio, lp.hub_pv,
+            k_hub_decide<<<grid_items(m, 256), 256, 0, c.stream>>>(hv.hubs, m, part, g.vw, vol, lam, ratio, lp.hub_pv,
                                                                        lp.hub_best, out);
             c.kt_end(tk, 0.0);
             if (tk >= 0) acct_add(c, c.kt_counter(tk), acct.p + 2);
@@ -2262,7 +2380,7 @@ static void local_move_t(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g,
         }
     }
     relabel(c, s, nfull, best_part, best);
-    s.hub_kv.reset();
+    s.drop_hubs();
 }
 
 // afterburner_filter_strict (src/local_mover.cpp:131-213): exact sequential
@@ -2376,7 +2494,7 @@ void local_move_strict(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, i
         trc.end(k, tr);
     }
     relabel(c, s, n, best_part, best);
-    s.hub_kv.reset();
+    s.drop_hubs();
 }
 
 i64 sweep_once(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, const i32* part, const i64* vol, i64 L,
@@ -2404,7 +2522,7 @@ i64 sweep_once(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, const i32
     copy_dev(c, dest, s.dest, n * sizeof(i32));
     copy_dev(c, gain, s.gain, n * sizeof(float));
     c.sync();
-    s.hub_kv.reset();
+    s.drop_hubs();
     return km;
 }
 
@@ -2812,7 +2930,7 @@ void local_move_batch(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, co
         }
     }
     relabel_batch(c, s, bl, best_part, best, active);
-    s.hub_kv.reset();
+    s.drop_hubs();
 }
 
 }  // namespace pggc
