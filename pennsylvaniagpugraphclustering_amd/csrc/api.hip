@@ -1057,6 +1057,7 @@ int pggc_louvain(pggc_ctx* ctx, const pggc_graph* gg, pggc_state* st, int constr
         CTX_CHECK(ctx);
         DGraph g = view_of(gg);
         RefineData rd = rd_of(st);
+        know_max_weight(ctx->c, g);
         RunStats rs;
         Renum rtop;
         louvain_part(ctx->c, ctx->ms, g, rd, constrained != 0, constraint, part_out, rs, nullptr,
@@ -1071,6 +1072,7 @@ int pggc_leiden(pggc_ctx* ctx, const pggc_graph* gg, pggc_state* st, int plus, i
         CTX_CHECK(ctx);
         DGraph g = view_of(gg);
         RefineData rd = rd_of(st);
+        know_max_weight(ctx->c, g);
         RunStats rs;
         Renum rtop;
         leiden_part(ctx->c, ctx->ms, g, rd, plus != 0, improve != 0, input, part_out, rs, nullptr,
@@ -1091,7 +1093,7 @@ int pggc_cluster(pggc_ctx* ctx, const pggc_graph* gg, int algo, int objective, d
             g.wk = W_UNIT;
         }
         Ctx& c = ctx->c;
-        if (g.wk != W_UNIT && g.nnz > 0) g.wmax = max_weight(c, g);  // read by every plan and contraction
+        know_max_weight(c, g);
         c.seed = seed;
         c.draws = 0;
         Buf<i64> vol(c, g.n + 1);

@@ -168,6 +168,7 @@ void louvain_batch(Ctx& c, MoveScratch& ms, const std::vector<DGraph>& gs, const
         g0.w = nullptr;
         g0.wk = W_UNIT;
     }
+    know_max_weight(c, g0);
     // ---- per-instance state (cluster_data per instance, one label space)
     BatchState st;
     st.K = K;

@@ -127,7 +127,7 @@ void own_weight(Ctx& c, const DGraph& g, const i32* labels, i64* out);
 // the same; the sweeps read 4 instead of 8 weight bytes per edge and the level
 // holds 8 instead of 12 bytes per nonzero) and int64 otherwise, or always with
 // `to`: when the finer level's weights sum to less than 2^31 they are written
-// as int32 at once, else after a max reduction.
+// as int32 at once, else after a max reduction (contract_widths).
 // With `to` the columns and int64 weights go to the caller's arrays instead of
 // out's (nothing is written there when they do not fit cap); the copy from out's
 // took 0.4 of 7.0 ms for 100M coarse nonzeros.
@@ -140,6 +140,9 @@ void contract(Ctx& c, const DGraph& g, const i32* vcmap, i64 nc, OwnedGraph& out
 
 // largest weight of g as an unsigned value (a negative weight is huge); g.nnz > 0
 u64 max_weight(Ctx& c, const DGraph& g);
+// g.wmax of a weighted graph, read once by the calls whose plans and contractions
+// ask for it
+void know_max_weight(Ctx& c, DGraph& g);
 
 // next.vw[map[i]] += g.vw[i]  (src/clustering_methods.cpp:33-38)
 void coarsen_vertex_weights(Ctx& c, const DGraph& g, const i32* map, i64 nc, i64* out);

@@ -7,6 +7,7 @@
 #include "graph.h"
 #include "hash.h"
 #include "select.h"
+#include "widths.h"
 
 namespace pggc {
 
@@ -193,7 +194,6 @@ __global__ void __launch_bounds__(256) k_cscatter(const i32* vcmap, i64 n, const
 // Merge classes by bound (the summed degrees of a row's members): LDS tables
 // for bounds up to C_BOUND[q], then big rows and empty ones.
 constexpr int C_BIG = 5, C_EMPTY = 6, C_CLS = 7;
-constexpr i64 C_TOP = 8192;  // largest bound merged in LDS
 struct MergeClass {
     const i64* bound;
     __device__ __forceinline__ int operator()(i64 u) const {
@@ -752,9 +752,10 @@ static void narrow_weights(Ctx& c, OwnedGraph& g) {
 }
 
 // AT: sums of rows merged in LDS; TT: staged weights; OT: weights written to
-// `ow` (out.w or out.w32, allocated here), or int64 ones to the caller's arrays
+// `ow` (out.w or out.w32, allocated here), or int64 ones to the caller's arrays;
+// packed: the big rows' tables have one word per slot (one CAS per new key)
 template <class AT, class TT, class OT>
-static void contract_t(Ctx& c, const DGraph& g, const i32* vcmap, i64 nc, OwnedGraph& out, Buf<OT>& ow,
+static void contract_t(Ctx& c, const DGraph& g, const i32* vcmap, i64 nc, bool packed, OwnedGraph& out, Buf<OT>& ow,
                        const ContractTo* to) {
     const i64 n = g.n;
     // member counts, bounds and coarse degrees, zeroed by one launch
@@ -798,9 +799,6 @@ static void contract_t(Ctx& c, const DGraph& g, const i32* vcmap, i64 nc, OwnedG
         k_goff_sizes<<<grid_items(n2, 256), 256, 0, c.stream>>>(big, n2, bound, nc, goff);
         PGGC_LAUNCH_CHECK();
         scan_i64(c, goff, goff, n2);
-        // packed tables (one CAS per new key) when every coarse weight fits
-        // 32 bits
-        const bool packed = sizeof(TT) == 4;
         k_member_degs<<<grid_items(n, 256), 256, 0, c.stream>>>(members, g.rp, n, mdp);
         PGGC_LAUNCH_CHECK();
         scan_i64(c, mdp, mdp, n);
@@ -917,24 +915,25 @@ static void contract_t(Ctx& c, const DGraph& g, const i32* vcmap, i64 nc, OwnedG
     }
 }
 
+void know_max_weight(Ctx& c, DGraph& g) {
+    if (g.wk != W_UNIT && g.nnz > 0 && g.wmax == 0) g.wmax = max_weight(c, g);
+}
+
 void contract(Ctx& c, const DGraph& g, const i32* vcmap, i64 nc, OwnedGraph& out, const ContractTo* to) {
-    // all weights together below 2^31: every coarse weight and sum fits 32 bits
-    const u64 top = (u64)1 << 31;
-    const bool small = g.wsmall || (g.wk == W_UNIT ? (u64)g.nnz < top
-                                                   : g.wmax > 0 && g.wmax < top && (u64)g.nnz * g.wmax < top);
-    if (small && !to) {
-        contract_t<u32, i32>(c, g, vcmap, nc, out, out.w32, nullptr);
+    DGraph f = g;
+    if (!g.wsmall) know_max_weight(c, f);
+    const ContractWidths w = contract_widths(g.nnz, g.wk == W_UNIT ? 1 : f.wmax, g.wsmall);
+    if (w.small && !to) {
+        contract_t<u32, i32>(c, g, vcmap, nc, true, out, out.w32, nullptr);
         return;
     }
-    if (small) {
-        contract_t<u32, i32>(c, g, vcmap, nc, out, out.w, to);
-    } else {
-        // 32-bit sums in LDS when the weights are small enough for C_TOP of them
-        const u64 mx = g.wk == W_UNIT ? 1 : g.wmax ? g.wmax : g.nnz > 0 ? max_weight(c, g) : 1;
-        if (mx <= 0xffffffffull / C_TOP) contract_t<u32, i64>(c, g, vcmap, nc, out, out.w, to);
-        else contract_t<i64, i64>(c, g, vcmap, nc, out, out.w, to);
-        if (!to) narrow_weights(c, out);
+    if (w.small) {
+        contract_t<u32, i32>(c, g, vcmap, nc, true, out, out.w, to);
+        return;
     }
+    if (w.sum32) contract_t<u32, i64>(c, g, vcmap, nc, w.packed, out, out.w, to);
+    else contract_t<i64, i64>(c, g, vcmap, nc, w.packed, out, out.w, to);
+    if (!to) narrow_weights(c, out);
 }
 
 }  // namespace pggc

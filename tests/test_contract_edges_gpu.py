@@ -53,3 +53,34 @@ def test_rows_at_table_sizes(gpu_ctx, kind, weights, leaf_groups):
     assert np.array_equal(rp.cpu().numpy(), rrp)
     assert np.array_equal(col.cpu().numpy(), rcol)
     assert np.array_equal(w.cpu().numpy(), rw)
+
+
+@pytest.mark.parametrize("bound", [2 ** 31, 2 ** 32])
+@pytest.mark.parametrize("over", [0, 1])
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("leaf_groups", [1, 700])
+def test_total_weight_at_width_edges(gpu_ctx, bound, over, wide, leaf_groups):
+    """Equal weights whose sum over the graph is the largest below 2^31 or 2^32,
+    or the next one above: the edges of 32-bit staging and of one-word tables.
+    With one group of leaves a coarse weight is half of the sum; pggc_contract
+    and the coarse levels of a whole run."""
+    from pennsylvaniagpugraphclustering_amd import clustering as C
+    g = stars("spread", None, 3)
+    w1 = (bound - 1) // g.nnz + over
+    assert (g.nnz * w1 < bound) == (over == 0)
+    w = np.full(g.nnz, w1, np.int32)
+    vc = np.concatenate([np.arange(LEAVES) % leaf_groups, leaf_groups + np.arange(len(DEGREES)) * (leaf_groups > 1)])
+    vc = vc.astype(np.int32)
+    nc = int(vc.max()) + 1
+    print(f"contract total {g.nnz * w1} groups={leaf_groups} wide={wide}", flush=True)
+    dg = C.DeviceGraph(g.rp, g.col, w.astype(np.int64) if wide else w, None, objective="WMod")
+    rp, col, cw = C.build_coarse_graph(dg, vc, nc)
+    rrp, rcol, rw = O.contract(g.rp, g.col, w, vc, nc)
+    assert np.array_equal(rp.cpu().numpy(), rrp)
+    assert np.array_equal(col.cpu().numpy(), rcol)
+    assert np.array_equal(cw.cpu().numpy(), rw)
+    if leaf_groups > 1:
+        vw = dg.vtx_w.cpu().numpy()
+        q, part, info = C.cluster(dg, "louvain", "WMod", 1.0, 1, seed=2)
+        oq, op, oi = O.cluster(g.rp, g.col, w, vw, "WMod", 1.0, "louvain", 1, seed=2)
+        assert q == oq and np.array_equal(part.cpu().numpy(), op) and info["sweeps"] == oi["sweeps"]
