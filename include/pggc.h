@@ -148,6 +148,8 @@ int pggc_ctx_set_sweep_trace(pggc_ctx* ctx, pggc_sweep_fn fn, void* user);
  *     scoring of vertices with 64 < degree <= 512: 64 (default), 128, 256.
  *   PGGC_KNOB_TABLE_SLOTS_PER_EDGE: LDS hash-table slots per edge of a degree
  *     class's bound, 64 < degree <= 2048: 2 (default) or 4.
+ *     Both without effect on levels of at most 8,192 vertices of degree 65 to
+ *     2048, which are scored in one launch of 256 threads and 2 slots.
  *   PGGC_KNOB_HUB_UPDATE_DIV, PGGC_KNOB_HUB_LDS_MAX_DEGREE (2048 or 4096),
  *     PGGC_KNOB_HUB_EDGES_PER_ITEM (512, 1024, 2048),
  *     PGGC_KNOB_HUB_SLOTS_PER_ITEM (2048, 4096, 8192) and PGGC_KNOB_HUB_BUILD:
@@ -160,10 +162,11 @@ int pggc_ctx_set_sweep_trace(pggc_ctx* ctx, pggc_sweep_fn fn, void* user);
  *     copy of the level with vertices in descending degree order (rows keep
  *     their entry order; labels, priorities and new cluster ids follow the
  *     original ids, so results are identical) or on the level itself.  1:
- *     always the copy; 2 (default): the copy on large levels whose edges
- *     gather on few vertices, and on the top level when the call makes more
- *     than one top-level pass (pggc_cluster with ex_iters != 0); 0: never.
- *     Not used with the active-set predictor on.
+ *     always the copy (of coarse levels, while the copies of a run hold at
+ *     most 1/16 of the device's memory together); 2 (default): the copy on
+ *     large levels whose edges gather on few vertices, and on the top level
+ *     when the call makes more than one top-level pass (pggc_cluster with
+ *     ex_iters != 0); 0: never.  Not used with the active-set predictor on.
  *   PGGC_KNOB_CONTRACT_BATCH: the contraction merges its largest coarse rows
  *     in HBM hash tables and sorts them in batches of rows holding at most
  *     this many table slots (default 2^30) and a quarter as many sort
@@ -183,10 +186,9 @@ int pggc_ctx_set_sweep_trace(pggc_ctx* ctx, pggc_sweep_fn fn, void* user);
 #define PGGC_KNOB_COUNT 11
 int pggc_ctx_set_knob(pggc_ctx* ctx, int knob, int64_t value);
 int pggc_ctx_get_knob(pggc_ctx* ctx, int knob, int64_t* value);
-/* Autotuner of the execution-shape knobs (no counterpart in the reference):
- * coordinate descent in the order hub LDS max degree, table threads, table
- * slots per edge, hub edges per item, hub slots per item, hub update divisor;
- * each candidate value is timed on one pLouvain clustering of g
+/* Autotuner of the execution-shape knobs that have an effect (no counterpart in
+ * the reference): coordinate descent in the order table threads, table slots
+ * per edge; each value is timed on one pLouvain clustering of g
  * (louvain_part, src/clustering_methods.cpp:139-222; best of reps runs after
  * an untimed one), and the fastest value is kept on ctx.  report (host, nullable): up to cap rows of
  * (knob, value, microseconds); *nrows (nullable) receives the rows timed.

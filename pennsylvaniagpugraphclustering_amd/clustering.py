@@ -88,10 +88,9 @@ class Context:
              "hub_lds_max_degree": 4, "hub_edges_per_item": 5, "hub_slots_per_item": 6, "raw_sweeps": 7,
              "hub_build": 8, "renumber": 9, "contract_batch": 10}
 
-    # values the execution-shape knobs accept (results are identical for all)
-    KNOB_VALUES = {"table_threads": (64, 128, 256), "table_slots_per_edge": (2, 4),
-                   "hub_lds_max_degree": (2048, 4096), "hub_edges_per_item": (512, 1024, 2048),
-                   "hub_slots_per_item": (2048, 4096, 8192), "hub_update_div": (16, 32, 64)}
+    # values of the knobs that the autotuner times (results are identical for
+    # all); the hub knobs are accepted and have no effect
+    KNOB_VALUES = {"table_threads": (64, 128, 256), "table_slots_per_edge": (2, 4)}
 
     def set_knob(self, name, value):
         """Tuning knob of the HIP path (gnn_max_sweeps: predicted sweeps per
@@ -104,7 +103,7 @@ class Context:
         return v.value
 
     def autotune(self, g, objective="Mod", reps=2):
-        """pggc_autotune: coordinate descent over the execution-shape knobs,
+        """pggc_autotune: coordinate descent over the knobs of KNOB_VALUES,
         timing one pLouvain clustering of g per value; the fastest values stay
         set.  Returns (chosen {knob: value}, [(knob, value, us), ...])."""
         names = {v: k for k, v in self.KNOBS.items()}

@@ -699,18 +699,17 @@ int pggc_gnn_eval(pggc_ctx* ctx, const pggc_graph* gg, const int32_t* part, cons
     });
 }
 
-// candidate values of the execution-shape knobs (what the kernels are
-// instantiated for); the other knobs take any value >= 0
+// accepted values of the execution-shape knobs (of the tables', what the kernels
+// are instantiated for); the other knobs take any value >= 0
 static const std::vector<int64_t>* knob_candidates(int knob) {
     static const std::vector<int64_t> threads{64, 128, 256}, spe{2, 4}, lds{2048, 4096}, edges{512, 1024, 2048},
-        slots{2048, 4096, 8192}, div{16, 32, 64};
+        slots{2048, 4096, 8192};
     switch (knob) {
         case PGGC_KNOB_TABLE_THREADS: return &threads;
         case PGGC_KNOB_TABLE_SLOTS_PER_EDGE: return &spe;
         case PGGC_KNOB_HUB_LDS_MAX_DEGREE: return &lds;
         case PGGC_KNOB_HUB_EDGES_PER_ITEM: return &edges;
         case PGGC_KNOB_HUB_SLOTS_PER_ITEM: return &slots;
-        case PGGC_KNOB_HUB_UPDATE_DIV: return &div;  // the autotuner's range (any value >= 0 is accepted)
         default: return nullptr;
     }
 }
@@ -718,10 +717,7 @@ static const std::vector<int64_t>* knob_candidates(int knob) {
 static void set_knob(Ctx& c, int knob, int64_t value) {
     if (value < 0) throw Error(PGGC_EINVAL, "knob value must be >= 0");
     const std::vector<int64_t>* cand = knob_candidates(knob);
-    const bool shape = knob == PGGC_KNOB_TABLE_THREADS || knob == PGGC_KNOB_TABLE_SLOTS_PER_EDGE ||
-                       knob == PGGC_KNOB_HUB_LDS_MAX_DEGREE || knob == PGGC_KNOB_HUB_EDGES_PER_ITEM ||
-                       knob == PGGC_KNOB_HUB_SLOTS_PER_ITEM;
-    if (shape && std::find(cand->begin(), cand->end(), value) == cand->end())
+    if (cand && std::find(cand->begin(), cand->end(), value) == cand->end())
         throw Error(PGGC_EINVAL, "knob value is not one the kernels are built for");
     switch (knob) {
         case PGGC_KNOB_HUB_UPDATE_DIV: c.hub_update_div = value; break;
@@ -737,7 +733,6 @@ static void set_knob(Ctx& c, int knob, int64_t value) {
         case PGGC_KNOB_CONTRACT_BATCH: c.contract_batch = std::max<int64_t>(value, 1); break;
         default: throw Error(PGGC_EINVAL, "unknown knob");
     }
-    if (shape) c.knob_epoch++;  // level plans depend on these
 }
 
 static int64_t get_knob(const Ctx& c, int knob) {
@@ -779,8 +774,8 @@ int pggc_ctx_get_knob(pggc_ctx* ctx, int knob, int64_t* value) {
     });
 }
 
-// Coordinate descent over the execution-shape knobs: each knob in turn
-// takes every candidate value, one pLouvain clustering of g (louvain_part:
+// Coordinate descent over the knobs that change how a kernel runs: each in turn
+// takes every accepted value, one pLouvain clustering of g (louvain_part:
 // every level down and up, the unit of the ex_iters loop) is timed, and the
 // fastest value is kept.  A first untimed run per value builds the plans.
 int pggc_autotune(pggc_ctx* ctx, const pggc_graph* gg, int objective, int reps, int64_t* report, int cap,
@@ -796,8 +791,7 @@ int pggc_autotune(pggc_ctx* ctx, const pggc_graph* gg, int objective, int reps, 
         Buf<i64> vol(c, std::max<i64>(n, 1));
         Buf<i32> part(c, std::max<i64>(n, 1));
         int rows = 0;
-        const int order[] = {PGGC_KNOB_HUB_LDS_MAX_DEGREE, PGGC_KNOB_TABLE_THREADS, PGGC_KNOB_TABLE_SLOTS_PER_EDGE,
-                             PGGC_KNOB_HUB_EDGES_PER_ITEM, PGGC_KNOB_HUB_SLOTS_PER_ITEM, PGGC_KNOB_HUB_UPDATE_DIV};
+        const int order[] = {PGGC_KNOB_TABLE_THREADS, PGGC_KNOB_TABLE_SLOTS_PER_EDGE};
         for (int knob : order) {
             const std::vector<int64_t>& cand = *knob_candidates(knob);
             int64_t best_v = get_knob(c, knob);

@@ -55,7 +55,6 @@ struct LevelPlan {
     Buf<u64> hub_best;
     i64 hub_blocks = 0, hub_edges = 0, hub_chunks = 0, hub_starts = 0, nhalf = 0;
     bool hub32 = false;   // their row sums fit 32 bits
-    u64 epoch = ~(u64)0;
     i64 nlds = 0, hub0 = 0, nhub = 0;
     bool agg32 = false;  // sums of rows of degree <= 8192 fit 32 bits
     i64 max_deg = 0;  // of the hub class (0 without hubs)

@@ -272,10 +272,9 @@ __global__ void k_hub_shape(const i64* rp, const i32* list, i64 m, i64* out) {
 }
 
 void plan_level(Ctx& c, const DGraph& g, LevelPlan& p) {
-    if (p.key == (const void*)g.rp && p.n == g.n && p.epoch == c.knob_epoch) return;
+    if (p.key == (const void*)g.rp && p.n == g.n) return;
     p.key = g.rp;
     p.n = g.n;
-    p.epoch = c.knob_epoch;
     {
         const int tk = c.kt_begin(KS_ORDER);
         const i64 n = g.n, nb = ceil_div(std::max<i64>(n, 1), PL_TILE);

@@ -68,6 +68,23 @@ def test_every_knob_value_gives_identical_results(gpu_ctx, graphs_under_test, al
         _set_all(gpu_ctx, DEFAULTS)
 
 
+def test_autotune_times_knobs_with_an_effect(gpu_ctx, graphs_under_test):
+    """The table knobs only; the hub knobs, which no kernel reads, keep what
+    the caller set."""
+    dg, obj = graphs_under_test["hub30k"]
+    kept = {"hub_lds_max_degree": 4096, "hub_edges_per_item": 512, "hub_slots_per_item": 2048, "hub_update_div": 16}
+    try:
+        _set_all(gpu_ctx, kept)
+        chosen, table = gpu_ctx.autotune(dg, obj, reps=1)
+        assert [r[:2] for r in table] == [("table_threads", 64), ("table_threads", 128), ("table_threads", 256),
+                                          ("table_slots_per_edge", 2), ("table_slots_per_edge", 4)]
+        assert set(chosen) == {"table_threads", "table_slots_per_edge"}
+        for k, v in kept.items():
+            assert gpu_ctx.get_knob(k) == v
+    finally:
+        _set_all(gpu_ctx, DEFAULTS)
+
+
 def test_knob_values_are_checked(gpu_ctx):
     from pennsylvaniagpugraphclustering_amd import _lib
     with pytest.raises(_lib.PggcError):
