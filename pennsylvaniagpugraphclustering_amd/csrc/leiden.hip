@@ -113,7 +113,7 @@ template <bool LAST, class WT>
 __device__ __forceinline__ u64 hn_best(const i32* __restrict__ col, WT W, const u64* __restrict__ well, i64 s, i64 e,
                                        i64 first, i64 step, i32 ci, float multi, i32 seed) {
     u64 best = 0;
-    for (i64 jb = s + first; jb < e; jb += step * HN_U) {
+    for (i64 jb = s + first; __any(jb < e); jb += step * HN_U) {  // wave-uniform loop control
         i32 v[HN_U];
         u64 o[HN_U];
 #pragma unroll
@@ -122,10 +122,10 @@ __device__ __forceinline__ u64 hn_best(const i32* __restrict__ col, WT W, const 
             v[u] = j < e ? col[j] : -1;
         }
 #pragma unroll
-        for (int u = 0; u < HN_U; u++) o[u] = v[u] >= 0 ? well[v[u]] : (u64)0xffffffffu;
+        for (int u = 0; u < HN_U; u++) o[u] = v[u] >= 0 ? well[v[u]] : 0;
 #pragma unroll
         for (int u = 0; u < HN_U; u++) {
-            if (well_cluster(o[u]) != ci) continue;
+            if (v[u] < 0 || well_cluster(o[u]) != ci) continue;
             const i64 j = jb + u * step;
             const float val = fmaf(-multi, well_weight(o[u]), (float)W(j));
             if (!(val >= 0.0f)) continue;
@@ -151,18 +151,19 @@ __global__ void __launch_bounds__(256) k_hn_weighted(const i64* __restrict__ rp,
     constexpr bool LAST = G == HN_G;
     const int lane = threadIdx.x & (G - 1);
     const i64 x = block_id() * (256 / G) + threadIdx.x / G;
-    i32 i = -1;
-    i64 s = 0;
-    u64 best = 0;
+    i32 i = -1, ci = -1;
+    i64 s = 0, e = 0;
+    float multi = 0.0f;
     if (x < m) {
         i = list[x];
-        s = rp[i];
+        s = e = rp[i];
         const u64 me = well[i];
-        const i32 ci = well_cluster(me);
-        if (!hn_skips(seed, i, ci))
-            best = hn_best<LAST>(col, W, well, s, rp[i + 1], lane, G, ci, gamma * well_weight(me), seed);
+        ci = well_cluster(me);
+        multi = gamma * well_weight(me);
+        if (!hn_skips(seed, i, ci)) e = rp[i + 1];
     }
-    xlane_fence(best);  // the groups' loops end at different iterations
+    u64 best = hn_best<LAST>(col, W, well, s, e, lane, G, ci, multi, seed);
+    xlane_fence(best);
 #pragma unroll
     for (int o = G / 2; o > 0; o >>= 1) {
         const u64 b = __shfl_xor(best, o, G);

@@ -741,17 +741,18 @@ __global__ void __launch_bounds__(BS) k_score_table(const i64* __restrict__ rp, 
         keys[q] = EMPTY_KEY;
         vals[q] = 0;
     }
+    AT pv = 0;  // (summed before the inserts: probing ends lane by lane)
+#pragma unroll
+    for (int q = 0; q < R; q++) pv += r[q].part == p ? w[q] : (AT)0;
+    pv = block_reduce<BS>(pv, [](AT a, AT b) { return a + b; });
     __syncthreads();
-    AT pv = 0;
     u32 h[R];
 #pragma unroll
     for (int q = 0; q < R; q++) {
         h[q] = 0;
-        if (r[q].part == EMPTY_KEY) continue;
-        if (r[q].part == p) pv += w[q];
-        else h[q] = table_add_slot(keys, vals, (u32)S, r[q].part, w[q]);
+        if (r[q].part == EMPTY_KEY || r[q].part == p) continue;
+        h[q] = table_add_slot(keys, vals, (u32)S, r[q].part, w[q]);
     }
-    pv = block_reduce<BS>(pv, [](AT a, AT b) { return a + b; });
     __syncthreads();
     float multi, p_conn, b;
     own_terms((i64)pv, vol[p], wi, lam(i), lam.rt(i, ratio), multi, p_conn, b);
