@@ -21,6 +21,23 @@ def hub_graph(n=30000, hub_deg=20000, seed=5, weights=None):
     return graphs.from_edges(n, src, dst, w)
 
 
+def many_table_rows(degrees, m=8500, n=60000, weights=None, seed=21):
+    """m vertices of degree 65 to 95 over a shared pool, after one vertex of each
+    of `degrees`: more table rows than a level may have to be scored in one
+    launch (TABLE_ONE_LAUNCH in csrc/localmove.hip)."""
+    rng = np.random.default_rng(seed)
+    k = len(degrees)
+    d = np.concatenate([np.asarray(degrees), rng.integers(65, 96, m)])
+    # a random run of consecutive pool vertices each (distinct neighbours)
+    first = rng.integers(0, n - k - m - int(d.max()), len(d))
+    src = np.repeat(np.arange(len(d)), d)
+    dst = k + m + np.repeat(first, d) + np.arange(len(src)) - np.repeat(np.cumsum(d) - d, d)
+    w = None if weights is None else rng.integers(weights[0], weights[1] + 1, len(src))
+    g = graphs.from_edges(n, src, dst, w)
+    assert np.array_equal(g.degrees()[:len(d)], d)
+    return g
+
+
 def cases():
     return {
         "karate": (graphs.karate(), "Mod"),

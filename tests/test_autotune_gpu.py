@@ -1,13 +1,14 @@
 """The execution-shape knobs (threads per vertex and slots per edge of the
-LDS-table scoring, the LDS/HBM cut-off for hubs, hub build and scan item
-sizes, the hub-table update divisor, the hub-table build method, the
-top-level renumbering, the contraction's batch size) change time only: every value gives
-the same clustering, bit for bit, as the defaults.  The autotuner times each
-candidate and keeps the fastest, so it cannot change results either."""
+LDS-table scoring, the renumbering of levels, the contraction's batch size, and
+the hub knobs, which are accepted without effect) change time only: every value
+gives the same clustering, bit for bit, as the defaults.  The table knobs choose
+kernels on levels of more than 8,192 rows of degree 65 to 2048 only; one of the
+graphs has such a level.  The autotuner times each value of the table knobs and
+keeps the fastest, so it cannot change results either."""
 import numpy as np
 import pytest
 
-from tests.graphcases import hub_graph
+from tests.graphcases import hub_graph, many_table_rows
 from pennsylvaniagpugraphclustering_amd import graphs
 
 pytestmark = pytest.mark.gpu
@@ -23,7 +24,10 @@ def graphs_under_test():
     out = {}
     for name, (g, obj) in {"hub30k": (hub_graph(), "Mod"),
                            "hub30k_w": (hub_graph(seed=9, weights=(1, 10)), "WMod"),
-                           "rmat16": (graphs.rmat(16, 16, seed=2), "Mod")}.items():
+                           "rmat16": (graphs.rmat(16, 16, seed=2), "Mod"),
+                           "rows9k": (many_table_rows([200, 500, 1000, 2000]), "Mod")}.items():
+        if name == "rows9k":
+            assert ((g.degrees() > 64) & (g.degrees() <= 2048)).sum() > 8192
         out[name] = (C.DeviceGraph.from_csr(g, obj), obj)
     return out
 
@@ -52,8 +56,7 @@ def test_every_knob_value_gives_identical_results(gpu_ctx, graphs_under_test, al
             variants = [{k: v} for k, vals in gpu_ctx.KNOB_VALUES.items() for v in vals if v != DEFAULTS[k]]
             variants.append({"table_threads": 256, "table_slots_per_edge": 4, "hub_lds_max_degree": 4096,
                              "hub_edges_per_item": 512, "hub_slots_per_item": 2048, "hub_update_div": 0})
-            # hub tables built by edge items with HBM atomics, for every hub
-            # and for every other hub (the rest from LDS slices)
+            # accepted, without effect
             variants += [{"hub_build": 1}, {"hub_build": 2}, {"hub_build": 2, "hub_update_div": 0}]
             variants += [{"renumber": 0}, {"renumber": 1}, {"contract_batch": 4096}]
             for var in variants:

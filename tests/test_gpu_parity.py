@@ -251,10 +251,9 @@ def test_full_clustering_rmat16(gpu_ctx, algo):
 @pytest.mark.parametrize("algo,ex_iters", [("louvain", -1), ("leiden+", 0)])
 def test_wide_hub_tables(gpu_ctx, hub_build, algo, ex_iters):
     """Edge weights of 2^20..2^21 on the hub graph: the hub's row weight
-    (about 3e10) does not fit the packed 32-bit table slots, so the hub
-    tables hold separate keys and 64-bit weights; a degree-20,000 hub has a
-    table of two LDS slices.  Every build method (LDS slices, edge items with
-    HBM atomics, a mix of both) gives the oracle's clustering."""
+    (about 3e10) does not fit 32 bits, so its LDS tables hold 64-bit sums; a
+    degree-20,000 hub has four slices.  Every value of the hub_build knob, which
+    is accepted without effect, gives the oracle's clustering."""
     g = hub_graph(seed=11, weights=(1 << 20, 1 << 21))
     vw = g.vertex_weights("WMod")
     print(f"cluster hub30k wide {algo} hub_build={hub_build}", flush=True)

@@ -55,3 +55,31 @@ def test_improve_with_isolated_vertices(gpu_ctx, objective, labels, plus):
             gpu_ctx.set_knob("renumber", 2)
     assert np.array_equal(res[0][0], res[1][0])
     assert res[0][1:] == res[1][1:]
+
+
+@pytest.mark.parametrize("objective", ["Mod", "CPM", "WMod"])
+@pytest.mark.parametrize("groups", [1, 40, 3000])
+def test_constrained_pass_with_isolated_vertices(gpu_ctx, objective, groups):
+    """A constrained pLouvain pass from singletons, where the isolated vertices
+    are left out and the others gather 16-byte records with their constraint: in
+    one group, in a few that mix isolated and other vertices, and with every
+    vertex a group of its own (no move under the constraint, so the strict local
+    move runs, and then the passes without the constraint)."""
+    import torch
+    from pennsylvaniagpugraphclustering_amd import clustering as C
+    g = sparse_graph((1, 20) if objective == "WMod" else None)
+    dg = C.DeviceGraph.from_csr(g, objective)
+    cons = np.random.default_rng(8).permutation(g.n) % groups
+    res = []
+    for knob in (0, 1):
+        gpu_ctx.set_knob("renumber", knob)
+        try:
+            st, vol = C.state_init(dg, objective, 0.2 if objective == "CPM" else 1.0)
+            print(f"constrained {objective} groups={groups} renumber={knob}", flush=True)
+            c = torch.from_numpy(cons.astype(np.int32)).cuda()
+            out = C.louvain_part(dg, st, constrained=True, constraint=c)
+            res.append((out.cpu().numpy(), st.obj, st.uncut, st.label_count))
+        finally:
+            gpu_ctx.set_knob("renumber", 2)
+    assert np.array_equal(res[0][0], res[1][0])
+    assert res[0][1:] == res[1][1:]
