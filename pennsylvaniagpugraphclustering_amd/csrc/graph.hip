@@ -921,8 +921,9 @@ void know_max_weight(Ctx& c, DGraph& g) {
 
 void contract(Ctx& c, const DGraph& g, const i32* vcmap, i64 nc, OwnedGraph& out, const ContractTo* to) {
     DGraph f = g;
-    if (!g.wsmall) know_max_weight(c, f);
-    const ContractWidths w = contract_widths(g.nnz, g.wk == W_UNIT ? 1 : f.wmax, g.wsmall);
+    if (nc <= 1) f.wsmall = true;  // no coarse edges
+    if (!f.wsmall) know_max_weight(c, f);
+    const ContractWidths w = contract_widths(f.nnz, f.wk == W_UNIT ? 1 : f.wmax, f.wsmall);
     if (w.small && !to) {
         contract_t<u32, i32>(c, g, vcmap, nc, true, out, out.w32, nullptr);
         return;

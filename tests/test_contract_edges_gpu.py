@@ -84,3 +84,14 @@ def test_total_weight_at_width_edges(gpu_ctx, bound, over, wide, leaf_groups):
         q, part, info = C.cluster(dg, "louvain", "WMod", 1.0, 1, seed=2)
         oq, op, oi = O.cluster(g.rp, g.col, w, vw, "WMod", 1.0, "louvain", 1, seed=2)
         assert q == oq and np.array_equal(part.cpu().numpy(), op) and info["sweeps"] == oi["sweeps"]
+
+
+@pytest.mark.parametrize("weights", [None, (1, 50), (2 ** 30, 2 ** 31 - 1)])
+def test_one_cluster(gpu_ctx, weights):
+    """Every vertex in one cluster: one empty row, whatever the weights."""
+    from pennsylvaniagpugraphclustering_amd import clustering as C
+    g = stars("spread", weights, 3)
+    dg = C.DeviceGraph.from_csr(g, "Mod" if weights is None else "WMod")
+    print(f"contract into one cluster w={weights}", flush=True)
+    rp, col, w = C.build_coarse_graph(dg, np.zeros(g.n, np.int32), 1)
+    assert rp.cpu().tolist() == [0, 0] and col.numel() == 0 and w.numel() == 0
