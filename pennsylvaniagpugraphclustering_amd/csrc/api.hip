@@ -170,10 +170,10 @@ constexpr int LEIDEN_MAX_STALLS = 8;
 // pays (renum_build) or the call makes several top-level passes (reuse) with
 // it at 2 (the default), never at 0 or with the active-set predictor on, whose
 // features follow the vertex order.
-// Copies that no knob or reuse asks for hold at most RN_MEM of the device's
-// memory: a top level's copy, and those of a run's coarse levels together.  On
-// graphs of billions of edges the finer levels go without, as their hierarchy
-// takes most of the memory.
+// A top level's copy that neither the knob nor reuse asks for holds at most
+// RN_MEM of the device's memory, and so do those of a run's coarse levels
+// together.  On graphs of billions of edges the finer levels go without, as
+// their hierarchy takes most of the memory.
 constexpr double RN_MEM = 1.0 / 16;
 static double renum_bytes(const DGraph& g) { return 32.0 * g.n + (g.wk == W_I64 ? 12.0 : 8.0) * g.nnz; }
 static Renum* top_renum(Ctx& c, MoveScratch& ms, const DGraph& g, Renum& r, bool reuse) {
@@ -196,14 +196,14 @@ static Renum* coarse_renum(Ctx& c, MoveScratch& ms, std::vector<Level>& levels, 
     return l.rn->copied ? l.rn.get() : nullptr;
 }
 
-// local_move at one level; rn (when set) is the top level renumbered
+// local_move at one level; rn (when set) is the level renumbered
 static void move_level(Ctx& c, MoveScratch& ms, LevelPlan& lp, const DGraph& g, i32* part, RefineData& rfd,
                        bool is_initial, bool constrained, i32* cons, bool SA, RunStats& rs, Renum* rn) {
     if (rn) local_move_renum(c, ms, *rn, part, rfd, is_initial, constrained, cons, SA, &rs.mv);
     else local_move(c, ms, lp, g, part, rfd, is_initial, constrained, cons, SA, &rs.mv);
 }
 
-// Contraction of a level; at the top level with rn set, through the
+// Contraction of a level; with rn set, through the
 // renumbered copy (the same coarse graph: coarse ids are the labels, coarse
 // rows are sorted and their weights are integer sums), whose rows gather
 // the map with more locality.  rn->part is the local mover's scratch and

@@ -18,14 +18,14 @@ enum KSlot {
     KS_SCORE_GROUP = 0,  // k_score_groups
     KS_SCORE_TABLE,      // k_score_table / k_score_raw (LDS tables, block arg-max)
     KS_SCORE_HUB,        // hub scoring: k_hub_gather, k_hub_score (k_hub_raw), k_hub_decide
-    KS_AFTERBURNER,      // k_ab_small / k_ab_wave / k_ab_block
+    KS_AFTERBURNER,      // k_ab_lanes, k_ab_block (k_ab_pack)
     KS_MOVES,            // k_mvp_moves + k_move_edges + k_apply_moves
     KS_CONTRACT_AGG,     // k_cagg (LDS merge of coarse rows)
     KS_CONTRACT_BIG,     // k_cbig_insert + k_cbig_extract
     KS_CONTRACT_COPY,    // k_crow_copy
     KS_EVAL,             // k_eval_uncut
     KS_LEIDEN,           // leidenR refinement (all its kernels)
-    KS_ORDER,            // ordering pass (classes + two stable partitions)
+    KS_ORDER,            // ordering pass (two stable partitions by class)
     KS_COUNT
 };
 
@@ -175,13 +175,11 @@ void fill_i32(Ctx& c, i32* p, i64 n, i32 v);
 void fill_i64(Ctx& c, i64* p, i64 n, i64 v);
 void iota_i32(Ctx& c, i32* p, i64 n);
 void copy_dev(Ctx& c, void* dst, const void* src, size_t bytes);  // on c.stream
-// host -> device copy, done when it returns: the bytes go through a pinned
-// coherent staging area and a copy kernel on the stream, so later kernels
-// read them through the same cache path as data written by kernels
-// Host to device in stream order; src may be changed at once.
+// Host to device in stream order; src may be changed at once.  The bytes go
+// through the pinned coherent staging area and a copy kernel on the stream, so
+// later kernels read them through the same cache path as data written by kernels.
 void copy_h2d(Ctx& c, void* dst, const void* src, size_t bytes);
-// Device to host, for several arrays with one wait: count values of each src
-// into dst.
+// Device to host, for several arrays with one wait.
 struct Fetch {
     void* dst;
     const void* src;

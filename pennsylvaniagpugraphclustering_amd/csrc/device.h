@@ -24,16 +24,6 @@ __device__ __forceinline__ i64 wave_sum_i64(i64 v) {
     return v;
 }
 
-__device__ __forceinline__ u64 wave_max_u64(u64 v) {
-    xlane_fence(v);
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        u64 y = __shfl_xor(v, o);
-        v = y > v ? y : v;
-    }
-    return v;
-}
-
 // group reductions over `G` consecutive lanes (G a power of two <= 64)
 template <int G>
 __device__ __forceinline__ i64 group_sum_i64(i64 v) {
@@ -42,6 +32,7 @@ __device__ __forceinline__ i64 group_sum_i64(i64 v) {
     for (int o = G / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, G);
     return v;
 }
+
 // Block reductions through an LDS halving tree (no lane shuffles, so they
 // are safe after loops whose lanes exit at different iterations).  BS is the
 // block size (a power of two); every thread must call them and receives the

@@ -36,7 +36,6 @@ struct OwnedGraph {
     }
 };
 
-// Stable degree bucketing (src/ordering.cpp:131-164).
 // out[r] += the weights of row r's edges whose neighbour passes Pass()(key[r],
 // key[neighbour]); out is zeroed by the caller, sums are exact integers.
 //
@@ -109,6 +108,7 @@ __global__ void __launch_bounds__(256) k_row_sums(const i64* __restrict__ rp, co
 }
 
 __device__ __forceinline__ int order_class(i64 d) { return d < LARGE_CUTOFF ? 0 : (d < MASSIVE_CUTOFF ? 1 : 2); }
+// Stable degree bucketing (src/ordering.cpp:131-164).
 struct Orders {
     Buf<i32> o1, o2;
     i64 off_large = 0, off_large2 = 0, off_mid = 0, off_mid2 = 0;

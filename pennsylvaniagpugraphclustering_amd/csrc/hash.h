@@ -52,9 +52,6 @@ __device__ __forceinline__ void ptable_add_from(u64* tab, u32 mask, i32 key, u64
     }
     atomicAdd((unsigned long long*)&tab[h], (unsigned long long)w);
 }
-__device__ __forceinline__ void ptable_add(u64* tab, u32 mask, i32 key, u64 w) {
-    ptable_add_from(tab, mask, key, w, slot_hash(key, mask));
-}
 
 // Work-item pre-aggregation: a block merges the (key, weight) pairs of one
 // work item (at most LSLOTS / 2 pairs) in an LDS table, then adds each

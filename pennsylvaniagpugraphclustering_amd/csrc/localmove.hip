@@ -97,8 +97,9 @@ __host__ __device__ __forceinline__ int score_class(i64 d) {
 // small levels, bound by launches (direct_sweep)
 constexpr i64 DIRECT_MAX = (i64)1 << 18, DIRECT_NNZ = (i64)1 << 22;
 // Level of at most this many rows of degree 65 to 2048: one launch for their
-// five classes (the chip holds 5 of its 256-thread blocks per CU, 1,280 at once; a
-// class of its own takes 5 to 9 us of a launch's latency however few its rows).
+// five classes (its 256-thread blocks take 33 KB of LDS each with 32-bit sums, so a
+// CU holds 4 of them and the chip 1,024 at once; a class of its own takes 5 to 9
+// us of a launch's latency however few its rows).
 // At 2,048 rows, and only without longer ones, a CPM run of 30,011 vertices took 2.94
 // ms, 2.70 now, weighted pLeiden+ on R-MAT scale 17 28.7, 27.3 now; at the 12,000 to
 // 200,000 rows of R-MAT scale 22's levels the classes' own widths are better.
@@ -517,10 +518,6 @@ __device__ __forceinline__ T group_reduce(T v, Op op) {
 template <int G, class T>
 __device__ __forceinline__ T group_max(T v) {
     return group_reduce<G>(v, [](T a, T b) { return a > b ? a : b; });
-}
-template <int G, class T>
-__device__ __forceinline__ T group_add(T v) {
-    return group_reduce<G>(v, [](T a, T b) { return a + b; });
 }
 // over the block; every thread gets the result
 template <int BS, class T, class Op>
@@ -1278,11 +1275,11 @@ static void score_all(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, co
     const ScoreArgs<LT> a{L, part, vol, RecView{s.rec.p, cons ? s.rec16.p : nullptr}, cons, lam, ratio, out};
     PGGC_WDISPATCH(g, {
         using WT = decltype(W);
-        using A64 = typename std::conditional<IsUnit<WT>::v, u32, i64>::type;  // sums of unit rows fit 32 bits
+        constexpr bool unit = IsUnit<WT>::v;  // (agg32 and hub32 hold)
         i64 m;
         int tk = c.kt_begin(KS_SCORE_GROUP);
         if (lp.agg32) launch_groups<u32>(c, g, W, a, st, raw);
-        else launch_groups<A64>(c, g, W, a, st, raw);
+        else if constexpr (!unit) launch_groups<i64>(c, g, W, a, st, raw);
         c.kt_end(tk, 0.0);
         if (tk >= 0) acct_add(c, c.kt_counter(tk), acct.p);
         tk = c.kt_begin(KS_SCORE_TABLE);
@@ -1295,8 +1292,8 @@ static void score_all(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, co
                                                                        part, vol, a.rv, cons, lam, ratio, out);
         } else if (lp.agg32) {
             launch_tables<u32>(c, lp, g, W, a);
-        } else {
-            launch_tables<A64>(c, lp, g, W, a);
+        } else if constexpr (!unit) {
+            launch_tables<i64>(c, lp, g, W, a);
         }
         c.kt_end(tk, 0.0);
         if (tk >= 0) acct_add(c, c.kt_counter(tk), acct.p + 1);
@@ -1304,10 +1301,13 @@ static void score_all(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, co
             const HubView hv{L + lp.hub0, lp.hub_pre, m, ceil_div(m, NXCD), lp.hub_blocks};
             if (!raw) s.ensure_hubs(c, lp);
             tk = c.kt_begin(KS_SCORE_HUB);
-            if (raw && lp.hub32) PGGC_HUB_RAW(HUB_SLOTS32);
-            else if (raw) PGGC_HUB_RAW(HUB_SLOTS64);
-            else if (lp.hub32) PGGC_HUB(HUB_SLOTS32, u32);
-            else PGGC_HUB(HUB_SLOTS64, A64);
+            if (lp.hub32) {
+                if (raw) PGGC_HUB_RAW(HUB_SLOTS32);
+                else PGGC_HUB(HUB_SLOTS32, u32);
+            } else if constexpr (!unit) {
+                if (raw) PGGC_HUB_RAW(HUB_SLOTS64);
+                else PGGC_HUB(HUB_SLOTS64, i64);
+            }
             k_hub_decide<<<grid_items(m, 256), 256, 0, c.stream>>>(hv.hubs, m, part, g.vw, vol, lam, ratio, lp.hub_pv,
                                                                        lp.hub_best, out);
             c.kt_end(tk, 0.0);

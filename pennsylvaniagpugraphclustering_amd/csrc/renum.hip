@@ -1,4 +1,4 @@
-// Internal degree order of the top level for the local mover.
+// Internal degree order of a level for its local mover.
 #include "renum.h"
 
 #include "device.h"
