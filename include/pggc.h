@@ -170,8 +170,10 @@ int pggc_ctx_set_sweep_trace(pggc_ctx* ctx, pggc_sweep_fn fn, void* user);
  *   PGGC_KNOB_CONTRACT_BATCH: the contraction merges its largest coarse rows
  *     in HBM hash tables and sorts them in batches of rows holding at most
  *     this many table slots (default 2^30) and a quarter as many sort
- *     entries, which bounds its memory on graphs of billions of edges; the
- *     coarse graph is the same for every value >= 1. */
+ *     entries, which bounds its memory on graphs of billions of edges.  The
+ *     scoring of vertices of degree above 8192 takes batches of at most as
+ *     many edges (and at most 1/64 of the device's memory).  Results are the
+ *     same for every value >= 1. */
 #define PGGC_KNOB_HUB_UPDATE_DIV 0
 #define PGGC_KNOB_GNN_MAX_SWEEPS 1
 #define PGGC_KNOB_TABLE_THREADS 2

@@ -49,11 +49,18 @@ struct LevelPlan {
     // the smaller classes, the others (from list entry hub0 on) in chunks of
     // their edges and slices of their clusters' hash range: hub_pre holds the
     // prefixes of their edges, chunks and bucket starts and of the slices of
-    // groups of 8 hubs (k_hub_sizes; hub_edges, hub_chunks, hub_starts and
-    // hub_blocks in all).  hub_pv and hub_best are zero between sweeps.
+    // groups of 8 hubs (k_hub_sizes).  hub_pv and hub_best are zero between
+    // sweeps.  They are scored in batches of whole groups, [h0, h1) with the
+    // batch's sizes, normally one.
     Buf<i64> hub_pre, hub_pv;
     Buf<u64> hub_best;
-    i64 hub_blocks = 0, hub_edges = 0, hub_chunks = 0, hub_starts = 0, nhalf = 0;
+    struct HubBatch {
+        i64 h0, h1, edges, chunks, starts, blocks;
+    };
+    std::vector<HubBatch> hub_batches;
+    i64 hub_blocks = 0;     // of all hubs
+    size_t hub_words = 0;   // 8-byte words of scratch for the largest batch
+    i64 nhalf = 0;
     bool hub32 = false;   // their row sums fit 32 bits
     i64 nlds = 0, hub0 = 0, nhub = 0;
     bool agg32 = false;  // sums of rows of degree <= 8192 fit 32 bits
@@ -80,18 +87,15 @@ struct MoveScratch {
     Buf<u64> mvp;  // per vertex: cluster | moved << 31, and the cluster after this sweep's moves
     Buf<u64> rec;     // per vertex: cluster and its volume as fp32 (scoring)
     Buf<uint4> rec16; // the same with the cluster's constraint value, when there is one
-    // the large hubs' gathered entries, while a local move runs: cluster and
-    // volume, weight (32 or 64 bits), and the bucket starts of every chunk
-    Buf<u64> hub_kv;
-    Buf<u32> hub_kw;
-    Buf<unsigned short> hub_st;
+    // the gathered entries of a batch of large hubs, while a local move runs:
+    // cluster and volume, then the weights (32 or 64 bits), then the bucket
+    // starts of every chunk
+    Buf<u64> hub_buf;
     Buf<u64> sqpart;  // partial sums of k_finish
     Buf<i32> part, dest, cand, moves, flag, tmp, tmp2;
     Buf<float> gain;
     Buf<i64> prio, scal;
     void ensure(Ctx& c, i64 n);
-    void ensure_hubs(Ctx& c, const LevelPlan& lp);
-    void drop_hubs();
 };
 
 void plan_level(Ctx& c, const DGraph& g, LevelPlan& p);

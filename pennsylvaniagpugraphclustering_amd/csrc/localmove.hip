@@ -15,6 +15,7 @@
 #include <chrono>
 #include <type_traits>
 
+#include "batching.h"
 #include "device.h"
 #include "gnn.h"
 #include "hash.h"
@@ -65,28 +66,6 @@ void MoveScratch::ensure(Ctx& c, i64 n) {
     prio = Buf<i64>(c, cap + 1);
     scal = Buf<i64>(c, SC_COUNT);
     sqpart = Buf<u64>(c, 2 * FIN_BLOCKS);
-}
-
-// the large hubs' gathered entries
-void MoveScratch::ensure_hubs(Ctx& c, const LevelPlan& lp) {
-    if (hub_kv.n < (size_t)lp.hub_edges) {
-        hub_kv.reset();
-        hub_kv = Buf<u64>(c, lp.hub_edges);
-    }
-    const size_t words = lp.hub32 ? lp.hub_edges : 2 * lp.hub_edges;
-    if (hub_kw.n < words) {
-        hub_kw.reset();
-        hub_kw = Buf<u32>(c, words);
-    }
-    if (hub_st.n < (size_t)lp.hub_starts) {
-        hub_st.reset();
-        hub_st = Buf<unsigned short>(c, lp.hub_starts);
-    }
-}
-void MoveScratch::drop_hubs() {
-    hub_kv.reset();
-    hub_kw.reset();
-    hub_st.reset();
 }
 
 // ------------------------------------------------------------- level plan
@@ -227,27 +206,40 @@ __global__ void k_hub_sizes(const i64* rp, const i32* hubs, i64 m, int slots, i6
         sz[3 * m + x] = hub_slices(rp[i + 1] - rp[i], slots);
     }
 }
-// The scanned sizes of a level's m hubs: rows of hub_pre, each relative to its
+// A batch of m hubs: its rows of the scanned sizes, each relative to the batch's
 // first entry.
 struct HubView {
     const i32* hubs;
-    const i64* pre;
+    const i64 *edges, *chunks, *starts, *groups;
     i64 m, ng, nblk;
-    __device__ __forceinline__ i64 edge0(i64 h) const { return pre[h]; }
-    __device__ __forceinline__ i64 chunk0(i64 h) const { return pre[m + h] - pre[m]; }
-    __device__ __forceinline__ i64 start0(i64 h) const { return pre[2 * m + h] - pre[2 * m]; }
+    __device__ __forceinline__ i64 edge0(i64 h) const { return edges[h] - edges[0]; }
+    __device__ __forceinline__ i64 chunk0(i64 h) const { return chunks[h] - chunks[0]; }
+    __device__ __forceinline__ i64 start0(i64 h) const { return starts[h] - starts[0]; }
     // block -> hub and slice; false for padding.  The largest hubs come first.
     __device__ __forceinline__ bool slice(i64 bid, i64& h, i64& sl) const {
         if (bid >= nblk) return false;
-        const i64* g0 = pre + 3 * m;
         const i64 b = nblk - 1 - bid;
-        const i64 q = b / NXCD + g0[0];
-        const i64 g = upper_row(g0, 0, ng, q);
+        const i64 q = b / NXCD + groups[0];
+        const i64 g = upper_row(groups, 0, ng, q);
         h = g * NXCD + b % NXCD;
-        sl = q - g0[g];
+        sl = q - groups[g];
         return h < m;
     }
 };
+// the hubs [h0, h1) of a level's, h0 a multiple of NXCD
+static HubView hub_view(const LevelPlan& p, i64 h0, i64 h1, i64 blocks) {
+    const i64* pre = p.hub_pre.p + h0;
+    return HubView{p.sc_list.p + p.hub0 + h0, pre, pre + p.nhub, pre + 2 * p.nhub,
+                   p.hub_pre.p + 3 * p.nhub + h0 / NXCD, h1 - h0, ceil_div(h1 - h0, NXCD), blocks};
+}
+// Batches of hubs hold at most this share of the device's memory (a larger group
+// of hubs is a batch of its own): scratch for all hub edges at once, up to 20 GB
+// on R-MAT scale 27, made the allocator give blocks back and take them again, and
+// a pLeiden+ pass took 21.4 s, with batches 18.2.
+constexpr double HUB_MEM = 1.0 / 64;
+static size_t hub_scratch(const LevelPlan::HubBatch& b, bool sum32) {
+    return (size_t)(b.edges + (sum32 ? ceil_div(b.edges, 2) : b.edges) + ceil_div(b.starts, 4));
+}
 
 __global__ void k_hub_deg_keys(const i64* rp, const i32* list, i64 m, u64* keys, i32* vals) {
     const i64 x = thread_item();
@@ -344,10 +336,25 @@ void plan_level(Ctx& c, const DGraph& g, LevelPlan& p) {
         Fetch f[4];
         for (int k = 0; k < 4; k++) f[k] = Fetch{&e[k], p.hub_pre.p + at[k], sizeof(i64)};
         copy_d2h(c, f, 4);
-        p.hub_edges = e[0];
-        p.hub_chunks = e[1] - e[0];
-        p.hub_starts = e[2] - e[1];
         p.hub_blocks = (e[3] - e[2]) * NXCD;
+        p.hub_batches.assign(1, LevelPlan::HubBatch{0, m, e[0], e[1] - e[0], e[2] - e[1], p.hub_blocks});
+        const i64 cap = std::min<i64>(c.contract_batch, (i64)(HUB_MEM * (double)c.mem_total) / (p.hub32 ? 12 : 16));
+        if (e[0] > cap) {
+            std::vector<i64> pre, ge(ng + 1);
+            const Fetch all = fetch(pre, p.hub_pre.p, (size_t)np + 1);
+            copy_d2h(c, &all, 1);
+            for (i64 k = 0; k <= ng; k++) ge[k] = pre[std::min(k * NXCD, m)];
+            const std::vector<i64> cuts = batch_cuts(ge, cap, nullptr);
+            p.hub_batches.clear();
+            for (size_t q = 0; q + 1 < cuts.size(); q++) {
+                const i64 h0 = cuts[q] * NXCD, h1 = std::min(cuts[q + 1] * NXCD, m);
+                p.hub_batches.push_back({h0, h1, pre[h1] - pre[h0], pre[m + h1] - pre[m + h0],
+                                         pre[2 * m + h1] - pre[2 * m + h0],
+                                         (pre[3 * m + cuts[q + 1]] - pre[3 * m + cuts[q]]) * NXCD});
+            }
+        }
+        p.hub_words = 0;
+        for (const LevelPlan::HubBatch& b : p.hub_batches) p.hub_words = std::max(p.hub_words, hub_scratch(b, p.hub32));
     }
 }
 
@@ -869,7 +876,7 @@ __global__ void __launch_bounds__(HUB_GT) k_hub_gather(const i64* __restrict__ r
     __shared__ u32 hist[HUB_BUCKETS];
     const i64 b = block_id();
     if (b >= hv.chunk0(hv.m)) return;
-    const i64 h = upper_row(hv.pre + hv.m, 0, hv.m, b + hv.pre[hv.m]);
+    const i64 h = upper_row(hv.chunks, 0, hv.m, b + hv.chunks[0]);
     const i32 i = hv.hubs[h];
     if (dest[i] == NO_MOVE) return;
     const int t = threadIdx.x;
@@ -1265,13 +1272,16 @@ static void score_all(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, co
     k_hub_raw<SL><<<grid_blocks(lp.hub_blocks), 256, 0, c.stream>>>(g.rp, g.col, W, g.vw, hv, part, vol, a.rv, cons, \
                                                                     lam, ratio, dest, lp.hub_best)
 #define PGGC_HUB(SL, AT)                                                                                             \
-    do {                                                                                                             \
-        AT* kw = (AT*)(void*)s.hub_kw.p;                                                                             \
-        k_hub_gather<SL, AT><<<grid_blocks(lp.hub_chunks), HUB_GT, 0, c.stream>>>(                                   \
-            g.rp, g.col, W, hv, part, a.rv, cons, dest, s.hub_kv, kw, s.hub_st, lp.hub_pv);                          \
-        k_hub_score<SL, 1024, AT><<<grid_blocks(lp.hub_blocks), 1024, 0, c.stream>>>(                                \
-            g.rp, g.vw, hv, part, vol, lam, ratio, dest, s.hub_kv, kw, s.hub_st, lp.hub_pv, lp.hub_best);            \
-    } while (0)
+    for (const LevelPlan::HubBatch& hb : lp.hub_batches) {                                                           \
+        const HubView bv = hub_view(lp, hb.h0, hb.h1, hb.blocks);                                                    \
+        u64* kv = s.hub_buf;                                                                                         \
+        AT* kw = (AT*)(void*)(kv + hb.edges);                                                                        \
+        unsigned short* hs = (unsigned short*)(void*)(kv + hub_scratch(hb, sizeof(AT) == 4) - ceil_div(hb.starts, 4)); \
+        k_hub_gather<SL, AT><<<grid_blocks(hb.chunks), HUB_GT, 0, c.stream>>>(                                       \
+            g.rp, g.col, W, bv, part, a.rv, cons, dest, kv, kw, hs, lp.hub_pv.p + hb.h0);                            \
+        k_hub_score<SL, 1024, AT><<<grid_blocks(hb.blocks), 1024, 0, c.stream>>>(                                    \
+            g.rp, g.vw, bv, part, vol, lam, ratio, dest, kv, kw, hs, lp.hub_pv.p + hb.h0, lp.hub_best.p + hb.h0);    \
+    }
     const ScoreArgs<LT> a{L, part, vol, RecView{s.rec.p, cons ? s.rec16.p : nullptr}, cons, lam, ratio, out};
     PGGC_WDISPATCH(g, {
         using WT = decltype(W);
@@ -1298,15 +1308,18 @@ static void score_all(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, co
         c.kt_end(tk, 0.0);
         if (tk >= 0) acct_add(c, c.kt_counter(tk), acct.p + 1);
         if ((m = lp.nhub) > 0) {
-            const HubView hv{L + lp.hub0, lp.hub_pre, m, ceil_div(m, NXCD), lp.hub_blocks};
-            if (!raw) s.ensure_hubs(c, lp);
+            const HubView hv = hub_view(lp, 0, m, lp.hub_blocks);
+            if (!raw && s.hub_buf.n < lp.hub_words) {
+                s.hub_buf.reset();
+                s.hub_buf = Buf<u64>(c, lp.hub_words);
+            }
             tk = c.kt_begin(KS_SCORE_HUB);
             if (lp.hub32) {
                 if (raw) PGGC_HUB_RAW(HUB_SLOTS32);
-                else PGGC_HUB(HUB_SLOTS32, u32);
+                else PGGC_HUB(HUB_SLOTS32, u32)
             } else if constexpr (!unit) {
                 if (raw) PGGC_HUB_RAW(HUB_SLOTS64);
-                else PGGC_HUB(HUB_SLOTS64, i64);
+                else PGGC_HUB(HUB_SLOTS64, i64)
             }
             k_hub_decide<<<grid_items(m, 256), 256, 0, c.stream>>>(hv.hubs, m, part, g.vw, vol, lam, ratio, lp.hub_pv,
                                                                        lp.hub_best, out);
@@ -2380,7 +2393,7 @@ static void local_move_t(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g,
         }
     }
     relabel(c, s, nfull, best_part, best);
-    s.drop_hubs();
+    s.hub_buf.reset();
 }
 
 // afterburner_filter_strict (src/local_mover.cpp:131-213): exact sequential
@@ -2494,7 +2507,7 @@ void local_move_strict(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, i
         trc.end(k, tr);
     }
     relabel(c, s, n, best_part, best);
-    s.drop_hubs();
+    s.hub_buf.reset();
 }
 
 i64 sweep_once(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, const i32* part, const i64* vol, i64 L,
@@ -2522,7 +2535,7 @@ i64 sweep_once(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, const i32
     copy_dev(c, dest, s.dest, n * sizeof(i32));
     copy_dev(c, gain, s.gain, n * sizeof(float));
     c.sync();
-    s.drop_hubs();
+    s.hub_buf.reset();
     return km;
 }
 
@@ -2930,7 +2943,7 @@ void local_move_batch(Ctx& c, MoveScratch& s, LevelPlan& lp, const DGraph& g, co
         }
     }
     relabel_batch(c, s, bl, best_part, best, active);
-    s.drop_hubs();
+    s.hub_buf.reset();
 }
 
 }  // namespace pggc

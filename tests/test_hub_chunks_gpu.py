@@ -1,7 +1,7 @@
 """Hubs scored in chunks of 4,096 edges and slices of their clusters' hash
 range: one sweep at the edges of the chunks and of the slices, with all their
 neighbours in two clusters, in a few and in one each, with and without a
-constraint, 32-bit and 64-bit sums, and hubs of more slices than a chunk has
+constraint, 32-bit and 64-bit sums, in one batch and in several, and hubs of more slices than a chunk has
 buckets, bit-identical to the oracle; and scoring time that grows with the
 degree, not with its square."""
 import numpy as np
@@ -37,7 +37,8 @@ DEGREES = [8193, 10923, 12287, 12288, 12289, 16383, 16384, 16385, 20481, 65536, 
 @pytest.mark.parametrize("weights", [None, (1, 30), (1 << 29, (1 << 30) - 1)])
 @pytest.mark.parametrize("labels", [2, 60, 0])
 @pytest.mark.parametrize("constrained", [False, True])
-def test_hubs_at_chunk_edges(gpu_ctx, weights, labels, constrained):
+@pytest.mark.parametrize("batched", [False, True])
+def test_hubs_at_chunk_edges(gpu_ctx, weights, labels, constrained, batched):
     rng = np.random.default_rng(5)
     m = len(DEGREES)
     n = 110000
@@ -52,8 +53,13 @@ def test_hubs_at_chunk_edges(gpu_ctx, weights, labels, constrained):
     if labels:
         part[:L] = np.arange(L)
     cons = rng.integers(0, 2, L).astype(np.int32) if constrained else None
-    print(f"hub sweep labels={labels} weights={weights} constrained={constrained}", flush=True)
-    check_sweep(g, part, L, cons)
+    print(f"hub sweep labels={labels} weights={weights} constrained={constrained} batched={batched}", flush=True)
+    try:
+        if batched:  # every 8 hubs a batch of their own
+            gpu_ctx.set_knob("contract_batch", 1)
+        check_sweep(g, part, L, cons)
+    finally:
+        gpu_ctx.set_knob("contract_batch", 1 << 30)
 
 
 @pytest.mark.parametrize("weights,degree", [(None, 8500000), ((1 << 29, (1 << 30) - 1), 5700000)])
