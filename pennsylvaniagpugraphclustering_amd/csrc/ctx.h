@@ -94,7 +94,7 @@ struct Ctx {
     // always, 2 where it pays
     int renumber = 2;
     // big-row contraction batches: table slots per batch (sort entries per
-    // batch: a quarter of it)
+    // batch: a quarter of it); edges per batch of large hubs
     i64 contract_batch = (i64)1 << 30;
     // the active-set predictor runs on at most this many sweeps of a
     // local-move call (0: on every eligible sweep)
